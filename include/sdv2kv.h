@@ -210,9 +210,11 @@ typedef struct sdv2_attn_params {
   const int64_t* rope_start_frame; /* host [B]                                     */
   /* sdv2_dtype of q, both caches and out.  SDV2_BF16 (0): the matrix-core
    * kernel.  SDV2_F32: what the reference's fallback operator computes on fp32
-   * tensors (causal_model.py:111-157) - products, sums and softmax in fp32,
-   * one key range (num_splits, workspace and rope_freqs must be unset: fp32
-   * queries arrive rotated), strides in multiples of 4 elements.             */
+   * tensors (causal_model.py:111-157) - products, sums and softmax in fp32
+   * (num_splits is ignored and rope_freqs must be unset: fp32 queries arrive
+   * rotated), strides in multiples of 4 elements.  With a workspace of
+   * sdv2_swa_attn_f32_workspace_bytes() the key range is split to fill the
+   * chip; without one (NULL, or too small) it is walked whole.               */
   int32_t dtype;
   /* Optional q RMSNorm inside the call (needs rope_freqs and SDV2_BF16): q is
    * the raw q projection, q_norm_weight the norm's weight (device, bf16,
@@ -229,6 +231,9 @@ int sdv2_swa_attn_default_splits(int32_t rows, int32_t q_tokens, int32_t heads, 
 /* bytes of workspace needed for `num_splits` (0 = default); 0 when unsplit */
 size_t sdv2_swa_attn_workspace_bytes(int32_t rows, int32_t q_tokens, int32_t heads,
                                      int32_t max_seq_len, int32_t num_splits);
+/* the same for SDV2_F32 tensors, whose kernel picks its own splits; one workspace
+ * may serve both kinds of call */
+size_t sdv2_swa_attn_f32_workspace_bytes(int32_t rows, int32_t q_tokens, int32_t heads, int32_t max_seq_len);
 int sdv2_swa_attn_fwd(const sdv2_attn_params* p);
 
 /* ------------------------------------------------------------------------

@@ -38,6 +38,7 @@ EXPORTED_SYMBOLS = (
     "sdv2_kv_append_rope",
     "sdv2_swa_attn_default_splits",
     "sdv2_swa_attn_workspace_bytes",
+    "sdv2_swa_attn_f32_workspace_bytes",
     "sdv2_swa_attn_fwd",
     "sdv2_swa_attn_fwd_static",
     "sdv2_sink_similarity_workspace_bytes",
@@ -195,6 +196,8 @@ def lib() -> C.CDLL:
     handle.sdv2_swa_attn_default_splits.argtypes = [C.c_int32] * 4
     handle.sdv2_swa_attn_workspace_bytes.restype = C.c_size_t
     handle.sdv2_swa_attn_workspace_bytes.argtypes = [C.c_int32] * 5
+    handle.sdv2_swa_attn_f32_workspace_bytes.restype = C.c_size_t
+    handle.sdv2_swa_attn_f32_workspace_bytes.argtypes = [C.c_int32] * 4
     handle.sdv2_swa_attn_fwd.restype = C.c_int
     handle.sdv2_swa_attn_fwd.argtypes = [C.POINTER(AttnParams)]
     handle.sdv2_swa_attn_fwd_static.restype = C.c_int

@@ -1278,7 +1278,7 @@ extern "C" int sdv2_swa_attn_fwd_static(const sdv2_attn_params* p) {
   if (!p) return SDV2_ERR_INVALID_ARG;
   if (p->rows <= 0 || p->q_tokens <= 0 || p->heads <= 0 || p->max_seq_len < 0)
     return attn_fwd(p, nullptr, 0);                       // nothing to split: same answers as the plain entry point
-  if (p->dtype == SDV2_F32) return attn_fwd(p, nullptr, 0);   // fp32 walks one key range: no scratch, whatever num_splits says
+  if (p->dtype == SDV2_F32) return attn_fwd(p, nullptr, 0);   // fp32 without scratch walks one key range, whatever num_splits says
   const int splits = p->num_splits > 0 ? p->num_splits
                                        : sdv2_swa_attn_default_splits(p->rows, p->q_tokens, p->heads, p->max_seq_len);
   SplitPlan plan;
@@ -1295,7 +1295,7 @@ extern "C" int sdv2_swa_attn_fwd_static(const sdv2_attn_params* p) {
 namespace {
 
 int attn_fwd(const sdv2_attn_params* p, void* workspace, size_t workspace_bytes) {
-  if (p->dtype == SDV2_F32) return sdv2::attn_fwd_f32(p);        // fp32 arithmetic, one key range: no workspace
+  if (p->dtype == SDV2_F32) return sdv2::attn_fwd_f32(p, workspace, workspace_bytes);        // fp32 arithmetic
   if (p->dtype != SDV2_BF16) return SDV2_ERR_UNSUPPORTED;
   if (p->head_dim != kD) return SDV2_ERR_UNSUPPORTED;
   if (p->rows < 0 || p->q_tokens < 0 || p->heads <= 0 || p->max_seq_len < 0) return SDV2_ERR_INVALID_ARG;

@@ -378,8 +378,8 @@ def swa_attention(
     q [B,S,H,128] bf16; k_cache/v_cache [B,L,H,128] bf16 views with any row /
     token / head strides; seq_lens int32 [B] on the device (None = L).  All
     three may be fp32 instead (the reference's CPU-runnable configuration): the
-    result is then computed in fp32 throughout, by a plain kernel that walks the
-    whole key range (q rotated beforehand, ``num_splits`` ignored).
+    result is then computed in fp32 throughout, on the fp32 matrix instructions
+    (q rotated beforehand, ``num_splits`` ignored).
     With ``mask_block_tokens`` = b in (0, S) and ``chunk_key_start`` (int32 [B]
     on the device, or host ints: where each row's own chunk sits in the cache)
     query token t does not see the chunk's later blocks
@@ -391,7 +391,7 @@ def swa_attention(
                            % (q.dtype, k_cache.dtype, v_cache.dtype))
     fp32 = q.dtype == torch.float32
     if fp32 and (rope is not None or static_scratch):
-        raise RuntimeError("fp32 attention takes rotated queries and one key range (no rope=, no static_scratch=)")
+        raise RuntimeError("fp32 attention takes rotated queries (no rope=) and no static_scratch=")
     rows, q_tokens, heads, _ = q.shape
     if k_cache.shape[0] != rows or k_cache.shape[2] != heads or v_cache.shape != k_cache.shape:
         raise RuntimeError(f"cache view {tuple(k_cache.shape)} / {tuple(v_cache.shape)} does not match q {tuple(q.shape)}")
@@ -405,10 +405,11 @@ def swa_attention(
     lib = _capi.lib()
     max_seq_len = k_cache.shape[1]
     if fp32:
-        num_splits = 1          # the fp32 kernel walks the whole key range
-    elif num_splits <= 0:
-        num_splits = lib.sdv2_swa_attn_default_splits(rows, q_tokens, heads, max_seq_len)
-    need = 0 if static_scratch else lib.sdv2_swa_attn_workspace_bytes(rows, q_tokens, heads, max_seq_len, num_splits)
+        need = lib.sdv2_swa_attn_f32_workspace_bytes(rows, q_tokens, heads, max_seq_len)    # (it picks its own splits)
+    else:
+        if num_splits <= 0:
+            num_splits = lib.sdv2_swa_attn_default_splits(rows, q_tokens, heads, max_seq_len)
+        need = 0 if static_scratch else lib.sdv2_swa_attn_workspace_bytes(rows, q_tokens, heads, max_seq_len, num_splits)
     if workspace is not None and not getattr(workspace, "_sdv2_workspace", False):
         raise RuntimeError("workspace= takes a buffer made by ops.new_workspace() (zero-filled ticket words)")
     if need and (workspace is None or workspace.numel() * workspace.element_size() < need):

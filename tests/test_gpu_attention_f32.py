@@ -108,3 +108,41 @@ def test_fp32_and_bf16_do_not_mix(gpu_device):
     kf = torch.zeros(1, 8, 1, 128, device=gpu_device)
     with pytest.raises(RuntimeError):
         ops.swa_attention(q, kf, kf, rope=(table, (2, 2), [0]))
+
+
+@pytest.mark.parametrize(
+    "rows,S,H,L,seq",
+    [
+        (1, 128, 1, 1024, None),            # whole query and key tiles, split key range
+        (1, 129, 2, 1023, None),            # one query row in the second tile, one key short of a tile
+        (2, 33, 1, 4097, [4097, 1]),        # most key ranges, all but the first of row 1's empty
+        (1, 1, 1, 4000, None),
+        (1, 160, 13, 321, None),            # pairs that do not divide over the XCDs
+    ],
+)
+def test_fp32_split_key_ranges(gpu_device, rows, S, H, L, seq):
+    """A call that is split over key ranges, twice on one workspace, against the oracle and against
+    the same call walked whole (no workspace)."""
+    import ctypes as C
+
+    from streamdiffusionv2_amd import _capi, ops
+
+    torch.manual_seed(77)
+    q, k, v = torch.randn(rows, S, H, 128), torch.randn(rows, L, H, 128), torch.randn(rows, L, H, 128)
+    lens = seq if seq is not None else [L] * rows
+    want = oracle.attention_fp32_reference(q, k, v, lens)
+    qd, kd, vd = q.to(gpu_device), _to_device(k, gpu_device, True), _to_device(v, gpu_device, True)
+    sl = torch.tensor(lens, dtype=torch.int32, device=gpu_device)
+    assert _capi.lib().sdv2_swa_attn_f32_workspace_bytes(rows, S, H, L) > 0
+    first, again = ops.swa_attention(qd, kd, vd, sl), ops.swa_attention(qd, kd, vd, sl)
+    p = _capi.AttnParams()
+    whole = torch.empty_like(qd)
+    p.q, p.k_cache, p.v_cache, p.out, p.seq_lens = (t.data_ptr() for t in (qd, kd, vd, whole, sl))
+    p.q_stride, p.k_stride, p.v_stride, p.out_stride = (ops._stride3(t, "t") for t in (qd, kd, vd, whole))
+    p.rows, p.q_tokens, p.heads, p.head_dim, p.max_seq_len, p.dtype = rows, S, H, 128, L, _capi.DTYPE_F32
+    p.stream = torch.cuda.current_stream().cuda_stream
+    _capi.check(_capi.lib().sdv2_swa_attn_fwd(C.byref(p)), "sdv2_swa_attn_fwd")
+    torch.cuda.synchronize()
+    assert torch.equal(first, again)
+    _check(first.cpu(), want)
+    _check(whole.cpu(), want)
