@@ -35,7 +35,7 @@ PEAK_HBM_GBS = 8000.0       # MI355X HBM3E
 # only used for the kernels it was taken on: same key-range split count, same
 # kernel sources (hash below); otherwise `traffic` is null and stderr says why.
 TRAFFIC_JSON = os.path.join(ROOT, "profiles", "hbm_traffic.json")
-KERNEL_SOURCES = ("swa_attn_fwd.hip", "kv_append_rope.hip", "rope_device.h", "sdv2kv_internal.h")
+KERNEL_SOURCES = ("swa_attn_fwd.hip", "swa_attn_fwd_m16.hip", "attn_device.h", "kv_append_rope.hip", "rope_device.h", "sdv2kv_internal.h")
 
 
 def kernel_source_hash() -> str:
@@ -81,8 +81,9 @@ def record_traffic(args, w):
             raise SystemExit(f"no counter_collection.csv under {args.record_traffic}/{sub}")
         total, count = collections.defaultdict(float), collections.Counter()
         for row in csv.DictReader(open(files[0])):
-            for short in ("swa_attn_fwd_kernel", "kv_append_rope_kernel", "copy16_kernel"):
-                if short in row["Kernel_Name"]:
+            for short, names in (("swa_attn_fwd_kernel", ("swa_attn_fwd_kernel", "swa_attn_fwd_m16_kernel")),
+                                 ("kv_append_rope_kernel", ("kv_append_rope_kernel",)), ("copy16_kernel", ("copy16_kernel",))):
+                if any(n in row["Kernel_Name"] for n in names):
                     total[short] += float(row["Counter_Value"])
                     count[short] += 1
         return {k: total[k] / count[k] for k in total}

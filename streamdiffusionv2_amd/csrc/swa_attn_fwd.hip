@@ -56,23 +56,14 @@
 #include "sdv2kv_profile.h"
 #include "sdv2kv_internal.h"
 #include "rope_device.h"
+#include "attn_device.h"
 
 namespace {
 
-typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
-typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2;
-typedef __attribute__((ext_vector_type(4))) short s16x4;
-typedef __attribute__((ext_vector_type(8))) short s16x8;
-typedef __attribute__((ext_vector_type(16))) float f32x16;
-typedef __attribute__((ext_vector_type(2))) float f32x2;
-typedef __attribute__((ext_vector_type(4))) uint32_t u32x4;
-typedef __attribute__((ext_vector_type(2))) uint32_t u32x2;
-typedef __attribute__((ext_vector_type(2))) _Float16 f16x2;
-typedef __attribute__((ext_vector_type(8))) _Float16 f16x8;
-typedef __attribute__((address_space(3))) char lds_char;
-typedef __attribute__((address_space(3))) int lds_int;
+using namespace sdv2::attn;
 
-constexpr int kD = SDV2_HEAD_DIM;           // 128
+typedef __attribute__((ext_vector_type(4))) float f32x4;
+
 constexpr int kWaves = 8;                   // two waves per SIMD, one 32-row query block each
 constexpr int kThreads = kWaves * 64;
 // The global->LDS transfers of a tile are issued by the first wave of every
@@ -80,14 +71,9 @@ constexpr int kThreads = kWaves * 64;
 // eight issuing, both waves of a SIMD are held at the same moment right after
 // the barrier, with four the other one keeps the matrix pipe fed (measured
 // 0.5-1.5 % faster; two or one issuing waves fall far behind the rest).
-constexpr int kIssuers = 4;
-constexpr int kPieces = 16 / kIssuers;      // global->LDS instructions per issuing wave and matrix tile
-constexpr int kQBlock = 32;                 // query rows per wave
+static_assert(kIssuers == 4, "the first wave of every SIMD");
 constexpr int kQTile = kWaves * kQBlock;    // 256
-constexpr int kKTile = 64;
-constexpr int kTileBytes = kKTile * kD * 2; // 16 KB per matrix
 constexpr int kStages = 3;
-constexpr int kStageBytes = 16384;          // epilogue staging per wave: 32 rows x 512 B
 // Two flag words of the workgroup sit behind the tile buffers and the staging
 // areas, so that setting and reading them needs no barrier of its own.
 constexpr int kLdsFlags = 2 * kStages * kTileBytes > kWaves * kStageBytes ? 2 * kStages * kTileBytes
@@ -95,8 +81,6 @@ constexpr int kLdsFlags = 2 * kStages * kTileBytes > kWaves * kStageBytes ? 2 * 
 constexpr int kLdsBytes = kLdsFlags + 256;
 constexpr float kLog2e = 1.4426950408889634f;
 constexpr int kCuSlots = 256;               // one workgroup per CU
-constexpr int kMaxDevices = 64;
-constexpr int kPartBlockHalves = kQBlock * kD;   // one block's partial output: 32 x 128 fp16 = 8 KB
 // The ticket words of a split call sit in a region of FIXED size at the head of
 // the workspace, whatever the shape: a region that grew with the shape would
 // overlap, for a larger call, what an earlier smaller call left of its partial
@@ -112,126 +96,7 @@ constexpr int kLdsVBase = kStages * kTileBytes;
 constexpr int kLdsVRel(int buf) { return buf * kTileBytes; }
 constexpr int kLdsV(int buf) { return kLdsVBase + kLdsVRel(buf); }
 
-struct AttnKernelArgs {
-  const uint16_t* q;
-  const uint16_t* k;
-  const uint16_t* v;
-  uint16_t* out;
-  const int32_t* seq_lens;
-  sdv2_stride3 q_st, k_st, v_st, o_st;
-  int32_t rows, q_tokens, heads, max_seq_len;
-  // Key ranges per (row, head): num_splits, except that of every group_pairs
-  // consecutive (row, head) pairs the last more_pairs take num_splits + 1.
-  // (Uniform: group_pairs = rows * heads, more_pairs = 0.)
-  int32_t num_splits, group_pairs, more_pairs;
-  float scale_log2;            // softmax_scale * log2(e)
-  int32_t mask_block_tokens;   // 0 = no mask inside the chunk
-  const int32_t* chunk_start;  // device [rows]: cache position of the chunk's own first key
-  // Split calls.  Partial results are kept per 32-row query block in the order
-  // the registers hold them (see store_partial), q_blocks = ceil(q_tokens / 32).
-  int32_t q_blocks;
-  int32_t* tickets;            // [row][head][query tile], zero between calls
-  uint16_t* part_o;            // [split][row][head][block][8 KB] fp16: normalised output / row scale
-  float* part_lse;             // [split][row][head][block][32]   log2 sum exp
-  float* part_scale;           // [split][row][head][block][32]   largest magnitude of the normalised row
-  // Rotation of the queries inside the kernel (q is then the chunk's query
-  // BEFORE RoPE): the complex128 table, or null when q arrives rotated.
-  const double2* freqs;
-  int32_t grid_w, frame_tokens, split_t, split_h;
-  int64_t start_frame[SDV2_MAX_ROWS];
-  // RMSNorm of the queries inside the kernel (q is then the raw projection):
-  // the norm weight [heads * 128] and 1 / rms per (row, token), or null
-  const uint16_t* q_norm_w;
-  const float* q_inv_rms;
-};
-
 __device__ __forceinline__ int swz(int r) { return ((r & 3) << 2) | ((r >> 2) & 3); }
-
-// v_max without the NaN-quieting canonicalisation fmaxf() drags in.
-__device__ __forceinline__ float vmax(float a, float b) {
-  float r;
-  asm("v_max_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
-  return r;
-}
-
-// exchange between the two lanes that share a query column (lane and lane ^ 32)
-__device__ __forceinline__ float half_max(float x) {
-  auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
-  return vmax(__uint_as_float(r[0]), __uint_as_float(r[1]));
-}
-__device__ __forceinline__ float half_sum(float x) {
-  auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
-  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
-}
-
-__device__ __forceinline__ uint32_t pack_bf16x2(float lo, float hi) {
-  // fptrunc <2 x float> -> <2 x bfloat> selects v_cvt_pk_bf16_f32 (nearest-even)
-  const f32x2 x = {lo, hi};
-  return __builtin_bit_cast(uint32_t, __builtin_convertvector(x, bf16x2));
-}
-
-// two floats -> packed fp16 pair (lo in the low half), nearest-even
-__device__ __forceinline__ uint32_t pack_f16x2(float lo, float hi) {
-  const f32x2 x = {lo, hi};
-  return __builtin_bit_cast(uint32_t, __builtin_convertvector(x, f16x2));
-}
-
-// acc + lo + hi of a packed bf16 pair (v_dot2c_f32_bf16 against (1, 1))
-__device__ __forceinline__ float add_bf16_pair(uint32_t packed, float acc) {
-  const bf16x2 ones = {(__bf16)1.0f, (__bf16)1.0f};
-  return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2, packed), ones, acc, false);
-}
-
-// ---------------------------------------------------------------------------
-// LDS reads with hand-placed waits.  The compiler treats every LDS access as
-// possibly aliasing an in-flight global->LDS transfer and would drain all
-// counters before each dependent MFMA; issuing the reads as asm and tying an
-// explicit s_waitcnt to the fragment about to be consumed keeps several reads
-// in flight behind the matrix pipe.  LDS returns data in issue order, so
-// lgkmcnt(N) means "all but the newest N reads have landed".
-// ---------------------------------------------------------------------------
-template <int... I, typename F>
-__device__ __forceinline__ void static_for_impl(std::integer_sequence<int, I...>, F&& f) {
-  (f(std::integral_constant<int, I>{}), ...);
-}
-template <int N, typename F>
-__device__ __forceinline__ void static_for(F&& f) {
-  static_for_impl(std::make_integer_sequence<int, N>{}, f);
-}
-
-template <int kOffset>
-__device__ __forceinline__ u32x4 lds_read_b128(uint32_t addr) {
-  u32x4 r;
-  asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(r) : "v"(addr), "n"(kOffset));
-  return r;
-}
-template <int kOffset>
-__device__ __forceinline__ u32x2 lds_read_tr16_b64(uint32_t addr) {
-  u32x2 r;
-  asm volatile("ds_read_b64_tr_b16 %0, %1 offset:%2" : "=v"(r) : "v"(addr), "n"(kOffset));
-  return r;
-}
-// The same reads for the exact pass, which is not pipelined: the value is
-// waited for inside the statement and handed to compiler-generated MFMAs.
-// (Absolute per-lane addresses as in the fast pass: taking them relative to
-// the LDS base would keep a second copy of all sixteen alive across the
-// streaming loop.)
-__device__ __forceinline__ bf16x8 lds_read_b128_now(uint32_t addr) {
-  u32x4 r;
-  asm volatile("ds_read_b128 %0, %1\n\ts_waitcnt lgkmcnt(0)" : "=v"(r) : "v"(addr) : "memory");
-  return __builtin_bit_cast(bf16x8, r);
-}
-__device__ __forceinline__ bf16x8 lds_read_tr16_b64x2_now(uint32_t addr_lo, uint32_t addr_hi) {
-  u32x2 lo, hi;
-  asm volatile("ds_read_b64_tr_b16 %0, %2\n\tds_read_b64_tr_b16 %1, %3\n\ts_waitcnt lgkmcnt(0)"
-               : "=&v"(lo), "=&v"(hi) : "v"(addr_lo), "v"(addr_hi) : "memory");
-  return __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3));
-}
-// Optimisation passes may sink pure arithmetic down to its first use, which
-// here is a whole pipeline slot later.  Passing a value through an empty
-// volatile asm fixes the point by which it has to be computed.
-__device__ __forceinline__ void pin(float& x) { asm volatile("" : "+v"(x)); }
-__device__ __forceinline__ void pin(uint32_t& x) { asm volatile("" : "+v"(x)); }
 
 // The MFMAs of the fast pass are asm as well.  Left to itself the
 // compiler keeps every MFMA accumulator in the accumulation registers, but the
@@ -276,19 +141,6 @@ __device__ __forceinline__ void mfma_o(f32x16& d, const u32x4& a, const u32x4& b
 // (0..15, kPieces per issuing wave) fills rows 4i..4i+3; lane l lands on row 4i + l/16,
 // physical chunk l%16, so it must fetch logical chunk (l%16) ^ g(row).
 // ---------------------------------------------------------------------------
-// 16 bytes per lane from (wave-uniform base + this lane's 32-bit offset) to
-// (wave-uniform LDS address + 16 * lane).  Written as asm so that the address
-// stays "SGPR pair + one VGPR" instead of a 64-bit pointer per lane.
-__device__ __forceinline__ void dma16(const char* uniform_base, uint32_t lane_off, uint32_t lds_dst) {
-  asm volatile(
-      "s_mov_b32 m0, %2\n\t"
-      "s_nop 0\n\t"
-      "global_load_lds_dwordx4 %0, %1"
-      :
-      : "v"(lane_off), "s"(uniform_base), "s"(lds_dst)
-      : "memory");
-}
-
 // One 64-key tile of K or of V.  `off` holds this lane's four byte offsets
 // from the tile's first key row.  The last, partial tile redirects rows at or
 // past the valid length to the last valid key (their scores are masked), so
@@ -312,58 +164,6 @@ __device__ __forceinline__ void issue_matrix_tile(const char* base, uint32_t tok
   }
 }
 
-// ---------------------------------------------------------------------------
-// Partial results travel between workgroups that may sit on different XCDs,
-// each behind its own L2.  Fences would make that safe by writing back and
-// invalidating a whole L2 per workgroup (measured: 13 us per workgroup, and the
-// K / V lines the neighbours are streaming go with it).  Instead every access
-// to a partial result is itself device-coherent, as a relaxed atomic access of
-// agent scope is (the sc1 scope bit: the store writes through to memory, the
-// load does not hit in a stale line), and the ticket orders them: a workgroup
-// draws its ticket only after its stores have been acknowledged (vmcnt(0),
-// barrier), and the last one reads only after it has drawn.  The 16-byte
-// accesses have no atomic spelling in the language, so they are asm (8-byte
-// atomics were measured 4 % of the whole kernel slower).
-// ---------------------------------------------------------------------------
-__device__ __forceinline__ void store_coherent_x4(void* base, const u32x4& w0, const u32x4& w1, const u32x4& w2,
-                                                  const u32x4& w3) {
-  asm volatile(
-      "global_store_dwordx4 %0, %1, off sc1\n\t"
-      "global_store_dwordx4 %0, %2, off offset:1024 sc1\n\t"
-      "global_store_dwordx4 %0, %3, off offset:2048 sc1\n\t"
-      "global_store_dwordx4 %0, %4, off offset:3072 sc1"
-      :
-      : "v"(base), "v"(w0), "v"(w1), "v"(w2), "v"(w3)
-      : "memory");
-}
-// One block's partial output as this lane holds it: eight 16-byte pieces 1 KB
-// apart.  Issue and wait are ONE asm statement: between a load's issue and its
-// return the compiler believes the destination registers hold the value, and
-// is free to copy them elsewhere and reuse them - as an address, say - for the
-// load to overwrite when it lands.
-__device__ __forceinline__ void load_coherent_x8(const char* base, u32x4 (&w)[8]) {
-  asm volatile(
-      "global_load_dwordx4 %0, %8, off sc1\n\t"
-      "global_load_dwordx4 %1, %8, off offset:1024 sc1\n\t"
-      "global_load_dwordx4 %2, %8, off offset:2048 sc1\n\t"
-      "global_load_dwordx4 %3, %8, off offset:3072 sc1\n\t"
-      "global_load_dwordx4 %4, %9, off sc1\n\t"
-      "global_load_dwordx4 %5, %9, off offset:1024 sc1\n\t"
-      "global_load_dwordx4 %6, %9, off offset:2048 sc1\n\t"
-      "global_load_dwordx4 %7, %9, off offset:3072 sc1\n\t"
-      "s_waitcnt vmcnt(0)"
-      : "=&v"(w[0]), "=&v"(w[1]), "=&v"(w[2]), "=&v"(w[3]), "=&v"(w[4]), "=&v"(w[5]), "=&v"(w[6]), "=&v"(w[7])
-      : "v"(base), "v"(base + 4096)
-      : "memory");
-}
-__device__ __forceinline__ void store_coherent(float* p, float x) {
-  __hip_atomic_store(reinterpret_cast<uint32_t*>(p), __float_as_uint(x), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-__device__ __forceinline__ float load_coherent(const float* p) {
-  return __uint_as_float(
-      __hip_atomic_load(reinterpret_cast<const uint32_t*>(p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
-}
-
 // The compiler does not know that the asm MFMAs are still in flight when the
 // asm statement retires, so wherever code it generates may touch S or O right
 // after a slot (register moves at control-flow joins, the epilogue) the matrix
@@ -371,6 +171,14 @@ __device__ __forceinline__ float load_coherent(const float* p) {
 // may be read.  The tag makes every use textually distinct, otherwise identical
 // drains at the ends of sibling branches are merged into one AFTER the join,
 // behind the very moves they are meant to precede.
+// Row sums of the packed weights: one 16x16x32 MFMA per 16 keys, whose A operand
+// (`pick`, see LaneConst) adds up, for every lane, the weights of the lane's own
+// query.  (v_dot2c_f32_bf16 did it on the vector side, two weights an instruction,
+// but waits for the matrix pipe to run empty: some 20 cycles each.)
+__device__ __forceinline__ void mfma_row_sum(f32x4& d, const u32x4& pick, const u32x4& p) {
+  asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(d) : "a"(pick), "v"(p));
+}
+
 template <int kTag>
 __device__ __forceinline__ void mfma_drain(f32x16 (&oacc)[4], f32x16 (&s)[2]) {
   asm volatile("s_nop 15\n\ts_nop 15 ; matrix pipe drained, site %6"
@@ -379,6 +187,7 @@ __device__ __forceinline__ void mfma_drain(f32x16 (&oacc)[4], f32x16 (&s)[2]) {
 }
 
 struct LaneConst {
+  u32x4 pick;             // bf16 ones where the lane's k group holds weights of the queries of the lane's row group, else zeros
   uint32_t k_addr[8];     // K fragment of d-step ks: key row lane%32 of a 32-key block
   uint32_t v_addr[4][2];  // V^T fragment of d block db, key sub-quad j, within a 16-key step
   float c2;               // softmax scale * log2(e)
@@ -415,7 +224,7 @@ __device__ __forceinline__ void mask_block(f32x16& s, int key0, int seq, int hf,
 // ---------------------------------------------------------------------------
 template <bool kMask, int kPar, int kKOff, int kVOff, bool kDoS, bool kDoPV, bool kDoSM>
 __device__ __forceinline__ void slot(const LaneConst& c, const bf16x8 (&qf)[8], f32x16 (&s)[2], u32x4 (&p)[2][2],
-                                     f32x16 (&oacc)[4], float& l, int key0, int key_end) {
+                                     f32x16 (&oacc)[4], f32x4& l, int key0, int key_end) {
   // Fragment pairs are requested one group early: with a second wave on the
   // SIMD to cover the wait that is enough and measured 2-3 % faster than two
   // (fewer fragments in flight); none ahead is 4 % slower.
@@ -480,9 +289,7 @@ __device__ __forceinline__ void slot(const LaneConst& c, const bf16x8 (&qf)[8], 
       if constexpr (t >= 2 && t - 2 < kSteps && ((t - 2) & 1) == 1) {
         constexpr int u = t - 2, g = u / 2;
         uint32_t packed = pack_bf16x2(weight[u - 1], weight[u]);
-        l = add_bf16_pair(packed, l);
         pin(packed);
-        pin(l);
         p[kPar][g >> 2][g & 3] = packed;
       }
     }
@@ -504,6 +311,7 @@ __device__ __forceinline__ void slot(const LaneConst& c, const bf16x8 (&qf)[8], 
     if constexpr (i == 1 && kDoPV) mfma_o<later>(oacc[db], vfrag[g], p[kPar ^ 1][kk]);
 
     softmax_step(tc);
+    if constexpr (kDoPV && (t & 7) == 7) mfma_row_sum(l, c.pick, p[kPar ^ 1][kk]);
     __builtin_amdgcn_sched_barrier(0);
   });
   softmax_step(std::integral_constant<int, kSteps>{});
@@ -516,28 +324,28 @@ __device__ __forceinline__ void slot(const LaneConst& c, const bf16x8 (&qf)[8], 
 // coming and meets the barriers; only the waves whose fast result was unsafe
 // (`compute`) redo their block.
 // ---------------------------------------------------------------------------
-__device__ __forceinline__ void exact_pass(const LaneConst& c, const bf16x8 (&qf)[8], f32x16 (&oacc)[4], float& m_run,
-                                           float& l_run, bool compute, const char* kbase, const char* vbase,
+template <typename Key0>
+__device__ __forceinline__ void exact_pass(const Key0& key0_of, LaneConst& c, const bf16x8 (&qf)[8], f32x16 (&oacc)[4],
+                                           f32x4& l_sum, bool compute, const char* kbase, const char* vbase,
                                            uint32_t k_tok_bytes, uint32_t v_tok_bytes, const uint32_t (&k_ld)[kPieces],
                                            const uint32_t (&v_ld)[kPieces], int tile_begin, int n, int seq,
                                            uint32_t lds_addr0, lds_char* lds, int wave_u, int lane) {
+  float m_run = -INFINITY, l_run = 0.f;
   if (compute) {
-    m_run = -INFINITY;
-    l_run = 0.f;
 #pragma unroll
     for (int db = 0; db < 4; ++db)
 #pragma unroll
       for (int i = 0; i < 16; ++i) oacc[db][i] = 0.f;
   }
   auto issue = [&](int T) {
-    const int key0 = (tile_begin + T) * kKTile;
+    const int key0 = key0_of(tile_begin + T);
     issue_matrix_tile(kbase, k_tok_bytes, k_ld, key0, seq, lds_addr0 + kLdsK(T & 1), wave_u, lane);
     issue_matrix_tile(vbase, v_tok_bytes, v_ld, key0, seq, lds_addr0 + kLdsV(T & 1), wave_u, lane);
   };
   __syncthreads();       // everyone is done with the buffers of the fast pass
   issue(0);
   for (int T = 0; T < n; ++T) {
-    const int key0 = (tile_begin + T) * kKTile;
+    const int key0 = key0_of(tile_begin + T);
     const int kb_off = kLdsK(T & 1), vb_off = kLdsVRel(T & 1);
     if (T + 1 < n) {
       issue(T + 1);      // into the buffer tile T - 1 left at the barrier that ended the last trip
@@ -602,6 +410,10 @@ __device__ __forceinline__ void exact_pass(const LaneConst& c, const bf16x8 (&qf
     }
     __syncthreads();     // tile T's buffer is free for tile T + 2
   }
+  if (compute) {
+    l_sum[0] = half_sum(l_run);
+    c.neg_ref = -m_run * c.c2;
+  }
 }
 
 // This lane's query row as the B operand of S^T = K Q^T: d-step ks takes the
@@ -609,42 +421,22 @@ __device__ __forceinline__ void exact_pass(const LaneConst& c, const bf16x8 (&qf
 // the query before rotation and is rotated here, in the arithmetic of the
 // append kernel (IEEE double, no fused multiply-add, double -> float -> bf16),
 // so the kernel sees bit for bit the Q' the append would have stored.
-struct QueryRope {
-  const double2* freqs;        // null: the query arrives rotated
-  int64_t start_frame;         // of this cache row
-  int32_t grid_w, frame_tokens, split_t, split_h;
-  // With norm_w (this head's 128 norm weights, offset like qp) the row is the
-  // raw q projection: every slice is normalised with the token's 1 / rms as
-  // the append kernel's fused norm would have done it (sdv2::normalise: two
-  // roundings to bf16), then rotated.
-  const uint16_t* norm_w;
-  float inv_rms;
-};
-
 __device__ __forceinline__ void load_query(const QueryRope& rope, const uint16_t* qp, int token, int hf,
                                            bf16x8 (&qf)[8]) {
-  if (rope.freqs == nullptr) {
+  const int fi = token / rope.frame_tokens;
+  const int rem = token - fi * rope.frame_tokens;
+  const int hi = rem / rope.grid_w;
+  const int wi = rem - hi * rope.grid_w;
+  const int64_t frame = rope.start_frame + fi;
 #pragma unroll
-    for (int ks = 0; ks < 8; ++ks) qf[ks] = *reinterpret_cast<const bf16x8*>(qp + 16 * ks);
-  } else {
-    const int fi = token / rope.frame_tokens;
-    const int rem = token - fi * rope.frame_tokens;
-    const int hi = rem / rope.grid_w;
-    const int wi = rem - hi * rope.grid_w;
-    const int64_t frame = rope.start_frame + fi;
-#pragma unroll
-    for (int ks = 0; ks < 8; ++ks) {
-      double2 cs[4];
-      sdv2::load_rotation(rope.freqs, kD / 2, rope.split_t, rope.split_h, 2 * ks + hf, frame, hi, wi, cs);
-      sdv2::Vec8<uint16_t> x = sdv2::Vec8<uint16_t>::load(qp + 16 * ks);
-      if (rope.norm_w) x = sdv2::normalise(x, rope.inv_rms, sdv2::Vec8<uint16_t>::load(rope.norm_w + 16 * ks));
-      const sdv2::Vec8<uint16_t> y = sdv2::rotate(x, cs);
-      qf[ks] = __builtin_bit_cast(bf16x8, y.raw);
-    }
+  for (int ks = 0; ks < 8; ++ks) {
+    double2 cs[4];
+    sdv2::load_rotation(rope.freqs, kD / 2, rope.split_t, rope.split_h, 2 * ks + hf, frame, hi, wi, cs);
+    sdv2::Vec8<uint16_t> x = sdv2::Vec8<uint16_t>::load(qp + 16 * ks);
+    if (rope.norm_w) x = sdv2::normalise(x, rope.inv_rms, sdv2::Vec8<uint16_t>::load(rope.norm_w + 16 * ks));
+    const sdv2::Vec8<uint16_t> y = sdv2::rotate(x, cs);
+    qf[ks] = __builtin_bit_cast(bf16x8, y.raw);
   }
-  // the value is (re)defined in the register class every later use names, so it is never copied back and forth
-#pragma unroll
-  for (int ks = 0; ks < 8; ++ks) asm volatile("" : "+a"(qf[ks]));
 }
 
 template <bool kMask>
@@ -660,66 +452,35 @@ void swa_attn_fwd_kernel(const AttnKernelArgs a) {
   const int wave = tid >> 6;
   const int wave_u = __builtin_amdgcn_readfirstlane(wave);
   const int hf = lane >> 5;                 // which half of the wave
-  // Workgroups are dealt to the eight XCDs round robin by id, and each XCD has
-  // its own L2.  Work items are ordered so that the query tiles of one (row,
-  // head, key split) are neighbours, and XCD x takes the x-th eighth of that
-  // list: the workgroups that stream the same K / V run on the same XCD at the
-  // same time and all but the first fetch of a tile hit in L2.
-  //
-  // With a mixed split count a group of (row, head) pairs is one XCD's share:
-  // its pairs with fewer, longer key ranges come first, so that the workgroups
-  // the dispatcher hands out last are the short ones (longest first is what
-  // packs unequal pieces best onto the CUs).
-  int qtile, head, row, split, nsplits;
-  const int nq = (a.q_tokens + kQTile - 1) / kQTile;
-  {
-    const int per_lo = nq * a.num_splits, per_hi = per_lo + nq;
-    const int lo_pairs = a.group_pairs - a.more_pairs;
-    const int per_group = lo_pairs * per_lo + a.more_pairs * per_hi;
-    const int total = (a.heads * a.rows / a.group_pairs) * per_group;
-    const int xcd = blockIdx.x & 7;
-    const int first = (int)(((int64_t)xcd * total) >> 3);
-    const int end = (int)(((int64_t)(xcd + 1) * total) >> 3);
-    const int item = first + (blockIdx.x >> 3);
-    if (item >= end) return;
-    const int group = item / per_group;
-    int r = item - group * per_group;
-    int pair = group * a.group_pairs;
-    if (r < lo_pairs * per_lo) {
-      nsplits = a.num_splits;
-      pair += r / per_lo;
-      r %= per_lo;
-    } else {
-      nsplits = a.num_splits + 1;
-      r -= lo_pairs * per_lo;
-      pair += lo_pairs + r / per_hi;
-      r %= per_hi;
-    }
-    qtile = r % nq;
-    split = r / nq;
-    head = pair % a.heads;
-    row = pair / a.heads;
-  }
+  WorkItem w;
+  if (!w.decode(a, blockIdx.x)) return;
+  const int qtile = w.qtile, head = w.head, row = w.row, split = w.split, nsplits = w.nsplits;
 
   int seq = a.seq_lens ? a.seq_lens[row] : a.max_seq_len;
   seq = seq < a.max_seq_len ? seq : a.max_seq_len;
   seq = seq < 0 ? 0 : seq;
   const int ntiles = (seq + kKTile - 1) / kKTile;
-  const int per_split = (ntiles + nsplits - 1) / nsplits;
+  // With the mask inside the chunk the tiles [hole, hole + skipped) hold nothing but keys that are hidden from
+  // every query of this workgroup (from the last one, that is: earlier queries see fewer): they are not streamed,
+  // and the key ranges are cut from what is left.
+  int hole = 0x7fffffff, skipped = 0;
+  if constexpr (kMask) {
+    const int first = a.chunk_start[row], bt = a.mask_block_tokens;
+    const int q_last = qtile * kQTile + kQTile < a.q_tokens ? qtile * kQTile + kQTile - 1 : a.q_tokens - 1;
+    const int lo = first + (q_last / bt + 1) * bt, hi = first + a.q_tokens;
+    const int h0 = (lo + kKTile - 1) / kKTile, h1 = hi >= seq ? ntiles : hi / kKTile;
+    if (h1 > h0) { hole = h0; skipped = h1 - h0; }
+  }
+  auto key0_of = [&](int tile) { return (tile < hole ? tile : tile + skipped) * kKTile; };
+  const int per_split = (ntiles - skipped + nsplits - 1) / nsplits;
   const int tile_begin = split * per_split;
   int tile_end = tile_begin + per_split;
-  tile_end = tile_end < ntiles ? tile_end : ntiles;
+  tile_end = tile_end < ntiles - skipped ? tile_end : ntiles - skipped;
   const int n = tile_end - tile_begin;       // tiles this workgroup streams
 
-  // (the transfers take their base addresses from scalar registers: say so to the compiler)
-  auto uniform = [](const void* ptr) {
-    const uint64_t x = reinterpret_cast<uint64_t>(ptr);
-    const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)x), hi = __builtin_amdgcn_readfirstlane((uint32_t)(x >> 32));
-    return reinterpret_cast<const char*>(((uint64_t)hi << 32) | lo);
-  };
   const uint32_t lds_addr0 = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)lds);
-  const char* kbase = uniform(a.k + row * a.k_st.row + head * a.k_st.head);
-  const char* vbase = uniform(a.v + row * a.v_st.row + head * a.v_st.head);
+  const char* kbase = uniform_pointer(a.k + row * a.k_st.row + head * a.k_st.head);
+  const char* vbase = uniform_pointer(a.v + row * a.v_st.row + head * a.v_st.head);
   const uint32_t k_tok_bytes = (uint32_t)(a.k_st.token * 2);
   const uint32_t v_tok_bytes = (uint32_t)(a.v_st.token * 2);
 
@@ -733,16 +494,26 @@ void swa_attn_fwd_kernel(const AttnKernelArgs a) {
   }
   // T is the tile index inside this workgroup's range
   auto issue_k = [&](int T, int buf) {
-    issue_matrix_tile(kbase, k_tok_bytes, k_ld, (tile_begin + T) * kKTile, seq, lds_addr0 + kLdsK(buf), wave_u, lane);
+    issue_matrix_tile(kbase, k_tok_bytes, k_ld, key0_of(tile_begin + T), seq, lds_addr0 + kLdsK(buf), wave_u, lane);
   };
   auto issue_v = [&](int T, int buf) {
-    issue_matrix_tile(vbase, v_tok_bytes, v_ld, (tile_begin + T) * kKTile, seq, lds_addr0 + kLdsV(buf), wave_u, lane);
+    issue_matrix_tile(vbase, v_tok_bytes, v_ld, key0_of(tile_begin + T), seq, lds_addr0 + kLdsV(buf), wave_u, lane);
   };
 
-  // The transfers the first two slots need go out first; the query rows are
-  // fetched (and rotated) behind them, the rest of the look-ahead after that:
-  // ordinary loads return in order with the transfers, so whatever is issued
-  // ahead of the query rows is what the first wait for them also waits for.
+  // ---- this lane's query row, and the first tiles -----------------------------
+  // Loads return in the order they were issued.  A query that arrives rotated is
+  // asked for ahead of the first tiles, so that both come back in one trip to
+  // memory; one that is to be rotated here needs several trips for the rotation
+  // table and is fetched behind the tiles the first two slots need, the rest of
+  // the look-ahead after it.
+  const int q_row = qtile * kQTile + wave * kQBlock + (lane & 31);
+  const int q_row_c = q_row < a.q_tokens ? q_row : a.q_tokens - 1;
+  const uint16_t* q_ptr = a.q + row * a.q_st.row + (int64_t)q_row_c * a.q_st.token + head * a.q_st.head + 8 * hf;
+  bf16x8 qf[8];
+  if (a.freqs == nullptr) {
+#pragma unroll
+    for (int ks = 0; ks < 8; ++ks) qf[ks] = *reinterpret_cast<const bf16x8*>(q_ptr + 16 * ks);
+  }
   if (n > 0) {
     issue_k(0, 0);
     issue_v(0, 0);
@@ -757,26 +528,18 @@ void swa_attn_fwd_kernel(const AttnKernelArgs a) {
     if (tid == 0) flags[0] = 0;       // "a wave found an unsafe row sum": read behind the barrier that ends the loop
   }
 
-  // ---- this lane's query row -------------------------------------------------
-  const int q_row = qtile * kQTile + wave * kQBlock + (lane & 31);
-  bf16x8 qf[8];
-  {
-    const int q_row_c = q_row < a.q_tokens ? q_row : a.q_tokens - 1;
+  if (a.freqs != nullptr) {
     QueryRope rope;
     rope.freqs = a.freqs;
     rope.grid_w = a.grid_w; rope.frame_tokens = a.frame_tokens; rope.split_t = a.split_t; rope.split_h = a.split_h;
-    // (constant indices and selects: indexing the by-value argument block with a run-time
-    // row would move the whole block, its pointers included, out of scalar registers)
-    rope.start_frame = a.start_frame[0];
-    static_for<SDV2_MAX_ROWS - 1>([&](auto ic) {
-      constexpr int i = decltype(ic)::value + 1;
-      rope.start_frame = row == i ? a.start_frame[i] : rope.start_frame;
-    });
+    rope.start_frame = row_start_frame(a, row);
     rope.norm_w = a.q_norm_w ? a.q_norm_w + head * kD + 8 * hf : nullptr;
     rope.inv_rms = a.q_norm_w ? a.q_inv_rms[(int64_t)row * a.q_tokens + q_row_c] : 1.0f;
-    load_query(rope, a.q + row * a.q_st.row + (int64_t)q_row_c * a.q_st.token + head * a.q_st.head + 8 * hf, q_row_c,
-               hf, qf);
+    load_query(rope, q_ptr, q_row_c, hf, qf);
   }
+  // the value is (re)defined in the register class every later use names, so it is never copied back and forth
+#pragma unroll
+  for (int ks = 0; ks < 8; ++ks) asm volatile("" : "+a"(qf[ks]));
   if (n > 0) {
     // every buffer a slot may read starts with real (finite) data, also where the tile does not exist
     issue_v(n > 1 ? 1 : n - 1, 1);
@@ -785,6 +548,14 @@ void swa_attn_fwd_kernel(const AttnKernelArgs a) {
 
   // ---- per-lane LDS read addresses ------------------------------------------
   LaneConst c;
+  {
+    // as the B operand of a 16x16x32 MFMA the packed weights of 16 keys put query lane % 32 into k group lane / 16:
+    // groups 0 and 2 the first sixteen queries, 1 and 3 the others.  Result row m = 4 (lane / 16) + i is to add up
+    // the groups of its own lanes' queries.
+    const uint32_t one = ((lane >> 4) & 1) == ((lane >> 2) & 1) ? 0x3f803f80u : 0u;
+    c.pick = u32x4{one, one, one, one};
+    asm volatile("" : "+a"(c.pick));      // (one copy for the whole kernel: a constant formed in front of an asm MFMA is read too early)
+  }
   c.c2 = a.scale_log2;
   c.neg_ref = 0.f;
   c.hf = hf;
@@ -834,8 +605,7 @@ void swa_attn_fwd_kernel(const AttnKernelArgs a) {
   for (int i = 0; i < 2; ++i)
 #pragma unroll
     for (int j = 0; j < 2; ++j) p[i][j] = u32x4{0u, 0u, 0u, 0u};
-  float l_run = 0.f;                 // this lane's share of the row sum
-  float m_run = 0.f;                 // the row's exponent reference, in score units
+  f32x4 l_run = {0.f, 0.f, 0.f, 0.f};   // the row's sum of weights, the same in every register
   bool unsafe = false;
 
   // Tile T (64 keys) = blocks 2T, 2T+1, in K / V buffers T % 3.  Slot 2T needs
@@ -855,11 +625,11 @@ void swa_attn_fwd_kernel(const AttnKernelArgs a) {
   // exist) are masked to -inf, so their weights are exact zeros against
   // whatever finite data the buffers still hold.  In the first slot P(-1) is
   // zero likewise.
-  const int key_end = seq < tile_end * kKTile ? seq : tile_end * kKTile;
+  const int key_end = seq;
   auto do_tile = [&](auto buf_c, int T) {
     constexpr int kB = decltype(buf_c)::value;              // T % 3
     constexpr int kBNext = (kB + 1) % kStages, kBPrev = (kB + 2) % kStages;
-    const int key0 = (tile_begin + T) * kKTile;
+    const int key0 = key0_of(tile_begin + T);
     slot<kMask, 0, kLdsK(kB) + 32 * 256, kLdsVRel(kBPrev) + 32 * 256, true, true, true>(c, qf, s, p, oacc, l_run, key0,
                                                                                         key_end);
     if (T + 3 < n) {
@@ -912,7 +682,6 @@ void swa_attn_fwd_kernel(const AttnKernelArgs a) {
         for (int i = 1; i < 16; ++i) ref = vmax(ref, s[0][i]);
         ref = half_max(ref);
         ref = (ref > -0x1p120f && ref < 0x1p120f) ? ref : 0.f;      // also false for NaN
-        m_run = ref;
         c.neg_ref = -ref * c.c2;
       }
       // Three tiles per trip, one per buffer; the last trip stops after the last
@@ -929,23 +698,29 @@ void swa_attn_fwd_kernel(const AttnKernelArgs a) {
       // buffer) empties the pipeline.  The code addresses V buffer 2; the lane
       // addresses are moved when the last tile sits in another buffer.
       {
-        LaneConst cf = c;
+        // (in place and back again: a copy of the addresses does not fit the registers)
         const uint32_t shift = (uint32_t)(((n - 1) % kStages - 2) * kTileBytes);
 #pragma unroll
         for (int db = 0; db < 4; ++db)
 #pragma unroll
-          for (int j = 0; j < 2; ++j) cf.v_addr[db][j] = c.v_addr[db][j] + shift;
-        slot<kMask, 0, 0, kLdsVRel(2) + 32 * 256, false, true, false>(cf, qf, s, p, oacc, l_run, 0, key_end);
+          for (int j = 0; j < 2; ++j) c.v_addr[db][j] += shift;
+        slot<kMask, 0, 0, kLdsVRel(2) + 32 * 256, false, true, false>(c, qf, s, p, oacc, l_run, 0, key_end);
+#pragma unroll
+        for (int db = 0; db < 4; ++db)
+#pragma unroll
+          for (int j = 0; j < 2; ++j) c.v_addr[db][j] -= shift;
       }
       mfma_drain<0>(oacc, s);
+      asm volatile("" : "+a"(l_run));
       // Checked once, after the last tile: a sum that overflowed stays inf or NaN, one
       // that underflowed stays tiny.  With the mask inside the chunk a sum of exactly
       // zero is legitimate when every key of this workgroup's range is hidden from
       // the lane's query (its split then contributes nothing).
       {
-        const float l_tot = half_sum(l_run);
+        const float l_tot = l_run[0];
         bool ok = l_tot >= 0x1p-100f && l_tot <= 0x1p100f;
-        if constexpr (kMask) ok |= l_tot == 0.f && tile_begin * kKTile >= c.m_lo && key_end <= c.m_hi;
+        if constexpr (kMask) ok |= l_tot == 0.f && key0_of(tile_begin) >= c.m_lo &&
+              (key0_of(tile_end - 1) + kKTile < seq ? key0_of(tile_end - 1) + kKTile : seq) <= c.m_hi;
         unsafe = __builtin_amdgcn_ballot_w64(!ok) != 0;
       }
     }
@@ -957,15 +732,34 @@ void swa_attn_fwd_kernel(const AttnKernelArgs a) {
     __syncthreads();
     const int redo = flags[0];
     if (redo)
-      exact_pass(c, qf, oacc, m_run, l_run, unsafe, kbase, vbase, k_tok_bytes, v_tok_bytes, k_ld, v_ld, tile_begin, n,
+      exact_pass(key0_of, c, qf, oacc, l_run, unsafe, kbase, vbase, k_tok_bytes, v_tok_bytes, k_ld, v_ld, tile_begin, n,
                  seq, lds_addr0, lds, wave_u, lane);
   }
 
   // ---- epilogue ---------------------------------------------------------------
   // (every wave is done with the K / V buffers: the barrier above, or the last one of the exact pass)
   const int block = qtile * kWaves + wave;              // this wave's 32-row block within the (row, head)
-  float l_tot = half_sum(l_run);
+  const float l_tot = l_run[0];
   float inv = l_tot > 0.f ? 1.0f / l_tot : 0.f;
+
+  // A lane holds one query row's values scattered over the 128 dims, so direct
+  // stores would touch 32 rows with 16 or 32 bytes each.  Instead every wave
+  // stages its 32-row block in its own part of the (now idle) LDS, 16-byte
+  // chunks XOR-swizzled by row, and writes whole rows of 256 bytes.  LDS
+  // operations of one wave complete in order, so the block needs no barrier of
+  // its own.
+  lds_char* stage = lds + wave * kStageBytes;
+  auto stage_out = [&](int db, const f32x16& o) {
+    const int r = lane & 31;
+#pragma unroll
+    for (int gq = 0; gq < 4; ++gq) {
+      u32x2 x;
+      x[0] = pack_bf16x2(o[4 * gq] * inv, o[4 * gq + 1] * inv);
+      x[1] = pack_bf16x2(o[4 * gq + 2] * inv, o[4 * gq + 3] * inv);
+      const int chunk = db * 4 + gq;
+      *reinterpret_cast<__attribute__((address_space(3))) u32x2*>(stage + r * 256 + ((chunk ^ (r & 15)) << 4) + hf * 8) = x;
+    }
+  };
 
   if (nsplits > 1) {
     // Partial result of a key range: the normalised row divided by its largest
@@ -1003,7 +797,7 @@ void swa_attn_fwd_kernel(const AttnKernelArgs a) {
       }
       if (hf == 0) {
         store_coherent(a.part_lse + blk * kQBlock + lane,
-                       l_tot > 0.f ? m_run * c.c2 + __builtin_amdgcn_logf(l_tot) : -INFINITY);
+                       l_tot > 0.f ? __builtin_amdgcn_logf(l_tot) - c.neg_ref : -INFINITY);
         store_coherent(a.part_scale + blk * kQBlock + lane, row_scale);
       }
     }
@@ -1014,7 +808,7 @@ void swa_attn_fwd_kernel(const AttnKernelArgs a) {
     __builtin_amdgcn_s_waitcnt(0x0F70);       // vmcnt(0)
     __syncthreads();
     if (tid == 0) {
-      int32_t* ticket = a.tickets + ((int64_t)row * a.heads + head) * nq + qtile;
+      int32_t* ticket = a.tickets + ((int64_t)row * a.heads + head) * a.q_tiles + qtile;
       const int drawn = __hip_atomic_fetch_add(ticket, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       const int last = drawn == nsplits - 1;
       if (last) __hip_atomic_store(ticket, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -1025,12 +819,14 @@ void swa_attn_fwd_kernel(const AttnKernelArgs a) {
 
     // combine: out = sum_s 2^(lse_s - LSE) O_s over the ranges in their fixed
     // order (every range, this workgroup's own included, as it lies in memory:
-    // the sum does not depend on which workgroup happens to be last)
+    // the sum does not depend on which workgroup happens to be last).  A trip to
+    // memory costs the same microsecond and a half whatever it carries, so the
+    // statistics of four ranges travel with half of their outputs, and the other
+    // half follows (all of it at once does not fit the registers).
     const int r32 = lane & 31;
-    constexpr int kBatch = 8;         // ranges whose statistics are fetched together
-    float wsum = 0.f;
-    float lse[kBatch], scale[kBatch], ws[kBatch];
-    // log-sum-exp and row scale of the ranges of a batch; the loads go out together
+    constexpr int kBatch = 4;
+    float lse_max = -INFINITY;
+    float lse[kBatch], scale[kBatch];
     auto fetch = [&](int s0) {
 #pragma unroll
       for (int u = 0; u < kBatch; ++u) {
@@ -1039,72 +835,62 @@ void swa_attn_fwd_kernel(const AttnKernelArgs a) {
         scale[u] = load_coherent(a.part_scale + (sp * slab + blk0) * kQBlock + r32);
       }
     };
-    fetch(0);
-    float lse_max = lse[0];
+    auto part_at = [&](int sp, int half) {
+      return reinterpret_cast<const char*>(a.part_o + ((sp < nsplits ? sp : nsplits - 1) * slab + blk0) * kPartBlockHalves +
+                                           lane * 8) + half * 4096;
+    };
 #pragma unroll
-    for (int u = 1; u < kBatch; ++u) lse_max = fmaxf(lse_max, lse[u]);         // (entries past the last range repeat it)
-    for (int sp = kBatch; sp < nsplits; ++sp)
-      lse_max = fmaxf(lse_max, load_coherent(a.part_lse + (sp * slab + blk0) * kQBlock + r32));
+    for (int half = 0; half < 2; ++half) {
+      f32x16 acc[2];
 #pragma unroll
-    for (int db = 0; db < 4; ++db)
+      for (int db = 0; db < 2; ++db)
 #pragma unroll
-      for (int i = 0; i < 16; ++i) oacc[db][i] = 0.f;
-    for (int s0 = 0; s0 < nsplits; s0 += kBatch) {
-      if (s0 > 0) fetch(s0);
+        for (int i = 0; i < 16; ++i) acc[db][i] = 0.f;
+      float wsum = 0.f;
+      for (int s0 = 0; s0 < nsplits; s0 += kBatch) {
+        u32x4 x[kBatch][4];
+        if (half == 0 || nsplits > kBatch) fetch(s0);
+        load_coherent_4x4(part_at(s0, half), part_at(s0 + 1, half), part_at(s0 + 2, half), part_at(s0 + 3, half), x);
+        if (half == 0 && s0 == 0) {
 #pragma unroll
-      for (int u = 0; u < kBatch; ++u) {
-        const float w = (s0 + u >= nsplits || lse[u] == -INFINITY) ? 0.f : __builtin_amdgcn_exp2f(lse[u] - lse_max);
-        wsum += w;
-        ws[u] = w * scale[u];         // weight times the row's fp16 scale
-      }
+          for (int u = 0; u < kBatch; ++u) lse_max = fmaxf(lse_max, lse[u]);         // (entries past the last range repeat it)
+          for (int sp = kBatch; sp < nsplits; ++sp)
+            lse_max = fmaxf(lse_max, load_coherent(a.part_lse + (sp * slab + blk0) * kQBlock + r32));
+        }
 #pragma unroll
-      for (int u = 0; u < kBatch; ++u) {
-        if (s0 + u >= nsplits) break;
-        u32x4 x[8];
-        load_coherent_x8(
-            reinterpret_cast<const char*>(a.part_o + ((s0 + u) * slab + blk0) * kPartBlockHalves + lane * 8), x);
+        for (int u = 0; u < kBatch; ++u) {
+          const float e = (s0 + u >= nsplits || lse[u] == -INFINITY) ? 0.f : __builtin_amdgcn_exp2f(lse[u] - lse_max);
+          wsum += e;
+          const float w2 = e * scale[u];             // weight times the row's fp16 scale
+          if (s0 + u < nsplits)
 #pragma unroll
-        for (int j = 0; j < 8; ++j) {
-          const int db = j >> 1, i0 = 8 * (j & 1);
-          const f16x8 h = __builtin_bit_cast(f16x8, x[j]);
+            for (int j = 0; j < 4; ++j) {
+              const f16x8 h = __builtin_bit_cast(f16x8, x[u][j]);
 #pragma unroll
-          for (int e = 0; e < 8; ++e) oacc[db][i0 + e] += ws[u] * static_cast<float>(h[e]);
+              for (int i = 0; i < 8; ++i) acc[j >> 1][8 * (j & 1) + i] += w2 * static_cast<float>(h[i]);
+            }
         }
       }
+      inv = wsum > 0.f ? 1.0f / wsum : 0.f;
+      stage_out(2 * half, acc[0]);
+      stage_out(2 * half + 1, acc[1]);
     }
-    inv = wsum > 0.f ? 1.0f / wsum : 0.f;
   } else if (idle) {
     return;
+  } else {
+#pragma unroll
+    for (int db = 0; db < 4; ++db) stage_out(db, oacc[db]);
   }
 
-  // A lane holds one query row's values scattered over the 128 dims, so direct
-  // stores would touch 32 rows with 16 or 32 bytes each.  Instead every wave
-  // stages its 32-row block in its own 16 KB of the (now idle) LDS, 16-byte
-  // chunks XOR-swizzled by row, and writes whole rows of 256 bytes.  LDS
-  // operations of one wave complete in order, so the block needs no barrier of
-  // its own.
-  lds_char* stage = lds + wave * kStageBytes;
   const int q0 = qtile * kQTile + wave * kQBlock;
-  const int r = lane & 31;
-#pragma unroll
-  for (int db = 0; db < 4; ++db)
-#pragma unroll
-    for (int g = 0; g < 4; ++g) {
-      u32x2 w;
-      w[0] = pack_bf16x2(oacc[db][4 * g] * inv, oacc[db][4 * g + 1] * inv);
-      w[1] = pack_bf16x2(oacc[db][4 * g + 2] * inv, oacc[db][4 * g + 3] * inv);
-      const int chunk = db * 4 + g;
-      *reinterpret_cast<__attribute__((address_space(3))) u32x2*>(stage + r * 256 + ((chunk ^ (r & 15)) << 4) + hf * 8) =
-          w;
-    }
   uint16_t* dst = a.out + row * a.o_st.row + head * a.o_st.head + (int64_t)q0 * a.o_st.token;
   const int j = lane & 15;
 #pragma unroll
   for (int it = 0; it < 8; ++it) {
     const int rr = 4 * it + (lane >> 4);
-    const u32x4 w = *reinterpret_cast<__attribute__((address_space(3))) const u32x4*>(
+    const u32x4 x = *reinterpret_cast<__attribute__((address_space(3))) const u32x4*>(
         stage + rr * 256 + ((j ^ (rr & 15)) << 4));
-    if (q0 + rr < a.q_tokens) *reinterpret_cast<u32x4*>(dst + rr * a.o_st.token + j * 8) = w;
+    if (q0 + rr < a.q_tokens) *reinterpret_cast<u32x4*>(dst + rr * a.o_st.token + j * 8) = x;
   }
 }
 
@@ -1381,12 +1167,20 @@ int attn_fwd(const sdv2_attn_params* p, void* workspace, size_t workspace_bytes)
     a.part_scale = reinterpret_cast<float*>(ws + w.part_scale);
   }
 
+  set_work_list(&a, kQTile);
   hipStream_t stream = static_cast<hipStream_t>(p->stream);
   const int64_t nq_tiles = (p->q_tokens + kQTile - 1) / kQTile;
   const int64_t items = ((int64_t)p->rows * p->heads / plan.group) *
                         (nq_tiles * ((int64_t)(plan.group - plan.more) * plan.base + (int64_t)plan.more * (plan.base + 1)));
   if (items > (1 << 28)) return SDV2_ERR_INVALID_ARG;
   dim3 grid((unsigned)(8 * ((items + 7) / 8)));
+  // Which kernel.  The one on 16x16x32 matrix instructions takes 1.51 us per 64-key tile of a full CU where this one
+  // takes 1.65, and a microsecond more to fill its deeper pipeline: they meet at 12 tiles (1536 queries x 40 heads,
+  // one key range: 768 keys 30.5 against 30.7 us, 384 keys 22.1 against 21.3, 3072 keys 84.5 against 90.4).  The mask
+  // inside the chunk costs the other kernel, whose lanes own two queries each, more than it gains.
+  constexpr int kTilesForM16 = 12;
+  if (a.mask_block_tokens == 0 && (p->max_seq_len + kKTile - 1) / kKTile >= kTilesForM16 * plan.base)
+    return sdv2::attn::launch_m16(a, grid.x, stream);
   // The tile buffers (96 KB) or the epilogue staging (16 KB per wave) exceed the static limit:
   // ask for the dynamic size once per device.
   // The kernel exists twice: the mask inside the chunk costs the plain

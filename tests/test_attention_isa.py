@@ -139,3 +139,29 @@ def test_register_budget(assembly):
     text = "\n".join(assembly)
     counts = [int(x) for x in re.findall(r"\.vgpr_count:\s+(\d+)", text)]
     assert len(counts) == 2 and max(counts) <= 256, counts
+
+
+@pytest.fixture(scope="module")
+def assembly_m16():
+    out = os.path.join(ROOT, "build", "isa_check")
+    os.makedirs(out, exist_ok=True)
+    path = os.path.join(out, "swa_attn_fwd_m16.s")
+    cmd = [build_ext.hipcc_path(), *build_ext.HIPCC_FLAGS, f"-I{os.path.join(ROOT, 'include')}", f"-I{build_ext.CSRC}",
+           "-S", "--cuda-device-only", str(build_ext.CSRC / "swa_attn_fwd_m16.hip"), "-o", path]
+    res = subprocess.run(cmd, capture_output=True, text=True)
+    assert res.returncode == 0, res.stderr[-2000:]
+    return open(path).read().split("\n")
+
+
+def test_the_same_promises_for_the_16x16_kernel(assembly_m16):
+    start = next(i for i, l in enumerate(assembly_m16) if re.match(r"^_Z\S*swa_attn_fwd_m16_kernel\S*:", l))
+    end = next(i for i in range(start, len(assembly_m16)) if assembly_m16[i].strip().startswith(".Lfunc_end"))
+    body = assembly_m16[start:end]
+    problems, n_mfma = early_reads(instructions(body))
+    assert n_mfma >= 256 and not problems, problems[:10]
+    loop = next(i for i, l in enumerate(body) if "Loop Header" in l)
+    hot = body[loop:next(i for i, l in enumerate(body) if "matrix pipe drained, site 0" in l)]
+    assert sum("v_mfma_f32_16x16x32_bf16" in l for l in hot) >= 128
+    assert not [l.strip() for l in hot if re.search(r"\bscratch_(load|store)", l)]
+    counts = [int(x) for x in re.findall(r"\.vgpr_count:\s+(\d+)", "\n".join(assembly_m16))]
+    assert len(counts) == 1 and counts[0] <= 256, counts

@@ -379,3 +379,59 @@ def test_one_extreme_query_row_costs_less_than_a_second_launch(gpu_device):
     _check(out.cpu()[:, rows], want)
     print(f"plain {plain * 1e3:.1f} us, one extreme row {extreme * 1e3:.1f} us", flush=True)
     assert extreme < 3.0 * plain, (plain, extreme)
+
+
+# the kernel on 16x16x32 matrix instructions takes unmasked calls of at least 12 tiles (of 64 keys) per key range
+@pytest.mark.parametrize("rows,S,H,L,seq,splits,head_major", [
+    (1, 256, 2, 768, None, 1, True),             # exactly 12 whole tiles, whole query tile
+    (1, 257, 1, 769, None, 1, True),             # one query row in the second tile, one key in the 13th
+    (1, 255, 3, 831, None, 1, False),            # one key short of a tile
+    (1, 1, 1, 800, None, 1, True),               # one query
+    (1, 33, 2, 1600, None, 2, True),             # a second block of one row, split
+    (2, 31, 5, 2320, [2320, 1], 3, True),        # ranges with nothing in them
+    (3, 64, 2, 1900, [1900, 33, 700], 2, False),
+    (1, 300, 8, 3000, None, 2 | (0 << 8), True),
+    (1, 300, 16, 3000, None, 2 | (1 << 8), True),  # two split counts
+    (1, 40, 2, 6000, None, 6, True),             # more ranges than are combined at once
+])
+def test_attention_on_16x16_matrix_instructions(gpu_device, rows, S, H, L, seq, splits, head_major):
+    """Against the fp32 oracle at the edges of tiles, ranges and blocks; twice on one workspace, same bits; and
+    again with scores far outside the range of the fixed-reference softmax."""
+    from streamdiffusionv2_amd import ops
+
+    torch.manual_seed(4)
+    lens = seq if seq is not None else [L] * rows
+    sl = torch.tensor(lens, dtype=torch.int32, device=gpu_device)
+
+    def on_device(t):
+        return t.permute(0, 2, 1, 3).contiguous().to(gpu_device).permute(0, 2, 1, 3) if head_major else t.to(gpu_device)
+
+    for scale in (1.0, 30.0):
+        q, k, v = (torch.randn(rows, n, H, 128) for n in (S, L, L))
+        q[:, S // 2:] *= scale                    # (30: scores of several hundred, either way, on half of the rows)
+        q, k, v = q.bfloat16(), k.bfloat16(), v.bfloat16()
+        print(f"rows={rows} S={S} H={H} L={L} splits={splits:#x} scale={scale}", flush=True)
+        want = oracle.attention_fp32_reference(q, k, v, lens)
+        got, again = (ops.swa_attention(q.to(gpu_device), on_device(k), on_device(v), sl, num_splits=splits) for _ in range(2))
+        torch.cuda.synchronize()
+        _check(got.cpu(), want)
+        assert torch.equal(got.view(torch.int16), again.view(torch.int16))
+
+
+@pytest.mark.parametrize("frames,bt_frames", [(3, 1), (3, 2), (2, 1)])
+def test_masked_attention_skips_hidden_tiles(gpu_device, frames, bt_frames):
+    """With the mask inside the chunk the tiles that are hidden from every query of a workgroup are not streamed:
+    chunks at the head, in the middle and at the end of the cache, unsplit and split."""
+    from streamdiffusionv2_amd import ops
+
+    torch.manual_seed(8)
+    ft, H = 300, 2                                # 300 tokens a frame: hidden ranges end inside tiles
+    S, L = frames * ft, 2000
+    q, k, v = (torch.randn(1, n, H, 128).bfloat16() for n in (S, L, L))
+    for start in (0, 520, L - S):
+        want = oracle.attention_fp32_reference(q, k, v, [L], [start], bt_frames * ft)
+        for splits in (1, 3):
+            got = ops.swa_attention(q.to(gpu_device), k.to(gpu_device), v.to(gpu_device), None, num_splits=splits,
+                                    chunk_key_start=[start], mask_block_tokens=bt_frames * ft)
+            torch.cuda.synchronize()
+            _check(got.cpu(), want)
