@@ -236,19 +236,15 @@ class RingKVPath:
             for frame in range(dst // frame_tokens, min(self.sink_size, (dst + tokens - 1) // frame_tokens + 1)):
                 kept["stale"][i] |= 1 << frame
 
-    def _layer_launcher(self, q, k, v, kv_cache, table, grid, qk_norm=None, keep_roped_q=False):
+    def _layer_launcher(self, q, k, v, kv_cache, table, grid, qk_norm=None):
         """The cached launch descriptors for this layer, rebuilt when the
-        cache, the shapes, the grid or the norm weights change.  keep_roped_q:
-        the caller wants the normalised, rotated query back, so the append
-        writes it (otherwise, with the norm folded in, no such tensor exists)."""
+        cache, the shapes, the grid or the norm weights change."""
         launcher = getattr(self, "_launcher", None)
-        in_attention = not (keep_roped_q and qk_norm is not None)
         if launcher is None or not launcher.matches(q, k, v, kv_cache, table, qk_norm) \
-                or launcher.rope_in_attention != in_attention \
                 or (launcher.ap.grid_f, launcher.ap.grid_h, launcher.ap.grid_w) != tuple(grid):
             launcher = ops.LayerLauncher(kv_cache["k"], kv_cache["v"], kv_cache["global_end_index"],
                                          kv_cache["local_end_index"], table, grid, q, k, v, qk_norm=qk_norm,
-                                         rope_in_attention=in_attention)
+                                         rope_in_attention=False)
             self._launcher = launcher
         if launcher.forced_splits != self.num_splits:
             launcher.forced_splits = self.num_splits
@@ -349,15 +345,11 @@ class RingKVPath:
             if q.dtype == torch.bfloat16 and rows <= ops._capi.MAX_ROWS:
                 # steady-state fast path: launch descriptors are built once per
                 # (cache, shape) and only patched per call
-                launcher = self._layer_launcher(q, k, v, kv_cache, table, (f, h, w), qk_norm, return_roped_query)
+                launcher = self._layer_launcher(q, k, v, kv_cache, table, (f, h, w), qk_norm)
                 start_frames = [c // frame_tokens for c in starts]
                 out = launcher.launch(q, k, v, start_frames, plan, seq, mask_tokens, override)
                 if return_roped_query:
-                    # the attention kernel rotates q on the fly and keeps no copy: the
-                    # stand-alone rotation gives the same bits (one arithmetic for both)
-                    if launcher.roped_q is not None:
-                        return out, launcher.roped_q.clone()
-                    return out, ops.causal_rope_apply(q, [(f, h, w)] * rows, table, torch.tensor(start_frames))
+                    return out, launcher.roped_q.clone()
                 return out
 
             roped_q = ops.kv_append_rope(

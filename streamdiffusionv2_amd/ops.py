@@ -330,6 +330,30 @@ def _workspace(dev: torch.device, nbytes: int, pool: Optional[dict] = None) -> t
     return ws
 
 
+_ROPED_QUERIES: dict = {}
+
+
+def _roped_query_scratch(dev: torch.device, elems: int) -> torch.Tensor:
+    """Where a layer call's append leaves the rotated query for its attention:
+    one bf16 buffer per (device, stream), grown on demand.  The two launches
+    follow each other on the stream, so the layers of a model share it."""
+    key = (dev, _stream_ptr(dev))
+    buf = _ROPED_QUERIES.get(key)
+    if buf is None or buf.numel() < elems:
+        buf = torch.empty(elems, dtype=torch.bfloat16, device=dev)
+        _ROPED_QUERIES[key] = buf
+    return buf
+
+
+def release_scratch() -> None:
+    """Give back the scratch buffers kept per (device, stream): split-KV and
+    sink-similarity workspaces, rotated queries.  Calls already enqueued keep
+    what they use until the stream is past them (the allocator's own rule); not
+    for programs that still replay graphs captured over these calls."""
+    for pool in (_WORKSPACES, _SIM_WORKSPACES, _ROPED_QUERIES):
+        pool.clear()
+
+
 def chunk_starts_tensor(starts, rows: int, q_tokens: int, max_seq_len: int, dev) -> torch.Tensor:
     """Per-row cache position of the chunk's own keys as the int32 device
     tensor the attention kernel reads; host values are range-checked here."""
@@ -654,16 +678,18 @@ class LayerLauncher:
                           tuple(v_cache.stride()), global_end_index.data_ptr(), local_end_index.data_ptr())
         self.k_cache, self.v_cache = k_cache, v_cache
         self.lib = _capi.lib()
-        # The query is rotated where it is consumed, inside the attention kernel,
-        # so the append moves K and V only.  With the q / k norm folded into the
-        # append the append still reads q - the norm needs the sum of squares of
-        # whole tokens - but only leaves 1 / rms per token (``q_inv_rms``) for the
-        # attention kernel, which normalises and rotates.  On request
-        # (rope_in_attention=False) the append rotates q as well and hands the
-        # attention the rotated copy in ``roped_q``.
+        # Where the query is rotated.  rope_in_attention: where it is consumed,
+        # inside the attention kernel; the append then moves K and V only (and, with
+        # the q / k norm folded in, leaves 1 / rms per q token in ``q_inv_rms``).
+        # Otherwise (what RingKVPath does) by the append, which hands the attention
+        # the rotated copy: a third more bytes for the append, once per query and
+        # spread over the chip, against 3.5 us of table reads and double arithmetic
+        # at the start of every attention workgroup, once per key range of the query
+        # (whole layer call at 3120 queries x 12 heads against themselves: 103 -> 97 us;
+        # 1560 x 40 against 9360 keys: 332 -> 322 us).
         self.rope_in_attention = bool(rope_in_attention)
-        self.roped_q = None if self.rope_in_attention else torch.empty(
-            (rows, tokens, heads, HEAD_DIM), dtype=torch.bfloat16, device=dev)
+        self._roped = None                           # the scratch the last call's rotated query went to
+        self.roped_elems = rows * tokens * heads * HEAD_DIM
         self.q_inv_rms = torch.empty((rows, tokens), dtype=torch.float32, device=dev) \
             if self.rope_in_attention and qk_norm is not None else None
         self.sf = (C.c_int64 * rows)()
@@ -674,9 +700,10 @@ class LayerLauncher:
         ap = _capi.AppendParams()
         ap.k_in_stride = _stride3(k_like, "k")
         ap.v_in_stride = _stride3(v_like, "v")
+        roped_stride = _capi.Stride3(tokens * heads * HEAD_DIM, heads * HEAD_DIM, HEAD_DIM)
         if not self.rope_in_attention:
             ap.q_in_stride = _stride3(q_like, "q")
-            ap.q_out, ap.q_out_stride = self.roped_q.data_ptr(), _stride3(self.roped_q, "q_out")
+            ap.q_out_stride = roped_stride
         elif self.q_inv_rms is not None:
             ap.q_in_stride = _stride3(q_like, "q")
             ap.q_inv_rms = self.q_inv_rms.data_ptr()
@@ -710,7 +737,7 @@ class LayerLauncher:
             if self.q_inv_rms is not None:
                 at.q_norm_weight, at.q_inv_rms = qk_norm[0].data_ptr(), self.q_inv_rms.data_ptr()
         else:
-            at.q, at.q_stride = self.roped_q.data_ptr(), _stride3(self.roped_q, "q")
+            at.q_stride = roped_stride
         at.k_cache, at.k_stride = k_cache.data_ptr(), _stride3(k_cache, "k_cache")
         at.v_cache, at.v_stride = v_cache.data_ptr(), _stride3(v_cache, "v_cache")
         at.rows, at.q_tokens, at.heads, at.head_dim = rows, tokens, heads, HEAD_DIM
@@ -757,7 +784,9 @@ class LayerLauncher:
             if self.q_inv_rms is not None:
                 ap.q_in = q.data_ptr()
         else:
+            self._roped = _roped_query_scratch(self.dev, self.roped_elems)
             ap.q_in = q.data_ptr()
+            ap.q_out = at.q = self._roped.data_ptr()
         stream = _stream_ptr(self.dev)
         ap.stream = stream
         span = plan.max_seq_len
@@ -779,6 +808,14 @@ class LayerLauncher:
         at.seq_lens = seq_lens.data_ptr() if seq_lens is not None else None
         at.stream = stream
         return out
+
+    @property
+    def roped_q(self) -> Optional[torch.Tensor]:
+        """The last call's rotated query (a scratch every layer on the stream
+        writes in turn: copy it), or None when the attention rotates it."""
+        if self._roped is None:
+            return None
+        return self._roped[:self.roped_elems].view(self.rows, self.tokens, self.heads, HEAD_DIM)
 
     def set_timers(self, append: Optional[KernelTimer] = None, attention: Optional[KernelTimer] = None) -> None:
         """Attach (or, with None, detach) kernel timers for the next launches."""
