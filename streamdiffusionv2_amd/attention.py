@@ -10,7 +10,6 @@ two HIP kernels and no device-to-host copy.
 """
 from __future__ import annotations
 
-import copy
 import time
 from typing import List, Optional
 
@@ -30,15 +29,25 @@ class WanRMSNorm(nn.Module):
         self.weight = nn.Parameter(torch.ones(dim))
 
     def forward(self, x):
-        if not torch.is_grad_enabled() and ops.rms_norm_supported(x, self.weight):
+        if not torch.is_grad_enabled():
             # one launch of the library's kernel (the bits of the expression below on the CPU)
             # instead of the seven kernels the expression becomes on the device
-            return ops.rms_norm(x, self.weight.detach(), self.eps)
+            out = ops.rms_norm_or_none(x, self.weight, self.eps)
+            if out is not None:
+                return out
         xf = x.float()
         return (xf * torch.rsqrt(xf.pow(2).mean(dim=-1, keepdim=True) + self.eps)).type_as(x) * self.weight
 
 
 _HOST_LIST_CACHE: dict = {}
+
+
+def _flat_list(t: torch.Tensor) -> list:
+    out = t.tolist()                      # (flattened as a list: a reshape first costs five times the reading)
+    dim = t.dim()
+    if dim == 2:
+        return [x for row in out for x in row]
+    return out if dim == 1 else t.reshape(-1).tolist()
 
 
 def _host_ints(value, slot: str, rows: Optional[int] = None) -> List[int]:
@@ -50,16 +59,16 @@ def _host_ints(value, slot: str, rows: Optional[int] = None) -> List[int]:
     ``kv_cache_starts`` that way (causal_stream_inference.py:268-269) - and is
     read every time."""
     if isinstance(value, torch.Tensor):
-        version = ring.tensor_version(value)
-        if value.device.type == "cpu" or version is None:
-            out = value.reshape(-1).tolist()
+        version = ring.tensor_version(value) if value.is_cuda else None
+        if version is None:
+            out = _flat_list(value)
         else:
-            stamp = (version, value.data_ptr(), tuple(value.shape))
+            stamp = (version, value.data_ptr(), value.shape)
             hit = _HOST_LIST_CACHE.get(slot)
             if hit is not None and hit[0] is value and hit[1] == stamp:
                 out = hit[2]
             else:
-                out = value.reshape(-1).tolist()
+                out = _flat_list(value)
                 _HOST_LIST_CACHE[slot] = (value, stamp, out)
     elif isinstance(value, (list, tuple)):
         out = list(value)
@@ -241,7 +250,7 @@ class RingKVPath:
         cache, the shapes, the grid or the norm weights change."""
         launcher = getattr(self, "_launcher", None)
         if launcher is None or not launcher.matches(q, k, v, kv_cache, table, qk_norm) \
-                or (launcher.ap.grid_f, launcher.ap.grid_h, launcher.ap.grid_w) != tuple(grid):
+                or launcher.grid != tuple(grid):
             launcher = ops.LayerLauncher(kv_cache["k"], kv_cache["v"], kv_cache["global_end_index"],
                                          kv_cache["local_end_index"], table, grid, q, k, v, qk_norm=qk_norm,
                                          rope_in_attention=False)
@@ -302,7 +311,7 @@ class RingKVPath:
 
         # Planning advances the host's ring state (queues, pass counter, index mirror) before the launches
         # are validated: a call that fails - a frame beyond the RoPE table, say - must leave it where it was.
-        undo = (copy.deepcopy(self._evict_idx), kv_cache.get("current_step"))
+        undo = ([list(queue) for queue in self._evict_idx], kv_cache.get("current_step"))
         try:
             # planned as if no row refreshed; _settle() corrects the host state later where one did
             plan = ring.plan_append(kv_cache, self._evict_idx, starts, q.shape[1], frame_tokens, self.sink_size)
@@ -501,7 +510,7 @@ class CausalWanSelfAttention(nn.Module, RingKVPath):
                 and self.num_heads <= 64:
             # the two RMSNorms run inside the append kernel
             q, k = q.view(b, s, n, d), k.view(b, s, n, d)
-            norm = (self.norm_q.weight.detach(), self.norm_k.weight.detach(), self.eps)
+            norm = (self.norm_q.weight, self.norm_k.weight, self.eps)
             out = self.attend(q, k, v, grid_sizes, freqs, kv_cache, current_start, qk_norm=norm)
         else:
             q = self.norm_q(q).view(b, s, n, d)

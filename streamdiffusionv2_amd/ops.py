@@ -24,7 +24,7 @@ def _require_gpu(*tensors: torch.Tensor) -> torch.device:
     for t in tensors:
         if t is None:
             continue
-        if t.device.type != "cuda":
+        if not t.is_cuda:
             raise RuntimeError(
                 "sdv2kv operators run on the GPU only (tensor on %s); there is no CPU path" % t.device
             )
@@ -42,11 +42,9 @@ def _stride3(t: torch.Tensor, name: str) -> _capi.Stride3:
 
 
 def _stream_ptr(dev: torch.device) -> int:
-    return torch.cuda.current_stream(dev).cuda_stream
-
-
-def _current_device_index() -> int:
-    return torch.cuda.current_device()
+    # (the handle itself; torch.cuda.current_stream() wraps it in an object first, three microseconds a call)
+    index = dev.index
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if index is None else index)
 
 
 class _NoSwitch:
@@ -81,7 +79,7 @@ def device_freqs(freqs: torch.Tensor, device: torch.device) -> torch.Tensor:
         version = freqs._version
     except RuntimeError:            # created under torch.inference_mode(): no edit counter
         version = None
-    key = (id(freqs), version, freqs.data_ptr(), str(device))
+    key = (id(freqs), version, freqs.data_ptr(), device)
     hit = _FREQS_CACHE.get(key)
     if hit is not None and hit[0] is freqs:
         return hit[1]
@@ -316,13 +314,13 @@ def reset_workspace_tickets(dev: torch.device) -> None:
             ws[:TICKET_BYTES].zero_()
 
 
-def _workspace(dev: torch.device, nbytes: int, pool: Optional[dict] = None) -> torch.Tensor:
+def _workspace(dev: torch.device, nbytes: int, pool: Optional[dict] = None, stream: Optional[int] = None) -> torch.Tensor:
     """Scratch for split-KV partials, one buffer per (device, stream), grown on
     demand and reused.  Calls on one stream run one after another, so they can
     share a buffer; calls on different streams may overlap in time and must not
     (their tickets and partial results would mix), so each stream gets its own."""
     pool = _WORKSPACES if pool is None else pool
-    key = (dev, _stream_ptr(dev))
+    key = (dev, _stream_ptr(dev) if stream is None else stream)
     ws = pool.get(key)
     if ws is None or ws.numel() < nbytes:
         ws = new_workspace(dev, nbytes)
@@ -333,11 +331,11 @@ def _workspace(dev: torch.device, nbytes: int, pool: Optional[dict] = None) -> t
 _ROPED_QUERIES: dict = {}
 
 
-def _roped_query_scratch(dev: torch.device, elems: int) -> torch.Tensor:
+def _roped_query_scratch(dev: torch.device, elems: int, stream: int) -> torch.Tensor:
     """Where a layer call's append leaves the rotated query for its attention:
     one bf16 buffer per (device, stream), grown on demand.  The two launches
     follow each other on the stream, so the layers of a model share it."""
-    key = (dev, _stream_ptr(dev))
+    key = (dev, stream)
     buf = _ROPED_QUERIES.get(key)
     if buf is None or buf.numel() < elems:
         buf = torch.empty(elems, dtype=torch.bfloat16, device=dev)
@@ -367,6 +365,43 @@ def chunk_starts_tensor(starts, rows: int, q_tokens: int, max_seq_len: int, dev)
         if x < 0 or x + q_tokens > max_seq_len:
             raise RuntimeError(f"chunk_key_start {x} puts the chunk outside the {max_seq_len}-key view")
     return torch.tensor([int(x) for x in starts], dtype=torch.int32).to(dev, non_blocking=True)
+
+
+# Descriptors of the attention calls seen, everything filled in that shapes, strides and dtypes decide: checking
+# and filling them costs more host time than the rest of a call, and a program has a handful of layouts.
+_ATTN_LAYOUTS: dict = {}
+_MAX_ATTN_LAYOUTS = 256
+
+
+def _attn_layout(q, k_cache, v_cache, out, num_splits: int, static_scratch: bool, rope: bool):
+    """(descriptor as bytes, workspace bytes it needs, rows, query tokens, heads, keys)."""
+    if q.dtype not in _DTYPES or k_cache.dtype != q.dtype or v_cache.dtype != q.dtype:
+        raise RuntimeError("swa_attention takes q and both caches in one dtype, bf16 or fp32; got %s/%s/%s"
+                           % (q.dtype, k_cache.dtype, v_cache.dtype))
+    fp32 = q.dtype == torch.float32
+    if fp32 and (rope or static_scratch):
+        raise RuntimeError("fp32 attention takes rotated queries (no rope=) and no static_scratch=")
+    rows, q_tokens, heads, _ = q.shape
+    if k_cache.shape[0] != rows or k_cache.shape[2] != heads or v_cache.shape != k_cache.shape:
+        raise RuntimeError(f"cache view {tuple(k_cache.shape)} / {tuple(v_cache.shape)} does not match q {tuple(q.shape)}")
+    lib = _capi.lib()
+    max_seq_len = k_cache.shape[1]
+    if fp32:
+        need = lib.sdv2_swa_attn_f32_workspace_bytes(rows, q_tokens, heads, max_seq_len)    # (it picks its own splits)
+    else:
+        if num_splits <= 0:
+            num_splits = lib.sdv2_swa_attn_default_splits(rows, q_tokens, heads, max_seq_len)
+        need = 0 if static_scratch else lib.sdv2_swa_attn_workspace_bytes(rows, q_tokens, heads, max_seq_len, num_splits)
+    p = _capi.AttnParams()
+    p.q_stride = _stride3(q, "q")
+    p.k_stride, p.v_stride = _stride3(k_cache, "k_cache"), _stride3(v_cache, "v_cache")
+    p.out_stride = _stride3(out, "out") if out is not None else \
+        _capi.Stride3(q_tokens * heads * HEAD_DIM, heads * HEAD_DIM, HEAD_DIM)
+    p.rows, p.q_tokens, p.heads, p.head_dim = rows, q_tokens, heads, HEAD_DIM
+    p.max_seq_len = max_seq_len
+    p.num_splits = num_splits
+    p.dtype = _DTYPES[q.dtype]
+    return bytes(p), need, rows, q_tokens, heads, max_seq_len
 
 
 def swa_attention(
@@ -410,50 +445,39 @@ def swa_attention(
     [start + (t // b + 1) * b, start + S).
     """
     dev = _require_gpu(q, k_cache, v_cache, seq_lens, out, workspace)
-    if q.dtype not in _DTYPES or k_cache.dtype != q.dtype or v_cache.dtype != q.dtype:
-        raise RuntimeError("swa_attention takes q and both caches in one dtype, bf16 or fp32; got %s/%s/%s"
-                           % (q.dtype, k_cache.dtype, v_cache.dtype))
-    fp32 = q.dtype == torch.float32
-    if fp32 and (rope is not None or static_scratch):
-        raise RuntimeError("fp32 attention takes rotated queries (no rope=) and no static_scratch=")
-    rows, q_tokens, heads, _ = q.shape
-    if k_cache.shape[0] != rows or k_cache.shape[2] != heads or v_cache.shape != k_cache.shape:
-        raise RuntimeError(f"cache view {tuple(k_cache.shape)} / {tuple(v_cache.shape)} does not match q {tuple(q.shape)}")
+    if out is not None and (out.dtype != q.dtype or out.shape != q.shape):
+        raise RuntimeError("out must have q's dtype and shape")
+    key = (q.shape, q.stride(), q.dtype, k_cache.shape, k_cache.stride(), k_cache.dtype, v_cache.shape, v_cache.stride(),
+           v_cache.dtype, None if out is None else out.stride(), num_splits, static_scratch, rope is None)
+    layout = _ATTN_LAYOUTS.get(key)
+    if layout is None:
+        layout = _attn_layout(q, k_cache, v_cache, out, num_splits, static_scratch, rope is not None)
+        if len(_ATTN_LAYOUTS) >= _MAX_ATTN_LAYOUTS:
+            _ATTN_LAYOUTS.clear()
+        _ATTN_LAYOUTS[key] = layout
+    template, need, rows, q_tokens, heads, max_seq_len = layout
     if seq_lens is not None and (seq_lens.dtype != torch.int32 or seq_lens.numel() != rows or not seq_lens.is_contiguous()):
         raise RuntimeError("seq_lens must be a contiguous int32 tensor with one entry per row")
     if out is None:
-        out = torch.empty((rows, q_tokens, heads, HEAD_DIM), dtype=q.dtype, device=dev)
-    elif out.dtype != q.dtype or tuple(out.shape) != tuple(q.shape):
-        raise RuntimeError("out must have q's dtype and shape")
+        out = torch.empty(q.shape, dtype=q.dtype, device=dev)
 
     lib = _capi.lib()
-    max_seq_len = k_cache.shape[1]
-    if fp32:
-        need = lib.sdv2_swa_attn_f32_workspace_bytes(rows, q_tokens, heads, max_seq_len)    # (it picks its own splits)
-    else:
-        if num_splits <= 0:
-            num_splits = lib.sdv2_swa_attn_default_splits(rows, q_tokens, heads, max_seq_len)
-        need = 0 if static_scratch else lib.sdv2_swa_attn_workspace_bytes(rows, q_tokens, heads, max_seq_len, num_splits)
+    stream = _stream_ptr(dev)
     if workspace is not None and not getattr(workspace, "_sdv2_workspace", False):
         raise RuntimeError("workspace= takes a buffer made by ops.new_workspace() (zero-filled ticket words)")
     if need and (workspace is None or workspace.numel() * workspace.element_size() < need):
-        workspace = _workspace(dev, need)
+        workspace = _workspace(dev, need, stream=stream)
 
-    p = _capi.AttnParams()
-    p.q, p.q_stride = q.data_ptr(), _stride3(q, "q")
-    p.k_cache, p.k_stride = k_cache.data_ptr(), _stride3(k_cache, "k_cache")
-    p.v_cache, p.v_stride = v_cache.data_ptr(), _stride3(v_cache, "v_cache")
-    p.out, p.out_stride = out.data_ptr(), _stride3(out, "out")
-    p.seq_lens = seq_lens.data_ptr() if seq_lens is not None else None
-    p.rows, p.q_tokens, p.heads, p.head_dim = rows, q_tokens, heads, HEAD_DIM
-    p.max_seq_len = max_seq_len
-    p.num_splits = num_splits
-    p.dtype = _DTYPES[q.dtype]
-    p.softmax_scale = float(softmax_scale) if softmax_scale else 0.0
+    p = _capi.AttnParams.from_buffer_copy(template)
+    p.q, p.k_cache, p.v_cache, p.out = q.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), out.data_ptr()
+    if seq_lens is not None:
+        p.seq_lens = seq_lens.data_ptr()
+    if softmax_scale:
+        p.softmax_scale = float(softmax_scale)
     if need:
         p.workspace = workspace.data_ptr()
         p.workspace_bytes = workspace.numel() * workspace.element_size()
-    p.stream = _stream_ptr(dev)
+    p.stream = stream
     if mask_block_tokens:
         chunk_key_start = chunk_starts_tensor(chunk_key_start, rows, q_tokens, max_seq_len, dev)
         p.mask_block_tokens = int(mask_block_tokens)
@@ -655,10 +679,6 @@ class LayerLauncher:
     built once per (cache, shape) and patched per call.
     """
 
-    @staticmethod
-    def _sig(t):
-        return (tuple(t.shape), tuple(t.stride()), t.dtype)
-
     def __init__(self, k_cache, v_cache, global_end_index, local_end_index, freqs_table, grid, q_like, k_like=None,
                  v_like=None, qk_norm=None, rope_in_attention=True):
         k_like = q_like if k_like is None else k_like
@@ -673,9 +693,11 @@ class LayerLauncher:
         dev = _require_gpu(k_cache, v_cache, global_end_index, local_end_index, freqs_table, q_like)
         self.dev = dev
         self.rows, self.tokens, self.heads = rows, tokens, heads
-        self.in_sig = (self._sig(q_like), self._sig(k_like), self._sig(v_like))
-        self.cache_sig = (k_cache.data_ptr(), v_cache.data_ptr(), tuple(k_cache.shape), tuple(k_cache.stride()),
-                          tuple(v_cache.stride()), global_end_index.data_ptr(), local_end_index.data_ptr())
+        self.in_shape = q_like.shape
+        self.in_strides = (q_like.stride(), k_like.stride(), v_like.stride())
+        self.cache_shape = k_cache.shape
+        self.cache_strides = (k_cache.stride(), v_cache.stride())
+        self.cache_ptrs = (k_cache.data_ptr(), v_cache.data_ptr(), global_end_index.data_ptr(), local_end_index.data_ptr())
         self.k_cache, self.v_cache = k_cache, v_cache
         self.lib = _capi.lib()
         # Where the query is rotated.  rope_in_attention: where it is consumed,
@@ -712,7 +734,7 @@ class LayerLauncher:
         ap.freqs, ap.freq_rows = freqs_table.data_ptr(), freqs_table.shape[0]
         ap.dtype = _capi.DTYPE_BF16
         ap.rows, ap.tokens, ap.heads, ap.head_dim = rows, tokens, heads, HEAD_DIM
-        ap.grid_f, ap.grid_h, ap.grid_w = (int(x) for x in grid)
+        self.grid = ap.grid_f, ap.grid_h, ap.grid_w = tuple(int(x) for x in grid)
         ap.cache_tokens = k_cache.shape[1]
         ap.start_frame = C.cast(self.sf, C.POINTER(C.c_int64))
         ap.dst_start = C.cast(self.ds, C.POINTER(C.c_int64))
@@ -720,11 +742,12 @@ class LayerLauncher:
         ap.local_end_index = local_end_index.data_ptr()
         ap.new_global_end = C.cast(self.ng, C.POINTER(C.c_int64))
         ap.new_local_end = C.cast(self.nl, C.POINTER(C.c_int64))
-        self.qk_norm = qk_norm
+        self.norm_args = None
         if qk_norm is not None:
             _check_norm(qk_norm, q_like.dtype, heads, dev)
-            ap.q_norm_weight, ap.k_norm_weight = qk_norm[0].data_ptr(), qk_norm[1].data_ptr()
-            ap.norm_eps = float(qk_norm[2])
+            self.norm_args = ap.q_norm_weight, ap.k_norm_weight, ap.norm_eps = \
+                qk_norm[0].data_ptr(), qk_norm[1].data_ptr(), float(qk_norm[2])
+            self.norm_weights = qk_norm[:2]          # held: the descriptor keeps their addresses
         self.ap, self.ap_ref = ap, C.byref(ap)
         self.freqs_table = freqs_table
 
@@ -735,7 +758,7 @@ class LayerLauncher:
             at.rope_grid_h, at.rope_grid_w = int(grid[1]), int(grid[2])
             at.rope_start_frame = C.cast(self.sf, C.POINTER(C.c_int64))
             if self.q_inv_rms is not None:
-                at.q_norm_weight, at.q_inv_rms = qk_norm[0].data_ptr(), self.q_inv_rms.data_ptr()
+                at.q_norm_weight, at.q_inv_rms = self.norm_args[0], self.q_inv_rms.data_ptr()
         else:
             at.q_stride = roped_stride
         at.k_cache, at.k_stride = k_cache.data_ptr(), _stride3(k_cache, "k_cache")
@@ -744,22 +767,22 @@ class LayerLauncher:
         self.at, self.at_ref = at, C.byref(at)
         self.span = -1
         self.workspace_need = 0
-        self.out_stride = None
+        at.out_stride = roped_stride                 # contiguous, like the rotated query
         self.forced_splits = 0                       # 0 = the library's own choice
         self.timers = (None, None)
 
     def matches(self, q, k, v, kv_cache, freqs_table, qk_norm=None) -> bool:
-        if (self._sig(q), self._sig(k), self._sig(v)) != self.in_sig or freqs_table is not self.freqs_table:
+        shape, strides, bf16 = self.in_shape, self.in_strides, torch.bfloat16
+        if freqs_table is not self.freqs_table or q.shape != shape or k.shape != shape or v.shape != shape \
+                or q.stride() != strides[0] or k.stride() != strides[1] or v.stride() != strides[2] \
+                or q.dtype != bf16 or k.dtype != bf16 or v.dtype != bf16:
             return False
-        if (qk_norm is None) != (self.qk_norm is None):
-            return False
-        if qk_norm is not None and (qk_norm[0].data_ptr() != self.qk_norm[0].data_ptr()
-                                    or qk_norm[1].data_ptr() != self.qk_norm[1].data_ptr()
-                                    or float(qk_norm[2]) != float(self.qk_norm[2])):
+        if self.norm_args != (None if qk_norm is None else (qk_norm[0].data_ptr(), qk_norm[1].data_ptr(), qk_norm[2])):
             return False
         kc, vc = kv_cache["k"], kv_cache["v"]
-        return self.cache_sig == (kc.data_ptr(), vc.data_ptr(), tuple(kc.shape), tuple(kc.stride()), tuple(vc.stride()),
-                                  kv_cache["global_end_index"].data_ptr(), kv_cache["local_end_index"].data_ptr())
+        return self.cache_ptrs == (kc.data_ptr(), vc.data_ptr(), kv_cache["global_end_index"].data_ptr(),
+                                   kv_cache["local_end_index"].data_ptr()) \
+            and kc.shape == self.cache_shape and (kc.stride(), vc.stride()) == self.cache_strides
 
     def patch(self, q, k, v, start_frames, plan, seq_lens: Optional[torch.Tensor] = None,
               mask_block_tokens: int = 0, dst_start_override: Optional[torch.Tensor] = None) -> torch.Tensor:
@@ -773,22 +796,21 @@ class LayerLauncher:
         if mask_block_tokens:
             self.chunk_starts = chunk_starts_tensor(plan.dst_start, self.rows, self.tokens, plan.max_seq_len, self.dev)
             at.chunk_key_start = self.chunk_starts.data_ptr()
-        for i in range(self.rows):
-            self.sf[i] = start_frames[i]
-            self.ds[i] = plan.dst_start[i]
-            self.ng[i] = plan.new_global_end[i]
-            self.nl[i] = plan.new_local_end[i]
+        self.sf[:] = start_frames
+        self.ds[:] = plan.dst_start
+        self.ng[:] = plan.new_global_end
+        self.nl[:] = plan.new_local_end
         ap.k_in, ap.v_in = k.data_ptr(), v.data_ptr()
+        stream = _stream_ptr(self.dev)
         if self.rope_in_attention:
             at.q = q.data_ptr()
             if self.q_inv_rms is not None:
                 ap.q_in = q.data_ptr()
         else:
-            self._roped = _roped_query_scratch(self.dev, self.roped_elems)
+            self._roped = roped = _roped_query_scratch(self.dev, self.roped_elems, stream)
             ap.q_in = q.data_ptr()
-            ap.q_out = at.q = self._roped.data_ptr()
-        stream = _stream_ptr(self.dev)
-        ap.stream = stream
+            ap.q_out = at.q = roped.data_ptr()
+        ap.stream = at.stream = stream
         span = plan.max_seq_len
         if span != self.span:
             self.span = span
@@ -798,15 +820,12 @@ class LayerLauncher:
             self.workspace_need = self.lib.sdv2_swa_attn_workspace_bytes(self.rows, self.tokens, self.heads, span,
                                                                          at.num_splits)
         if self.workspace_need:
-            ws = _workspace(self.dev, self.workspace_need)      # this stream's; may have been regrown by another shape
+            # this stream's; may have been regrown by another shape
+            ws = _workspace(self.dev, self.workspace_need, stream=stream)
             at.workspace, at.workspace_bytes = ws.data_ptr(), ws.numel()
-        out = torch.empty((self.rows, self.tokens, self.heads, HEAD_DIM), dtype=torch.bfloat16, device=self.dev)
-        if self.out_stride is None:
-            self.out_stride = _stride3(out, "out")
-            at.out_stride = self.out_stride
+        out = torch.empty(self.in_shape, dtype=torch.bfloat16, device=self.dev)
         at.out = out.data_ptr()
         at.seq_lens = seq_lens.data_ptr() if seq_lens is not None else None
-        at.stream = stream
         return out
 
     @property
@@ -836,11 +855,7 @@ class LayerLauncher:
         """Append + attention for one call; returns the attention output
         [rows, S, H, 128]."""
         out = self.patch(q, k, v, start_frames, plan, seq_lens, mask_block_tokens, dst_start_override)
-        if _current_device_index() != self.dev.index:
-            with torch.cuda.device(self.dev):
-                self.run_append()
-                self.run_attention()
-        else:
+        with _on_device(self.dev):
             self.run_append()
             self.run_attention()
         return out
@@ -881,10 +896,15 @@ def flash_attention(q, k, v, q_lens=None, k_lens=None, dropout_p=0.0, softmax_sc
                 (softmax_scale if softmax_scale is not None else HEAD_DIM ** -0.5)
     if k_lens is not None:
         k_lens = k_lens.to(device=q.device, dtype=torch.int32).contiguous()
-    qb, kb, vb = (t if t.dtype == torch.bfloat16 else t.to(torch.bfloat16) for t in (q, k, v))
-    if qb.stride(-1) != 1:
-        qb = qb.contiguous()
-    out = swa_attention(qb, kb, vb, k_lens, softmax_scale=scale)
+    if out_dtype != torch.bfloat16:
+        q = q.to(torch.bfloat16)
+    if k.dtype != torch.bfloat16:
+        k = k.to(torch.bfloat16)
+    if v.dtype != torch.bfloat16:
+        v = v.to(torch.bfloat16)
+    if q.stride(-1) != 1:
+        q = q.contiguous()
+    out = swa_attention(q, k, v, k_lens, softmax_scale=scale)
     return out if out_dtype == torch.bfloat16 else out.to(out_dtype)
 
 
@@ -933,6 +953,8 @@ def _norm_rows(t: torch.Tensor):
     """(rows, elements between rows) of a tensor [..., width] whose rows are
     contiguous and evenly spaced, else None."""
     width = t.shape[-1]
+    if t.is_contiguous():
+        return t.numel() // width, width
     if width > 1 and t.stride(-1) != 1:
         return None
     rows = t.numel() // width
@@ -952,15 +974,28 @@ def _norm_rows(t: torch.Tensor):
     return rows, step
 
 
+def _norm_input(x: torch.Tensor, weight: torch.Tensor):
+    """:func:`_norm_rows` of x if :func:`rms_norm` can take it, else None."""
+    width = x.shape[-1] if x.dim() else 0
+    if not (x.is_cuda and x.dtype in _DTYPES and weight.dtype == x.dtype and weight.device == x.device
+            and width > 0 and width % HEAD_DIM == 0 and width // HEAD_DIM <= 64 and weight.numel() == width
+            and weight.is_contiguous() and x.data_ptr() % 16 == 0 and weight.data_ptr() % 16 == 0):
+        return None
+    return _norm_rows(x)
+
+
 def rms_norm_supported(x: torch.Tensor, weight: torch.Tensor) -> bool:
     """Can :func:`rms_norm` take this input?  (A device tensor of a dtype the
     library knows; rows of a multiple of 128 up to 8192 contiguous elements, 16-byte
     aligned and evenly spaced; a contiguous weight of the same dtype.)"""
-    width = x.shape[-1] if x.dim() else 0
-    return (x.is_cuda and x.dtype in _DTYPES and weight.dtype == x.dtype and weight.device == x.device
-            and width > 0 and width % HEAD_DIM == 0 and width // HEAD_DIM <= 64 and weight.numel() == width
-            and weight.is_contiguous() and x.data_ptr() % 16 == 0 and weight.data_ptr() % 16 == 0
-            and _norm_rows(x) is not None)
+    return _norm_input(x, weight) is not None
+
+
+def rms_norm_or_none(x: torch.Tensor, weight: torch.Tensor, eps: float) -> Optional[torch.Tensor]:
+    """:func:`rms_norm`, or None for an input it does not take."""
+    rows = _norm_input(x, weight)
+    return None if rows is None else _launch_norm(x, weight, eps, torch.empty(x.shape, dtype=x.dtype, device=x.device),
+                                                  rows, x.shape[-1])
 
 
 def rms_norm(x: torch.Tensor, weight: torch.Tensor, eps: float, out: Optional[torch.Tensor] = None) -> torch.Tensor:
@@ -971,24 +1006,25 @@ def rms_norm(x: torch.Tensor, weight: torch.Tensor, eps: float, out: Optional[to
     elements, a common distance apart); ``out`` defaults to a new contiguous
     tensor and may be x itself."""
     dev = _require_gpu(x, weight)
-    if not rms_norm_supported(x, weight):
+    x_rows = _norm_input(x, weight)
+    if x_rows is None:
         raise RuntimeError(f"rms_norm takes bf16 / fp32 rows of a multiple of 128 up to 8192 contiguous, 16-byte aligned, "
                            f"evenly spaced elements with a contiguous weight of the same dtype and width, got x "
                            f"{tuple(x.shape)} {x.dtype} strides {x.stride()}, weight {tuple(weight.shape)} {weight.dtype}")
-    width = x.shape[-1]
-    tokens, x_step = _norm_rows(x)
     if out is None:
         out = torch.empty(x.shape, dtype=x.dtype, device=dev)
     elif out.shape != x.shape or out.dtype != x.dtype or out.device != dev:
         raise RuntimeError("out must have x's shape, dtype and device")
-    rows = _norm_rows(out)
-    if rows is None or out.data_ptr() % 16:
+    out_rows = _norm_rows(out)
+    if out_rows is None or out.data_ptr() % 16:
         raise RuntimeError("out: rows must be contiguous, 16-byte aligned and evenly spaced")
-    p = _capi.RmsNormParams()
-    p.x, p.out, p.weight = x.data_ptr(), out.data_ptr(), weight.data_ptr()
-    p.x_token_stride, p.out_token_stride = x_step, rows[1]
-    p.tokens, p.width, p.dtype, p.eps = tokens, width, _DTYPES[x.dtype], float(eps)
-    p.stream = _stream_ptr(dev)
+    return _launch_norm(x, weight, eps, out, x_rows, out_rows[1])
+
+
+def _launch_norm(x, weight, eps, out, x_rows, out_step):
+    dev = x.device
+    p = _capi.RmsNormParams(x.data_ptr(), out.data_ptr(), weight.data_ptr(), x_rows[1], out_step, x_rows[0], x.shape[-1],
+                            _DTYPES[x.dtype], eps, _stream_ptr(dev))
     with _on_device(dev):
         _capi.check(_capi.lib().sdv2_rms_norm(C.byref(p)), "sdv2_rms_norm")
     return out
