@@ -357,8 +357,10 @@ class RingKVPath:
                 launcher = self._layer_launcher(q, k, v, kv_cache, table, (f, h, w), qk_norm)
                 start_frames = [c // frame_tokens for c in starts]
                 out = launcher.launch(q, k, v, start_frames, plan, seq, mask_tokens, override)
+                # (not held from call to call: the allocator hands the memory to the next layer)
+                roped_q, launcher.roped_q = launcher.roped_q, None
                 if return_roped_query:
-                    return out, launcher.roped_q.clone()
+                    return out, roped_q
                 return out
 
             roped_q = ops.kv_append_rope(

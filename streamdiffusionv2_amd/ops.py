@@ -328,27 +328,12 @@ def _workspace(dev: torch.device, nbytes: int, pool: Optional[dict] = None, stre
     return ws
 
 
-_ROPED_QUERIES: dict = {}
-
-
-def _roped_query_scratch(dev: torch.device, elems: int, stream: int) -> torch.Tensor:
-    """Where a layer call's append leaves the rotated query for its attention:
-    one bf16 buffer per (device, stream), grown on demand.  The two launches
-    follow each other on the stream, so the layers of a model share it."""
-    key = (dev, stream)
-    buf = _ROPED_QUERIES.get(key)
-    if buf is None or buf.numel() < elems:
-        buf = torch.empty(elems, dtype=torch.bfloat16, device=dev)
-        _ROPED_QUERIES[key] = buf
-    return buf
-
-
 def release_scratch() -> None:
     """Give back the scratch buffers kept per (device, stream): split-KV and
-    sink-similarity workspaces, rotated queries.  Calls already enqueued keep
-    what they use until the stream is past them (the allocator's own rule); not
-    for programs that still replay graphs captured over these calls."""
-    for pool in (_WORKSPACES, _SIM_WORKSPACES, _ROPED_QUERIES):
+    sink-similarity workspaces.  Calls already enqueued keep what they use until
+    the stream is past them (the allocator's own rule); not for programs that
+    still replay graphs captured over these calls."""
+    for pool in (_WORKSPACES, _SIM_WORKSPACES):
         pool.clear()
 
 
@@ -710,8 +695,10 @@ class LayerLauncher:
         # (whole layer call at 3120 queries x 12 heads against themselves: 103 -> 97 us;
         # 1560 x 40 against 9360 keys: 332 -> 322 us).
         self.rope_in_attention = bool(rope_in_attention)
-        self._roped = None                           # the scratch the last call's rotated query went to
-        self.roped_elems = rows * tokens * heads * HEAD_DIM
+        # The rotated query of the last patched call, a tensor of that call's own: a second thread
+        # may append on the same stream between this call's two launches, and a graph that captured
+        # them keeps the memory in its pool.  (None when the attention rotates.)
+        self.roped_q = None
         self.q_inv_rms = torch.empty((rows, tokens), dtype=torch.float32, device=dev) \
             if self.rope_in_attention and qk_norm is not None else None
         self.sf = (C.c_int64 * rows)()
@@ -807,9 +794,9 @@ class LayerLauncher:
             if self.q_inv_rms is not None:
                 ap.q_in = q.data_ptr()
         else:
-            self._roped = roped = _roped_query_scratch(self.dev, self.roped_elems, stream)
+            self.roped_q = torch.empty(self.in_shape, dtype=torch.bfloat16, device=self.dev)
             ap.q_in = q.data_ptr()
-            ap.q_out = at.q = roped.data_ptr()
+            ap.q_out = at.q = self.roped_q.data_ptr()
         ap.stream = at.stream = stream
         span = plan.max_seq_len
         if span != self.span:
@@ -827,14 +814,6 @@ class LayerLauncher:
         at.out = out.data_ptr()
         at.seq_lens = seq_lens.data_ptr() if seq_lens is not None else None
         return out
-
-    @property
-    def roped_q(self) -> Optional[torch.Tensor]:
-        """The last call's rotated query (a scratch every layer on the stream
-        writes in turn: copy it), or None when the attention rotates it."""
-        if self._roped is None:
-            return None
-        return self._roped[:self.roped_elems].view(self.rows, self.tokens, self.heads, HEAD_DIM)
 
     def set_timers(self, append: Optional[KernelTimer] = None, attention: Optional[KernelTimer] = None) -> None:
         """Attach (or, with None, detach) kernel timers for the next launches."""

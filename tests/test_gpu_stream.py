@@ -199,6 +199,34 @@ def test_kernel_timers_measure_each_kernel(gpu_device):
         t.close()
 
 
+def test_two_layer_calls_may_interleave_on_one_stream(gpu_device):
+    """Two threads on one stream can enqueue their layers' launches in any
+    order (the library releases the interpreter while it launches): append,
+    append, attention, attention gives what the calls give one after another."""
+    from streamdiffusionv2_amd import ops, ring, rope
+
+    heads, grid, S, cap = 2, (1, 8, 16), 128, 512
+    table = ops.device_freqs(rope.build_freqs(), gpu_device)
+    plan = ring.AppendPlan([3 * S], [11 * S], [cap])
+    calls, want = [], []
+    for seed in range(2):
+        gen = torch.Generator(device=gpu_device).manual_seed(seed)
+        cache = ring.new_kv_cache(1, 1, cap, heads, 1, device=gpu_device)[0]
+        for name in ("k", "v"):
+            cache[name].normal_(generator=gen)
+        qkv = [torch.randn(1, S, heads, 128, device=gpu_device, generator=gen).bfloat16() for _ in range(3)]
+        launcher = ops.LayerLauncher(cache["k"], cache["v"], cache["global_end_index"], cache["local_end_index"],
+                                     table, grid, *qkv, rope_in_attention=False)
+        want.append(launcher.launch(*qkv, [10], plan).clone())
+        calls.append((launcher, qkv))
+    outs = [launcher.patch(*qkv, [10], plan) for launcher, qkv in calls]
+    for step in ("run_append", "run_attention"):
+        for launcher, _ in calls:
+            getattr(launcher, step)()
+    for got, ref in zip(outs, want):
+        assert torch.equal(_bits(got), _bits(ref))
+
+
 def test_layer_call_replays_from_a_hip_graph(gpu_device):
     """The library neither allocates nor synchronises, so a layer call (append,
     split attention, merge) can be captured into a HIP graph.  A captured call
