@@ -969,20 +969,63 @@ bool decode_splits(int32_t encoded, int32_t rows, int32_t heads, SplitPlan* plan
   return plan->most() <= 64;
 }
 
+// What a call takes, in microseconds.
+//
+// The kernels of 256-row query tiles (one workgroup per CU): `base` ranges per (row, head), of every eighth of the
+// pairs `more` with one range more.  Workgroups cost their tiles of 64 keys and a start and end worth 4.25; handed
+// out longest first they end after `span` tile times.  A tile time is 1.18 us while half the CUs work and grows to
+// 1.56 when all do: the board's power is what they share.  Leaving partial results and combining them costs 4.1 us,
+// 5 more for a second batch of four ranges, and what the results move.  Fitted to 38 shapes with all their plans
+// (624 plans within 25 % of their shape's best: 5 % rms; the plan it picks costs 1 % more than the best one on
+// average, 8 % at worst.  A model without the power term took 6.4 % more at 3120 x 12 against themselves, 14 % at
+// 4 x 1024 x 12 against 6144 and 900 x 40 against 2700.)
+double tile_kernels_us(int32_t rows, int32_t q_tokens, int32_t heads, int32_t max_seq_len, int base, int more) {
+  constexpr double kStart = 4.25, kCall = 3.8, kTile = 1.18, kPower = 0.38, kFree = 0.54;
+  const int nq = (q_tokens + kQTile - 1) / kQTile, ntiles = (max_seq_len + kKTile - 1) / kKTile;
+  const int64_t pairs = (int64_t)rows * heads;
+  const double length = (ntiles + base - 1) / base + kStart;
+  double span, busy, ranges = base;              // busy: of the chip, in tile times
+  if (more == 0) {
+    const int64_t workgroups = pairs * nq * base;
+    span = (double)((workgroups + kCuSlots - 1) / kCuSlots) * length;
+    busy = workgroups * length / kCuSlots;
+  } else {
+    // Workgroups of two lengths, one XCD's share of them handed out as the dispatcher does: the next one, longest
+    // first, to the CU that is free first
+    constexpr int kCusPerXcd = kCuSlots / 8;
+    const int group = (int)(pairs / 8);
+    const double shorter = (ntiles + base) / (base + 1) + kStart;
+    double free_at[kCusPerXcd] = {};
+    auto hand_out = [&](int count, double x) {
+      for (int i = 0; i < count; ++i) {
+        int cu = 0;
+        for (int c = 1; c < kCusPerXcd; ++c)
+          if (free_at[c] < free_at[cu]) cu = c;
+        free_at[cu] += x;
+      }
+    };
+    const int n_long = (group - more) * nq * base, n_short = more * nq * (base + 1);
+    hand_out(n_long, length);
+    hand_out(n_short, shorter);
+    span = 0;
+    for (double t : free_at) span = t > span ? t : span;
+    busy = (n_long * length + n_short * shorter) / kCusPerXcd;
+    ranges += (double)more / group;
+  }
+  const double load = busy / span;
+  double us = kCall + span * (kTile + (load > kFree ? (load - kFree) / (1 - kFree) * kPower : 0));
+  if (base > 1 || more > 0)
+    us += 4.1 + (base + (more > 0) > 4 ? 5.0 : 0.0) + ranges * pairs * q_tokens * (kD * 2 * 0.14e-6);
+  return us;
+}
+
 }  // namespace
 
 extern "C" int sdv2_swa_attn_default_splits(int32_t rows, int32_t q_tokens, int32_t heads, int32_t max_seq_len) {
   if (rows <= 0 || q_tokens <= 0 || heads <= 0 || max_seq_len <= 0) return 1;
-  // One workgroup per CU.  With s key-range splits there are qwork * s
-  // workgroups; they run in ceil(qwork * s / 256) rounds, each as long as one
-  // workgroup's tile count plus a fixed start / end cost of about three tile
-  // times.  Writing and combining the partial results
-  // costs roughly one tile time per 3.5 MB of them per split.  Constants fitted
-  // to measurements on the five benchmark shapes.
   const int nq = (q_tokens + kQTile - 1) / kQTile;
   const int64_t pairs = (int64_t)rows * heads;
-  const int64_t qwork = pairs * nq;
-  if (qwork > kMaxTickets) return 1;
+  if (pairs * nq > kMaxTickets) return 1;
   // (the answer depends on the shape alone and costs a small simulation: the last one is remembered)
   static std::mutex lock;
   static int32_t last_shape[4] = {0, 0, 0, 0};
@@ -994,52 +1037,23 @@ extern "C" int sdv2_swa_attn_default_splits(int32_t rows, int32_t q_tokens, int3
       return last_answer;
   }
   const int ntiles = (max_seq_len + kKTile - 1) / kKTile;
-  const double partial_tiles = (double)rows * heads * q_tokens * kD * 4 / 7.0e6;
+  constexpr int kLeastTiles = 6;                 // of a range
+  auto us = [&](int base, int more) { return tile_kernels_us(rows, q_tokens, heads, max_seq_len, base, more); };
   int best = 1;
-  double best_cost = 1e300;
-  for (int sp = 1; sp <= 8; ++sp) {
-    const int per = (ntiles + sp - 1) / sp;
-    if (sp > 1 && per < 6) break;
-    const int64_t rounds = (qwork * sp + kCuSlots - 1) / kCuSlots;
-    const double cost = (double)rounds * (per + 3) + (sp > 1 ? sp * partial_tiles : 0.0);
-    if (cost < best_cost - 1e-9) { best_cost = cost; best = sp; }
+  double best_us = us(1, 0);
+  for (int base = 2; base <= 8 && (ntiles + base - 1) / base >= kLeastTiles; ++base) {
+    const double t = us(base, 0);
+    if (t < best_us) { best_us = t; best = base; }
   }
-  // A uniform count can leave the last round of workgroups mostly empty (1120
-  // workgroups are 4.4 rounds of 256).  When the (row, head) pairs divide over
-  // the eight XCDs, some pairs of each XCD's share may take one range more:
-  // workgroups of two lengths, the long ones dispatched first, fill the 32 CUs
-  // of an XCD more evenly.  Simulated as the dispatcher works (next workgroup
-  // to the CU that is free first); taken when it beats the best uniform count
-  // by 3 %.
-  if (pairs % 8 == 0 && pairs / 8 >= 2 && pairs / 8 <= 255) {
-    const int group = (int)(pairs / 8);
-    constexpr int kCusPerXcd = kCuSlots / 8;
-    double mixed_cost = 1e300;
-    int mixed = 0;
-    for (int sp = 1; sp <= 7; ++sp) {
-      const int per_lo = (ntiles + sp - 1) / sp, per_hi = (ntiles + sp) / (sp + 1);
-      if (per_hi < 6) break;
-      for (int more = 1; more < group; ++more) {
-        double busy[kCusPerXcd] = {};
-        auto hand_out = [&](int count, double length) {
-          for (int i = 0; i < count; ++i) {
-            int cu = 0;
-            for (int c = 1; c < kCusPerXcd; ++c)
-              if (busy[c] < busy[cu]) cu = c;
-            busy[cu] += length;
-          }
-        };
-        hand_out((group - more) * nq * sp, per_lo + 3);
-        hand_out(more * nq * (sp + 1), per_hi + 3);
-        double span = 0;
-        for (double b : busy) span = b > span ? b : span;
-        const double ranges = ((double)(group - more) * sp + (double)more * (sp + 1)) / group;
-        const double cost = span + ranges * partial_tiles;
-        if (cost < mixed_cost - 1e-9) { mixed_cost = cost; mixed = sp | (more << 8); }
+  // A uniform count can leave the last round of workgroups mostly empty (1120 workgroups are 4.4 rounds of 256).  When
+  // the (row, head) pairs divide over the eight XCDs, some pairs of each XCD's share may take one range more.  (Where
+  // that is a matter of one per cent, uniform ranges are taken.)
+  if (pairs % 8 == 0 && pairs / 8 >= 2 && pairs / 8 <= 255)
+    for (int base = 1; base <= 7 && (ntiles + base) / (base + 1) >= kLeastTiles; ++base)
+      for (int more = 1; more < (int)(pairs / 8); ++more) {
+        const double t = us(base, more);
+        if (t < best_us * ((best >> 8) ? 1.0 : 0.99)) { best_us = t; best = base | (more << 8); }
       }
-    }
-    if (mixed_cost < 0.97 * best_cost) best = mixed;
-  }
   std::lock_guard<std::mutex> guard(lock);
   last_shape[0] = rows; last_shape[1] = q_tokens; last_shape[2] = heads; last_shape[3] = max_seq_len;
   last_answer = best;
@@ -1167,8 +1181,8 @@ int attn_fwd(const sdv2_attn_params* p, void* workspace, size_t workspace_bytes)
     a.part_scale = reinterpret_cast<float*>(ws + w.part_scale);
   }
 
-  set_work_list(&a, kQTile);
   hipStream_t stream = static_cast<hipStream_t>(p->stream);
+  set_work_list(&a, kQTile);
   const int64_t nq_tiles = (p->q_tokens + kQTile - 1) / kQTile;
   const int64_t items = ((int64_t)p->rows * p->heads / plan.group) *
                         (nq_tiles * ((int64_t)(plan.group - plan.more) * plan.base + (int64_t)plan.more * (plan.base + 1)));
