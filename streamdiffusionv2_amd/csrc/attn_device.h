@@ -12,6 +12,7 @@
 
 #include "sdv2kv.h"
 #include "sdv2kv_internal.h"
+#include "rope_device.h"
 
 namespace sdv2 {
 namespace attn {
@@ -22,6 +23,7 @@ typedef __attribute__((ext_vector_type(4))) short s16x4;
 typedef __attribute__((ext_vector_type(8))) short s16x8;
 typedef __attribute__((ext_vector_type(16))) float f32x16;
 typedef __attribute__((ext_vector_type(2))) float f32x2;
+typedef __attribute__((ext_vector_type(4))) float f32x4;
 typedef __attribute__((ext_vector_type(4))) uint32_t u32x4;
 typedef __attribute__((ext_vector_type(2))) uint32_t u32x2;
 typedef __attribute__((ext_vector_type(2))) _Float16 f16x2;
@@ -292,6 +294,48 @@ __device__ __forceinline__ int64_t row_start_frame(const AttnKernelArgs& a, int 
   return frame;
 }
 
+// ---- the 16x16x32 kernels ------------------------------------------------------
+// Where 16-byte chunk c of LDS row r (a key) is stored: position c ^ swz16(r).  A
+// linear map of the four low bits of r with two properties.  Its upper three bits
+// differ on any eight consecutive rows: a V read takes 8 keys x 32 bytes per half
+// wave.  And swz16(12) = 1: a 16-byte K read is served to lanes 0-3, 12-15 and 20-27
+// together (then 4-11, 16-19 and 28-31), that is, to keys 0-3 and 12-15 of one chunk
+// and 4-11 of the next, and those two sets of positions must not meet.  Measured: no
+// bank conflicts (with a swizzle that has the first property alone, 1.3 cycles per read).
+__device__ __forceinline__ int swz16(int r) { return (r & 3) << 1 | ((r >> 2 ^ r >> 3) & 1) << 3 | (r >> 3 & 1); }
+
+// over the four lanes that share a query column (lane, lane ^ 16, lane ^ 32, lane ^ 48)
+__device__ __forceinline__ float col_max(float x) {
+  x = half_max(x);
+  auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  return vmax(__uint_as_float(r[0]), __uint_as_float(r[1]));
+}
+__device__ __forceinline__ float col_sum(float x) {
+  x = half_sum(x);
+  auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+
+// One query row as the B operand of S^T = K Q^T: d-step ks takes the 8 elements
+// 32 ks + 8 g of the row.  The row is the query before rotation and is rotated
+// here, in the arithmetic of the append kernel, after the
+// RMSNorm of the raw projection when the norm's weight is given.
+__device__ __forceinline__ void load_query(const QueryRope& rope, const uint16_t* qp, int token, int g, bf16x8 (&qf)[4]) {
+  const int fi = token / rope.frame_tokens;
+  const int rem = token - fi * rope.frame_tokens;
+  const int hi = rem / rope.grid_w;
+  const int wi = rem - hi * rope.grid_w;
+  const int64_t frame = rope.start_frame + fi;
+#pragma unroll
+  for (int ks = 0; ks < 4; ++ks) {
+    double2 cs[4];
+    sdv2::load_rotation(rope.freqs, kD / 2, rope.split_t, rope.split_h, 4 * ks + g, frame, hi, wi, cs);
+    sdv2::Vec8<uint16_t> x = sdv2::Vec8<uint16_t>::load(qp + 32 * ks);
+    if (rope.norm_w) x = sdv2::normalise(x, rope.inv_rms, sdv2::Vec8<uint16_t>::load(rope.norm_w + 32 * ks));
+    qf[ks] = __builtin_bit_cast(bf16x8, sdv2::rotate(x, cs).raw);
+  }
+}
+
 // (the transfers take their base addresses from scalar registers: say so to the compiler)
 __device__ __forceinline__ const char* uniform_pointer(const void* ptr) {
   const uint64_t x = reinterpret_cast<uint64_t>(ptr);
@@ -354,6 +398,8 @@ inline void set_work_list(AttnKernelArgs* a, int q_tile_rows) {
 
 // the kernel on 16x16x32 matrix instructions (swa_attn_fwd_m16.hip)
 int launch_m16(const AttnKernelArgs& a, uint32_t workgroups, hipStream_t stream);
+// the kernel whose waves share the keys of one query block (swa_attn_fwd_wave.hip)
+int launch_wave(const AttnKernelArgs& a, uint32_t workgroups, hipStream_t stream);
 
 }  // namespace attn
 }  // namespace sdv2

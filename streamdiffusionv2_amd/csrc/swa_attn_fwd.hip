@@ -62,8 +62,6 @@ namespace {
 
 using namespace sdv2::attn;
 
-typedef __attribute__((ext_vector_type(4))) float f32x4;
-
 constexpr int kWaves = 8;                   // two waves per SIMD, one 32-row query block each
 constexpr int kThreads = kWaves * 64;
 // The global->LDS transfers of a tile are issued by the first wave of every
@@ -1019,6 +1017,15 @@ double tile_kernels_us(int32_t rows, int32_t q_tokens, int32_t heads, int32_t ma
   return us;
 }
 
+// The kernel whose workgroups are 32-row query blocks (swa_attn_fwd_wave.hip): 256 keys take 1.22 us, and up to 256
+// workgroups run at once.  Measured against the other kernels with their best splits: 256 x 12 against 512 keys 9.0
+// (17.0) us, 1536 keys 13.7 (21.6), 3072 keys 20.9 (27.4), 9360 keys 51.9 (44.8); 300 workgroups (780 x 12) against
+// 512 keys 16.3 (17.1), 1536 keys 25.7 (22.8); 588 workgroups against 512 keys 23.6 (17.5).
+double wave_kernel_us(int32_t rows, int32_t q_tokens, int32_t heads, int32_t max_seq_len) {
+  const int64_t workgroups = (int64_t)rows * heads * ((q_tokens + kQBlock - 1) / kQBlock);
+  return 2.4 + (double)((workgroups + kCuSlots - 1) / kCuSlots) * (4.6 + 1.22 * ((max_seq_len + 255) / 256));
+}
+
 }  // namespace
 
 extern "C" int sdv2_swa_attn_default_splits(int32_t rows, int32_t q_tokens, int32_t heads, int32_t max_seq_len) {
@@ -1054,6 +1061,7 @@ extern "C" int sdv2_swa_attn_default_splits(int32_t rows, int32_t q_tokens, int3
         const double t = us(base, more);
         if (t < best_us * ((best >> 8) ? 1.0 : 0.99)) { best_us = t; best = base | (more << 8); }
       }
+  if (wave_kernel_us(rows, q_tokens, heads, max_seq_len) < best_us) best = 1;        // (which attn_fwd then picks)
   std::lock_guard<std::mutex> guard(lock);
   last_shape[0] = rows; last_shape[1] = q_tokens; last_shape[2] = heads; last_shape[3] = max_seq_len;
   last_answer = best;
@@ -1182,13 +1190,19 @@ int attn_fwd(const sdv2_attn_params* p, void* workspace, size_t workspace_bytes)
   }
 
   hipStream_t stream = static_cast<hipStream_t>(p->stream);
+  // Which kernel, first: one key range, and few enough query blocks that the waves had better share those than the keys
+  if (splits == 1 && wave_kernel_us(p->rows, p->q_tokens, p->heads, p->max_seq_len) <
+                         tile_kernels_us(p->rows, p->q_tokens, p->heads, p->max_seq_len, 1, 0)) {
+    set_work_list(&a, kQBlock);
+    return sdv2::attn::launch_wave(a, 8u * (((uint32_t)a.total_items + 7u) / 8u), stream);
+  }
   set_work_list(&a, kQTile);
   const int64_t nq_tiles = (p->q_tokens + kQTile - 1) / kQTile;
   const int64_t items = ((int64_t)p->rows * p->heads / plan.group) *
                         (nq_tiles * ((int64_t)(plan.group - plan.more) * plan.base + (int64_t)plan.more * (plan.base + 1)));
   if (items > (1 << 28)) return SDV2_ERR_INVALID_ARG;
   dim3 grid((unsigned)(8 * ((items + 7) / 8)));
-  // Which kernel.  The one on 16x16x32 matrix instructions takes 1.51 us per 64-key tile of a full CU where this one
+  // Which of the other two.  The one on 16x16x32 matrix instructions takes 1.51 us per 64-key tile of a full CU where this one
   // takes 1.65, and a microsecond more to fill its deeper pipeline: they meet at 12 tiles (1536 queries x 40 heads,
   // one key range: 768 keys 30.5 against 30.7 us, 384 keys 22.1 against 21.3, 3072 keys 84.5 against 90.4).  The mask
   // inside the chunk costs the other kernel, whose lanes own two queries each, more than it gains.

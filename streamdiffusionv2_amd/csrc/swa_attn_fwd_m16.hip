@@ -40,14 +40,8 @@
 // rescaled.  A wave that finds a row sum outside [2^-100, 2^100] after its last
 // tile redoes its block with the running-maximum recurrence (exact_pass).
 //
-// LDS tile layout: row r (key) holds sixteen 16-byte chunks; chunk c is stored
-// at position c ^ swz16(r), a linear map of the four low bits of r with two
-// properties.  Its upper three bits differ on any eight consecutive rows: a V read
-// takes 8 keys x 32 bytes per half wave.  And swz16(12) = 1: a 16-byte K read is
-// served to lanes 0-3, 12-15 and 20-27 together (then 4-11, 16-19 and 28-31), that
-// is, to keys 0-3 and 12-15 of one chunk and 4-11 of the next, and those two sets of
-// positions must not meet.  Measured: no bank conflicts (with a swizzle that has the
-// first property alone, 1.3 cycles per read).
+// LDS tile layout: row r (key) holds sixteen 16-byte chunks; chunk c is stored at
+// position c ^ swz16(r) (attn_device.h).
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -62,8 +56,6 @@
 namespace {
 
 using namespace sdv2::attn;
-
-typedef __attribute__((ext_vector_type(4))) float f32x4;
 
 constexpr int kWaves = 8;
 constexpr int kThreads = kWaves * 64;
@@ -81,20 +73,6 @@ static_assert(kWaves * kStage16 <= kLdsFlags, "the epilogue stages in the tile b
 // relative to the first V buffer with the base folded into the address register.
 constexpr int kLdsBuf(int buf) { return buf * kTileBytes; }
 constexpr int kLdsVBase = kStages * kTileBytes;
-
-__device__ __forceinline__ int swz16(int r) { return (r & 3) << 1 | ((r >> 2 ^ r >> 3) & 1) << 3 | (r >> 3 & 1); }
-
-// over the four lanes that share a query column (lane, lane ^ 16, lane ^ 32, lane ^ 48)
-__device__ __forceinline__ float col_max(float x) {
-  x = half_max(x);
-  auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
-  return vmax(__uint_as_float(r[0]), __uint_as_float(r[1]));
-}
-__device__ __forceinline__ float col_sum(float x) {
-  x = half_sum(x);
-  auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
-  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
-}
 
 // The MFMAs of the fast pass are asm with the register class of every operand
 // named: scores feed the vector ALU and stay in VGPRs, the output tile and the
@@ -422,26 +400,6 @@ __device__ __forceinline__ void exact_pass(LaneConst& c, const bf16x8 (&qf)[2][4
       lacc[qt][0] = col_sum(l_run[qt]);
       c.neg_ref[qt] = -m_run[qt] * c.c2;
     }
-}
-
-// One query row as the B operand of S^T = K Q^T: d-step ks takes the 8 elements
-// 32 ks + 8 g of the row.  The row is the query before rotation and is rotated
-// here, in the arithmetic of the append kernel, after the
-// RMSNorm of the raw projection when the norm's weight is given.
-__device__ __forceinline__ void load_query(const QueryRope& rope, const uint16_t* qp, int token, int g, bf16x8 (&qf)[4]) {
-  const int fi = token / rope.frame_tokens;
-  const int rem = token - fi * rope.frame_tokens;
-  const int hi = rem / rope.grid_w;
-  const int wi = rem - hi * rope.grid_w;
-  const int64_t frame = rope.start_frame + fi;
-#pragma unroll
-  for (int ks = 0; ks < 4; ++ks) {
-    double2 cs[4];
-    sdv2::load_rotation(rope.freqs, kD / 2, rope.split_t, rope.split_h, 4 * ks + g, frame, hi, wi, cs);
-    sdv2::Vec8<uint16_t> x = sdv2::Vec8<uint16_t>::load(qp + 32 * ks);
-    if (rope.norm_w) x = sdv2::normalise(x, rope.inv_rms, sdv2::Vec8<uint16_t>::load(rope.norm_w + 32 * ks));
-    qf[ks] = __builtin_bit_cast(bf16x8, sdv2::rotate(x, cs).raw);
-  }
 }
 
 __global__ __launch_bounds__(kThreads, 1)

@@ -165,3 +165,44 @@ def test_the_same_promises_for_the_16x16_kernel(assembly_m16):
     assert not [l.strip() for l in hot if re.search(r"\bscratch_(load|store)", l)]
     counts = [int(x) for x in re.findall(r"\.vgpr_count:\s+(\d+)", "\n".join(assembly_m16))]
     assert len(counts) == 1 and counts[0] <= 256, counts
+
+
+@pytest.fixture(scope="module")
+def assembly_wave():
+    out = os.path.join(ROOT, "build", "isa_check")
+    os.makedirs(out, exist_ok=True)
+    path = os.path.join(out, "swa_attn_fwd_wave.s")
+    cmd = [build_ext.hipcc_path(), *build_ext.HIPCC_FLAGS, f"-I{os.path.join(ROOT, 'include')}", f"-I{build_ext.CSRC}",
+           "-S", "--cuda-device-only", str(build_ext.CSRC / "swa_attn_fwd_wave.hip"), "-o", path]
+    res = subprocess.run(cmd, capture_output=True, text=True)
+    assert res.returncode == 0, res.stderr[-2000:]
+    return open(path).read().split("\n")
+
+
+def test_nothing_touches_a_query_on_its_way(assembly_wave):
+    """The small-call kernel requests a rotated query ahead of its first keys and waits for both together: until the
+    first of those waits (or the one for waves without a key) no instruction may name the query's registers."""
+    starts = [i for i, l in enumerate(assembly_wave) if re.match(r"^_Z\S*swa_attn_fwd_wave_kernel\S*:", l)]
+    assert len(starts) == 4
+    checked = 0
+    for st in starts:
+        end = next(i for i in range(st, len(assembly_wave)) if assembly_wave[i].strip().startswith(".Lfunc_end"))
+        body = assembly_wave[st:end]
+        last = next((i for i, l in enumerate(body) if "Q requested" in l), None)
+        if last is None:
+            continue                              # (the variants that rotate the query load it in the ordinary way)
+        checked += 1
+        query = set()
+        for mn, ops in instructions(body[last - 7:last + 1]):
+            assert mn == "global_load_dwordx4"
+            query |= registers(ops[0])
+        assert len(query) == 32
+        # in the order of the text: up to the wait behind the first fragment reads' request
+        for mn, ops in instructions(body[last + 1:]):
+            if mn == "s_waitcnt" and ops[0].startswith("vmcnt(8)"):
+                break
+            assert not any(registers(o) & query for o in ops), (mn, ops)
+    assert checked == 2
+    counts = [int(x) for x in re.findall(r"\.vgpr_count:\s+(\d+)", "\n".join(assembly_wave))]
+    assert len(counts) == 4 and max(counts) <= 256, counts
+    assert not any(re.search(r"\bscratch_(load|store)", l) for l in assembly_wave)

@@ -435,3 +435,51 @@ def test_masked_attention_skips_hidden_tiles(gpu_device, frames, bt_frames):
                                     chunk_key_start=[start], mask_block_tokens=bt_frames * ft)
             torch.cuda.synchronize()
             _check(got.cpu(), want)
+
+
+# the kernel whose waves share the keys of one 32-query block takes unsplit calls of up to 256 such blocks, and some more
+@pytest.mark.parametrize("rows,S,H,L,seq,block", [
+    (1, 1, 1, 1, None, 0),                       # one query, one key
+    (2, 31, 2, 16, [15, 16], 0),                 # the second half of the block starts where the first does
+    (2, 33, 1, 40, [17, 31], 0),                 # ... and inside it; one row in the second query block
+    (3, 32, 1, 64, [32, 33, 0], 0),              # a whole block, one key more, no key at all
+    (1, 64, 3, 255, None, 0),                    # every wave has one block, the last moved down by a key
+    (2, 40, 2, 900, [257, 513], 0),              # some waves one block more than others
+    (1, 256, 32, 96, None, 0),                   # 256 workgroups, most waves without a block
+    (1, 257, 32, 96, None, 0),                   # 288: not this kernel
+    (1, 90, 2, 333, None, 30),                   # mask inside the chunk, blocks of a row's own length
+    (2, 96, 2, 512, [512, 470], 32),             # hidden blocks left out
+    (1, 120, 2, 120, None, 10),                  # against itself
+])
+@pytest.mark.parametrize("head_major", [True, False])
+def test_attention_of_small_calls(gpu_device, rows, S, H, L, seq, block, head_major):
+    """Against the fp32 oracle at the edges of key blocks, waves and query blocks; rows without a key are zero; and
+    again with scores of several hundred either way (largest scores that differ between waves by hundreds)."""
+    from streamdiffusionv2_amd import ops
+
+    torch.manual_seed(6)
+    lens = seq if seq is not None else [L] * rows
+    sl = torch.tensor(lens, dtype=torch.int32, device=gpu_device)
+    starts = [max(0, n - S) for n in lens]
+    mask = (starts, block) if block else ()
+    kw = dict(chunk_key_start=starts, mask_block_tokens=block) if block else {}
+    live = [i for i, n in enumerate(lens) if n]
+
+    def on_device(t):
+        return t.permute(0, 2, 1, 3).contiguous().to(gpu_device).permute(0, 2, 1, 3) if head_major else t.to(gpu_device)
+
+    for scale in (1.0, 30.0):
+        q, k, v = (torch.randn(rows, n, H, 128) for n in (S, L, L))
+        q[:, S // 2:] *= scale
+        for i, n in enumerate(lens):
+            k[i, n:], v[i, n:] = float("nan"), float("inf")          # nothing past the last key may count
+        q, k, v = q.bfloat16(), k.bfloat16(), v.bfloat16()
+        print(f"rows={rows} S={S} H={H} L={L} block={block} scale={scale}", flush=True)
+        got = ops.swa_attention(q.to(gpu_device), on_device(k), on_device(v), sl, num_splits=1, **kw).cpu()
+        for i in range(rows):
+            if i not in live:
+                assert not got[i].any()
+                continue
+            n = lens[i]
+            _check(got[i:i + 1], oracle.attention_fp32_reference(q[i:i + 1], k[i:i + 1, :n], v[i:i + 1, :n], [n],
+                                                                 *(([mask[0][i]], mask[1]) if mask else ())))
