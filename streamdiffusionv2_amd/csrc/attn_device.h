@@ -73,6 +73,7 @@ struct AttnKernelArgs {
   FastDiv div_group, div_q_tiles, div_splits, div_splits_more, div_heads;
   float scale_log2;            // softmax_scale * log2(e)
   int32_t mask_block_tokens;   // 0 = no mask inside the chunk
+  FastDiv div_mask_block;      // by mask_block_tokens
   const int32_t* chunk_start;  // device [rows]: cache position of the chunk's own first key
   // Split calls.  Partial results are kept per 32-row query block in the order
   // the registers hold them (see store_partial), q_blocks = ceil(q_tokens / 32).

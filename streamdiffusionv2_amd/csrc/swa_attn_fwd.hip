@@ -1145,6 +1145,7 @@ int attn_fwd(const sdv2_attn_params* p, void* workspace, size_t workspace_bytes)
     if (!p->chunk_key_start) return SDV2_ERR_INVALID_ARG;
     a.chunk_start = p->chunk_key_start;
     a.mask_block_tokens = p->mask_block_tokens;
+    a.div_mask_block = FastDiv::by((uint32_t)p->mask_block_tokens);
   }
 
   if (p->rope_freqs) {
@@ -1204,10 +1205,11 @@ int attn_fwd(const sdv2_attn_params* p, void* workspace, size_t workspace_bytes)
   dim3 grid((unsigned)(8 * ((items + 7) / 8)));
   // Which of the other two.  The one on 16x16x32 matrix instructions takes 1.51 us per 64-key tile of a full CU where this one
   // takes 1.65, and a microsecond more to fill its deeper pipeline: they meet at 12 tiles (1536 queries x 40 heads,
-  // one key range: 768 keys 30.5 against 30.7 us, 384 keys 22.1 against 21.3, 3072 keys 84.5 against 90.4).  The mask
-  // inside the chunk costs the other kernel, whose lanes own two queries each, more than it gains.
+  // one key range: 768 keys 30.5 against 30.7 us, 384 keys 22.1 against 21.3, 3072 keys 84.5 against 90.4).  With the
+  // mask inside the chunk likewise (3807 queries x 12 heads in blocks of 1269 against 11421 keys, the layer call: 264
+  // against 274 us).
   constexpr int kTilesForM16 = 12;
-  if (a.mask_block_tokens == 0 && (p->max_seq_len + kKTile - 1) / kKTile >= kTilesForM16 * plan.base)
+  if ((p->max_seq_len + kKTile - 1) / kKTile >= kTilesForM16 * plan.base)
     return sdv2::attn::launch_m16(a, grid.x, stream);
   // The tile buffers (96 KB) or the epilogue staging (16 KB per wave) exceed the static limit:
   // ask for the dynamic size once per device.

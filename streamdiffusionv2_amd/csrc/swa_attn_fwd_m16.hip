@@ -163,17 +163,32 @@ struct LaneConst {
   float c2;               // softmax scale * log2(e)
   float neg_ref[2];       // minus the query's exponent reference, in log2 units (0 until it is chosen)
   int g4;                 // 4 * (lane / 16)
+  // Block-causal mask inside the chunk: the chunk's own keys are [m_first, m_hi), blocks of m_block; a query sees the
+  // blocks up to its own.  m_lo: the first key hidden from the wave's first query (all wave-uniform; what a lane's own
+  // two queries see is worked out again in the few blocks that need it: registers are short).
+  int m_first, m_lo, m_hi, m_block, q_first;
+  FastDiv m_div;
 };
 
-// s[kt][qt]: scores of keys key0 + 16 kt + 4 g + i; those at or past the end of the valid keys count for nothing
+// s[kt][qt]: scores of keys key0 + 16 kt + 4 g + i; those at or past the end of the valid keys count for nothing, nor
+// do those the mask inside the chunk hides
+template <bool kMask>
 __device__ __forceinline__ void mask_block(f32x4 (&s)[2][2], const LaneConst& c, int key0, int seq) {
 #pragma unroll
-  for (int kt = 0; kt < 2; ++kt)
+  for (int qt = 0; qt < 2; ++qt) {
+    int m_lo = 0x7fffffff;
+    if constexpr (kMask) {
+      const int n16 = __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0)) & 15;
+      m_lo = c.m_first + (c.m_div(c.q_first + 16 * qt + n16) + 1) * c.m_block;
+    }
 #pragma unroll
-    for (int qt = 0; qt < 2; ++qt)
+    for (int kt = 0; kt < 2; ++kt)
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
-        if (key0 + 16 * kt + c.g4 + i >= seq) s[kt][qt][i] = -INFINITY;
+      for (int i = 0; i < 4; ++i) {
+        const int key = key0 + 16 * kt + c.g4 + i;
+        if (key >= seq || (kMask && key >= m_lo && key < c.m_hi)) s[kt][qt][i] = -INFINITY;
+      }
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -206,7 +221,7 @@ __device__ __forceinline__ u32x4 read_k(const LaneConst& c, int g) {
 }
 
 // kKNext / kVNext: where the coming slot reads; kNext false: there is none
-template <int kPar, int kKOff, int kVOff, int kKNext, int kVNext, bool kDoS, bool kDoPV, bool kDoSM, bool kNext>
+template <bool kMask, int kPar, int kKOff, int kVOff, int kKNext, int kVNext, bool kDoS, bool kDoPV, bool kDoSM, bool kNext>
 __device__ __forceinline__ void slot(const LaneConst& c, const bf16x8 (&qf)[2][4], f32x4 (&s)[2][2][2], u32x4 (&p)[2][2],
                                      f32x4 (&oacc)[8][2], f32x4 (&lacc)[2], Ahead& ahead, int key0, int key_end) {
   f32x4 (&s_cur)[2][2] = s[kPar];
@@ -220,11 +235,15 @@ __device__ __forceinline__ void slot(const LaneConst& c, const bf16x8 (&qf)[2][4
   }
 
   if constexpr (kDoSM) {
-    // The last, partial tile.  The test value goes through an empty asm so that the compiler cannot fold this
-    // uniform, rarely taken branch into the per-lane compares and hoist those.
+    // The last, partial tile, and blocks with hidden keys.  The test value goes through an empty asm so that the
+    // compiler cannot fold this uniform, rarely taken branch into the per-lane compares and hoist those.
     int masked = key0 + 32 - key_end;
+    if constexpr (kMask) {
+      const int into_hidden = key0 + 32 - c.m_lo < c.m_hi - key0 ? key0 + 32 - c.m_lo : c.m_hi - key0;
+      masked = masked > into_hidden ? masked : into_hidden;
+    }
     asm volatile("" : "+s"(masked));
-    if (masked > 0) mask_block(s_cur, c, key0, key_end);
+    if (masked > 0) mask_block<kMask>(s_cur, c, key0, key_end);
   }
   __builtin_amdgcn_sched_barrier(0);
 
@@ -311,11 +330,12 @@ __device__ __forceinline__ void slot(const LaneConst& c, const bf16x8 (&qf)[2][4
 // Conventional online softmax with a running maximum over the workgroup's key
 // range, tiles double-buffered.  Every wave keeps the tiles coming and meets the
 // barriers; only the waves whose fast result was unsafe redo their block.
+template <bool kMask, typename KeyOf>
 __device__ __forceinline__ void exact_pass(LaneConst& c, const bf16x8 (&qf)[2][4], f32x4 (&oacc)[8][2], f32x4 (&lacc)[2],
                                            bool compute, const char* kbase, const char* vbase,
                                            uint32_t k_tok_bytes, uint32_t v_tok_bytes, const uint32_t (&k_ld)[kPieces],
                                            const uint32_t (&v_ld)[kPieces], int tile_begin, int n, int seq,
-                                           uint32_t lds_addr0, int wave_u, int lane) {
+                                           KeyOf key0_of, uint32_t lds_addr0, int wave_u, int lane) {
   float m_run[2] = {-INFINITY, -INFINITY}, l_run[2] = {0.f, 0.f};
   if (compute) {
 #pragma unroll
@@ -325,7 +345,7 @@ __device__ __forceinline__ void exact_pass(LaneConst& c, const bf16x8 (&qf)[2][4
     }
   }
   auto issue = [&](int T) {
-    const int key0 = (tile_begin + T) * kKTile;
+    const int key0 = key0_of(tile_begin + T);
     issue_tile(kbase, k_tok_bytes, k_ld, key0, seq, lds_addr0 + kLdsBuf(T & 1), wave_u, lane);
     issue_tile(vbase, v_tok_bytes, v_ld, key0, seq, lds_addr0 + kLdsVBase + kLdsBuf(T & 1), wave_u, lane);
   };
@@ -342,7 +362,7 @@ __device__ __forceinline__ void exact_pass(LaneConst& c, const bf16x8 (&qf)[2][4
     __syncthreads();     // tile T has landed for every wave
     if (compute) {
       for (int kb = 0; kb < 2; ++kb) {             // 32 keys at a time
-        const int key0 = (tile_begin + T) * kKTile + 32 * kb;
+        const int key0 = key0_of(tile_begin + T) + 32 * kb;
         f32x4 s[2][2];
 #pragma unroll
         for (int kt = 0; kt < 2; ++kt) {
@@ -354,7 +374,7 @@ __device__ __forceinline__ void exact_pass(LaneConst& c, const bf16x8 (&qf)[2][4
             for (int qt = 0; qt < 2; ++qt) s[kt][qt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf, qf[qt][ks], s[kt][qt], 0, 0, 0);
           }
         }
-        if (key0 + 32 > seq) mask_block(s, c, key0, seq);
+        if (key0 + 32 > seq || (kMask && key0 + 32 > c.m_lo && key0 < c.m_hi)) mask_block<kMask>(s, c, key0, seq);
         u32x4 pf[2];
 #pragma unroll
         for (int qt = 0; qt < 2; ++qt) {
@@ -402,6 +422,7 @@ __device__ __forceinline__ void exact_pass(LaneConst& c, const bf16x8 (&qf)[2][4
     }
 }
 
+template <bool kMask>
 __global__ __launch_bounds__(kThreads, 1)
 void swa_attn_fwd_m16_kernel(const AttnKernelArgs a) {
   extern __shared__ __attribute__((aligned(1024))) char smem[];
@@ -422,10 +443,22 @@ void swa_attn_fwd_m16_kernel(const AttnKernelArgs a) {
   seq = seq < a.max_seq_len ? seq : a.max_seq_len;
   seq = seq < 0 ? 0 : seq;
   const int ntiles = (seq + kKTile - 1) / kKTile;
-  const int per_split = (ntiles + nsplits - 1) / nsplits;
+  // With the mask inside the chunk the tiles [hole, hole + skipped) hold nothing but keys that are hidden from
+  // every query of this workgroup (from the last one, that is): they are not streamed, and the key ranges are cut
+  // from what is left.
+  int hole = 0x7fffffff, skipped = 0;
+  if constexpr (kMask) {
+    const int first = a.chunk_start[row], bt = a.mask_block_tokens;
+    const int q_last = qtile * kQTile + kQTile < a.q_tokens ? qtile * kQTile + kQTile - 1 : a.q_tokens - 1;
+    const int lo = first + (a.div_mask_block(q_last) + 1) * bt, hi = first + a.q_tokens;
+    const int h0 = (lo + kKTile - 1) / kKTile, h1 = hi >= seq ? ntiles : hi / kKTile;
+    if (h1 > h0) { hole = h0; skipped = h1 - h0; }
+  }
+  auto key0_of = [=](int tile) { return (kMask && tile >= hole ? tile + skipped : tile) * kKTile; };
+  const int per_split = (ntiles - skipped + nsplits - 1) / nsplits;
   const int tile_begin = split * per_split;
   int tile_end = tile_begin + per_split;
-  tile_end = tile_end < ntiles ? tile_end : ntiles;
+  tile_end = tile_end < ntiles - skipped ? tile_end : ntiles - skipped;
   const int n = tile_end - tile_begin;       // tiles this workgroup streams
 
   const uint32_t lds_addr0 = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)lds);
@@ -444,10 +477,10 @@ void swa_attn_fwd_m16_kernel(const AttnKernelArgs a) {
   }
   // T is the tile index inside this workgroup's range
   auto issue_k = [&](int T, int buf) {
-    issue_tile(kbase, k_tok_bytes, k_ld, (tile_begin + T) * kKTile, seq, lds_addr0 + kLdsBuf(buf), wave_u, lane);
+    issue_tile(kbase, k_tok_bytes, k_ld, key0_of(tile_begin + T), seq, lds_addr0 + kLdsBuf(buf), wave_u, lane);
   };
   auto issue_v = [&](int T, int buf) {
-    issue_tile(vbase, v_tok_bytes, v_ld, (tile_begin + T) * kKTile, seq, lds_addr0 + kLdsVBase + kLdsBuf(buf), wave_u, lane);
+    issue_tile(vbase, v_tok_bytes, v_ld, key0_of(tile_begin + T), seq, lds_addr0 + kLdsVBase + kLdsBuf(buf), wave_u, lane);
   };
 
   // ---- this lane's two query rows, and the first tiles ------------------------
@@ -519,6 +552,14 @@ void swa_attn_fwd_m16_kernel(const AttnKernelArgs a) {
   c.c2 = a.scale_log2;
   c.neg_ref[0] = c.neg_ref[1] = 0.f;
   c.g4 = 4 * g;
+  if constexpr (kMask) {
+    c.m_block = a.mask_block_tokens;
+    c.m_div = a.div_mask_block;
+    c.q_first = qtile * kQTile + wave_u * kQBlock;
+    c.m_first = __builtin_amdgcn_readfirstlane(a.chunk_start[row]);
+    c.m_hi = c.m_first + a.q_tokens;
+    c.m_lo = __builtin_amdgcn_readfirstlane(c.m_first + (c.m_div(c.q_first) + 1) * c.m_block);
+  }
   {
     // K (A operand): key = lane%16 of the 16-key tile, chunk = 4*ks + g
     const int base = n16 * 256 + ((g ^ swz16(n16)) << 4);
@@ -559,7 +600,7 @@ void swa_attn_fwd_m16_kernel(const AttnKernelArgs a) {
   // the same code; scores of keys at or beyond the end of the range are masked to
   // -inf, so their weights are exact zeros against whatever finite data the
   // buffers still hold.
-  const int key_end = seq < tile_end * kKTile ? seq : tile_end * kKTile;
+  const int key_end = seq;
   Ahead ahead;
   auto land = [&](int T) {           // what must have landed by the barrier of tile T has
     if (T + 3 < n) {
@@ -572,13 +613,13 @@ void swa_attn_fwd_m16_kernel(const AttnKernelArgs a) {
   auto do_tile = [&](auto buf_c, int T) {
     constexpr int kB = decltype(buf_c)::value;              // T % kStages
     constexpr int kBNext = (kB + 1) % kStages, kBPrev = (kB + kStages - 1) % kStages;
-    const int key0 = (tile_begin + T) * kKTile;
-    slot<0, kLdsBuf(kB) + kHalf, kLdsBuf(kBPrev) + kHalf, kLdsBuf(kBNext), kLdsBuf(kB), true, true, true, true>(
+    const int key0 = key0_of(tile_begin + T);
+    slot<kMask, 0, kLdsBuf(kB) + kHalf, kLdsBuf(kBPrev) + kHalf, kLdsBuf(kBNext), kLdsBuf(kB), true, true, true, true>(
         c, qf, s, p, oacc, lacc, ahead, key0, key_end);
     land(T);
     if (T + 4 < n) issue_k(T + 4, kB);
     if (T + 3 < n) issue_v(T + 3, kBPrev);
-    slot<1, kLdsBuf(kBNext), kLdsBuf(kB), kLdsBuf(kBNext) + kHalf, kLdsBuf(kB) + kHalf, true, true, true, true>(
+    slot<kMask, 1, kLdsBuf(kBNext), kLdsBuf(kB), kLdsBuf(kBNext) + kHalf, kLdsBuf(kB) + kHalf, true, true, true, true>(
         c, qf, s, p, oacc, lacc, ahead, key0 + 32, key_end);
   };
   using B0 = std::integral_constant<int, 0>;
@@ -612,7 +653,7 @@ void swa_attn_fwd_m16_kernel(const AttnKernelArgs a) {
         ahead.k[g] = read_k<kLdsBuf(0)>(c, g);
         ahead.v[g] = read_v<kLdsBuf(kStages - 1) + kHalf>(c, g);
       }
-      slot<1, kLdsBuf(0), kLdsBuf(kStages - 1) + kHalf, kLdsBuf(0) + kHalf, kLdsBuf(kStages - 1) + kHalf, true, false, false, true>(
+      slot<kMask, 1, kLdsBuf(0), kLdsBuf(kStages - 1) + kHalf, kLdsBuf(0) + kHalf, kLdsBuf(kStages - 1) + kHalf, true, false, false, true>(
           c, qf, s, p, oacc, lacc, ahead, 0, key_end);
       mfma_drain<1>(oacc, s);
 #pragma unroll
@@ -650,7 +691,7 @@ void swa_attn_fwd_m16_kernel(const AttnKernelArgs a) {
         const uint32_t shift = (uint32_t)(((n - 1) % kStages - (kStages - 1)) * kTileBytes);
 #pragma unroll
         for (int db = 0; db < 8; ++db) c.v_addr[db] += shift;
-        slot<0, 0, kLdsBuf(kStages - 1) + kHalf, 0, 0, false, true, false, false>(
+        slot<kMask, 0, 0, kLdsBuf(kStages - 1) + kHalf, 0, 0, false, true, false, false>(
             c, qf, s, p, oacc, lacc, ahead, 0, key_end);
 #pragma unroll
         for (int db = 0; db < 8; ++db) c.v_addr[db] -= shift;
@@ -663,7 +704,14 @@ void swa_attn_fwd_m16_kernel(const AttnKernelArgs a) {
 #pragma unroll
       for (int qt = 0; qt < 2; ++qt) {
         const float l_tot = lacc[qt][0];
-        ok &= l_tot >= 0x1p-100f && l_tot <= 0x1p100f;
+        bool fine = l_tot >= 0x1p-100f && l_tot <= 0x1p100f;
+        if constexpr (kMask) {
+          // (zero is right where every key of this range is hidden from the query)
+          const int m_lo = c.m_first + (c.m_div(q_row + 16 * qt) + 1) * c.m_block;
+          const int last = key0_of(tile_end - 1) + kKTile;
+          fine |= l_tot == 0.f && key0_of(tile_begin) >= m_lo && (last < seq ? last : seq) <= c.m_hi;
+        }
+        ok &= fine;
       }
       unsafe = __builtin_amdgcn_ballot_w64(!ok) != 0;
     }
@@ -675,8 +723,8 @@ void swa_attn_fwd_m16_kernel(const AttnKernelArgs a) {
     __syncthreads();
     const int redo = flags[0];
     if (redo)
-      exact_pass(c, qf, oacc, lacc, unsafe, kbase, vbase, k_tok_bytes, v_tok_bytes, k_ld, v_ld, tile_begin, n,
-                 seq, lds_addr0, wave_u, lane);
+      exact_pass<kMask>(c, qf, oacc, lacc, unsafe, kbase, vbase, k_tok_bytes, v_tok_bytes, k_ld, v_ld, tile_begin, n,
+                 seq, key0_of, lds_addr0, wave_u, lane);
   }
 
   // ---- epilogue ---------------------------------------------------------------
@@ -856,11 +904,13 @@ int sdv2::attn::launch_m16(const AttnKernelArgs& a, uint32_t workgroups, hipStre
   int device = 0;
   if (hipGetDevice(&device) != hipSuccess || device < 0 || device >= kMaxDevices) return SDV2_ERR_LAUNCH;
   if (!lds_ready[device].load(std::memory_order_acquire)) {
-    if (hipFuncSetAttribute(reinterpret_cast<const void*>(swa_attn_fwd_m16_kernel),
-                            hipFuncAttributeMaxDynamicSharedMemorySize, kLdsBytes) != hipSuccess)
-      return SDV2_ERR_LAUNCH;
+    for (const void* kernel : {reinterpret_cast<const void*>(swa_attn_fwd_m16_kernel<false>),
+                               reinterpret_cast<const void*>(swa_attn_fwd_m16_kernel<true>)})
+      if (hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, kLdsBytes) != hipSuccess) return SDV2_ERR_LAUNCH;
     lds_ready[device].store(true, std::memory_order_release);
   }
-  sdv2::launch_timed(SDV2_KERNEL_ATTENTION, swa_attn_fwd_m16_kernel, dim3(workgroups), dim3(kThreads), kLdsBytes, stream, a);
+  auto launch = [&](auto kernel) { sdv2::launch_timed(SDV2_KERNEL_ATTENTION, kernel, dim3(workgroups), dim3(kThreads), kLdsBytes, stream, a); };
+  if (a.mask_block_tokens > 0) launch(swa_attn_fwd_m16_kernel<true>);
+  else launch(swa_attn_fwd_m16_kernel<false>);
   return hipGetLastError() == hipSuccess ? SDV2_OK : SDV2_ERR_LAUNCH;
 }

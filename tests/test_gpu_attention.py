@@ -483,3 +483,29 @@ def test_attention_of_small_calls(gpu_device, rows, S, H, L, seq, block, head_ma
             n = lens[i]
             _check(got[i:i + 1], oracle.attention_fp32_reference(q[i:i + 1], k[i:i + 1, :n], v[i:i + 1, :n], [n],
                                                                  *(([mask[0][i]], mask[1]) if mask else ())))
+
+
+@pytest.mark.parametrize("rows,S,H,L,block,splits,start", [
+    (1, 900, 2, 2400, 300, 3, 0),                # 12 tiles a range or more: the kernel on 16x16x32 matrix instructions
+    (1, 900, 2, 2400, 300, 3, 1501),             # the chunk is the last of the keys
+    (2, 333, 3, 1700, 37, 2, 700),               # blocks that end inside tiles, two rows
+    (1, 600, 15, 800, 200, 1, 130),              # unsplit: more query blocks than the kernel for small calls takes
+    (1, 320, 2, 2304, 64, 3, 1),                 # a range of which early queries see nothing but hidden keys
+])
+def test_masked_attention_on_16x16_matrix_instructions(gpu_device, rows, S, H, L, block, splits, start):
+    """Mask inside the chunk, whole tiles of hidden keys left out, against the fp32 oracle; and again with scores that
+    leave the range of the fixed-reference softmax."""
+    from streamdiffusionv2_amd import ops
+
+    torch.manual_seed(9)
+    start = min(start, L - S)
+    lens = [L] * rows
+    for scale in (1.0, 30.0):
+        q, k, v = (torch.randn(rows, n, H, 128) for n in (S, L, L))
+        q[:, S // 2:] *= scale
+        q, k, v = q.bfloat16(), k.bfloat16(), v.bfloat16()
+        print(f"rows={rows} S={S} H={H} L={L} block={block} splits={splits} scale={scale}", flush=True)
+        want = oracle.attention_fp32_reference(q, k, v, lens, [start] * rows, block)
+        got = ops.swa_attention(q.to(gpu_device), k.to(gpu_device), v.to(gpu_device), None, num_splits=splits,
+                                chunk_key_start=[start] * rows, mask_block_tokens=block)
+        _check(got.cpu(), want)
