@@ -159,7 +159,7 @@ constexpr int kNormMaxSteps = 16;           // heads <= 64
 constexpr int kNormWaves = 4;
 
 template <typename T, int kStepsPerWave, bool kWriteQ>
-__global__ __launch_bounds__(64 * kNormWaves)
+__global__ __launch_bounds__(64 * kNormWaves, sizeof(T) == 2 && kStepsPerWave <= 3 ? 4 : 2)
 void kv_append_norm_rope_kernel(const AppendKernelArgs a) {
 #pragma clang fp contract(off)
   const int lane = threadIdx.x & 63;
@@ -169,41 +169,39 @@ void kv_append_norm_rope_kernel(const AppendKernelArgs a) {
   const int tok = blockIdx.x;
   const int row = blockIdx.z;
 
-  if (blockIdx.x == 0 && threadIdx.x == 0) {
-    if (a.global_end) a.global_end[row] = a.new_global[row];
-    if (a.local_end) a.local_end[row] = a.new_local[row];
-  }
-
+  // Everything the token needs is asked for here, in one trip to memory: a load behind a store would wait for the
+  // store's acknowledgement as well (they share a counter), and one load per head step waited for where it is used
+  // was a trip per step.  Lanes whose head does not exist ask for the last one's and store nothing.
   const int64_t e0 = sub * 8;
-  const int64_t dst_tok = row_dst_start(a, row) + tok;
   const T* qi = static_cast<const T*>(a.q_in) + row * a.q_in_st.row + tok * a.q_in_st.token + e0;
   const T* ki = static_cast<const T*>(a.k_in) + row * a.k_in_st.row + tok * a.k_in_st.token + e0;
   const T* vi = static_cast<const T*>(a.v_in) + row * a.v_in_st.row + tok * a.v_in_st.token + e0;
-  T* kc = static_cast<T*>(a.k_cache) + row * a.k_st.row + dst_tok * a.k_st.token + e0;
-  T* vc = static_cast<T*>(a.v_cache) + row * a.v_st.row + dst_tok * a.v_st.token + e0;
+  const T* wqp = static_cast<const T*>(a.q_norm_w) + e0;
+  const T* wkp = static_cast<const T*>(a.k_norm_w) + e0;
   const int steps = (a.heads + 3) >> 2;
 
-  sdv2::Vec8<T> q[kStepsPerWave], k[kStepsPerWave];
+  sdv2::Vec8<T> q[kStepsPerWave], k[kStepsPerWave], v[kStepsPerWave], wq[kStepsPerWave], wk[kStepsPerWave];
 #pragma unroll
   for (int i = 0; i < kStepsPerWave; ++i) {
     const int j = wave + kNormWaves * i;
-    const int h = 4 * j + head_in_step;
-    if (j < steps && h < a.heads) {
-      q[i] = sdv2::Vec8<T>::load(qi + h * a.q_in_st.head);
-      k[i] = sdv2::Vec8<T>::load(ki + h * a.k_in_st.head);
-      sdv2::Vec8<T>::load(vi + h * a.v_in_st.head).store(vc + h * a.v_st.head);
+    const int h = 4 * j + head_in_step, hh = h < a.heads ? h : a.heads - 1;
+    if (j < steps) {                         // (wave-uniform)
+      k[i] = sdv2::Vec8<T>::load(ki + hh * a.k_in_st.head);
+      q[i] = sdv2::Vec8<T>::load(qi + hh * a.q_in_st.head);
+      v[i] = sdv2::Vec8<T>::load(vi + hh * a.v_in_st.head);
+      wk[i] = sdv2::Vec8<T>::load(wkp + hh * 128);
+      if constexpr (kWriteQ) wq[i] = sdv2::Vec8<T>::load(wqp + hh * 128);
     } else {
-      q[i] = sdv2::Vec8<T>::zero();
-      k[i] = sdv2::Vec8<T>::zero();
+      k[i] = q[i] = v[i] = wk[i] = wq[i] = sdv2::Vec8<T>::zero();
     }
   }
-
   const int fi = tok / a.frame_tokens;
   const int rem = tok - fi * a.frame_tokens;
   const int hi = rem / a.grid_w;
   const int wi = rem - hi * a.grid_w;
   double2 cs[4];
   sdv2::load_rotation(a.freqs, a.pairs, a.split_t, a.split_h, sub, a.start_frame[row] + fi, hi, wi, cs);
+  const int64_t dst_tok = row_dst_start(a, row) + tok;
 
   __shared__ float squares[kNormWaves][2][64 * 8];     // per wave: one step's squares of k and of q
   __shared__ float block_sums[2][kNormMaxSteps][32];   // k / q, step, accumulator
@@ -222,11 +220,13 @@ void kv_append_norm_rope_kernel(const AppendKernelArgs a) {
         squares[wave][1][lane * 8 + e] = q[i].getf(e) * q[i].getf(e);
       }
       // (LDS operations of one wave complete in order: no barrier between the stores and the loads)
+      // (all sixteen asked for at once; those past a trailing partial block are there and left out)
       const int count = j < full ? 16 : tail;
-      float block = 0.f;
+      float x[16], block = 0.f;
 #pragma unroll
-      for (int m = 0; m < 16; ++m)
-        if (m < count) block += squares[wave][which][(c + 4 * m) * 8 + t];
+      for (int m = 0; m < 16; ++m) x[m] = squares[wave][which][(c + 4 * m) * 8 + t];
+#pragma unroll
+      for (int m = 0; m < 16; ++m) block = m < count ? block + x[m] : block;
       block_sums[which][j][chain] = block;
     }
   }
@@ -255,21 +255,27 @@ void kv_append_norm_rope_kernel(const AppendKernelArgs a) {
   const float width = static_cast<float>(a.heads * 128);
   const float rq = 1.0f / sqrtf(ssq_q / width + a.norm_eps);
   const float rk = 1.0f / sqrtf(ssq_k / width + a.norm_eps);
-  if (a.q_inv_rms && threadIdx.x == 0) a.q_inv_rms[(int64_t)row * a.tokens + tok] = rq;
-  const T* wq = static_cast<const T*>(a.q_norm_w) + e0;
-  const T* wk = static_cast<const T*>(a.k_norm_w) + e0;
+  T* kc = static_cast<T*>(a.k_cache) + row * a.k_st.row + dst_tok * a.k_st.token + e0;
+  T* vc = static_cast<T*>(a.v_cache) + row * a.v_st.row + dst_tok * a.v_st.token + e0;
 #pragma unroll
   for (int i = 0; i < kStepsPerWave; ++i) {
-    const int j = wave + kNormWaves * i;
-    const int h = 4 * j + head_in_step;
-    if (j < steps && h < a.heads) {
-      const sdv2::Vec8<T> kn = sdv2::normalise(k[i], rk, sdv2::Vec8<T>::load(wk + h * 128));
-      sdv2::rotate(kn, cs).store(kc + h * a.k_st.head);
-      if constexpr (kWriteQ) {
-        T* qo = static_cast<T*>(a.q_out) + row * a.q_out_st.row + tok * a.q_out_st.token + e0;
-        const sdv2::Vec8<T> qn = sdv2::normalise(q[i], rq, sdv2::Vec8<T>::load(wq + h * 128));
-        sdv2::rotate(qn, cs).store(qo + h * a.q_out_st.head);
-      }
+    const int h = 4 * (wave + kNormWaves * i) + head_in_step;
+    const sdv2::Vec8<T> kr = sdv2::rotate(sdv2::normalise(k[i], rk, wk[i]), cs);
+    if (h < a.heads) {
+      v[i].store(vc + h * a.v_st.head);
+      kr.store(kc + h * a.k_st.head);
+    }
+    if constexpr (kWriteQ) {
+      T* qo = static_cast<T*>(a.q_out) + row * a.q_out_st.row + tok * a.q_out_st.token + e0;
+      const sdv2::Vec8<T> qr = sdv2::rotate(sdv2::normalise(q[i], rq, wq[i]), cs);
+      if (h < a.heads) qr.store(qo + h * a.q_out_st.head);
+    }
+  }
+  if (threadIdx.x == 0) {
+    if (a.q_inv_rms) a.q_inv_rms[(int64_t)row * a.tokens + tok] = rq;
+    if (blockIdx.x == 0) {
+      if (a.global_end) a.global_end[row] = a.new_global[row];
+      if (a.local_end) a.local_end[row] = a.new_local[row];
     }
   }
 }

@@ -163,10 +163,12 @@ __device__ __forceinline__ void wave_sum_squares(const Vec8<T> (&k)[kSteps], con
         scratch[1][lane * 8 + i] = q[j].getf(i) * q[j].getf(i);
       }
       const int count = j < full ? 16 : tail;
-      float block = 0.f;
+      // (all sixteen asked for at once; those past a trailing partial block are there and left out)
+      float x[16], block = 0.f;
 #pragma unroll
-      for (int m = 0; m < 16; ++m)
-        if (m < count) block += scratch[which][(c + 4 * m) * 8 + t];
+      for (int m = 0; m < 16; ++m) x[m] = scratch[which][(c + 4 * m) * 8 + t];
+#pragma unroll
+      for (int m = 0; m < 16; ++m) block = m < count ? block + x[m] : block;
       if (j < full) blocks += block;
       else trailing = block;
     }
