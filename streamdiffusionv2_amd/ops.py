@@ -352,6 +352,28 @@ def chunk_starts_tensor(starts, rows: int, q_tokens: int, max_seq_len: int, dev)
     return torch.tensor([int(x) for x in starts], dtype=torch.int32).to(dev, non_blocking=True)
 
 
+_CHUNK_STARTS: dict = {}
+_MAX_CHUNK_STARTS = 256
+
+
+def _chunk_starts_on(starts, rows: int, q_tokens: int, max_seq_len: int, dev, stream: int) -> torch.Tensor:
+    """:func:`chunk_starts_tensor`, with host values shipped once: a stream's
+    chunks land in a handful of slots, and the copy costs 4.6 us of the stream
+    and more of the host per call.  Filed by value, per stream (the copy is
+    ordered with that stream's launches alone), never taken out again (a
+    captured graph may hold the address), not filled from inside a capture
+    (there the copy has yet to run)."""
+    if starts is None or isinstance(starts, torch.Tensor):
+        return chunk_starts_tensor(starts, rows, q_tokens, max_seq_len, dev)
+    key = (dev, stream, q_tokens, max_seq_len, rows, tuple(int(x) for x in starts))
+    hit = _CHUNK_STARTS.get(key)
+    if hit is None:
+        hit = chunk_starts_tensor(starts, rows, q_tokens, max_seq_len, dev)
+        if len(_CHUNK_STARTS) < _MAX_CHUNK_STARTS and not torch.cuda.is_current_stream_capturing():
+            _CHUNK_STARTS[key] = hit
+    return hit
+
+
 # Descriptors of the attention calls seen, everything filled in that shapes, strides and dtypes decide: checking
 # and filling them costs more host time than the rest of a call, and a program has a handful of layouts.
 _ATTN_LAYOUTS: dict = {}
@@ -464,7 +486,7 @@ def swa_attention(
         p.workspace_bytes = workspace.numel() * workspace.element_size()
     p.stream = stream
     if mask_block_tokens:
-        chunk_key_start = chunk_starts_tensor(chunk_key_start, rows, q_tokens, max_seq_len, dev)
+        chunk_key_start = _chunk_starts_on(chunk_key_start, rows, q_tokens, max_seq_len, dev, stream)
         p.mask_block_tokens = int(mask_block_tokens)
         p.chunk_key_start = chunk_key_start.data_ptr()
     if rope is not None:
@@ -776,19 +798,19 @@ class LayerLauncher:
         """Fill in what changes from call to call and allocate the output
         [rows, S, H, 128]; nothing is launched."""
         ap, at = self.ap, self.at
+        stream = _stream_ptr(self.dev)
         if dst_start_override is not None:
             _check_override(dst_start_override, self.rows, self.dev)
         ap.dst_start_override = dst_start_override.data_ptr() if dst_start_override is not None else None
         at.mask_block_tokens = mask_block_tokens
         if mask_block_tokens:
-            self.chunk_starts = chunk_starts_tensor(plan.dst_start, self.rows, self.tokens, plan.max_seq_len, self.dev)
+            self.chunk_starts = _chunk_starts_on(plan.dst_start, self.rows, self.tokens, plan.max_seq_len, self.dev, stream)
             at.chunk_key_start = self.chunk_starts.data_ptr()
         self.sf[:] = start_frames
         self.ds[:] = plan.dst_start
         self.ng[:] = plan.new_global_end
         self.nl[:] = plan.new_local_end
         ap.k_in, ap.v_in = k.data_ptr(), v.data_ptr()
-        stream = _stream_ptr(self.dev)
         if self.rope_in_attention:
             at.q = q.data_ptr()
             if self.q_inv_rms is not None:

@@ -509,3 +509,40 @@ def test_masked_attention_on_16x16_matrix_instructions(gpu_device, rows, S, H, L
         got = ops.swa_attention(q.to(gpu_device), k.to(gpu_device), v.to(gpu_device), None, num_splits=splits,
                                 chunk_key_start=[start] * rows, mask_block_tokens=block)
         _check(got.cpu(), want)
+
+
+def test_masked_calls_with_host_starts_on_two_streams(gpu_device):
+    """Host chunk starts are shipped once per value and stream: calls that alternate between starts and streams, and
+    one captured into a graph, give what a device tensor of the starts gives."""
+    from streamdiffusionv2_amd import ops
+
+    torch.manual_seed(10)
+    S, L, block = 96, 500, 32
+    q, k, v = (torch.randn(1, n, 2, 128, device=gpu_device).bfloat16() for n in (S, L, L))
+
+    def call(start):
+        return ops.swa_attention(q, k, v, None, chunk_key_start=start, mask_block_tokens=block)
+
+    starts = [0, 64, 131, L - S]
+    want = {s: call(torch.tensor([s], dtype=torch.int32, device=gpu_device)) for s in starts + [200]}
+    streams = [torch.cuda.Stream() for _ in range(2)]
+    torch.cuda.synchronize()
+    got = []
+    for s in starts * 2:
+        for stream in streams:
+            with torch.cuda.stream(stream):
+                got.append((s, call([s])))
+    torch.cuda.synchronize()
+    for s, out in got:
+        assert torch.equal(out.view(torch.int16), want[s].view(torch.int16)), s
+    with pytest.raises(RuntimeError, match="outside"):
+        call([L - S + 1])
+    graph, side = torch.cuda.CUDAGraph(), streams[0]           # (a stream on which the starts are there already)
+    with torch.cuda.graph(graph, stream=side):
+        out = call([64])
+    for _ in range(3):
+        graph.replay()
+        eager = call([200])
+        torch.cuda.synchronize()
+        assert torch.equal(out.view(torch.int16), want[64].view(torch.int16))
+        assert torch.equal(eager.view(torch.int16), want[200].view(torch.int16))
