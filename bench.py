@@ -35,7 +35,7 @@ PEAK_HBM_GBS = 8000.0       # MI355X HBM3E
 # only used for the kernels it was taken on: same key-range split count, same
 # kernel sources (hash below); otherwise `traffic` is null and stderr says why.
 TRAFFIC_JSON = os.path.join(ROOT, "profiles", "hbm_traffic.json")
-KERNEL_SOURCES = ("swa_attn_fwd.hip", "swa_attn_fwd_m16.hip", "attn_device.h", "kv_append_rope.hip", "rope_device.h", "sdv2kv_internal.h")
+KERNEL_SOURCES = ("swa_attn_fwd.hip", "swa_attn_fwd_m16.hip", "swa_attn_fwd_wave.hip", "attn_device.h", "kv_append_rope.hip", "rope_device.h", "sdv2kv_internal.h")
 
 
 def kernel_source_hash() -> str:
@@ -81,7 +81,7 @@ def record_traffic(args, w):
             raise SystemExit(f"no counter_collection.csv under {args.record_traffic}/{sub}")
         total, count = collections.defaultdict(float), collections.Counter()
         for row in csv.DictReader(open(files[0])):
-            for short, names in (("swa_attn_fwd_kernel", ("swa_attn_fwd_kernel", "swa_attn_fwd_m16_kernel")),
+            for short, names in (("swa_attn_fwd_kernel", ("swa_attn_fwd_kernel", "swa_attn_fwd_m16_kernel", "swa_attn_fwd_wave_kernel")),
                                  ("kv_append_rope_kernel", ("kv_append_rope_kernel",)), ("copy16_kernel", ("copy16_kernel",))):
                 if any(n in row["Kernel_Name"] for n in names):
                     total[short] += float(row["Counter_Value"])
@@ -400,8 +400,7 @@ def module_path_section(args, w, headline_ms):
 
     * ``fused_norm``: the path as CausalWanSelfAttention.forward drives it by
       default - raw q / k projections in, their RMSNorm folded into the append
-      (causal_model.py:212-218), the query normalised and rotated inside the
-      attention kernel;
+      (causal_model.py:212-218), which hands the attention the rotated query;
     * ``shipped_config``: the same with the shipped v2v settings, sink 3 and
       adaptive threshold 0.2 (configs/wan_causal_dmd_v2v.yaml:53-56).  The
       inputs carry a scene direction that changes every eighth chunk, so the
@@ -495,7 +494,7 @@ def module_path_section(args, w, headline_ms):
     out["fused_norm"]["kernel_ms_per_layer"] = {
         "append_with_norm": sum(t[0].elapsed_ms() for t in timers) / len(timers),
         "attention_with_q_norm": sum(t[1].elapsed_ms() for t in timers) / len(timers)}
-    out["fused_norm"]["append_bytes"] = w.append_bytes(with_q=True) * 5 // 6      # read q, k, v; write k', v
+    out["fused_norm"]["append_bytes"] = w.append_bytes(with_q=True)      # read q, k, v; write q', k', v
     out["fused_norm"]["append_GBps"] = out["fused_norm"]["append_bytes"] / (
         out["fused_norm"]["kernel_ms_per_layer"]["append_with_norm"] * 1e-3) / 1e9
     for t in timers:
@@ -663,8 +662,8 @@ def qk_norm_section(args, w):
         out[name] = e0.elapsed_time(e1) / n
     out["bytes_per_launch"] = w.append_bytes(with_q=True)
     # the fused kernel's own duration (timing events in its dispatch): as the operator returns the rotated
-    # query (read q, k, v; write q', k', v), and as the module path runs it (q is only read, for its sum of
-    # squares; the attention kernel normalises and rotates the raw q itself)
+    # query (read q, k, v; write q', k', v), as the module path runs it, and with q only read, for its sum of
+    # squares (callers whose attention normalises and rotates the raw q itself)
     inv_rms = torch.empty(B, S, dtype=torch.float32, device=dev)
 
     def fused_no_q_out(i):
@@ -902,7 +901,7 @@ def launch_floor_section(args, w):
     out = {}
     timer = ops.KernelTimer()
     lib = _capi.lib()
-    moved = w.append_bytes(with_q=False)
+    moved = w.append_bytes(with_q=True)
     for name, nbytes in (("empty_launch_us", 16), ("copy_of_append_bytes_us", moved // 2 // 16 * 16)):
         src = torch.empty(nbytes, dtype=torch.uint8, device=dev).random_(0, 255)
         dst = torch.empty_like(src)
@@ -1060,7 +1059,7 @@ def main():
     attn_s = g["attn_ms"] * 1e-3
     achieved_tflops = w.attn_flops() / attn_s / 1e12
     # the query is rotated inside the attention kernel: the append moves K and V only
-    append_gbs = w.append_bytes(with_q=False) / (g["append_ms"] * 1e-3) / 1e9
+    append_gbs = w.append_bytes(with_q=True) / (g["append_ms"] * 1e-3) / 1e9
     hbm = measured_traffic(w.name, g["splits"])
     result = {
         "metric": "kv_append_attn_tokens_per_s",
@@ -1107,7 +1106,7 @@ def main():
             "unit": "GB/s",
             "frac": append_gbs / PEAK_HBM_GBS,
             "traffic": hbm["append"] if hbm else None,
-            "bytes_per_launch": w.append_bytes(with_q=False),
+            "bytes_per_launch": w.append_bytes(with_q=True),
             "avg_launch_ms": g["append_ms"],
         },
         "kernel_ms_per_layer": {

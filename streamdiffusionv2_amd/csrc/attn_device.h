@@ -1,4 +1,4 @@
-// What the two bf16 attention kernels share (gfx950 only): the launch arguments,
+// What the bf16 attention kernels share (gfx950 only): the launch arguments,
 // the layout of a work list over (row, head, key range, query tile), LDS reads
 // and global->LDS transfers with hand-placed waits, packing, and the
 // device-coherent accesses that carry partial results between workgroups.

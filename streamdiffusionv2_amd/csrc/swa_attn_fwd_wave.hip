@@ -1,7 +1,7 @@
 // Sliding-window (sink + window) flash attention for small calls, for gfx950 (MI355X).
 //
 // Same operator and arguments as the kernel in swa_attn_fwd.hip (which see for the
-// reference lines it stands in for, and for the rule that picks one of the three).
+// reference lines it stands in for, and for the rules that pick one of the three).
 //
 // What bounds a small call is not the matrix pipe but how long one workgroup takes
 // and how few there are: 256 queries x 12 heads are 12 query tiles of the other
@@ -10,8 +10,10 @@
 // that call), the waves take the keys 32 at a time in turn, each by itself, and
 // meet once, in LDS, at the end: no barrier while the keys stream, no partial results
 // in memory, no ticket.  The price is that no wave shares a key it has fetched with
-// another: every workgroup streams all keys from L2, which is what bounds its
-// inner loop (a CU takes about 64 bytes a clock).
+// another: every workgroup streams all keys from L2, and those trips bound its
+// loop, 1.22 us per 256 keys (128 KB) whether 8 workgroups run or 240; the products
+// alone would take 0.8.  256 x 12 heads against 1536 keys: 21.6 us with the tile
+// kernels' best plan, 13.7 with this one; 512 keys 17.0 and 9.0.
 //
 // A wave's K and V blocks sit in 16 KB of LDS of its own; the next K block is requested
 // as soon as the fragments of this one are in registers, the next V block likewise.
