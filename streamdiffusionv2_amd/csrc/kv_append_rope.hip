@@ -70,6 +70,7 @@ __device__ __forceinline__ int64_t row_dst_start(const AppendKernelArgs& a, int 
 template <typename T, bool kWithQ, bool kWithKV>
 __global__ __launch_bounds__(kLanesPerRow * kTokensPerBlock)
 void kv_append_rope_kernel(const AppendKernelArgs a) {
+  sdv2::fetch_arguments<AppendKernelArgs>();
   const int lane = threadIdx.x & (kLanesPerRow - 1);
   const int tok = blockIdx.x * kTokensPerBlock + (threadIdx.x >> 4);
   const int row = blockIdx.z;
@@ -162,6 +163,7 @@ template <typename T, int kStepsPerWave, bool kWriteQ>
 __global__ __launch_bounds__(64 * kNormWaves, sizeof(T) == 2 && kStepsPerWave <= 3 ? 4 : 2)
 void kv_append_norm_rope_kernel(const AppendKernelArgs a) {
 #pragma clang fp contract(off)
+  sdv2::fetch_arguments<AppendKernelArgs>();
   const int lane = threadIdx.x & 63;
   const int wave = threadIdx.x >> 6;
   const int sub = lane & (kLanesPerRow - 1);            // 8-element slice of a head row

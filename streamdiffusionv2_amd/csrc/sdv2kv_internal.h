@@ -36,6 +36,22 @@ inline void launch_timed(int which, Kernel kernel, dim3 grid, dim3 block, uint32
     hipLaunchKernelGGL(kernel, grid, block, lds_bytes, stream, args);
 }
 
+// One word of every 64-byte line of the kernel's arguments, asked for together.  A fresh launch finds its arguments in
+// memory, and the compiler loads them where they are used: four or five trips one after another at the start of
+// every workgroup.  Behind this the rest come from the scalar cache.  For the short kernels: eight layers of 256
+// tokens x 12 heads against 1536 keys 178 -> 167 us.  (In the attention kernels of 256-row tiles it made no
+// difference; their launches are long, and their arguments crowd the scalar registers.)
+template <typename Args>
+__device__ __forceinline__ void fetch_arguments() {
+  const auto* words = (const __attribute__((address_space(4))) uint32_t*)__builtin_amdgcn_kernarg_segment_ptr();
+  constexpr int kLines = (sizeof(Args) + 63) / 64;
+  uint32_t x[kLines];
+#pragma unroll
+  for (int i = 0; i < kLines; ++i) x[i] = words[16 * i];
+#pragma unroll
+  for (int i = 0; i < kLines; ++i) asm volatile("" ::"s"(x[i]));
+}
+
 // float -> bfloat16 bit pattern, round-to-nearest-even, NaN -> 0x7FC0: the
 // rounding PyTorch applies when a float (or a double already narrowed to
 // float) is stored as bfloat16.

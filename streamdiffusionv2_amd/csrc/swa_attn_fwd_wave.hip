@@ -116,6 +116,7 @@ __global__ __launch_bounds__(kThreads, 1)
 void swa_attn_fwd_wave_kernel(const AttnKernelArgs a) {
   extern __shared__ __attribute__((aligned(1024))) char smem[];
   lds_char* lds = (lds_char*)smem;
+  sdv2::fetch_arguments<AttnKernelArgs>();
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
