@@ -245,9 +245,10 @@ int sdv2_swa_attn_fwd(const sdv2_attn_params* p);
  * the partial results of a split call go to SDV2_STATIC_SCRATCH_BYTES of
  * device memory that the library itself holds on every GPU it runs on, from
  * load to process exit.  A call whose sdv2_swa_attn_workspace_bytes() exceeds
- * that returns SDV2_ERR_SCRATCH_LIMIT and launches nothing (64 MiB covers the
- * Wan 1.3B and 14B shapes at 480p: one row of a 1560-token chunk against six
- * frames).  The call allocates and frees nothing and does not synchronise.
+ * that for a num_splits the caller gave returns SDV2_ERR_SCRATCH_LIMIT and
+ * launches nothing; where the plan is the library's own it is run unsplit (64 MiB
+ * covers the Wan 1.3B and 14B shapes at 480p: one row of a 1560-token chunk
+ * against six frames).  The call allocates and frees nothing and does not synchronise.
  * The scratch starts out zeroed and every call leaves its ticket words at zero
  * again, so nothing has to be cleared between calls, but all calls on one GPU
  * share it: two calls that overlap in time on one GPU - different streams,

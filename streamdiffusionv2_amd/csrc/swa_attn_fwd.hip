@@ -1093,8 +1093,13 @@ extern "C" int sdv2_swa_attn_fwd_static(const sdv2_attn_params* p) {
   if (!decode_splits(splits, p->rows, p->heads, &plan)) return SDV2_ERR_INVALID_ARG;   // as the plain entry point answers
   if (plan.most() <= 1) return attn_fwd(p, nullptr, 0);
   if (sdv2_swa_attn_workspace_bytes(p->rows, p->q_tokens, p->heads, p->max_seq_len, splits) >
-      (size_t)SDV2_STATIC_SCRATCH_BYTES)
-    return SDV2_ERR_SCRATCH_LIMIT;
+      (size_t)SDV2_STATIC_SCRATCH_BYTES) {
+    if (p->num_splits > 0) return SDV2_ERR_SCRATCH_LIMIT;
+    // the library's own choice of plan (often a matter of a per cent or two on calls this large) refuses nothing
+    sdv2_attn_params whole = *p;
+    whole.num_splits = 1;
+    return attn_fwd(&whole, nullptr, 0);
+  }
   void* ptr = static_scratch_address();
   if (!ptr) return SDV2_ERR_LAUNCH;
   return attn_fwd(p, ptr, SDV2_STATIC_SCRATCH_BYTES);

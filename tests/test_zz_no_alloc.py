@@ -108,6 +108,23 @@ def test_static_entry_point_refuses_more_than_it_holds(gpu_device):
     assert bool((of == 0.0).all())
 
 
+def test_static_entry_point_runs_unsplit_where_the_default_plan_does_not_fit(gpu_device):
+    from streamdiffusionv2_amd import _capi
+
+    lib = _capi.lib()
+    rows, q_tokens, heads, keys = 4, 2656, 12, 2121
+    splits = lib.sdv2_swa_attn_default_splits(rows, q_tokens, heads, keys)
+    assert lib.sdv2_swa_attn_workspace_bytes(rows, q_tokens, heads, keys, splits) > _capi.STATIC_SCRATCH_BYTES
+    torch.manual_seed(3)
+    q = torch.randn(rows, q_tokens, heads, 128, device=gpu_device).bfloat16()
+    kc, vc = (torch.randn(rows, keys, heads, 128, device=gpu_device).bfloat16() for _ in range(2))
+    got, want = torch.zeros_like(q), torch.ones_like(q)
+    _capi.check(lib.sdv2_swa_attn_fwd_static(C.byref(_attn_params(q, kc, vc, got, None, 0))), "static, default plan")
+    _capi.check(lib.sdv2_swa_attn_fwd(C.byref(_attn_params(q, kc, vc, want, None, 1))), "unsplit")
+    torch.cuda.synchronize()
+    assert torch.equal(got.view(torch.int16), want.view(torch.int16))
+
+
 def test_static_entry_point_at_the_wan_shapes(gpu_device):
     """The two shapes the 64 MiB are sized for: 1560 queries against 9360 keys
     with 12 heads (three key ranges) and with 40 heads (four)."""
