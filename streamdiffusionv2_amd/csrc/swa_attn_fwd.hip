@@ -1195,18 +1195,24 @@ int attn_fwd(const sdv2_attn_params* p, void* workspace, size_t workspace_bytes)
     a.part_scale = reinterpret_cast<float*>(ws + w.part_scale);
   }
 
+  // Work items of a launch on query tiles of q_tile_rows rows, counted in 64 bits before the 32-bit work list is made.
+  const int64_t per_query_tile = ((int64_t)p->rows * p->heads / plan.group) *
+                                 ((int64_t)(plan.group - plan.more) * plan.base + (int64_t)plan.more * (plan.base + 1));
+  auto work_items = [&](int q_tile_rows) { return per_query_tile * (((int64_t)p->q_tokens + q_tile_rows - 1) / q_tile_rows); };
+  const int64_t items = work_items(kQTile);
+  if (items > (1 << 28)) return SDV2_ERR_INVALID_ARG;
+
   hipStream_t stream = static_cast<hipStream_t>(p->stream);
-  // Which kernel, first: one key range, and few enough query blocks that the waves had better share those than the keys
-  if (splits == 1 && wave_kernel_us(p->rows, p->q_tokens, p->heads, p->max_seq_len) <
-                         tile_kernels_us(p->rows, p->q_tokens, p->heads, p->max_seq_len, 1, 0)) {
+  // Which kernel, first: one key range, and few enough query blocks that the waves had better share those than the keys.
+  // (A grid has fewer than 2^32 threads: up to eight times the workgroups must not carry an accepted call past that.)
+  constexpr int64_t kMostWaveItems = 1 << 22;
+  if (splits == 1 && work_items(kQBlock) <= kMostWaveItems &&
+      wave_kernel_us(p->rows, p->q_tokens, p->heads, p->max_seq_len) <
+          tile_kernels_us(p->rows, p->q_tokens, p->heads, p->max_seq_len, 1, 0)) {
     set_work_list(&a, kQBlock);
     return sdv2::attn::launch_wave(a, 8u * (((uint32_t)a.total_items + 7u) / 8u), stream);
   }
   set_work_list(&a, kQTile);
-  const int64_t nq_tiles = (p->q_tokens + kQTile - 1) / kQTile;
-  const int64_t items = ((int64_t)p->rows * p->heads / plan.group) *
-                        (nq_tiles * ((int64_t)(plan.group - plan.more) * plan.base + (int64_t)plan.more * (plan.base + 1)));
-  if (items > (1 << 28)) return SDV2_ERR_INVALID_ARG;
   dim3 grid((unsigned)(8 * ((items + 7) / 8)));
   // Which of the other two.  The one on 16x16x32 matrix instructions takes 1.51 us per 64-key tile of a full CU where this one
   // takes 1.65, and a microsecond more to fill its deeper pipeline: they meet at 12 tiles (1536 queries x 40 heads,

@@ -115,6 +115,28 @@ def test_argument_validation_without_gpu():
         _capi.check(_capi.SDV2_ERR_OUT_OF_RANGE, "x")
 
 
+@pytest.mark.parametrize("rows,q_tokens,heads,keys", [
+    (8191, 1, 65535, 64),          # one query block per (row, head): the kernel for small calls would be picked
+    (4096, 8192, 32768, 9360),     # 2^32 work items: nothing may be counted, or divided by, in 32 bits
+    (4096, 4096, 32768, 64),       # 2^31
+])
+def test_more_work_items_than_a_launch_holds_are_refused(rows, q_tokens, heads, keys):
+    """(in a process of its own: a wrapped count that ends in a division by zero would take this one along)"""
+    import subprocess
+    import sys
+
+    code = f"""
+import ctypes as C
+from streamdiffusionv2_amd import _capi
+a = _capi.AttnParams(q=256, k_cache=512, v_cache=768, out=1024, rows={rows}, q_tokens={q_tokens}, heads={heads},
+                     head_dim=128, max_seq_len={keys}, num_splits=1)
+print("status", _capi.lib().sdv2_swa_attn_fwd(C.byref(a)))
+"""
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    run = subprocess.run([sys.executable, "-c", code], cwd=root, capture_output=True, text=True, timeout=300)
+    assert run.returncode == 0 and f"status {_capi.SDV2_ERR_INVALID_ARG}" in run.stdout, (run.returncode, run.stdout, run.stderr)
+
+
 def test_split_heuristic_and_workspace_size():
     lib = _capi.lib()
     assert lib.sdv2_swa_attn_workspace_bytes(1, 1560, 12, 9360, 1) == 0
