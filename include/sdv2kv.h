@@ -31,7 +31,11 @@
 extern "C" {
 #endif
 
-#define SDV2KV_ABI_VERSION 12
+/* 13: sdv2_swa_attn_f32_workspace_bytes; a workspace given with SDV2_F32 is used
+ *     (12 ignored it), so its ticket words must be zero like any other's;
+ *     sdv2_swa_attn_fwd_static runs a call with num_splits = 0 unsplit where the
+ *     library's own plan needs more than SDV2_STATIC_SCRATCH_BYTES (12 refused it) */
+#define SDV2KV_ABI_VERSION 13
 #define SDV2_HEAD_DIM 128      /* causal_stream_inference.py:99-100 fixes 128 */
 #define SDV2_MAX_ROWS 16       /* rows (B) per sdv2_kv_append_rope call       */
 #define SDV2_MAX_SINK_FRAMES 16 /* sink frames per sdv2_sink_similarity call  */
@@ -214,7 +218,8 @@ typedef struct sdv2_attn_params {
    * (num_splits is ignored and rope_freqs must be unset: fp32 queries arrive
    * rotated), strides in multiples of 4 elements.  With a workspace of
    * sdv2_swa_attn_f32_workspace_bytes() the key range is split to fill the
-   * chip; without one (NULL, or too small) it is walked whole.               */
+   * chip (its ticket words must be zero); without one (NULL, too small or not
+   * 256-byte aligned) it is walked whole.                                    */
   int32_t dtype;
   /* Optional q RMSNorm inside the call (needs rope_freqs and SDV2_BF16): q is
    * the raw q projection, q_norm_weight the norm's weight (device, bf16,

@@ -12,7 +12,7 @@ from typing import Optional
 
 LIB_PATH = Path(__file__).resolve().parent / "_lib" / "libsdv2kv.so"
 
-ABI_VERSION = 12
+ABI_VERSION = 13
 HEAD_DIM = 128
 MAX_ROWS = 16
 
@@ -188,6 +188,11 @@ def lib() -> C.CDLL:
     handle = C.CDLL(str(LIB_PATH))
     handle.sdv2_abi_version.restype = C.c_int
     handle.sdv2_abi_version.argtypes = []
+    # (before any other symbol: a library of another version may lack some)
+    if handle.sdv2_abi_version() != ABI_VERSION:
+        raise ImportError(
+            f"{LIB_PATH} has ABI version {handle.sdv2_abi_version()}, expected {ABI_VERSION}: rebuild it"
+        )
     handle.sdv2_status_string.restype = C.c_char_p
     handle.sdv2_status_string.argtypes = [C.c_int]
     handle.sdv2_kv_append_rope.restype = C.c_int
@@ -227,10 +232,6 @@ def lib() -> C.CDLL:
     handle.sdv2_profile_mfma_stream.restype = C.c_int
     handle.sdv2_profile_mfma_stream.argtypes = [C.c_int, C.c_void_p, C.c_size_t, C.c_int32, C.c_void_p,
                                                 C.POINTER(C.c_double)]
-    if handle.sdv2_abi_version() != ABI_VERSION:
-        raise ImportError(
-            f"{LIB_PATH} has ABI version {handle.sdv2_abi_version()}, expected {ABI_VERSION}: rebuild it"
-        )
     _LIB = handle
     return handle
 

@@ -160,6 +160,22 @@ def test_missing_library_fails_loudly(monkeypatch, tmp_path):
         _capi.lib()
 
 
+def test_a_library_of_another_version_is_named_as_such(monkeypatch, tmp_path):
+    """It may lack symbols, or read a struct another way: the version is looked at before anything else."""
+    import shutil
+    import subprocess
+
+    if shutil.which("gcc") is None:
+        pytest.skip("no gcc")
+    # (12 is the last version without the fp32 workspace, whose fp32 calls took no workspace)
+    (tmp_path / "old.c").write_text("int sdv2_abi_version(void) { return 12; }")
+    subprocess.run(["gcc", "-shared", "-fPIC", str(tmp_path / "old.c"), "-o", str(tmp_path / "old.so")], check=True)
+    monkeypatch.setattr(_capi, "_LIB", None)
+    monkeypatch.setattr(_capi, "LIB_PATH", tmp_path / "old.so")
+    with pytest.raises(ImportError, match="ABI version 12"):
+        _capi.lib()
+
+
 def test_cpu_tensors_are_refused():
     from streamdiffusionv2_amd import ops
 
