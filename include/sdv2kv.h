@@ -34,8 +34,9 @@ extern "C" {
 /* 13: sdv2_swa_attn_f32_workspace_bytes; a workspace given with SDV2_F32 is used
  *     (12 ignored it), so its ticket words must be zero like any other's;
  *     sdv2_swa_attn_fwd_static runs a call with num_splits = 0 unsplit where the
- *     library's own plan needs more than SDV2_STATIC_SCRATCH_BYTES (12 refused it) */
-#define SDV2KV_ABI_VERSION 13
+ *     library's own plan needs more than SDV2_STATIC_SCRATCH_BYTES (12 refused it)
+ * 14: sdv2_attn_params.chunk_key_start_host */
+#define SDV2KV_ABI_VERSION 14
 #define SDV2_HEAD_DIM 128      /* causal_stream_inference.py:99-100 fixes 128 */
 #define SDV2_MAX_ROWS 16       /* rows (B) per sdv2_kv_append_rope call       */
 #define SDV2_MAX_SINK_FRAMES 16 /* sink frames per sdv2_sink_similarity call  */
@@ -202,7 +203,8 @@ typedef struct sdv2_attn_params {
    * else in the cache is older and stays visible.  0 (or b >= S) = no mask.  */
   int32_t mask_block_tokens;
   const int32_t* chunk_key_start;  /* device int32 [B], each in [0, L - S]; may be */
-                                   /* NULL when the mask is off                    */
+                                   /* NULL when the mask is off or                 */
+                                   /* chunk_key_start_host is given                */
   /* Optional RoPE of q inside the call.  rope_freqs = the device table of
    * sdv2_kv_append_rope (complex128 [rope_freq_rows, 64] as (re, im)), or NULL
    * when q is already rotated.  The chunk's S tokens are S / (grid_h * grid_w)
@@ -229,6 +231,12 @@ typedef struct sdv2_attn_params {
    * WanRMSNorm rounds, wan_base/modules/model.py:77-86) and then rotated.      */
   const void* q_norm_weight;
   const float* q_inv_rms;
+  /* What chunk_key_start says, from host memory instead (at most SDV2_MAX_ROWS
+   * rows): the values travel with the launch, so nothing has to be copied to the
+   * device, kept there or ordered with the stream.  Read during the call only;
+   * SDV2_ERR_OUT_OF_RANGE for a value outside [0, L - S].  With the mask on,
+   * exactly one of the two is set.                                             */
+  const int64_t* chunk_key_start_host;   /* host [B]                               */
 } sdv2_attn_params;
 
 /* the key-range split plan the library would pick for this shape, as num_splits carries it */

@@ -12,7 +12,7 @@ from typing import Optional
 
 LIB_PATH = Path(__file__).resolve().parent / "_lib" / "libsdv2kv.so"
 
-ABI_VERSION = 13
+ABI_VERSION = 14
 HEAD_DIM = 128
 MAX_ROWS = 16
 
@@ -108,6 +108,7 @@ class AttnParams(C.Structure):
         ("dtype", C.c_int32),
         ("q_norm_weight", C.c_void_p),
         ("q_inv_rms", C.c_void_p),
+        ("chunk_key_start_host", C.POINTER(C.c_int64)),
     ]
 
 

@@ -74,7 +74,6 @@ struct AttnKernelArgs {
   float scale_log2;            // softmax_scale * log2(e)
   int32_t mask_block_tokens;   // 0 = no mask inside the chunk
   FastDiv div_mask_block;      // by mask_block_tokens
-  const int32_t* chunk_start;  // device [rows]: cache position of the chunk's own first key
   // Split calls.  Partial results are kept per 32-row query block in the order
   // the registers hold them (see store_partial), q_blocks = ceil(q_tokens / 32).
   int32_t q_blocks;
@@ -91,7 +90,11 @@ struct AttnKernelArgs {
   // the norm weight [heads * 128] and 1 / rms per (row, token), or null
   const uint16_t* q_norm_w;
   const float* q_inv_rms;
+  sdv2::ChunkStarts chunk_starts;   // with the mask inside the chunk
 };
+__device__ __forceinline__ int row_chunk_start(const AttnKernelArgs& a, int row) {
+  return sdv2::row_chunk_start<offsetof(AttnKernelArgs, chunk_starts)>(a.chunk_starts, row);
+}
 
 // v_max without the NaN-quieting canonicalisation fmaxf() drags in.
 __device__ __forceinline__ float vmax(float a, float b) {

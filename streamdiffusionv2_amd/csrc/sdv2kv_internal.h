@@ -4,9 +4,10 @@
 
 #include <hip/hip_runtime.h>
 #include <hip/hip_ext.h>
+#include <stddef.h>
 #include <stdint.h>
 
-struct sdv2_attn_params;
+#include "sdv2kv.h"
 
 namespace sdv2 {
 
@@ -50,6 +51,36 @@ __device__ __forceinline__ void fetch_arguments() {
   for (int i = 0; i < kLines; ++i) x[i] = words[16 * i];
 #pragma unroll
   for (int i = 0; i < kLines; ++i) asm volatile("" ::"s"(x[i]));
+}
+
+// Cache positions of the chunk's own first key, one per row: the caller's device array, or host values that travel in
+// the launch's arguments.
+struct ChunkStarts {
+  const int32_t* device;               // null: `value`
+  int32_t value[SDV2_MAX_ROWS];
+};
+// Row `row` (wave-uniform) of the ChunkStarts at byte kOffset of the kernel's arguments, one scalar load either way.
+// (Read where the arguments lie: indexing the by-value block with a run-time row would move the whole block out of
+// scalar registers.)
+template <int kOffset>
+__device__ __forceinline__ int row_chunk_start(const ChunkStarts& starts, int row) {
+  typedef const __attribute__((address_space(4))) char* arg_bytes;
+  typedef const __attribute__((address_space(4))) int32_t* arg_words;
+  const arg_words carried = (arg_words)((arg_bytes)__builtin_amdgcn_kernarg_segment_ptr() + kOffset + offsetof(ChunkStarts, value));
+  return starts.device ? starts.device[row] : carried[row];
+}
+// host: fill `starts` from a call's parameters; the mask is on
+inline int set_chunk_starts(const sdv2_attn_params& p, ChunkStarts* starts) {
+  if ((p.chunk_key_start != nullptr) == (p.chunk_key_start_host != nullptr)) return SDV2_ERR_INVALID_ARG;
+  starts->device = p.chunk_key_start;
+  if (starts->device) return SDV2_OK;
+  if (p.rows > SDV2_MAX_ROWS) return SDV2_ERR_INVALID_ARG;
+  for (int i = 0; i < p.rows; ++i) {
+    const int64_t first = p.chunk_key_start_host[i];
+    if (first < 0 || first > (int64_t)p.max_seq_len - p.q_tokens) return SDV2_ERR_OUT_OF_RANGE;
+    starts->value[i] = (int32_t)first;
+  }
+  return SDV2_OK;
 }
 
 // float -> bfloat16 bit pattern, round-to-nearest-even, NaN -> 0x7FC0: the

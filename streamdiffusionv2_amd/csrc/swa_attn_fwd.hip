@@ -463,7 +463,7 @@ void swa_attn_fwd_kernel(const AttnKernelArgs a) {
   // and the key ranges are cut from what is left.
   int hole = 0x7fffffff, skipped = 0;
   if constexpr (kMask) {
-    const int first = a.chunk_start[row], bt = a.mask_block_tokens;
+    const int first = row_chunk_start(a, row), bt = a.mask_block_tokens;
     const int q_last = qtile * kQTile + kQTile < a.q_tokens ? qtile * kQTile + kQTile - 1 : a.q_tokens - 1;
     const int lo = first + (q_last / bt + 1) * bt, hi = first + a.q_tokens;
     const int h0 = (lo + kKTile - 1) / kKTile, h1 = hi >= seq ? ntiles : hi / kKTile;
@@ -559,7 +559,7 @@ void swa_attn_fwd_kernel(const AttnKernelArgs a) {
   c.hf = hf;
   if (kMask && a.mask_block_tokens > 0) {
     const int bt = a.mask_block_tokens;
-    const int first = a.chunk_start[row];
+    const int first = row_chunk_start(a, row);
     c.m_hi = __builtin_amdgcn_readfirstlane(first + a.q_tokens);
     c.wg_m_lo = __builtin_amdgcn_readfirstlane(first + ((qtile * kQTile) / bt + 1) * bt);
     c.m_lo = first + (q_row / bt + 1) * bt;
@@ -1147,8 +1147,8 @@ int attn_fwd(const sdv2_attn_params* p, void* workspace, size_t workspace_bytes)
   if (p->mask_block_tokens < 0) return SDV2_ERR_INVALID_ARG;
   if (p->mask_block_tokens > 0 && p->mask_block_tokens < p->q_tokens) {
     // a block as long as the chunk hides nothing: only shorter blocks switch the mask on
-    if (!p->chunk_key_start) return SDV2_ERR_INVALID_ARG;
-    a.chunk_start = p->chunk_key_start;
+    const int status = sdv2::set_chunk_starts(*p, &a.chunk_starts);
+    if (status != SDV2_OK) return status;
     a.mask_block_tokens = p->mask_block_tokens;
     a.div_mask_block = FastDiv::by((uint32_t)p->mask_block_tokens);
   }

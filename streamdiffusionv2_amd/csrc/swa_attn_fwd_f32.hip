@@ -91,12 +91,12 @@ struct AttnF32Args {
   int32_t rows, q_tokens, heads, max_seq_len;
   float scale_log2;            // softmax_scale * log2(e)
   int32_t mask_block_tokens;
-  const int32_t* chunk_start;
   int32_t splits, q_tiles, q_blocks;
   int32_t* tickets;            // [row][head][query tile]
   float* part_o;               // [split][row][head][block][16 KB]: sums of weights times values, in register order
   float* part_m;               // [split][row][head][block][32]: running maximum, log2 units
   float* part_l;               // [split][row][head][block][32]: sum of weights
+  sdv2::ChunkStarts chunk_starts;   // with the mask inside the chunk
 };
 
 __device__ __forceinline__ float half_max(float x) {
@@ -182,7 +182,7 @@ void swa_attn_fwd_f32_kernel(const AttnF32Args a) {
   // the chunk's own later blocks, hidden from this lane's query when the mask inside the chunk is on
   int m_lo = 0x7fffffff, m_hi = 0;
   if (a.mask_block_tokens > 0) {
-    const int first = a.chunk_start[row];
+    const int first = sdv2::row_chunk_start<offsetof(AttnF32Args, chunk_starts)>(a.chunk_starts, row);
     m_hi = first + a.q_tokens;
     m_lo = first + (q_row / a.mask_block_tokens + 1) * a.mask_block_tokens;
   }
@@ -467,8 +467,8 @@ int sdv2::attn_fwd_f32(const sdv2_attn_params* p, void* workspace, size_t worksp
   a.rows = p->rows; a.q_tokens = p->q_tokens; a.heads = p->heads; a.max_seq_len = p->max_seq_len;
   a.scale_log2 = (p->softmax_scale > 0.f ? p->softmax_scale : 0.08838834764831845f) * kLog2e;  // 1/sqrt(128)
   if (p->mask_block_tokens > 0 && p->mask_block_tokens < p->q_tokens) {
-    if (!p->chunk_key_start) return SDV2_ERR_INVALID_ARG;
-    a.chunk_start = p->chunk_key_start;
+    const int status = sdv2::set_chunk_starts(*p, &a.chunk_starts);
+    if (status != SDV2_OK) return status;
     a.mask_block_tokens = p->mask_block_tokens;
   }
   a.q_tiles = (p->q_tokens + kQTile - 1) / kQTile;

@@ -448,7 +448,7 @@ void swa_attn_fwd_m16_kernel(const AttnKernelArgs a) {
   // from what is left.
   int hole = 0x7fffffff, skipped = 0;
   if constexpr (kMask) {
-    const int first = a.chunk_start[row], bt = a.mask_block_tokens;
+    const int first = row_chunk_start(a, row), bt = a.mask_block_tokens;
     const int q_last = qtile * kQTile + kQTile < a.q_tokens ? qtile * kQTile + kQTile - 1 : a.q_tokens - 1;
     const int lo = first + (a.div_mask_block(q_last) + 1) * bt, hi = first + a.q_tokens;
     const int h0 = (lo + kKTile - 1) / kKTile, h1 = hi >= seq ? ntiles : hi / kKTile;
@@ -556,7 +556,7 @@ void swa_attn_fwd_m16_kernel(const AttnKernelArgs a) {
     c.m_block = a.mask_block_tokens;
     c.m_div = a.div_mask_block;
     c.q_first = qtile * kQTile + wave_u * kQBlock;
-    c.m_first = __builtin_amdgcn_readfirstlane(a.chunk_start[row]);
+    c.m_first = __builtin_amdgcn_readfirstlane(row_chunk_start(a, row));
     c.m_hi = c.m_first + a.q_tokens;
     c.m_lo = __builtin_amdgcn_readfirstlane(c.m_first + (c.m_div(c.q_first) + 1) * c.m_block);
   }

@@ -134,7 +134,7 @@ void swa_attn_fwd_wave_kernel(const AttnKernelArgs a) {
   // [hole, hole + skipped) are hidden from all of the workgroup's queries (from the last one, that is) and left out.
   int m_lo[2] = {0, 0}, m_lo_first = 0, m_hi = 0, hole = 0x7fffffff, skipped = 0;
   if constexpr (kMask) {
-    const int first = a.chunk_start[row], bt = a.mask_block_tokens;
+    const int first = row_chunk_start(a, row), bt = a.mask_block_tokens;
     const int q_last = q0 + kQBlock < a.q_tokens ? q0 + kQBlock - 1 : a.q_tokens - 1;
     m_hi = first + a.q_tokens;
     m_lo_first = first + (q0 / bt + 1) * bt;

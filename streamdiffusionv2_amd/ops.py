@@ -337,6 +337,14 @@ def release_scratch() -> None:
         pool.clear()
 
 
+def _check_chunk_starts(starts, rows: int, q_tokens: int, max_seq_len: int) -> None:
+    if starts is None or len(starts) != rows:
+        raise RuntimeError("mask_block_tokens needs chunk_key_start with one entry per row")
+    for x in starts:
+        if x < 0 or x + q_tokens > max_seq_len:
+            raise RuntimeError(f"chunk_key_start {x} puts the chunk outside the {max_seq_len}-key view")
+
+
 def chunk_starts_tensor(starts, rows: int, q_tokens: int, max_seq_len: int, dev) -> torch.Tensor:
     """Per-row cache position of the chunk's own keys as the int32 device
     tensor the attention kernel reads; host values are range-checked here."""
@@ -344,34 +352,8 @@ def chunk_starts_tensor(starts, rows: int, q_tokens: int, max_seq_len: int, dev)
         if starts.dtype != torch.int32 or starts.numel() != rows or starts.device != dev or not starts.is_contiguous():
             raise RuntimeError("chunk_key_start must be a contiguous int32 device tensor with one entry per row")
         return starts
-    if starts is None or len(starts) != rows:
-        raise RuntimeError("mask_block_tokens needs chunk_key_start with one entry per row")
-    for x in starts:
-        if x < 0 or x + q_tokens > max_seq_len:
-            raise RuntimeError(f"chunk_key_start {x} puts the chunk outside the {max_seq_len}-key view")
+    _check_chunk_starts(starts, rows, q_tokens, max_seq_len)
     return torch.tensor([int(x) for x in starts], dtype=torch.int32).to(dev, non_blocking=True)
-
-
-_CHUNK_STARTS: dict = {}
-_MAX_CHUNK_STARTS = 256
-
-
-def _chunk_starts_on(starts, rows: int, q_tokens: int, max_seq_len: int, dev, stream: int) -> torch.Tensor:
-    """:func:`chunk_starts_tensor`, with host values shipped once: a stream's
-    chunks land in a handful of slots, and the copy costs 4.6 us of the stream
-    and more of the host per call.  Filed by value, per stream (the copy is
-    ordered with that stream's launches alone), never taken out again (a
-    captured graph may hold the address), not filled from inside a capture
-    (there the copy has yet to run)."""
-    if starts is None or isinstance(starts, torch.Tensor):
-        return chunk_starts_tensor(starts, rows, q_tokens, max_seq_len, dev)
-    key = (dev, stream, q_tokens, max_seq_len, rows, tuple(int(x) for x in starts))
-    hit = _CHUNK_STARTS.get(key)
-    if hit is None:
-        hit = chunk_starts_tensor(starts, rows, q_tokens, max_seq_len, dev)
-        if len(_CHUNK_STARTS) < _MAX_CHUNK_STARTS and not torch.cuda.is_current_stream_capturing():
-            _CHUNK_STARTS[key] = hit
-    return hit
 
 
 # Descriptors of the attention calls seen, everything filled in that shapes, strides and dtypes decide: checking
@@ -486,9 +468,15 @@ def swa_attention(
         p.workspace_bytes = workspace.numel() * workspace.element_size()
     p.stream = stream
     if mask_block_tokens:
-        chunk_key_start = _chunk_starts_on(chunk_key_start, rows, q_tokens, max_seq_len, dev, stream)
         p.mask_block_tokens = int(mask_block_tokens)
-        p.chunk_key_start = chunk_key_start.data_ptr()
+        if isinstance(chunk_key_start, torch.Tensor) or rows > _capi.MAX_ROWS:
+            chunk_key_start = chunk_starts_tensor(chunk_key_start, rows, q_tokens, max_seq_len, dev)
+            p.chunk_key_start = chunk_key_start.data_ptr()
+        else:
+            # host values travel in the launch's arguments
+            _check_chunk_starts(chunk_key_start, rows, q_tokens, max_seq_len)
+            key_starts = _i64_array(chunk_key_start)
+            p.chunk_key_start_host = C.cast(key_starts, C.POINTER(C.c_int64))
     if rope is not None:
         table, grid_hw, start_frames = rope
         if table.dtype != torch.float64 or not table.is_contiguous() or table.device != dev:
@@ -773,6 +761,7 @@ class LayerLauncher:
         at.k_cache, at.k_stride = k_cache.data_ptr(), _stride3(k_cache, "k_cache")
         at.v_cache, at.v_stride = v_cache.data_ptr(), _stride3(v_cache, "v_cache")
         at.rows, at.q_tokens, at.heads, at.head_dim = rows, tokens, heads, HEAD_DIM
+        at.chunk_key_start_host = C.cast(self.ds, C.POINTER(C.c_int64))       # (where the append puts the chunk's keys)
         self.at, self.at_ref = at, C.byref(at)
         self.span = -1
         self.workspace_need = 0
@@ -804,8 +793,7 @@ class LayerLauncher:
         ap.dst_start_override = dst_start_override.data_ptr() if dst_start_override is not None else None
         at.mask_block_tokens = mask_block_tokens
         if mask_block_tokens:
-            self.chunk_starts = _chunk_starts_on(plan.dst_start, self.rows, self.tokens, plan.max_seq_len, self.dev, stream)
-            at.chunk_key_start = self.chunk_starts.data_ptr()
+            _check_chunk_starts(plan.dst_start, self.rows, self.tokens, plan.max_seq_len)
         self.sf[:] = start_frames
         self.ds[:] = plan.dst_start
         self.ng[:] = plan.new_global_end

@@ -131,6 +131,72 @@ def test_block_mask_with_exact_fallback_and_lengths(gpu_device):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("rows,S,L,splits,dtype", [
+    (16, 40, 300, 1, torch.bfloat16),          # every row the launch carries a value for; waves share a query block's keys
+    (16, 100, 700, 3, torch.bfloat16),         # 32x32x16 matrix instructions
+    (3, 300, 1600, 2, torch.bfloat16),         # 16x16x32
+    (16, 70, 333, 0, torch.float32),
+    (17, 40, 300, 1, torch.bfloat16),          # more rows than travel with a launch: a device copy for the call
+])
+def test_host_and_device_starts_agree(gpu_device, rows, S, L, splits, dtype):
+    from streamdiffusionv2_amd import ops
+
+    torch.manual_seed(5)
+    q, k, v = (torch.randn(rows, n, 2, 128, device=gpu_device).to(dtype) for n in (S, L, L))
+    starts = [(37 * r) % (L - S + 1) for r in range(rows - 1)] + [L - S]
+    out = [ops.swa_attention(q, k, v, None, num_splits=splits, chunk_key_start=s, mask_block_tokens=32)
+           for s in (starts, torch.tensor(starts, dtype=torch.int32, device=gpu_device))]
+    want = oracle.attention_fp32_reference(q.cpu(), k.cpu(), v.cpu(), [L] * rows, starts, 32)
+    assert torch.equal(out[0], out[1])
+    _close(out[0], want)
+
+
+@pytest.mark.gpu
+def test_host_starts_leave_nothing_behind(gpu_device):
+    """A long-lived program meets any number of chunk positions: none of them may stay on the device."""
+    from streamdiffusionv2_amd import ops
+
+    q = torch.zeros(1, 64, 1, 128, dtype=torch.bfloat16, device=gpu_device)
+    kv = torch.zeros(1, 512, 1, 128, dtype=torch.bfloat16, device=gpu_device)
+    out = torch.empty_like(q)
+
+    def call(start):
+        ops.swa_attention(q, kv, kv, None, out=out, num_splits=1, chunk_key_start=[start], mask_block_tokens=32)
+
+    call(0)
+    before = torch.cuda.memory_allocated()
+    for start in range(1, 301):
+        call(start)
+    torch.cuda.synchronize()
+    assert torch.cuda.memory_allocated() == before
+
+
+@pytest.mark.gpu
+def test_a_captured_call_carries_starts_it_never_saw_before(gpu_device):
+    """The position is part of the recorded launch: no copy from host memory that is gone by the replay."""
+    from streamdiffusionv2_amd import ops
+
+    torch.manual_seed(6)
+    S, L = 96, 500
+    q, k, v = (torch.randn(1, n, 2, 128, device=gpu_device).bfloat16() for n in (S, L, L))
+
+    def call(start):
+        return ops.swa_attention(q, k, v, None, chunk_key_start=start, mask_block_tokens=32)
+
+    want = {s: call(torch.tensor([s], dtype=torch.int32, device=gpu_device)) for s in (0, 77, 310)}
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = [call([s]) for s in (77, 310)]
+    for _ in range(3):
+        graph.replay()
+        eager = call([0])
+        torch.cuda.synchronize()
+        for s, got in ((77, out[0]), (310, out[1]), (0, eager)):
+            assert torch.equal(got.view(torch.int16), want[s].view(torch.int16)), s
+
+
+@pytest.mark.gpu
 def test_bad_mask_arguments(gpu_device):
     from streamdiffusionv2_amd import ops
 

@@ -137,6 +137,26 @@ print("status", _capi.lib().sdv2_swa_attn_fwd(C.byref(a)))
     assert run.returncode == 0 and f"status {_capi.SDV2_ERR_INVALID_ARG}" in run.stdout, (run.returncode, run.stdout, run.stderr)
 
 
+@pytest.mark.parametrize("dtype", [_capi.DTYPE_BF16, _capi.DTYPE_F32])
+def test_host_chunk_starts_are_checked(dtype):
+    """(every refusal comes before the first HIP call)"""
+    lib = _capi.lib()
+    a = _capi.AttnParams(q=256, k_cache=512, v_cache=768, out=1024, rows=2, q_tokens=64, heads=1, head_dim=128,
+                         max_seq_len=256, num_splits=1, dtype=dtype, mask_block_tokens=32)
+    assert lib.sdv2_swa_attn_fwd(C.byref(a)) == _capi.SDV2_ERR_INVALID_ARG           # the mask needs one of the two
+    for starts, status in (((0, 193), _capi.SDV2_ERR_OUT_OF_RANGE), ((-1, 0), _capi.SDV2_ERR_OUT_OF_RANGE),
+                           ((1 << 40, 0), _capi.SDV2_ERR_OUT_OF_RANGE)):
+        host = (C.c_int64 * 2)(*starts)
+        a.chunk_key_start_host = host
+        assert lib.sdv2_swa_attn_fwd(C.byref(a)) == status, starts
+    a.chunk_key_start_host = (C.c_int64 * 2)(0, 192)
+    a.chunk_key_start = 2048
+    assert lib.sdv2_swa_attn_fwd(C.byref(a)) == _capi.SDV2_ERR_INVALID_ARG           # and not both
+    a.chunk_key_start, a.rows = None, _capi.MAX_ROWS + 1
+    a.chunk_key_start_host = (C.c_int64 * (_capi.MAX_ROWS + 1))()
+    assert lib.sdv2_swa_attn_fwd(C.byref(a)) == _capi.SDV2_ERR_INVALID_ARG           # they travel with the launch
+
+
 def test_split_heuristic_and_workspace_size():
     lib = _capi.lib()
     assert lib.sdv2_swa_attn_workspace_bytes(1, 1560, 12, 9360, 1) == 0

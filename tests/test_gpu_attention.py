@@ -512,8 +512,8 @@ def test_masked_attention_on_16x16_matrix_instructions(gpu_device, rows, S, H, L
 
 
 def test_masked_calls_with_host_starts_on_two_streams(gpu_device):
-    """Host chunk starts are shipped once per value and stream: calls that alternate between starts and streams, and
-    one captured into a graph, give what a device tensor of the starts gives."""
+    """Host chunk starts travel with the launch: calls that alternate between starts and streams, and one captured into
+    a graph, give what a device tensor of the starts gives."""
     from streamdiffusionv2_amd import ops
 
     torch.manual_seed(10)
@@ -537,7 +537,7 @@ def test_masked_calls_with_host_starts_on_two_streams(gpu_device):
         assert torch.equal(out.view(torch.int16), want[s].view(torch.int16)), s
     with pytest.raises(RuntimeError, match="outside"):
         call([L - S + 1])
-    graph, side = torch.cuda.CUDAGraph(), streams[0]           # (a stream on which the starts are there already)
+    graph, side = torch.cuda.CUDAGraph(), streams[0]
     with torch.cuda.graph(graph, stream=side):
         out = call([64])
     for _ in range(3):
