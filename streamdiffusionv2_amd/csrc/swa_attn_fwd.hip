@@ -967,6 +967,26 @@ bool decode_splits(int32_t encoded, int32_t rows, int32_t heads, SplitPlan* plan
   return plan->most() <= 64;
 }
 
+// When one XCD is done with workgroups of two lengths, handed out as the dispatcher does: the next one, longest first, to
+// the CU that is free first.
+constexpr int kCusPerXcd = kCuSlots / 8;
+double two_lengths_span(int n_long, double length, int n_short, double shorter) {
+  double free_at[kCusPerXcd] = {};
+  auto hand_out = [&](int count, double x) {
+    for (int i = 0; i < count; ++i) {
+      int cu = 0;
+      for (int c = 1; c < kCusPerXcd; ++c)
+        if (free_at[c] < free_at[cu]) cu = c;
+      free_at[cu] += x;
+    }
+  };
+  hand_out(n_long, length);
+  hand_out(n_short, shorter);
+  double span = 0;
+  for (double t : free_at) span = t > span ? t : span;
+  return span;
+}
+
 // What a call takes, in microseconds.
 //
 // The kernels of 256-row query tiles (one workgroup per CU): `base` ranges per (row, head), of every eighth of the
@@ -988,25 +1008,10 @@ double tile_kernels_us(int32_t rows, int32_t q_tokens, int32_t heads, int32_t ma
     span = (double)((workgroups + kCuSlots - 1) / kCuSlots) * length;
     busy = workgroups * length / kCuSlots;
   } else {
-    // Workgroups of two lengths, one XCD's share of them handed out as the dispatcher does: the next one, longest
-    // first, to the CU that is free first
-    constexpr int kCusPerXcd = kCuSlots / 8;
     const int group = (int)(pairs / 8);
     const double shorter = (ntiles + base) / (base + 1) + kStart;
-    double free_at[kCusPerXcd] = {};
-    auto hand_out = [&](int count, double x) {
-      for (int i = 0; i < count; ++i) {
-        int cu = 0;
-        for (int c = 1; c < kCusPerXcd; ++c)
-          if (free_at[c] < free_at[cu]) cu = c;
-        free_at[cu] += x;
-      }
-    };
     const int n_long = (group - more) * nq * base, n_short = more * nq * (base + 1);
-    hand_out(n_long, length);
-    hand_out(n_short, shorter);
-    span = 0;
-    for (double t : free_at) span = t > span ? t : span;
+    span = two_lengths_span(n_long, length, n_short, shorter);
     busy = (n_long * length + n_short * shorter) / kCusPerXcd;
     ranges += (double)more / group;
   }
@@ -1015,6 +1020,26 @@ double tile_kernels_us(int32_t rows, int32_t q_tokens, int32_t heads, int32_t ma
   if (base > 1 || more > 0)
     us += 4.1 + (base + (more > 0) > 4 ? 5.0 : 0.0) + ranges * pairs * q_tokens * (kD * 2 * 0.14e-6);
   return us;
+}
+
+// Is a plan with two counts worth what it does to the result?  Partial results travel as fp16, scaled by the row's largest
+// magnitude: a (row, head) that two workgroups share comes out 0.2 to 0.5 % further from the exact result than one that
+// a single workgroup keeps in registers to the end (2-norm, 4 x 3132 x 40 against 9396 keys: 2.037e-3 and 2.028e-3 of the
+// result, nearly all of it the rounding of the weights and of the result itself to bf16).  So the busiest CU's queue of
+// tiles, starts and partial results counted, has to get shorter by 3 %.  What falls below that line are calls of more
+// than four rounds of workgroups that the model above would split for 1.0 to 1.6 %: staying whole costs them 1 to 3 %
+// (4 x 3132 x 40 against 9396 keys 2010 us whole, 1995 split; 4 x 2928 x 40 against 8784 1679 and 1646; 3 x 6090 x 40
+// against 18270 5467 and 5285; at worst, 4 x 4284 x 16 against themselves, 544 and 514).
+bool shortens_the_queue(int32_t rows, int32_t q_tokens, int32_t heads, int32_t max_seq_len, int base, int more) {
+  constexpr double kStart = 3, kTilesPerResult = kD * 4 / 7.0e6;             // a range's results: one tile time per 3.5 MB
+  const int nq = (q_tokens + kQTile - 1) / kQTile, ntiles = (max_seq_len + kKTile - 1) / kKTile;
+  const int64_t pairs = (int64_t)rows * heads;
+  const int group = (int)(pairs / 8);
+  const double whole = (double)((pairs * nq + kCuSlots - 1) / kCuSlots) * (ntiles + kStart);
+  const double split = two_lengths_span((group - more) * nq * base, (ntiles + base - 1) / base + kStart,
+                                        more * nq * (base + 1), (ntiles + base) / (base + 1) + kStart) +
+                       (base + (double)more / group) * (pairs * q_tokens * kTilesPerResult);
+  return split < 0.97 * whole;
 }
 
 // The kernel whose workgroups are 32-row query blocks (swa_attn_fwd_wave.hip): 256 keys take 1.22 us, and up to 256
@@ -1052,6 +1077,7 @@ extern "C" int sdv2_swa_attn_default_splits(int32_t rows, int32_t q_tokens, int3
     const double t = us(base, 0);
     if (t < best_us) { best_us = t; best = base; }
   }
+  const int uniform = best;
   // A uniform count can leave the last round of workgroups mostly empty (1120 workgroups are 4.4 rounds of 256).  When
   // the (row, head) pairs divide over the eight XCDs, some pairs of each XCD's share may take one range more.  (Where
   // that is a matter of one per cent, uniform ranges are taken.)
@@ -1061,6 +1087,10 @@ extern "C" int sdv2_swa_attn_default_splits(int32_t rows, int32_t q_tokens, int3
         const double t = us(base, more);
         if (t < best_us * ((best >> 8) ? 1.0 : 0.99)) { best_us = t; best = base | (more << 8); }
       }
+  if ((best >> 8) && !shortens_the_queue(rows, q_tokens, heads, max_seq_len, best & 0xff, best >> 8)) {
+    best = uniform;
+    best_us = us(uniform, 0);
+  }
   if (wave_kernel_us(rows, q_tokens, heads, max_seq_len) < best_us) best = 1;        // (which attn_fwd then picks)
   std::lock_guard<std::mutex> guard(lock);
   last_shape[0] = rows; last_shape[1] = q_tokens; last_shape[2] = heads; last_shape[3] = max_seq_len;

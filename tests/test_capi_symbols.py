@@ -173,6 +173,14 @@ def test_split_heuristic_and_workspace_size():
     assert lib.sdv2_swa_attn_default_splits(64, 8192, 16, 512) == 1        # short cache, huge grid
 
 
+@pytest.mark.parametrize("rows,q_tokens,heads,keys", [
+    (4, 3132, 40, 9396), (4, 2850, 40, 8550), (3, 5418, 40, 10836), (4, 1890, 36, 3780), (3, 3195, 40, 6390),
+    (4, 1647, 38, 3294), (4, 4284, 16, 4284)])
+def test_long_calls_are_not_split_for_a_per_cent(rows, q_tokens, heads, keys):
+    """Partial results are fp16: calls of many rounds that gain next to nothing from a second range stay whole."""
+    assert _capi.lib().sdv2_swa_attn_default_splits(rows, q_tokens, heads, keys) == 1
+
+
 def test_missing_library_fails_loudly(monkeypatch, tmp_path):
     monkeypatch.setattr(_capi, "_LIB", None)
     monkeypatch.setattr(_capi, "LIB_PATH", tmp_path / "nope.so")
