@@ -744,7 +744,8 @@ class LayerLauncher:
             _check_norm(qk_norm, q_like.dtype, heads, dev)
             self.norm_args = ap.q_norm_weight, ap.k_norm_weight, ap.norm_eps = \
                 qk_norm[0].data_ptr(), qk_norm[1].data_ptr(), float(qk_norm[2])
-            self.norm_weights = qk_norm[:2]          # held: the descriptor keeps their addresses
+            # held (their memory, whatever becomes of a module's parameter): the descriptor keeps the addresses
+            self.norm_weights = tuple(w.detach() for w in qk_norm[:2])
         self.ap, self.ap_ref = ap, C.byref(ap)
         self.freqs_table = freqs_table
 

@@ -260,6 +260,26 @@ def test_module_with_and_without_fusion(gpu_device):
     assert (y1.float() - y0.float()).abs().max().item() <= 3e-2
 
 
+def test_kept_descriptors_keep_the_norm_weights_memory(monkeypatch):
+    """A layer's kept launch descriptors are told from a changed weight by its address, so the memory at that address
+    must not go to another tensor meanwhile: not even when a module's weight gets other storage (``p.data = ...``,
+    ``module.to(dtype)``)."""
+    from streamdiffusionv2_amd import ops
+
+    monkeypatch.setattr(ops, "_require_gpu", lambda *t: t[0].device)          # (nothing is launched)
+    heads, tokens, cap = 2, 6, 12
+    cache = [torch.zeros(1, cap, heads, 128, dtype=torch.bfloat16) for _ in range(2)]
+    index = [torch.zeros(1, dtype=torch.long) for _ in range(2)]
+    q = torch.zeros(1, tokens, heads, 128, dtype=torch.bfloat16)
+    weights = [torch.nn.Parameter(torch.ones(heads * 128, dtype=torch.bfloat16)) for _ in range(2)]
+    launcher = ops.LayerLauncher(*cache, *index, torch.zeros(16, 64, 2, dtype=torch.float64), (1, 2, 3), q,
+                                 qk_norm=(*weights, 1e-6), rope_in_attention=False)
+    for w in weights:
+        w.data = torch.full_like(w, 2.0)
+    assert [w.data_ptr() for w in launcher.norm_weights] == list(launcher.norm_args[:2])
+    assert all(bool((w == 1).all()) for w in launcher.norm_weights)
+
+
 @pytest.mark.gpu
 def test_fused_norm_argument_errors(gpu_device):
     from streamdiffusionv2_amd import ops, rope
