@@ -765,7 +765,7 @@ class LayerLauncher:
         at.chunk_key_start_host = C.cast(self.ds, C.POINTER(C.c_int64))       # (where the append puts the chunk's keys)
         self.at, self.at_ref = at, C.byref(at)
         self.span = -1
-        self.workspace_need = 0
+        self.workspace_need, self.workspace = 0, None
         at.out_stride = roped_stride                 # contiguous, like the rotated query
         self.forced_splits = 0                       # 0 = the library's own choice
         self.timers = (None, None)
@@ -818,8 +818,9 @@ class LayerLauncher:
             self.workspace_need = self.lib.sdv2_swa_attn_workspace_bytes(self.rows, self.tokens, self.heads, span,
                                                                          at.num_splits)
         if self.workspace_need:
-            # this stream's; may have been regrown by another shape
-            ws = _workspace(self.dev, self.workspace_need, stream=stream)
+            # this stream's; may have been regrown by another shape (and, by another thread's call, between here
+            # and the launch: the one this call carries is held)
+            self.workspace = ws = _workspace(self.dev, self.workspace_need, stream=stream)
             at.workspace, at.workspace_bytes = ws.data_ptr(), ws.numel()
         out = torch.empty(self.in_shape, dtype=torch.bfloat16, device=self.dev)
         at.out = out.data_ptr()

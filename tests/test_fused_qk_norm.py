@@ -280,6 +280,34 @@ def test_kept_descriptors_keep_the_norm_weights_memory(monkeypatch):
     assert all(bool((w == 1).all()) for w in launcher.norm_weights)
 
 
+def test_a_patched_call_keeps_its_workspace_until_it_is_launched(monkeypatch):
+    """Between the filling-in of a call and its launch another thread may make the stream's workspace grow: the buffer
+    whose address the call carries must not be freed under it."""
+    import gc
+    import types
+    import weakref
+
+    from streamdiffusionv2_amd import ops
+
+    monkeypatch.setattr(ops, "_require_gpu", lambda *t: t[0].device)          # (nothing is launched)
+    monkeypatch.setattr(ops, "_stream_ptr", lambda dev: 0)
+    monkeypatch.setattr(ops, "_WORKSPACES", {})
+    heads, tokens, cap = 2, 6, 1200
+    cache = [torch.zeros(1, cap, heads, 128, dtype=torch.bfloat16) for _ in range(2)]
+    index = [torch.zeros(1, dtype=torch.long) for _ in range(2)]
+    q = torch.zeros(1, tokens, heads, 128, dtype=torch.bfloat16)
+    launcher = ops.LayerLauncher(*cache, *index, torch.zeros(16, 64, 2, dtype=torch.float64), (1, 2, 3), q,
+                                 rope_in_attention=False)
+    launcher.forced_splits = 2
+    plan = types.SimpleNamespace(dst_start=[0], new_global_end=[6], new_local_end=[6], max_seq_len=cap)
+    launcher.patch(q, q, q, [0], plan)
+    carried = weakref.ref(ops._WORKSPACES[(launcher.dev, 0)])
+    assert launcher.at.workspace == carried().data_ptr()
+    ops._workspace(launcher.dev, launcher.workspace_need + 1, stream=0)       # another call, a larger one
+    gc.collect()
+    assert carried() is not None and carried() is not ops._WORKSPACES[(launcher.dev, 0)]
+
+
 @pytest.mark.gpu
 def test_fused_norm_argument_errors(gpu_device):
     from streamdiffusionv2_amd import ops, rope
