@@ -328,15 +328,6 @@ def _workspace(dev: torch.device, nbytes: int, pool: Optional[dict] = None, stre
     return ws
 
 
-def release_scratch() -> None:
-    """Give back the scratch buffers kept per (device, stream): split-KV and
-    sink-similarity workspaces.  Calls already enqueued keep what they use until
-    the stream is past them (the allocator's own rule); not for programs that
-    still replay graphs captured over these calls."""
-    for pool in (_WORKSPACES, _SIM_WORKSPACES):
-        pool.clear()
-
-
 def _check_chunk_starts(starts, rows: int, q_tokens: int, max_seq_len: int) -> None:
     if starts is None or len(starts) != rows:
         raise RuntimeError("mask_block_tokens needs chunk_key_start with one entry per row")
