@@ -19,8 +19,6 @@ namespace attn {
 
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
 typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2;
-typedef __attribute__((ext_vector_type(4))) short s16x4;
-typedef __attribute__((ext_vector_type(8))) short s16x8;
 typedef __attribute__((ext_vector_type(16))) float f32x16;
 typedef __attribute__((ext_vector_type(2))) float f32x2;
 typedef __attribute__((ext_vector_type(4))) float f32x4;
@@ -125,12 +123,6 @@ __device__ __forceinline__ uint32_t pack_f16x2(float lo, float hi) {
   return __builtin_bit_cast(uint32_t, __builtin_convertvector(x, f16x2));
 }
 
-// acc + lo + hi of a packed bf16 pair (v_dot2c_f32_bf16 against (1, 1))
-__device__ __forceinline__ float add_bf16_pair(uint32_t packed, float acc) {
-  const bf16x2 ones = {(__bf16)1.0f, (__bf16)1.0f};
-  return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2, packed), ones, acc, false);
-}
-
 // ---------------------------------------------------------------------------
 // LDS reads with hand-placed waits.  The compiler treats every LDS access as
 // possibly aliasing an in-flight global->LDS transfer and would drain all
@@ -219,27 +211,10 @@ __device__ __forceinline__ void store_coherent_x4(void* base, const u32x4& w0, c
       : "v"(base), "v"(w0), "v"(w1), "v"(w2), "v"(w3)
       : "memory");
 }
-// One block's partial output as this lane holds it: eight 16-byte pieces 1 KB
-// apart.  Issue and wait are ONE asm statement: between a load's issue and its
-// return the compiler believes the destination registers hold the value, and
-// is free to copy them elsewhere and reuse them - as an address, say - for the
-// load to overwrite when it lands.
-__device__ __forceinline__ void load_coherent_x8(const char* base, u32x4 (&w)[8]) {
-  asm volatile(
-      "global_load_dwordx4 %0, %8, off sc1\n\t"
-      "global_load_dwordx4 %1, %8, off offset:1024 sc1\n\t"
-      "global_load_dwordx4 %2, %8, off offset:2048 sc1\n\t"
-      "global_load_dwordx4 %3, %8, off offset:3072 sc1\n\t"
-      "global_load_dwordx4 %4, %9, off sc1\n\t"
-      "global_load_dwordx4 %5, %9, off offset:1024 sc1\n\t"
-      "global_load_dwordx4 %6, %9, off offset:2048 sc1\n\t"
-      "global_load_dwordx4 %7, %9, off offset:3072 sc1\n\t"
-      "s_waitcnt vmcnt(0)"
-      : "=&v"(w[0]), "=&v"(w[1]), "=&v"(w[2]), "=&v"(w[3]), "=&v"(w[4]), "=&v"(w[5]), "=&v"(w[6]), "=&v"(w[7])
-      : "v"(base), "v"(base + 4096)
-      : "memory");
-}
-// four 1-KB-apart pieces of each of four blocks in one trip to memory
+// Four 16-byte pieces, 1 KB apart, of each of four blocks' partial outputs in one trip to memory.  Issue and wait
+// are ONE asm statement: between a load's issue and its return the compiler believes the destination registers hold
+// the value, and is free to copy them elsewhere and reuse them - as an address, say - for the load to overwrite when
+// it lands.
 __device__ __forceinline__ void load_coherent_4x4(const char* b0, const char* b1, const char* b2, const char* b3,
                                                   u32x4 (&w)[4][4]) {
   asm volatile(

@@ -162,13 +162,6 @@ __device__ __forceinline__ void issue_matrix_tile(const char* base, uint32_t tok
   }
 }
 
-// The compiler does not know that the asm MFMAs are still in flight when the
-// asm statement retires, so wherever code it generates may touch S or O right
-// after a slot (register moves at control-flow joins, the epilogue) the matrix
-// pipe is drained first: an 8-pass MFMA needs 18 wait states before its result
-// may be read.  The tag makes every use textually distinct, otherwise identical
-// drains at the ends of sibling branches are merged into one AFTER the join,
-// behind the very moves they are meant to precede.
 // Row sums of the packed weights: one 16x16x32 MFMA per 16 keys, whose A operand
 // (`pick`, see LaneConst) adds up, for every lane, the weights of the lane's own
 // query.  (v_dot2c_f32_bf16 did it on the vector side, two weights an instruction,
@@ -177,6 +170,13 @@ __device__ __forceinline__ void mfma_row_sum(f32x4& d, const u32x4& pick, const 
   asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(d) : "a"(pick), "v"(p));
 }
 
+// The compiler does not know that the asm MFMAs are still in flight when the
+// asm statement retires, so wherever code it generates may touch S or O right
+// after a slot (register moves at control-flow joins, the epilogue) the matrix
+// pipe is drained first: an 8-pass MFMA needs 18 wait states before its result
+// may be read.  The tag makes every use textually distinct, otherwise identical
+// drains at the ends of sibling branches are merged into one AFTER the join,
+// behind the very moves they are meant to precede.
 template <int kTag>
 __device__ __forceinline__ void mfma_drain(f32x16 (&oacc)[4], f32x16 (&s)[2]) {
   asm volatile("s_nop 15\n\ts_nop 15 ; matrix pipe drained, site %6"
@@ -902,10 +902,8 @@ struct WorkspaceLayout {
   size_t tickets, part_o, part_lse, part_scale, total;
 };
 WorkspaceLayout workspace_layout(int32_t rows, int32_t q_tokens, int32_t heads, int32_t num_splits) {
-  const size_t nq = (size_t)(q_tokens + kQTile - 1) / kQTile;
   const size_t blocks = (size_t)rows * heads * ((q_tokens + kQBlock - 1) / kQBlock);
   WorkspaceLayout w;
-  (void)nq;
   w.tickets = 0;
   w.part_o = (size_t)kMaxTickets * sizeof(int32_t);
   w.part_lse = w.part_o + (size_t)num_splits * blocks * kPartBlockHalves * sizeof(uint16_t);

@@ -277,8 +277,9 @@ __device__ __forceinline__ void slot(const LaneConst& c, const bf16x8 (&qf)[2][4
   static_for<8>([&](auto gc) {
     constexpr int g = decltype(gc)::value, a = g + kAhead;
     constexpr bool kSame = a < 8;                 // the reads of group a belong to this slot
-    // LDS returns in order: a fragment is there once at most the reads issued after it are in flight.  Those are the
-    // group's own V reads (behind its K read), the groups up to a, and group a's K read by the time V is waited for.
+    // LDS returns in order: a fragment is there once at most the reads issued after it are in flight.  A group's first
+    // product waits for its K and V reads together, until only the groups between it and a are in flight; in a slot
+    // without scores V waits by itself, and group a's K read may be in flight too.
     // (Groups below kAhead were requested by the slot before, which asks for both.)
     constexpr auto k_reads = [](int x) { return x >= 8 ? (kNext ? 1 : 0) : (x < kAhead || kDoS ? 1 : 0); };
     constexpr auto v_reads = [](int x) { return x >= 8 ? (kNext ? 2 : 0) : (x < kAhead || kDoPV ? 2 : 0); };
@@ -287,7 +288,7 @@ __device__ __forceinline__ void slot(const LaneConst& c, const bf16x8 (&qf)[2][4
       for (int x = g + 1; x < a; ++x) sum += k_reads(x) + v_reads(x);
       return sum;
     }();
-    constexpr int kPendingK = v_reads(g) + kBetween, kPendingV = kBetween + k_reads(a);
+    constexpr int kPendingV = kBetween + k_reads(a);
     using T0 = std::integral_constant<int, 2 * g>;
     using T1 = std::integral_constant<int, 2 * g + 1>;
 
