@@ -375,7 +375,7 @@ class RingKVPath:
             )
             mask = dict(chunk_key_start=list(plan.dst_start), mask_block_tokens=mask_tokens) if mask_tokens else {}
             # (fp32 storage, the reference's CPU-runnable configuration, is computed in
-            # fp32 throughout by a plain kernel; the matrix-core kernel is the bf16 one)
+            # fp32 throughout, on the fp32 matrix instructions)
             out = ops.swa_attention(roped_q, kv_cache["k"][:, :span], kv_cache["v"][:, :span], seq, **mask)
             if return_roped_query:
                 return out, roped_q
