@@ -286,6 +286,11 @@ def causal_rope_apply(x: torch.Tensor, grid_sizes, freqs: torch.Tensor, start_fr
 
 
 _WORKSPACES: dict = {}
+_CAPTURED_WORKSPACES: list = []       # (at most one per stream and growth step of its buffer)
+
+
+def _capturing(dev: torch.device) -> bool:
+    return dev.type == "cuda" and torch.cuda.is_current_stream_capturing()
 
 
 TICKET_BYTES = 65536          # head of an attention workspace (256 bytes for a sink-similarity one)
@@ -318,12 +323,21 @@ def _workspace(dev: torch.device, nbytes: int, pool: Optional[dict] = None, stre
     """Scratch for split-KV partials, one buffer per (device, stream), grown on
     demand and reused.  Calls on one stream run one after another, so they can
     share a buffer; calls on different streams may overlap in time and must not
-    (their tickets and partial results would mix), so each stream gets its own."""
+    (their tickets and partial results would mix), so each stream gets its own.
+
+    Under capture: a buffer that is there already is never freed again, however
+    the pool grows (the graph writes to it at every replay); one made inside the
+    capture is the graph's own and not filed (its zeros are part of the graph,
+    and nothing has filled it yet)."""
     pool = _WORKSPACES if pool is None else pool
     key = (dev, _stream_ptr(dev) if stream is None else stream)
     ws = pool.get(key)
-    if ws is None or ws.numel() < nbytes:
-        ws = new_workspace(dev, nbytes)
+    if ws is not None and ws.numel() >= nbytes:
+        if _capturing(dev) and not any(ws is kept for kept in _CAPTURED_WORKSPACES):
+            _CAPTURED_WORKSPACES.append(ws)
+        return ws
+    ws = new_workspace(dev, nbytes)
+    if not _capturing(dev):
         pool[key] = ws
     return ws
 

@@ -308,6 +308,34 @@ def test_a_patched_call_keeps_its_workspace_until_it_is_launched(monkeypatch):
     assert carried() is not None and carried() is not ops._WORKSPACES[(launcher.dev, 0)]
 
 
+def test_workspaces_under_capture(monkeypatch):
+    """(on the host, nothing is launched) A workspace that a capture has taken outlives the pool's growth; one made inside
+    a capture is not handed to later eager calls."""
+    import gc
+    import weakref
+
+    from streamdiffusionv2_amd import ops
+
+    dev = torch.device("cpu")
+    state = {"capturing": False}
+    monkeypatch.setattr(ops, "_capturing", lambda d: state["capturing"], raising=False)
+    pool = {}
+    state["capturing"] = True
+    inside = ops._workspace(dev, 1000, pool, stream=1)
+    assert inside.numel() == 1000 and pool == {}
+    state["capturing"] = False
+    first = ops._workspace(dev, 1000, pool, stream=1)
+    assert first is not inside and ops._workspace(dev, 900, pool, stream=1) is first
+    state["capturing"] = True
+    taken = weakref.ref(ops._workspace(dev, 1000, pool, stream=1))
+    assert taken() is first
+    state["capturing"] = False
+    del first
+    assert ops._workspace(dev, 2000, pool, stream=1).numel() == 2000
+    gc.collect()
+    assert taken() is not None
+
+
 @pytest.mark.gpu
 def test_fused_norm_argument_errors(gpu_device):
     from streamdiffusionv2_amd import ops, rope

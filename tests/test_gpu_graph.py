@@ -128,3 +128,31 @@ def test_layer_call_replays_from_a_hip_graph(gpu_device, adaptive):
             assert err.max().item() <= MAX_ABS and err.mean().item() <= MEAN_ABS
     if adaptive:
         assert refreshed - {-7}, "the decision kernel never ran in a replay"
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_split_call_captured_without_a_warm_up_of_its_stream(gpu_device, monkeypatch, dtype):
+    """The workspace is made inside the capture: every replay, with larger eager calls between them on the stream that
+    was captured, equals the eager result, and so do the eager calls."""
+    from streamdiffusionv2_amd import ops
+
+    torch.manual_seed(12)
+    side = torch.cuda.Stream()
+    monkeypatch.setattr(ops, "_WORKSPACES", {})           # (the stream's handle may have served another test)
+    q, k, v = (torch.randn(1, n, 3, 128, device=gpu_device).to(dtype) for n in (160, 2000, 2000))
+    qq = torch.randn(2, 160, 3, 128, device=gpu_device).to(dtype)
+    kk, vv = (torch.randn(2, 3000, 3, 128, device=gpu_device).to(dtype) for _ in range(2))
+    want, more = ops.swa_attention(q, k, v, num_splits=3), ops.swa_attention(qq, kk, vv, num_splits=4)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=side):
+        out = ops.swa_attention(q, k, v, num_splits=3)
+    for replay in range(4):
+        out.zero_()
+        torch.cuda.synchronize()
+        with torch.cuda.stream(side):
+            graph.replay()
+            eager = ops.swa_attention(qq, kk, vv, num_splits=4)
+        torch.cuda.synchronize()
+        assert torch.equal(out, want), replay
+        assert torch.equal(eager, more), replay
