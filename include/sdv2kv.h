@@ -35,8 +35,9 @@ extern "C" {
  *     (12 ignored it), so its ticket words must be zero like any other's;
  *     sdv2_swa_attn_fwd_static runs a call with num_splits = 0 unsplit where the
  *     library's own plan needs more than SDV2_STATIC_SCRATCH_BYTES (12 refused it)
- * 14: sdv2_attn_params.chunk_key_start_host */
-#define SDV2KV_ABI_VERSION 14
+ * 14: sdv2_attn_params.chunk_key_start_host
+ * 15: sdv2_cache_relayout_pair */
+#define SDV2KV_ABI_VERSION 15
 #define SDV2_HEAD_DIM 128      /* causal_stream_inference.py:99-100 fixes 128 */
 #define SDV2_MAX_ROWS 16       /* rows (B) per sdv2_kv_append_rope call       */
 #define SDV2_MAX_SINK_FRAMES 16 /* sink frames per sdv2_sink_similarity call  */
@@ -382,6 +383,11 @@ typedef struct sdv2_relayout_params {
 } sdv2_relayout_params;
 
 int sdv2_cache_relayout(const sdv2_relayout_params* p);
+
+/* The two calls in this order, K and V of a block, say.  Both are looked over
+ * before anything is launched; tensors of one shape, dtype and stream, the
+ * indices handed over with `first` alone, are one launch.                     */
+int sdv2_cache_relayout_pair(const sdv2_relayout_params* first, const sdv2_relayout_params* second);
 
 /* ------------------------------------------------------------------------
  * RMS norm over the model width, as a call of its own.

@@ -12,7 +12,7 @@ from typing import Optional
 
 LIB_PATH = Path(__file__).resolve().parent / "_lib" / "libsdv2kv.so"
 
-ABI_VERSION = 14
+ABI_VERSION = 15
 HEAD_DIM = 128
 MAX_ROWS = 16
 
@@ -45,6 +45,7 @@ EXPORTED_SYMBOLS = (
     "sdv2_sink_frame_sums_bytes",
     "sdv2_sink_similarity",
     "sdv2_cache_relayout",
+    "sdv2_cache_relayout_pair",
     "sdv2_rms_norm",
     "sdv2_event_create",
     "sdv2_event_destroy",
@@ -216,6 +217,8 @@ def lib() -> C.CDLL:
     handle.sdv2_sink_similarity.argtypes = [C.POINTER(SinkSimParams)]
     handle.sdv2_cache_relayout.restype = C.c_int
     handle.sdv2_cache_relayout.argtypes = [C.POINTER(RelayoutParams)]
+    handle.sdv2_cache_relayout_pair.restype = C.c_int
+    handle.sdv2_cache_relayout_pair.argtypes = [C.POINTER(RelayoutParams)] * 2
     handle.sdv2_rms_norm.restype = C.c_int
     handle.sdv2_rms_norm.argtypes = [C.POINTER(RmsNormParams)]
     handle.sdv2_event_create.restype = C.c_int

@@ -11,7 +11,7 @@ What is built here is everything on ONE device: the wire format and the two
 copies at its ends.  The reference broadcasts its token-major
 [B, cap, H, 128] tensors as they are; this package keeps a cache head-major in
 HBM, so a block is brought into the reference's wire layout by
-``export_block`` (one launch per tensor, ``sdv2_cache_relayout``) and absorbed
+``export_block`` (k and v in one launch, ``sdv2_cache_relayout_pair``) and absorbed
 by ``import_block`` (the same kernel the other way, with the index hand-over
 and the rank shift folded into the launch).  The transport between the two is
 the caller's: ``KVCacheManager`` takes it as the ``exchange`` callable, which on
@@ -100,8 +100,7 @@ def export_block(entry: dict, wire: Optional[BlockWire] = None) -> BlockWire:
     if wire is None:
         wire = new_wire_like(entry)
     src_idx = (entry["global_end_index"], entry["local_end_index"])
-    ops.cache_relayout(wire.k, entry["k"], (wire.global_end_index, wire.local_end_index), src_idx, 0)
-    ops.cache_relayout(wire.v, entry["v"])
+    ops.cache_relayout_pair((wire.k, wire.v), (entry["k"], entry["v"]), (wire.global_end_index, wire.local_end_index), src_idx)
     return wire
 
 
@@ -111,8 +110,7 @@ def import_block(entry: dict, wire: BlockWire, donor_rank: int, rank: int, frame
     keep their layout and identity) and ``global_end_index`` is shifted."""
     shift = global_end_shift(donor_rank, rank, frame_seq_length, time_step_length)
     dst_idx = (entry["global_end_index"], entry["local_end_index"])
-    ops.cache_relayout(entry["k"], wire.k, dst_idx, (wire.global_end_index, wire.local_end_index), shift)
-    ops.cache_relayout(entry["v"], wire.v)
+    ops.cache_relayout_pair((entry["k"], entry["v"]), (wire.k, wire.v), dst_idx, (wire.global_end_index, wire.local_end_index), shift)
     ring.forget_index_mirror(entry)      # the host copy of the indices is stale now
 
 

@@ -904,19 +904,7 @@ def flash_attention(q, k, v, q_lens=None, k_lens=None, dropout_p=0.0, softmax_sc
     return out if out_dtype == torch.bfloat16 else out.to(out_dtype)
 
 
-def cache_relayout(
-    dst: torch.Tensor,
-    src: torch.Tensor,
-    dst_indices: Optional[Tuple[torch.Tensor, torch.Tensor]] = None,
-    src_indices: Optional[Tuple[torch.Tensor, torch.Tensor]] = None,
-    global_end_shift: int = 0,
-    timer: Optional["KernelTimer"] = None,
-) -> None:
-    """``dst[...] = src[...]`` for two [rows, cap, heads, 128] tensors in any
-    stride order, plus, with both index pairs (global_end_index,
-    local_end_index) given, ``dst_global = src_global + global_end_shift`` and
-    ``dst_local = src_local`` in the same launch: one side of the block
-    hand-off of streamv2v/communication/kv_cache_manager.py:66-82."""
+def _relayout_params(dst, src, dst_indices, src_indices, global_end_shift):
     flat = [dst, src] + list(dst_indices or ()) + list(src_indices or ())
     dev = _require_gpu(*flat)
     if src.dtype not in _DTYPES or dst.dtype != src.dtype:
@@ -939,10 +927,44 @@ def cache_relayout(
         p.src_global_end_index, p.src_local_end_index = (t.data_ptr() for t in src_indices)
         p.global_end_shift = int(global_end_shift)
     p.stream = _stream_ptr(dev)
+    return p, dev
+
+
+def cache_relayout(
+    dst: torch.Tensor,
+    src: torch.Tensor,
+    dst_indices: Optional[Tuple[torch.Tensor, torch.Tensor]] = None,
+    src_indices: Optional[Tuple[torch.Tensor, torch.Tensor]] = None,
+    global_end_shift: int = 0,
+    timer: Optional["KernelTimer"] = None,
+) -> None:
+    """``dst[...] = src[...]`` for two [rows, cap, heads, 128] tensors in any
+    stride order, plus, with both index pairs (global_end_index,
+    local_end_index) given, ``dst_global = src_global + global_end_shift`` and
+    ``dst_local = src_local`` in the same launch: one side of the block
+    hand-off of streamv2v/communication/kv_cache_manager.py:66-82."""
+    p, dev = _relayout_params(dst, src, dst_indices, src_indices, global_end_shift)
     if timer is not None:
         timer.arm(_capi.KERNEL_RELAYOUT)
     with _on_device(dev):
         _capi.check(_capi.lib().sdv2_cache_relayout(C.byref(p)), "sdv2_cache_relayout")
+
+
+def cache_relayout_pair(
+    dst: Tuple[torch.Tensor, torch.Tensor],
+    src: Tuple[torch.Tensor, torch.Tensor],
+    dst_indices: Optional[Tuple[torch.Tensor, torch.Tensor]] = None,
+    src_indices: Optional[Tuple[torch.Tensor, torch.Tensor]] = None,
+    global_end_shift: int = 0,
+) -> None:
+    """:func:`cache_relayout` of two tensors, the indices with the first: K and
+    V of a block, one launch when both have the same shape and dtype."""
+    first, dev = _relayout_params(dst[0], src[0], dst_indices, src_indices, global_end_shift)
+    second, dev_second = _relayout_params(dst[1], src[1], None, None, 0)
+    if dev_second != dev:
+        raise RuntimeError(f"tensors on different devices: {dev} vs {dev_second}")
+    with _on_device(dev):
+        _capi.check(_capi.lib().sdv2_cache_relayout_pair(C.byref(first), C.byref(second)), "sdv2_cache_relayout_pair")
 
 
 def _norm_rows(t: torch.Tensor):

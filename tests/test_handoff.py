@@ -159,6 +159,36 @@ def test_relayout_round_trip(gpu_device, dtype, shape):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("cap,heads", [(1, 1), (7, 5), (8, 3), (15, 1), (16, 12), (17, 40), (33, 2)])
+def test_relayout_of_two_tensors(gpu_device, dtype, cap, heads):
+    """Around the 16 (bf16) and 8 (fp32) tokens of a workgroup; k and v with
+    strides of their own; a second tensor of another shape goes by itself."""
+    from streamdiffusionv2_amd import ops
+
+    rows = 2
+    gen = torch.Generator().manual_seed(cap * 100 + heads)
+    k, v, u = (torch.randn(rows, cap + extra, heads, 128, generator=gen).to(dtype) for extra in (0, 0, 3))
+    sg, sl = torch.tensor([100, 200], device=gpu_device), torch.tensor([30, 40], device=gpu_device)
+    wide = torch.zeros(rows, heads, cap + 5, 128, dtype=dtype, device=gpu_device)
+    src_v = wide.permute(0, 2, 1, 3)[:, :cap]                  # head-major, longer than the block
+    src_v.copy_(v)
+    for src, want in (((k.to(gpu_device), src_v), (k, v)), ((k.to(gpu_device), u.to(gpu_device)), (k, u))):
+        dst = (torch.zeros(rows, heads, want[0].shape[1], 128, dtype=dtype, device=gpu_device).permute(0, 2, 1, 3),
+               torch.zeros(rows, want[1].shape[1], heads, 128, dtype=dtype, device=gpu_device))
+        dg, dl = torch.zeros_like(sg), torch.zeros_like(sl)
+        ops.cache_relayout_pair(dst, src, (dg, dl), (sg, sl), 7)
+        torch.cuda.synchronize()
+        for got, ref in zip(dst, want):
+            assert torch.equal(_bits(got.cpu()), _bits(ref))
+        assert dg.tolist() == [107, 207] and dl.tolist() == [30, 40]
+    before = dst[0].clone()
+    with pytest.raises(RuntimeError):            # the second is refused: the first is not moved either
+        ops.cache_relayout_pair((dst[0], dst[1][:1].expand(rows, -1, -1, -1)), (torch.zeros_like(k, device=gpu_device), src[1]))
+    assert torch.equal(dst[0], before)
+
+
+@pytest.mark.gpu
 def test_relayout_indices_and_errors(gpu_device):
     from streamdiffusionv2_amd import ops
 
