@@ -13,6 +13,7 @@
 #include "sdv2kv.h"
 #include "sdv2kv_internal.h"
 #include "rope_device.h"
+#include "attn_tiles.h"
 
 namespace sdv2 {
 namespace attn {
@@ -38,22 +39,6 @@ constexpr int kPieces = 16 / kIssuers;      // global->LDS instructions per issu
 constexpr int kStageBytes = 16384;          // epilogue staging per wave
 constexpr int kMaxDevices = 64;
 constexpr int kPartBlockHalves = kQBlock * kD;   // one block's partial output: 32 x 128 fp16 = 8 KB
-
-// Division of a number below 2^31 by a launch constant without a division: the
-// work list is decoded by every workgroup before it can ask for its first tile,
-// and six integer divisions are a microsecond on the way there.
-struct FastDiv {
-  uint32_t mul, shift;
-  static FastDiv by(uint32_t d) {
-    FastDiv f{1, 0};
-    while ((1ull << f.shift) < d) ++f.shift;
-    f.mul = (uint32_t)(((1ull << 32) * ((1ull << f.shift) - d)) / d + 1);
-    return f;
-  }
-  __device__ __forceinline__ int operator()(int n) const {
-    return (int)((__umulhi((uint32_t)n, mul) + (uint32_t)n) >> shift);
-  }
-};
 
 struct AttnKernelArgs {
   const uint16_t* q;
@@ -90,9 +75,24 @@ struct AttnKernelArgs {
   const float* q_inv_rms;
   sdv2::ChunkStarts chunk_starts;   // with the mask inside the chunk
 };
-__device__ __forceinline__ int row_chunk_start(const AttnKernelArgs& a, int row) {
-  return sdv2::row_chunk_start<offsetof(AttnKernelArgs, chunk_starts)>(a.chunk_starts, row);
+template <typename Args>
+__device__ __forceinline__ int row_chunk_start(Args& a, int row) {
+  return sdv2::row_chunk_start<offsetof(AttnKernelArgs, chunk_starts)>(a.chunk_starts.device, row);
 }
+
+// The kernel's arguments, read where they lie each time: what is held from the start of a kernel to its end for the
+// few places that need it crowds the scalar registers of the loop between: seventy of them lived in vector registers, and
+// some of those in scratch memory.  (With the offsets of issue_tile out of the way too, no register of the m16 kernel is
+// spilled: six layers of 1560 x 12 heads against 9360 keys 556 -> 541 us, layer calls and all.)
+template <typename Args>
+using late_args = const __attribute__((address_space(4))) Args;
+template <typename Args>
+__device__ __forceinline__ late_args<Args>& read_late() {
+  auto* p = (late_args<Args>*)__builtin_amdgcn_kernarg_segment_ptr();
+  asm volatile("" : "+s"(p));
+  return *p;
+}
+__device__ __forceinline__ FastDiv read_div(late_args<FastDiv>& d) { return FastDiv{d.mul, d.shift}; }
 
 // v_max without the NaN-quieting canonicalisation fmaxf() drags in.
 __device__ __forceinline__ float vmax(float a, float b) {
@@ -264,7 +264,8 @@ struct QueryRope {
 
 // the row's first absolute frame (constant indices and selects: indexing the by-value argument block with a
 // run-time row would move the whole block, its pointers included, out of scalar registers)
-__device__ __forceinline__ int64_t row_start_frame(const AttnKernelArgs& a, int row) {
+template <typename Args>
+__device__ __forceinline__ int64_t row_start_frame(Args& a, int row) {
   int64_t frame = a.start_frame[0];
   static_for<SDV2_MAX_ROWS - 1>([&](auto ic) {
     constexpr int i = decltype(ic)::value + 1;

@@ -63,11 +63,11 @@ struct ChunkStarts {
 // (Read where the arguments lie: indexing the by-value block with a run-time row would move the whole block out of
 // scalar registers.)
 template <int kOffset>
-__device__ __forceinline__ int row_chunk_start(const ChunkStarts& starts, int row) {
+__device__ __forceinline__ int row_chunk_start(const int32_t* device, int row) {
   typedef const __attribute__((address_space(4))) char* arg_bytes;
   typedef const __attribute__((address_space(4))) int32_t* arg_words;
   const arg_words carried = (arg_words)((arg_bytes)__builtin_amdgcn_kernarg_segment_ptr() + kOffset + offsetof(ChunkStarts, value));
-  return starts.device ? starts.device[row] : carried[row];
+  return device ? device[row] : carried[row];
 }
 // host: fill `starts` from a call's parameters; the mask is on
 inline int set_chunk_starts(const sdv2_attn_params& p, ChunkStarts* starts) {

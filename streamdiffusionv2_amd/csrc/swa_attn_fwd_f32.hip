@@ -182,7 +182,7 @@ void swa_attn_fwd_f32_kernel(const AttnF32Args a) {
   // the chunk's own later blocks, hidden from this lane's query when the mask inside the chunk is on
   int m_lo = 0x7fffffff, m_hi = 0;
   if (a.mask_block_tokens > 0) {
-    const int first = sdv2::row_chunk_start<offsetof(AttnF32Args, chunk_starts)>(a.chunk_starts, row);
+    const int first = sdv2::row_chunk_start<offsetof(AttnF32Args, chunk_starts)>(a.chunk_starts.device, row);
     m_hi = first + a.q_tokens;
     m_lo = first + (q_row / a.mask_block_tokens + 1) * a.mask_block_tokens;
   }
