@@ -35,7 +35,9 @@ PEAK_HBM_GBS = 8000.0       # MI355X HBM3E
 # only used for the kernels it was taken on: same key-range split count, same
 # kernel sources (hash below); otherwise `traffic` is null and stderr says why.
 TRAFFIC_JSON = os.path.join(ROOT, "profiles", "hbm_traffic.json")
-KERNEL_SOURCES = ("swa_attn_fwd.hip", "swa_attn_fwd_m16.hip", "swa_attn_fwd_wave.hip", "attn_device.h", "kv_append_rope.hip", "rope_device.h", "sdv2kv_internal.h")
+KERNEL_SOURCES = ("swa_attn_fwd.hip", "swa_attn_fwd_m16.hip", "swa_attn_fwd_even.hip", "swa_attn_fwd_wave.hip", "attn_device.h",
+                  "attn_m16_device.h", "attn_wave_device.h", "attn_tiles.h", "attn_even_plan.h", "kv_append_rope.hip",
+                  "rope_device.h", "sdv2kv_internal.h")
 
 
 def kernel_source_hash() -> str:
@@ -81,7 +83,8 @@ def record_traffic(args, w):
             raise SystemExit(f"no counter_collection.csv under {args.record_traffic}/{sub}")
         total, count = collections.defaultdict(float), collections.Counter()
         for row in csv.DictReader(open(files[0])):
-            for short, names in (("swa_attn_fwd_kernel", ("swa_attn_fwd_kernel", "swa_attn_fwd_m16_kernel", "swa_attn_fwd_wave_kernel")),
+            for short, names in (("swa_attn_fwd_kernel", ("swa_attn_fwd_kernel", "swa_attn_fwd_m16_kernel", "swa_attn_fwd_even_kernel",
+                                                          "swa_attn_fwd_wave_kernel")),
                                  ("kv_append_rope_kernel", ("kv_append_rope_kernel",)), ("copy16_kernel", ("copy16_kernel",))):
                 if any(n in row["Kernel_Name"] for n in names):
                     total[short] += float(row["Counter_Value"])
@@ -95,7 +98,7 @@ def record_traffic(args, w):
     from streamdiffusionv2_amd import _capi
 
     rec = {
-        "splits": args.num_splits or _capi.lib().sdv2_swa_attn_default_splits(w.rows, w.chunk_tokens, w.heads, w.cache_tokens),
+        "splits": args.num_splits or _capi.lib().sdv2_swa_attn_plan(w.rows, w.chunk_tokens, w.heads, w.cache_tokens),
         "kernel_sources": kernel_source_hash(),
         "fetch_scale": f_scale, "write_scale": w_scale,
         "attn": (fetch["swa_attn_fwd_kernel"] * f_scale + write["swa_attn_fwd_kernel"] * w_scale) * 1024,
@@ -283,7 +286,7 @@ def gpu_bench(args, w):
         for x in t:
             if x:
                 x.close()
-    splits = args.num_splits or _capi.lib().sdv2_swa_attn_default_splits(B, S, H, w.cache_tokens)
+    splits = args.num_splits or _capi.lib().sdv2_swa_attn_plan(B, S, H, w.cache_tokens)
     fill_ms = None
     if args.fill_phase:
         # a second, fresh stream from chunk 0: latency of every chunk while the ring fills
@@ -1085,7 +1088,8 @@ def main():
             "chunk_tokens": w.chunk_tokens, "cache_tokens": w.cache_tokens,
             "grid": list(w.grid), "kv_splits": g["splits"] & 255,
             # of each XCD's share of the (row, head) pairs, how many take one key range more
-            "kv_splits_one_more_on_pairs_per_xcd": g["splits"] >> 8,
+            "kv_splits_one_more_on_pairs_per_xcd": g["splits"] >> 8 & 255,
+            "kv_equal_shares": g["splits"] == 1 << 20,
         },
         "roofline": {
             "kernel": "swa_attn_fwd_kernel",

@@ -36,8 +36,9 @@ extern "C" {
  *     sdv2_swa_attn_fwd_static runs a call with num_splits = 0 unsplit where the
  *     library's own plan needs more than SDV2_STATIC_SCRATCH_BYTES (12 refused it)
  * 14: sdv2_attn_params.chunk_key_start_host
- * 15: sdv2_cache_relayout_pair */
-#define SDV2KV_ABI_VERSION 15
+ * 15: sdv2_cache_relayout_pair
+ * 16: SDV2_SPLITS_EVEN, sdv2_swa_attn_plan */
+#define SDV2KV_ABI_VERSION 16
 #define SDV2_HEAD_DIM 128      /* causal_stream_inference.py:99-100 fixes 128 */
 #define SDV2_MAX_ROWS 16       /* rows (B) per sdv2_kv_append_rope call       */
 #define SDV2_MAX_SINK_FRAMES 16 /* sink frames per sdv2_sink_similarity call  */
@@ -242,6 +243,14 @@ typedef struct sdv2_attn_params {
 
 /* the key-range split plan the library would pick for this shape, as num_splits carries it */
 int sdv2_swa_attn_default_splits(int32_t rows, int32_t q_tokens, int32_t heads, int32_t max_seq_len);
+/* num_splits for equal shares: every workgroup of the launch gets the same amount of
+ * work, whole query tiles first and then a contiguous share of the key tiles that are
+ * left, so a query tile's keys may be cut anywhere; partial results are fp32.  For
+ * SDV2_BF16, queries that arrive rotated (no rope_freqs) and up to 16384 query tiles
+ * of 256 rows (else SDV2_ERR_UNSUPPORTED), and not by sdv2_swa_attn_fwd_static.      */
+#define SDV2_SPLITS_EVEN (1 << 20)
+/* sdv2_swa_attn_default_splits(), or SDV2_SPLITS_EVEN where that is the faster one */
+int sdv2_swa_attn_plan(int32_t rows, int32_t q_tokens, int32_t heads, int32_t max_seq_len);
 /* bytes of workspace needed for `num_splits` (0 = default); 0 when unsplit */
 size_t sdv2_swa_attn_workspace_bytes(int32_t rows, int32_t q_tokens, int32_t heads,
                                      int32_t max_seq_len, int32_t num_splits);

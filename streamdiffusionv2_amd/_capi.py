@@ -12,7 +12,7 @@ from typing import Optional
 
 LIB_PATH = Path(__file__).resolve().parent / "_lib" / "libsdv2kv.so"
 
-ABI_VERSION = 15
+ABI_VERSION = 16
 HEAD_DIM = 128
 MAX_ROWS = 16
 
@@ -37,6 +37,7 @@ EXPORTED_SYMBOLS = (
     "sdv2_status_string",
     "sdv2_kv_append_rope",
     "sdv2_swa_attn_default_splits",
+    "sdv2_swa_attn_plan",
     "sdv2_swa_attn_workspace_bytes",
     "sdv2_swa_attn_f32_workspace_bytes",
     "sdv2_swa_attn_fwd",
@@ -201,6 +202,8 @@ def lib() -> C.CDLL:
     handle.sdv2_kv_append_rope.argtypes = [C.POINTER(AppendParams)]
     handle.sdv2_swa_attn_default_splits.restype = C.c_int
     handle.sdv2_swa_attn_default_splits.argtypes = [C.c_int32] * 4
+    handle.sdv2_swa_attn_plan.restype = C.c_int
+    handle.sdv2_swa_attn_plan.argtypes = [C.c_int32] * 4
     handle.sdv2_swa_attn_workspace_bytes.restype = C.c_size_t
     handle.sdv2_swa_attn_workspace_bytes.argtypes = [C.c_int32] * 5
     handle.sdv2_swa_attn_f32_workspace_bytes.restype = C.c_size_t

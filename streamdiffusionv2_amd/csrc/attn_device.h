@@ -13,7 +13,7 @@
 #include "sdv2kv.h"
 #include "sdv2kv_internal.h"
 #include "rope_device.h"
-#include "attn_tiles.h"
+#include "attn_even_plan.h"
 
 namespace sdv2 {
 namespace attn {
@@ -241,6 +241,24 @@ __device__ __forceinline__ void load_coherent_4x4(const char* b0, const char* b1
       : "v"(b0), "v"(b1), "v"(b2), "v"(b3)
       : "memory");
 }
+// the same for 32 contiguous bytes per lane
+__device__ __forceinline__ void store_coherent_x2(void* base, const f32x4& w0, const f32x4& w1) {
+  asm volatile(
+      "global_store_dwordx4 %0, %1, off sc1\n\t"
+      "global_store_dwordx4 %0, %2, off offset:16 sc1"
+      :
+      : "v"(base), "v"(w0), "v"(w1)
+      : "memory");
+}
+__device__ __forceinline__ void load_coherent_x2(const void* base, f32x4& w0, f32x4& w1) {
+  asm volatile(
+      "global_load_dwordx4 %0, %2, off sc1\n\t"
+      "global_load_dwordx4 %1, %2, off offset:16 sc1\n\t"
+      "s_waitcnt vmcnt(0)"
+      : "=&v"(w0), "=&v"(w1)
+      : "v"(base)
+      : "memory");
+}
 __device__ __forceinline__ void store_coherent(float* p, float x) {
   __hip_atomic_store(reinterpret_cast<uint32_t*>(p), __float_as_uint(x), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
@@ -376,10 +394,23 @@ inline void set_work_list(AttnKernelArgs* a, int q_tile_rows) {
   a->div_heads = FastDiv::by((uint32_t)a->heads);
 }
 
+// what the kernel of equal shares is launched with (swa_attn_fwd_even.hip)
+struct EvenArgs {
+  AttnKernelArgs call;         // (first: its helpers read fields where the launch's arguments lie)
+  EvenPlan plan;
+  float* part_o;               // [workgroup][0: rest or middle of an item, 1: start of one][128 KB] fp32: normalised output
+  float* part_lse;             // [workgroup][the same][256]   log2 sum exp
+};
+constexpr int kEvenPartFloats = 256 * kD;
+constexpr int kEvenPartRows = 256;
+
 // the kernel on 16x16x32 matrix instructions (swa_attn_fwd_m16.hip)
 int launch_m16(const AttnKernelArgs& a, uint32_t workgroups, hipStream_t stream);
 // the kernel whose waves share the keys of one query block (swa_attn_fwd_wave.hip)
 int launch_wave(const AttnKernelArgs& a, uint32_t workgroups, hipStream_t stream);
+
+// the same with equal shares of the key tiles for all workgroups (swa_attn_fwd_even.hip)
+int launch_even(const EvenArgs& a, hipStream_t stream);
 
 }  // namespace attn
 }  // namespace sdv2

@@ -1,5 +1,7 @@
 // The streaming loop of the bf16 attention on 16x16x32 matrix instructions (gfx950
-// only): 8 waves = 256 query rows of one (row, head) against a range of its keys.
+// only): 8 waves = 256 query rows of one (row, head) against a range of its keys, for
+// the kernels that give a workgroup one such range (swa_attn_fwd_m16.hip) or a
+// share of several (swa_attn_fwd_even.hip).
 //
 // Keys stream through LDS in tiles of 64, four buffers per matrix, filled three tiles
 // ahead by global->LDS transfers that never touch registers; wave w owns the 32 query
@@ -443,14 +445,31 @@ __device__ __forceinline__ bool block_idle(late_args<AttnKernelArgs>& a, int qti
   return __builtin_amdgcn_readfirstlane(qtile * kQTile + wave * kQBlock >= a.q_tokens);
 }
 
+// A word of memory looked at by thread 0 before the range's last matrix instructions, for the time behind them.
+struct Peek {
+  const int32_t* word;       // null: nothing to look at
+  int want;
+  lds_int* found;            // was it that?  (for all threads, once stream_range is back)
+  __device__ __forceinline__ int begin() const {
+    return word && threadIdx.x == 0 ? __hip_atomic_load(word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0;
+  }
+  __device__ __forceinline__ void end(int seen) const {
+    if (word && threadIdx.x == 0) *found = seen == want;
+  }
+};
+struct NoPeek {
+  __device__ __forceinline__ int begin() const { return 0; }
+  __device__ __forceinline__ void end(int) const {}
+};
+
 // The workgroup's 256 query rows against entries [tile_begin, tile_end) of a tile list, the first
 // key of entry t being key0_of(t): sums of the weighted values
 // (oacc), the queries' row sums (l_sum) and the exponent references both are relative to (c.neg_ref).  Behind it every
 // wave is done with the tile buffers.
-template <bool kMask, typename KeyOf>
+template <bool kMask, typename KeyOf, typename LookAt = NoPeek>
 __device__ __forceinline__ void stream_range(late_args<AttnKernelArgs>& a, lds_char* lds, int qtile, int head, int row, int seq,
                                              KeyOf key0_of, int tile_begin, int tile_end, LaneConst& c,
-                                             f32x4 (&oacc)[8][2], float (&l_sum)[2]) {
+                                             f32x4 (&oacc)[8][2], float (&l_sum)[2], LookAt look = LookAt()) {
   lds_int* flags = reinterpret_cast<lds_int*>(lds + kLdsFlags);
   int tid = threadIdx.x;
   asm volatile("" : "+v"(tid));      // (what is derived from it is worked out per range, not held across them)
@@ -622,6 +641,7 @@ __device__ __forceinline__ void stream_range(late_args<AttnKernelArgs>& a, lds_c
   using B3 = std::integral_constant<int, 3>;
 
   const bool idle = block_idle(a, qtile, wave);
+  int seen = 0;
   if (n > 0) {
     // K tiles 0 and 1 and V tile 0 have landed once at most the four tiles requested behind them are in flight
     if (wave_u < kIssuers) {
@@ -681,6 +701,7 @@ __device__ __forceinline__ void stream_range(late_args<AttnKernelArgs>& a, lds_c
         asm volatile("s_waitcnt lgkmcnt(0)");
 #pragma unroll
         for (int g = 0; g < kAhead; ++g) asm volatile("" : "+v"(ahead.k[g]), "+v"(ahead.v[g]));
+        seen = look.begin();
         // (in place and back again: a copy of the addresses does not fit the registers)
         const uint32_t shift = (uint32_t)(((n - 1) % kStages - (kStages - 1)) * kTileBytes);
 #pragma unroll
@@ -701,10 +722,11 @@ __device__ __forceinline__ void stream_range(late_args<AttnKernelArgs>& a, lds_c
       for (int qt = 0; qt < 2; ++qt) {
         bool fine = l_sum[qt] >= 0x1p-100f && l_sum[qt] <= 0x1p100f;
         if constexpr (kMask) {
-          // (zero is right where every key of this range is hidden from the query)
+          // (zero is right where every key of this range is hidden from the query; a range that goes on from the
+          // last key to the first one holds some that are not)
           const int m_lo = c.m_first + (c.m_div(q_row + 16 * qt) + 1) * c.m_block;
           const int last = key0_of(tile_end - 1) + kKTile;
-          fine |= l_sum[qt] == 0.f && key0_of(tile_begin) >= m_lo && (last < seq ? last : seq) <= c.m_hi;
+          fine |= l_sum[qt] == 0.f && key0_of(tile_begin) >= m_lo && (last < seq ? last : seq) <= c.m_hi && last > key0_of(tile_begin);
         }
         ok &= fine;
       }
@@ -715,6 +737,7 @@ __device__ __forceinline__ void stream_range(late_args<AttnKernelArgs>& a, lds_c
     // with the K / V buffers (the epilogue stages its output there) and the flag, cleared before the
     // loop, holds every wave's word.
     if (unsafe && lane == 0) flags[0] = 1;
+    look.end(seen);
     __syncthreads();
     const int redo = flags[0];
     if (redo)

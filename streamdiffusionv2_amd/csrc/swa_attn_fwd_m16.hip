@@ -3,7 +3,7 @@
 //
 // Same operator, arguments, key-range splits and workspace as the kernel in
 // swa_attn_fwd.hip (which see for the reference lines it stands in for and for
-// the rules that pick one of the three); what differs is the matrix instruction,
+// the rules that pick one of the four); what differs is the matrix instruction,
 // with it every register layout, and the depth of the pipeline.
 //
 // What bounds it: on long launches the board's power, so what counts is the

@@ -384,7 +384,9 @@ def _attn_layout(q, k_cache, v_cache, out, num_splits: int, static_scratch: bool
         need = lib.sdv2_swa_attn_f32_workspace_bytes(rows, q_tokens, heads, max_seq_len)    # (it picks its own splits)
     else:
         if num_splits <= 0:
-            num_splits = lib.sdv2_swa_attn_default_splits(rows, q_tokens, heads, max_seq_len)
+            # (the static entry point has no room for equal shares, and their workgroups rotate no queries)
+            plan = lib.sdv2_swa_attn_default_splits if static_scratch or rope else lib.sdv2_swa_attn_plan
+            num_splits = plan(rows, q_tokens, heads, max_seq_len)
         need = 0 if static_scratch else lib.sdv2_swa_attn_workspace_bytes(rows, q_tokens, heads, max_seq_len, num_splits)
     p = _capi.AttnParams()
     p.q_stride = _stride3(q, "q")
@@ -818,8 +820,8 @@ class LayerLauncher:
         if span != self.span:
             self.span = span
             at.max_seq_len = span
-            at.num_splits = self.forced_splits or self.lib.sdv2_swa_attn_default_splits(
-                self.rows, self.tokens, self.heads, span)
+            plan = self.lib.sdv2_swa_attn_default_splits if self.rope_in_attention else self.lib.sdv2_swa_attn_plan
+            at.num_splits = self.forced_splits or plan(self.rows, self.tokens, self.heads, span)
             self.workspace_need = self.lib.sdv2_swa_attn_workspace_bytes(self.rows, self.tokens, self.heads, span,
                                                                          at.num_splits)
         if self.workspace_need:

@@ -1,0 +1,195 @@
+"""Attention with equal shares of the key tiles (num_splits = SDV2_SPLITS_EVEN):
+the integer arithmetic of the shares on the CPU, what the compiler made of the
+kernel, and its results against the fp32 oracle where a share can end badly -
+around a query tile of 256 rows, a block of 32, a key tile of 64, with rows of
+different lengths, with the mask inside the chunk, and with scores that force
+the running-maximum pass."""
+import os
+import re
+import shutil
+import subprocess
+
+import pytest
+import torch
+
+from oracle import sdv2_oracle as oracle
+from streamdiffusionv2_amd import _capi, build_ext
+from test_attention_isa import early_reads, instructions
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+EVEN = 1 << 20
+
+
+def test_every_tile_has_one_owner(tmp_path):
+    if shutil.which("g++") is None:
+        pytest.skip("no g++")
+    exe = str(tmp_path / "even_plan_check")
+    subprocess.run(["g++", "-std=c++17", "-O2", "-Wall", "-Werror", f"-I{build_ext.CSRC}",
+                    os.path.join(ROOT, "tests", "c_abi", "even_plan_check.cpp"), "-o", exe], check=True)
+    run = subprocess.run([exe], capture_output=True, text=True, timeout=120)
+    assert run.returncode == 0 and "3000 plans" in run.stdout, run.stdout
+
+
+def test_which_calls_get_equal_shares():
+    lib = _capi.lib()
+    for shape, plan in (((1, 1560, 40, 9360), EVEN), ((4, 4680, 12, 18720), EVEN),
+                        ((1, 256, 12, 1536), lib.sdv2_swa_attn_default_splits(1, 256, 12, 1536)),
+                        ((1, 1560, 12, 9360), lib.sdv2_swa_attn_default_splits(1, 1560, 12, 9360)),
+                        ((0, 1560, 12, 9360), 1)):
+        assert lib.sdv2_swa_attn_plan(*shape) == plan, shape
+    # tickets, and two results of 256 x 128 floats and 256 log-sum-exps for each of 256 workgroups, whatever the shape
+    assert lib.sdv2_swa_attn_workspace_bytes(1, 1560, 40, 9360, EVEN) == 65536 + 512 * 256 * (128 + 1) * 4
+    assert lib.sdv2_swa_attn_workspace_bytes(64, 65536, 64, 640, EVEN) == 0          # more query tiles than tickets
+
+
+def test_equal_shares_that_are_refused():
+    """(every refusal comes before the first HIP call)"""
+    import ctypes as C
+
+    lib = _capi.lib()
+
+    def params(**more):
+        p = _capi.AttnParams(q=256, k_cache=512, v_cache=768, out=1024, rows=1, q_tokens=512, heads=2, head_dim=128,
+                             max_seq_len=640, num_splits=EVEN)
+        for st in (p.q_stride, p.k_stride, p.v_stride, p.out_stride):
+            st.row, st.token, st.head = 1 << 20, 256, 128
+        for name, value in more.items():
+            setattr(p, name, value)
+        return C.byref(p)
+
+    assert lib.sdv2_swa_attn_fwd(params()) == _capi.SDV2_ERR_WORKSPACE
+    assert lib.sdv2_swa_attn_fwd(params(workspace=4096, workspace_bytes=65536)) == _capi.SDV2_ERR_WORKSPACE
+    assert lib.sdv2_swa_attn_fwd(params(rope_freqs=2048)) == _capi.SDV2_ERR_UNSUPPORTED
+    assert lib.sdv2_swa_attn_fwd(params(rows=64, q_tokens=65536, heads=64)) == _capi.SDV2_ERR_UNSUPPORTED
+    assert lib.sdv2_swa_attn_fwd(params(num_splits=EVEN | 2)) == _capi.SDV2_ERR_INVALID_ARG
+    assert lib.sdv2_swa_attn_fwd_static(params()) == _capi.SDV2_ERR_INVALID_ARG
+
+
+def test_the_streaming_loop_keeps_its_promises():
+    out = os.path.join(ROOT, "build", "isa_check")
+    os.makedirs(out, exist_ok=True)
+    path = os.path.join(out, "swa_attn_fwd_even.s")
+    cmd = [build_ext.hipcc_path(), *build_ext.HIPCC_FLAGS, f"-I{os.path.join(ROOT, 'include')}", f"-I{build_ext.CSRC}",
+           "-S", "--cuda-device-only", str(build_ext.CSRC / "swa_attn_fwd_even.hip"), "-o", path]
+    res = subprocess.run(cmd, capture_output=True, text=True)
+    assert res.returncode == 0, res.stderr[-2000:]
+    lines = open(path).read().split("\n")
+    starts = [i for i, l in enumerate(lines) if re.match(r"^_Z\S*swa_attn_fwd_even_kernel\S*:", l)]
+    assert len(starts) == 2                       # without and with the mask inside the chunk
+    for start in starts:
+        end = next(i for i in range(start, len(lines)) if lines[i].strip().startswith(".Lfunc_end"))
+        body = lines[start:end]
+        problems, n_mfma = early_reads(instructions(body))
+        assert n_mfma >= 256 and not problems, problems[:10]
+        first = next(i for i, l in enumerate(body) if "matrix pipe drained, site 1" in l)
+        last = next(i for i, l in enumerate(body) if "matrix pipe drained, site 0" in l)
+        loop = next(i for i in range(first, last) if "Loop Header" in body[i])
+        hot = body[loop:last]
+        assert sum("v_mfma_f32_16x16x32_bf16" in l for l in hot) >= 128
+        assert not [l.strip() for l in hot if re.search(r"\bscratch_(load|store)", l)]
+    assert max(int(x) for x in re.findall(r"\.vgpr_count:\s+(\d+)", "\n".join(lines))) <= 256
+
+
+def _close(got, want):
+    err = (got.float().cpu() - want).abs()
+    assert err.max().item() <= 2e-2 and err.mean().item() <= 2e-3, (err.max().item(), err.mean().item())
+
+
+def _inputs(rows, S, H, L, scale=1.0):
+    gen = torch.Generator().manual_seed(1000 * S + L)
+    q, k, v = (torch.randn(rows, n, H, 128, generator=gen) for n in (S, L, L))
+    return (q * scale).bfloat16(), (k * scale).bfloat16(), v.bfloat16()
+
+
+def _twice(q, k, v, lens, dev, **kw):
+    """The result, the same bits both times; the tickets are left at zero."""
+    from streamdiffusionv2_amd import ops
+
+    ws = ops.new_workspace(dev, _capi.lib().sdv2_swa_attn_workspace_bytes(q.shape[0], q.shape[1], q.shape[2], k.shape[1], EVEN))
+    out = [ops.swa_attention(q.to(dev), k.to(dev), v.to(dev), lens, num_splits=EVEN, workspace=ws, **kw) for _ in range(2)]
+    torch.cuda.synchronize()
+    assert torch.equal(out[0], out[1])
+    assert not ws[:65536].any()
+    return out[0]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows,S,H,L", [
+    (1, 256, 2, 1), (1, 256, 1, 64), (1, 255, 1, 65), (1, 20, 3, 700),      # one query tile, a tile that is not whole, a block
+    (1, 257, 3, 1100), (2, 288, 2, 640), (1, 289, 2, 129), (1, 384, 2, 333), (1, 385, 2, 700),      # rows past the last whole tile
+    (1, 512, 12, 127), (3, 1040, 4, 515), (2, 777, 5, 2000),                # shares of less than a tile, of about one, of several
+    (5, 600, 40, 130),                                                      # every workgroup takes a query tile whole first
+])
+def test_against_the_oracle(gpu_device, rows, S, H, L):
+    print(f"equal shares: {rows} x {S} x {H} against {L}", flush=True)
+    q, k, v = _inputs(rows, S, H, L)
+    _close(_twice(q, k, v, None, gpu_device), oracle.attention_fp32_reference(q, k, v, [L] * rows))
+
+
+@pytest.mark.gpu
+def test_rows_of_different_lengths(gpu_device):
+    q, k, v = _inputs(4, 600, 3, 1000)
+    lens = [1000, 1, 64, 517]
+    got = _twice(q, k, v, torch.tensor(lens, dtype=torch.int32, device=gpu_device), gpu_device)
+    _close(got, oracle.attention_fp32_reference(q, k, v, lens))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("device_starts", [False, True])
+@pytest.mark.parametrize("rows,S,L,block,starts", [
+    (1, 800, 1500, 100, [700]), (1, 777, 777, 259, [0]), (2, 544, 1200, 32, [656, 656]), (2, 544, 1200, 300, [0, 600]),
+    (1, 600, 650, 1, [17]),
+])
+def test_mask_inside_the_chunk(gpu_device, rows, S, L, block, starts, device_starts):
+    q, k, v = _inputs(rows, S, 5, L)
+    where = torch.tensor(starts, dtype=torch.int32, device=gpu_device) if device_starts else starts
+    got = _twice(q, k, v, None, gpu_device, chunk_key_start=where, mask_block_tokens=block)
+    _close(got, oracle.attention_fp32_reference(q, k, v, [L] * rows, starts, block))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("block", [0, 300])
+def test_scores_of_several_hundred(gpu_device, block):
+    """Pieces of an item whose exponent references differ by hundreds, some redone with a running maximum; a piece that
+    goes on from the last key to the first must not take hidden keys for all there is."""
+    q, k, v = _inputs(1, 600, 4, 900, scale=14.0)
+    kw = dict(chunk_key_start=[300], mask_block_tokens=block) if block else {}
+    want = oracle.attention_fp32_reference(q, k, v, [900], *(([300], block) if block else ()))
+    _close(_twice(q, k, v, None, gpu_device, **kw), want)
+
+
+@pytest.mark.gpu
+def test_cut_items_lose_nothing(gpu_device):
+    """Error against 64 bits of a call whose query tiles are nearly all cut, and of the same call whole: the pieces meet
+    in fp32, which adds some 2^-22 to the 2^-9 of the bf16 result - 1 % of room for the other exponent references."""
+    from streamdiffusionv2_amd import ops
+
+    q, k, v = (t.to(gpu_device) for t in _inputs(2, 1024, 40, 2000))       # (whole: 320 query tiles on the same matrix instructions)
+    want = torch.empty(q.shape, dtype=torch.float64, device=gpu_device)
+    for row in range(2):
+        for h in range(40):
+            s = q[row, :, h].double() @ k[row, :, h].double().t().contiguous() * 128 ** -0.5
+            want[row, :, h] = s.softmax(-1) @ v[row, :, h].double()
+    err = [((ops.swa_attention(q, k, v, None, num_splits=n).double() - want).norm() / want.norm()).item() for n in (1, EVEN)]
+    assert err[1] <= 1.01 * err[0], err
+
+
+@pytest.mark.gpu
+def test_equal_shares_in_a_graph(gpu_device):
+    """Recorded once, replayed on new inputs between eager calls of another shape on the same workspace."""
+    from streamdiffusionv2_amd import ops
+
+    q, k, v = (t.to(gpu_device) for t in _inputs(1, 700, 6, 1300))
+    q2, k2, v2 = (t.to(gpu_device) for t in _inputs(2, 300, 4, 800))
+    ops.swa_attention(q, k, v, num_splits=EVEN)
+    other = ops.swa_attention(q2, k2, v2, num_splits=EVEN)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = ops.swa_attention(q, k, v, num_splits=EVEN)
+    for i in range(4):
+        q.copy_(q.roll(i + 1, 1))
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, ops.swa_attention(q, k, v, num_splits=EVEN))
+        assert torch.equal(other, ops.swa_attention(q2, k2, v2, num_splits=EVEN))
