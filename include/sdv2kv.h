@@ -37,8 +37,9 @@ extern "C" {
  *     library's own plan needs more than SDV2_STATIC_SCRATCH_BYTES (12 refused it)
  * 14: sdv2_attn_params.chunk_key_start_host
  * 15: sdv2_cache_relayout_pair
- * 16: SDV2_SPLITS_EVEN, sdv2_swa_attn_plan */
-#define SDV2KV_ABI_VERSION 16
+ * 16: SDV2_SPLITS_EVEN, sdv2_swa_attn_plan
+ * 17: sdv2_linear, sdv2_linear_preferred */
+#define SDV2KV_ABI_VERSION 17
 #define SDV2_HEAD_DIM 128      /* causal_stream_inference.py:99-100 fixes 128 */
 #define SDV2_MAX_ROWS 16       /* rows (B) per sdv2_kv_append_rope call       */
 #define SDV2_MAX_SINK_FRAMES 16 /* sink frames per sdv2_sink_similarity call  */
@@ -427,6 +428,33 @@ typedef struct sdv2_rms_norm_params {
 } sdv2_rms_norm_params;
 
 int sdv2_rms_norm(const sdv2_rms_norm_params* p);
+
+/* ------------------------------------------------------------------------
+ * out = x weight^T + bias: the q, k, v and output projections around the
+ * attention (models/wan/causal_model.py:212-218, :389,
+ * wan_base/modules/model.py:181, :195), as nn.Linear computes them: products
+ * of bf16 accumulated in fp32, the bias added in fp32, one rounding.  Any m;
+ * n and k multiples of 64 (else SDV2_ERR_UNSUPPORTED).  Rows are k (x,
+ * weight) and n (out) contiguous elements, a multiple of 8 apart; x, weight
+ * and out 16-byte aligned, bias (or NULL) 8-byte.  out must not overlap x.
+ * ---------------------------------------------------------------------- */
+typedef struct sdv2_linear_params {
+  const void* x;               /* [m, k]                                       */
+  const void* weight;          /* [n, k]                                       */
+  const void* bias;            /* [n] or NULL                                  */
+  void* out;                   /* [m, n]                                       */
+  int64_t x_row_stride;        /* elements                                     */
+  int64_t weight_row_stride;
+  int64_t out_row_stride;
+  int64_t m;
+  int32_t n, k;
+  int32_t dtype;               /* sdv2_dtype of all four: SDV2_BF16            */
+  void* stream;                /* hipStream_t                                  */
+} sdv2_linear_params;
+
+int sdv2_linear(const sdv2_linear_params* p);
+/* 1 where the call is one round of the chip and faster than a general library's */
+int sdv2_linear_preferred(int64_t m, int32_t n, int32_t k);
 
 #ifdef __cplusplus
 }

@@ -23,7 +23,8 @@ typedef enum sdv2_profile_kernel {
   SDV2_KERNEL_SINK = 3,        /* sdv2_sink_similarity                         */
   SDV2_KERNEL_COPY = 4,        /* sdv2_copy_bytes                              */
   SDV2_KERNEL_NORM = 5,        /* sdv2_rms_norm                                */
-  SDV2_KERNEL_COUNT = 6
+  SDV2_KERNEL_LINEAR = 6,      /* sdv2_linear                                  */
+  SDV2_KERNEL_COUNT = 7
 } sdv2_profile_kernel;
 
 /* ------------------------------------------------------------------------

@@ -12,7 +12,7 @@ from typing import Optional
 
 LIB_PATH = Path(__file__).resolve().parent / "_lib" / "libsdv2kv.so"
 
-ABI_VERSION = 16
+ABI_VERSION = 17
 HEAD_DIM = 128
 MAX_ROWS = 16
 
@@ -28,7 +28,7 @@ STATIC_SCRATCH_BYTES = 64 << 20
 DTYPE_BF16 = 0
 DTYPE_F32 = 1
 
-KERNEL_APPEND, KERNEL_ATTENTION, KERNEL_RELAYOUT, KERNEL_SINK, KERNEL_COPY, KERNEL_NORM = range(6)
+KERNEL_APPEND, KERNEL_ATTENTION, KERNEL_RELAYOUT, KERNEL_SINK, KERNEL_COPY, KERNEL_NORM, KERNEL_LINEAR = range(7)
 STREAM_REGISTERS, STREAM_LDS_32_ROWS, STREAM_LDS_64_ROWS, STREAM_ATTENTION_MIX, STREAM_ATTENTION_MIX_64_ROWS = range(5)
 
 # every symbol include/sdv2kv.h and include/sdv2kv_profile.h declare
@@ -47,6 +47,8 @@ EXPORTED_SYMBOLS = (
     "sdv2_sink_similarity",
     "sdv2_cache_relayout",
     "sdv2_cache_relayout_pair",
+    "sdv2_linear",
+    "sdv2_linear_preferred",
     "sdv2_rms_norm",
     "sdv2_event_create",
     "sdv2_event_destroy",
@@ -154,6 +156,17 @@ class RmsNormParams(C.Structure):
     ]
 
 
+class LinearParams(C.Structure):
+    _fields_ = [
+        ("x", C.c_void_p), ("weight", C.c_void_p), ("bias", C.c_void_p), ("out", C.c_void_p),
+        ("x_row_stride", C.c_int64), ("weight_row_stride", C.c_int64), ("out_row_stride", C.c_int64),
+        ("m", C.c_int64),
+        ("n", C.c_int32), ("k", C.c_int32),
+        ("dtype", C.c_int32),
+        ("stream", C.c_void_p),
+    ]
+
+
 class RelayoutParams(C.Structure):
     _fields_ = [
         ("src", C.c_void_p), ("dst", C.c_void_p),
@@ -222,6 +235,10 @@ def lib() -> C.CDLL:
     handle.sdv2_cache_relayout.argtypes = [C.POINTER(RelayoutParams)]
     handle.sdv2_cache_relayout_pair.restype = C.c_int
     handle.sdv2_cache_relayout_pair.argtypes = [C.POINTER(RelayoutParams)] * 2
+    handle.sdv2_linear.restype = C.c_int
+    handle.sdv2_linear.argtypes = [C.POINTER(LinearParams)]
+    handle.sdv2_linear_preferred.restype = C.c_int
+    handle.sdv2_linear_preferred.argtypes = [C.c_int64, C.c_int32, C.c_int32]
     handle.sdv2_rms_norm.restype = C.c_int
     handle.sdv2_rms_norm.argtypes = [C.POINTER(RmsNormParams)]
     handle.sdv2_event_create.restype = C.c_int

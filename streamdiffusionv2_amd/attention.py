@@ -19,6 +19,24 @@ import torch.nn as nn
 from . import ops, ring
 
 
+def _unwatched(layer) -> bool:
+    """A plain Linear that nobody watches: a wrapped or replaced layer (an adapter, a quantised Linear) computes
+    something else than x W^T + b, and a hook expects its layer to be called."""
+    import torch.nn.modules.module as hooks
+    return type(layer) is nn.Linear and "forward" not in layer.__dict__ \
+        and not (layer._forward_hooks or layer._forward_pre_hooks or hooks._global_forward_hooks
+                 or hooks._global_forward_pre_hooks)
+
+
+def _linear(layer, x):
+    """``layer(x)``, by the library's kernel where it is faster and nothing expects the layer's own call."""
+    if _unwatched(layer):
+        out = ops.linear_or_none(x, layer.weight, layer.bias)
+        if out is not None:
+            return out
+    return layer(x)
+
+
 class WanRMSNorm(nn.Module):
     """RMS norm over the full model dim in fp32 (wan_base/modules/model.py:70-86)."""
 
@@ -414,9 +432,9 @@ class CausalWanSelfAttention(nn.Module, RingKVPath):
         self.fuse_qk_norm = True
 
         # The q, k and v projections (causal_model.py:212-218 calls the three
-        # Linears one after the other) run as ONE vendor GEMM on the three
-        # weights laid end to end: at 1560 tokens x 1536 the three launches take
-        # 60 us and the one 26 us, with the same bits out (every output element
+        # Linears one after the other) run as ONE product on the three
+        # weights laid end to end: at 1560 tokens x 1536 three launches of the vendor's take
+        # 60 us and one 26 us (the library's own 22), with the same bits out (every output element
         # is the same dot product over `dim`).  q, k and v are then strided views
         # of one [B, S, 3 * dim] tensor, which the kernels of the path read as
         # they are.  The packed copy of the weights (3 * dim * dim elements per
@@ -480,8 +498,10 @@ class CausalWanSelfAttention(nn.Module, RingKVPath):
         watched = _hooks._global_forward_hooks or _hooks._global_forward_pre_hooks
         packed = self._packed_qkv() if self.fuse_qkv_projection and not torch.is_grad_enabled() and not watched else None
         if packed is None:
-            return self.q(x), self.k(x), self.v(x)
-        y = nn.functional.linear(x, packed[0], packed[1])
+            return _linear(self.q, x), _linear(self.k, x), _linear(self.v, x)
+        y = ops.linear_or_none(x, packed[0], packed[1])
+        if y is None:
+            y = nn.functional.linear(x, packed[0], packed[1])
         d = self.dim
         return y[..., :d], y[..., d:2 * d], y[..., 2 * d:]
 
@@ -518,7 +538,7 @@ class CausalWanSelfAttention(nn.Module, RingKVPath):
             q = self.norm_q(q).view(b, s, n, d)
             k = self.norm_k(k).view(b, s, n, d)
             out = self.attend(q, k, v, grid_sizes, freqs, kv_cache, current_start)
-        return self.o(out.flatten(2))
+        return _linear(self.o, out.flatten(2))
 
 
 class WanT2VCrossAttention(nn.Module):
@@ -548,7 +568,7 @@ class WanT2VCrossAttention(nn.Module):
     def forward(self, x, context, context_lens, crossattn_cache=None):
         """x [B, L1, dim]; context [B, L2, dim]; context_lens [B] or None."""
         b, n, d = x.size(0), self.num_heads, self.head_dim
-        q = self.norm_q(self.q(x)).view(b, -1, n, d)
+        q = self.norm_q(_linear(self.q, x)).view(b, -1, n, d)
         if crossattn_cache is not None and crossattn_cache["is_init"]:
             k, v = crossattn_cache["k"], crossattn_cache["v"]
         else:
@@ -559,4 +579,4 @@ class WanT2VCrossAttention(nn.Module):
                 crossattn_cache["k"] = k
                 crossattn_cache["v"] = v
         out = ops.flash_attention(q, k, v, k_lens=context_lens)
-        return self.o(out.flatten(2))
+        return _linear(self.o, out.flatten(2))

@@ -1050,6 +1050,54 @@ def _launch_norm(x, weight, eps, out, x_rows, out_step):
     return out
 
 
+def _plain_call() -> bool:
+    """Nothing watches or rewrites tensor operations: no autograd (either mode), autocast, tracing or compilation, no
+    mode that wants to see them."""
+    return not (torch.is_grad_enabled() or torch.is_autocast_enabled("cuda") or torch.compiler.is_compiling()
+                or torch.jit.is_tracing() or torch.autograd.forward_ad._current_level >= 0
+                or torch._C._len_torch_dispatch_stack() or torch._C._len_torch_function_stack()
+                or torch._C._functorch.maybe_current_level() is not None)
+
+
+_PLAIN_TENSORS = (torch.Tensor, torch.nn.Parameter)
+_LINEAR_PREFERRED: dict = {}
+
+
+def linear_or_none(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor]) -> Optional[torch.Tensor]:
+    """``x weight^T + bias`` by the library's kernel where that is the faster one
+    (``sdv2_linear_preferred``: bf16, a chunk's worth of rows), else None: the
+    caller's nn.Linear, for everything the kernel does not take too."""
+    bf16 = torch.bfloat16
+    if not (x.is_cuda and x.dtype == bf16 and weight.dtype == bf16 and type(x) in _PLAIN_TENSORS
+            and type(weight) in _PLAIN_TENSORS and weight.dim() == 2 and x.dim() >= 2 and x.numel() and _plain_call()):
+        return None
+    n, k = weight.shape
+    if x.shape[-1] != k:
+        return None
+    m = x.numel() // k
+    key = (m, n, k)
+    preferred = _LINEAR_PREFERRED.get(key)
+    if preferred is None:
+        if len(_LINEAR_PREFERRED) >= _MAX_ATTN_LAYOUTS:
+            _LINEAR_PREFERRED.clear()
+        preferred = _LINEAR_PREFERRED[key] = bool(_capi.lib().sdv2_linear_preferred(m, n, k))
+    if not preferred:
+        return None
+    dev = x.device
+    rows = _norm_rows(x)
+    if rows is None or weight.device != dev or not weight.is_contiguous() or x.data_ptr() % 16 or weight.data_ptr() % 16:
+        return None
+    if bias is not None and not (type(bias) in _PLAIN_TENSORS and bias.dtype == bf16 and bias.device == dev
+                                 and bias.dim() == 1 and bias.is_contiguous() and bias.data_ptr() % 8 == 0):
+        return None
+    out = torch.empty((*x.shape[:-1], n), dtype=bf16, device=dev)
+    p = _capi.LinearParams(x.data_ptr(), weight.data_ptr(), bias.data_ptr() if bias is not None else None, out.data_ptr(),
+                           rows[1], k, n, m, n, k, _capi.DTYPE_BF16, _stream_ptr(dev))
+    with _on_device(dev):
+        _capi.check(_capi.lib().sdv2_linear(C.byref(p)), "sdv2_linear")
+    return out
+
+
 def copy_bytes(dst: torch.Tensor, src: torch.Tensor) -> None:
     """Plain 16-byte-vector copy with the library's own kernel (used to scale
     hardware counters against a transfer of known size)."""
