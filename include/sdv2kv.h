@@ -38,8 +38,10 @@ extern "C" {
  * 14: sdv2_attn_params.chunk_key_start_host
  * 15: sdv2_cache_relayout_pair
  * 16: SDV2_SPLITS_EVEN, sdv2_swa_attn_plan
- * 17: sdv2_linear, sdv2_linear_preferred */
-#define SDV2KV_ABI_VERSION 17
+ * 17: sdv2_linear, sdv2_linear_preferred
+ * 18: sdv2_linear_params.row_squares, sdv2_attn_params.q_row_squares and
+ *     q_norm_eps, sdv2_swa_attn_folds_norm */
+#define SDV2KV_ABI_VERSION 18
 #define SDV2_HEAD_DIM 128      /* causal_stream_inference.py:99-100 fixes 128 */
 #define SDV2_MAX_ROWS 16       /* rows (B) per sdv2_kv_append_rope call       */
 #define SDV2_MAX_SINK_FRAMES 16 /* sink frames per sdv2_sink_similarity call  */
@@ -240,7 +242,19 @@ typedef struct sdv2_attn_params {
    * SDV2_ERR_OUT_OF_RANGE for a value outside [0, L - S].  With the mask on,
    * exactly one of the two is set.                                             */
   const int64_t* chunk_key_start_host;   /* host [B]                               */
+  /* Optional RMSNorm of a query that is not rotated (the text cross-attention's):
+   * q is the raw projection, rows of heads * 128 elements, q_norm_weight as
+   * above, and q_row_squares what sdv2_linear stored beside it, sums of squares
+   * of 32 columns each (device float [B * S, heads * 4], 16-byte aligned); a
+   * row's 1 / rms is 1 / sqrt(sum / (heads * 128) + q_norm_eps).  No rope_freqs,
+   * q_inv_rms or mask, SDV2_BF16, and only where sdv2_swa_attn_folds_norm()
+   * says so (else SDV2_ERR_UNSUPPORTED).                                       */
+  const float* q_row_squares;
+  float q_norm_eps;
 } sdv2_attn_params;
+
+/* 1 where a call of this shape with default num_splits takes q_row_squares */
+int sdv2_swa_attn_folds_norm(int32_t rows, int32_t q_tokens, int32_t heads, int32_t max_seq_len);
 
 /* the key-range split plan the library would pick for this shape, as num_splits carries it */
 int sdv2_swa_attn_default_splits(int32_t rows, int32_t q_tokens, int32_t heads, int32_t max_seq_len);
@@ -450,6 +464,8 @@ typedef struct sdv2_linear_params {
   int32_t n, k;
   int32_t dtype;               /* sdv2_dtype of all four: SDV2_BF16            */
   void* stream;                /* hipStream_t                                  */
+  float* row_squares;          /* [m, n / 32] or NULL: sums of the squares of  */
+                               /* 32 columns each of out, as rounded           */
 } sdv2_linear_params;
 
 int sdv2_linear(const sdv2_linear_params* p);

@@ -12,7 +12,7 @@ from typing import Optional
 
 LIB_PATH = Path(__file__).resolve().parent / "_lib" / "libsdv2kv.so"
 
-ABI_VERSION = 17
+ABI_VERSION = 18
 HEAD_DIM = 128
 MAX_ROWS = 16
 
@@ -40,6 +40,7 @@ EXPORTED_SYMBOLS = (
     "sdv2_swa_attn_plan",
     "sdv2_swa_attn_workspace_bytes",
     "sdv2_swa_attn_f32_workspace_bytes",
+    "sdv2_swa_attn_folds_norm",
     "sdv2_swa_attn_fwd",
     "sdv2_swa_attn_fwd_static",
     "sdv2_sink_similarity_workspace_bytes",
@@ -113,6 +114,8 @@ class AttnParams(C.Structure):
         ("q_norm_weight", C.c_void_p),
         ("q_inv_rms", C.c_void_p),
         ("chunk_key_start_host", C.POINTER(C.c_int64)),
+        ("q_row_squares", C.c_void_p),
+        ("q_norm_eps", C.c_float),
     ]
 
 
@@ -164,6 +167,7 @@ class LinearParams(C.Structure):
         ("n", C.c_int32), ("k", C.c_int32),
         ("dtype", C.c_int32),
         ("stream", C.c_void_p),
+        ("row_squares", C.c_void_p),
     ]
 
 
@@ -219,6 +223,8 @@ def lib() -> C.CDLL:
     handle.sdv2_swa_attn_plan.argtypes = [C.c_int32] * 4
     handle.sdv2_swa_attn_workspace_bytes.restype = C.c_size_t
     handle.sdv2_swa_attn_workspace_bytes.argtypes = [C.c_int32] * 5
+    handle.sdv2_swa_attn_folds_norm.restype = C.c_int
+    handle.sdv2_swa_attn_folds_norm.argtypes = [C.c_int32] * 4
     handle.sdv2_swa_attn_f32_workspace_bytes.restype = C.c_size_t
     handle.sdv2_swa_attn_f32_workspace_bytes.argtypes = [C.c_int32] * 4
     handle.sdv2_swa_attn_fwd.restype = C.c_int

@@ -19,11 +19,11 @@ import torch.nn as nn
 from . import ops, ring
 
 
-def _unwatched(layer) -> bool:
-    """A plain Linear that nobody watches: a wrapped or replaced layer (an adapter, a quantised Linear) computes
-    something else than x W^T + b, and a hook expects its layer to be called."""
+def _unwatched(layer, kind=nn.Linear) -> bool:
+    """A plain Linear (or layer of another kind) that nobody watches: a wrapped or replaced layer (an adapter, a
+    quantised Linear) computes something else than x W^T + b, and a hook expects its layer to be called."""
     import torch.nn.modules.module as hooks
-    return type(layer) is nn.Linear and "forward" not in layer.__dict__ \
+    return type(layer) is kind and "forward" not in layer.__dict__ \
         and not (layer._forward_hooks or layer._forward_pre_hooks or hooks._global_forward_hooks
                  or hooks._global_forward_pre_hooks)
 
@@ -568,7 +568,8 @@ class WanT2VCrossAttention(nn.Module):
     def forward(self, x, context, context_lens, crossattn_cache=None):
         """x [B, L1, dim]; context [B, L2, dim]; context_lens [B] or None."""
         b, n, d = x.size(0), self.num_heads, self.head_dim
-        q = self.norm_q(_linear(self.q, x)).view(b, -1, n, d)
+        raw = self._raw_query(x, context, crossattn_cache)
+        q = (self.norm_q(_linear(self.q, x)) if raw is None else raw[0]).view(b, -1, n, d)
         if crossattn_cache is not None and crossattn_cache["is_init"]:
             k, v = crossattn_cache["k"], crossattn_cache["v"]
         else:
@@ -578,5 +579,27 @@ class WanT2VCrossAttention(nn.Module):
                 crossattn_cache["is_init"] = True
                 crossattn_cache["k"] = k
                 crossattn_cache["v"] = v
-        out = ops.flash_attention(q, k, v, k_lens=context_lens)
+        if raw is None:
+            out = ops.flash_attention(q, k, v, k_lens=context_lens)
+        else:
+            if context_lens is not None:
+                context_lens = context_lens.to(device=q.device, dtype=torch.int32).contiguous()
+            out = ops.swa_attention(q, k, v, context_lens, q_row_squares=(self.norm_q.weight, raw[1], self.norm_q.eps))
         return _linear(self.o, out.flatten(2))
+
+    def _raw_query(self, x, context, crossattn_cache):
+        """(q projection, sums of squares of its rows) where the attention normalises the query as it reads it, else
+        None.  (The norm as a launch of its own took 7.2 of a layer's 62 us.)"""
+        if not (x.dim() == 3 and self.head_dim == ops.HEAD_DIM and _unwatched(self.q) and _unwatched(self.norm_q, WanRMSNorm)
+                and self.q.weight.shape[0] == self.dim):
+            return None
+        keys = context
+        if crossattn_cache is not None and crossattn_cache["is_init"]:
+            keys = crossattn_cache["k"]
+            if keys.dtype != x.dtype or crossattn_cache["v"].dtype != x.dtype:
+                return None
+        elif keys.dtype != x.dtype or self.k.weight.dtype != x.dtype or self.v.weight.dtype != x.dtype:
+            return None
+        if not ops.folds_query_norm((x.size(0), x.size(1), self.dim), keys.shape[1], self.norm_q.weight, x.device):
+            return None
+        return ops.linear_or_none(x, self.q.weight, self.q.bias, row_squares=True)

@@ -73,6 +73,9 @@ struct AttnKernelArgs {
   // the norm weight [heads * 128] and 1 / rms per (row, token), or null
   const uint16_t* q_norm_w;
   const float* q_inv_rms;
+  // the same for a query that is not rotated: sums of squares of 32 columns each of (row, token), or null
+  const float* q_row_squares;
+  float q_norm_eps;
   sdv2::ChunkStarts chunk_starts;   // with the mask inside the chunk
 };
 template <typename Args>

@@ -53,9 +53,10 @@ struct LinearArgs {
   const uint16_t* w;
   const uint16_t* bias;
   uint16_t* out;
+  float* squares;                            // [row][n / 32], or null
   int64_t x_st, w_st, out_st;                // elements between rows
   int32_t m, stages;                         // rows; stages of the contraction
-  int32_t row_tiles, col_tiles;
+  int32_t row_tiles, col_tiles, square_groups;       // square_groups = n / 32
 };
 
 // Fragments in flight from LDS are nobody's to move: passing them through here, behind the wait, fixes that.
@@ -205,6 +206,30 @@ void linear_kernel(const LinearArgs a) {
     }
   }
   const int row0 = m0 + wm * 16 * kM;
+  if (a.squares != nullptr) {
+    // what a norm of the rows is to be made of: two fragments are 32 columns, four of each with every lane of a row
+    static_assert(kN % 2 == 0, "groups of 32 columns");
+#pragma unroll
+    for (int fm = 0; fm < kM; ++fm)
+#pragma unroll
+      for (int half = 0; half < kN / 2; ++half) {
+        float sum = 0.f;
+#pragma unroll
+        for (int fn = 2 * half; fn < 2 * half + 2; ++fn) {
+          const u32x2 y = *reinterpret_cast<__attribute__((address_space(3))) const u32x2*>(mine + (16 * fm + n16) * kOutBytes + 32 * fn + 8 * g);
+#pragma unroll
+          for (int i = 0; i < 2; ++i) {
+            const float lo = __uint_as_float(y[i] << 16), hi = __uint_as_float(y[i] & 0xffff0000u);
+            sum = __builtin_fmaf(lo, lo, sum);
+            sum = __builtin_fmaf(hi, hi, sum);
+          }
+        }
+        sum += __shfl_xor(sum, 16);
+        sum += __shfl_xor(sum, 32);
+        const int r = row0 + 16 * fm + n16;
+        if (g == 0 && r < a.m) a.squares[(int64_t)r * a.square_groups + (col0 >> 5) + half] = sum;
+      }
+  }
   uint16_t* dst = a.out + row0 * a.out_st + col0;
   constexpr int kChunks = 2 * kN;            // 16-byte chunks of a row
 #pragma unroll
@@ -282,7 +307,7 @@ extern "C" int sdv2_linear(const sdv2_linear_params* p) {
   if (!p->x || !p->weight || !p->out) return SDV2_ERR_INVALID_ARG;
   if ((reinterpret_cast<uintptr_t>(p->x) | reinterpret_cast<uintptr_t>(p->weight) | reinterpret_cast<uintptr_t>(p->out)) & 15)
     return SDV2_ERR_INVALID_ARG;
-  if (reinterpret_cast<uintptr_t>(p->bias) & 7) return SDV2_ERR_INVALID_ARG;
+  if ((reinterpret_cast<uintptr_t>(p->bias) & 7) || (reinterpret_cast<uintptr_t>(p->row_squares) & 3)) return SDV2_ERR_INVALID_ARG;
   // rows of 16-byte vectors that do not overlap; offsets within a tile's rows are 32-bit
   constexpr int64_t kMostStride = 1 << 22;
   for (int64_t st : {p->x_row_stride, p->weight_row_stride})
@@ -299,6 +324,8 @@ extern "C" int sdv2_linear(const sdv2_linear_params* p) {
   a.w_st = p->weight_row_stride;
   a.out_st = p->out_row_stride;
   a.m = (int32_t)p->m;
+  a.squares = p->row_squares;
+  a.square_groups = p->n / 32;
   a.stages = p->k / kDepth;
   a.row_tiles = (int32_t)((p->m + kTiles[i].m - 1) / kTiles[i].m);
   a.col_tiles = p->n / kTiles[i].n;

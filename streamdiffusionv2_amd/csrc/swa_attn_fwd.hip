@@ -437,6 +437,30 @@ __device__ __forceinline__ void load_query(const QueryRope& rope, const uint16_t
   }
 }
 
+// A raw projection that is not rotated, already requested: its RMSNorm as rms_norm.hip rounds it, the row's sum of
+// squares from the sums of 32 columns that the projection left.  The two lanes of a query take the heads in turn, and
+// their sums come in one trip, beside the query's own.  (As a launch of its own the norm of 3120 x 1536 took 7.2 us.)
+__device__ __forceinline__ void normalise_query(const AttnKernelArgs& a, int64_t token, int head, int hf, bf16x8 (&qf)[8]) {
+  constexpr int kBatch = 8;
+  const f32x4* const squares = reinterpret_cast<const f32x4*>(a.q_row_squares) + token * a.heads;
+  float sum = 0.f;
+  for (int h0 = hf; h0 < a.heads + hf; h0 += 2 * kBatch) {
+    f32x4 x[kBatch];
+#pragma unroll
+    for (int u = 0; u < kBatch; ++u) x[u] = squares[h0 + 2 * u < a.heads ? h0 + 2 * u : a.heads - 1];
+#pragma unroll
+    for (int u = 0; u < kBatch; ++u)
+      if (h0 + 2 * u < a.heads) sum += (x[u][0] + x[u][1]) + (x[u][2] + x[u][3]);
+  }
+  const float inv_rms = 1.0f / sqrtf(half_sum(sum) / (float)(a.heads * kD) + a.q_norm_eps);
+#pragma unroll
+  for (int ks = 0; ks < 8; ++ks) {
+    sdv2::Vec8<uint16_t> x;
+    x.raw = __builtin_bit_cast(uint4, qf[ks]);
+    qf[ks] = __builtin_bit_cast(bf16x8, sdv2::normalise(x, inv_rms, sdv2::Vec8<uint16_t>::load(a.q_norm_w + head * kD + 8 * hf + 16 * ks)).raw);
+  }
+}
+
 template <bool kMask>
 __global__ __launch_bounds__(kThreads, 1)
 void swa_attn_fwd_kernel(const AttnKernelArgs a) {
@@ -534,6 +558,8 @@ void swa_attn_fwd_kernel(const AttnKernelArgs a) {
     rope.norm_w = a.q_norm_w ? a.q_norm_w + head * kD + 8 * hf : nullptr;
     rope.inv_rms = a.q_norm_w ? a.q_inv_rms[(int64_t)row * a.q_tokens + q_row_c] : 1.0f;
     load_query(rope, q_ptr, q_row_c, hf, qf);
+  } else if (!kMask && a.q_row_squares != nullptr) {
+    normalise_query(a, ((int64_t)row * a.q_tokens + q_row_c), head, hf, qf);
   }
   // the value is (re)defined in the register class every later use names, so it is never copied back and forth
 #pragma unroll
@@ -1049,6 +1075,11 @@ double wave_kernel_us(int32_t rows, int32_t q_tokens, int32_t heads, int32_t max
   return 2.4 + (double)((workgroups + kCuSlots - 1) / kCuSlots) * (4.6 + 1.22 * ((max_seq_len + 255) / 256));
 }
 
+bool waves_share_queries(int32_t rows, int32_t q_tokens, int32_t heads, int32_t max_seq_len) {
+  return wave_kernel_us(rows, q_tokens, heads, max_seq_len) < tile_kernels_us(rows, q_tokens, heads, max_seq_len, 1, 0);
+}
+constexpr int kTilesForM16 = 12;               // key tiles from which swa_attn_fwd_m16.hip is taken: see attn_fwd
+
 // Equal shares (swa_attn_fwd_even.hip) -------------------------------------------------------------------------------
 // The plan for a shape on `workgroups` workgroups, or false where there is none.
 bool even_plan(int32_t rows, int32_t q_tokens, int32_t heads, int32_t max_seq_len, int workgroups, int rounds, EvenPlan* e) {
@@ -1170,6 +1201,12 @@ extern "C" int sdv2_swa_attn_plan(int32_t rows, int32_t q_tokens, int32_t heads,
   return even_us < 0.99 * us ? SDV2_SPLITS_EVEN : splits;
 }
 
+extern "C" int sdv2_swa_attn_folds_norm(int32_t rows, int32_t q_tokens, int32_t heads, int32_t max_seq_len) {
+  // the kernel of this file and one key range (the others have no room for it, or calls too long to notice)
+  return rows > 0 && q_tokens > 0 && heads > 0 && max_seq_len > 0 && (max_seq_len + kKTile - 1) / kKTile < kTilesForM16 &&
+         sdv2_swa_attn_plan(rows, q_tokens, heads, max_seq_len) == 1 && !waves_share_queries(rows, q_tokens, heads, max_seq_len);
+}
+
 extern "C" size_t sdv2_swa_attn_workspace_bytes(int32_t rows, int32_t q_tokens, int32_t heads,
                                                  int32_t max_seq_len, int32_t num_splits) {
   if (rows <= 0 || q_tokens <= 0 || heads <= 0) return 0;
@@ -1288,7 +1325,15 @@ int attn_fwd(const sdv2_attn_params* p, void* workspace, size_t workspace_bytes)
     a.split_h = a.split_t + third;
   }
 
-  if (p->q_norm_weight || p->q_inv_rms) {
+  if (p->q_row_squares) {
+    // the raw q projection: normalised as it is loaded
+    if (!p->q_norm_weight || p->q_inv_rms || p->rope_freqs || a.mask_block_tokens > 0) return SDV2_ERR_INVALID_ARG;
+    if (!aligned16(p->q_norm_weight) || !aligned16(p->q_row_squares) || !(p->q_norm_eps >= 0.f)) return SDV2_ERR_INVALID_ARG;
+    if (even || splits != 1 || !sdv2_swa_attn_folds_norm(p->rows, p->q_tokens, p->heads, p->max_seq_len)) return SDV2_ERR_UNSUPPORTED;
+    a.q_norm_w = static_cast<const uint16_t*>(p->q_norm_weight);
+    a.q_row_squares = p->q_row_squares;
+    a.q_norm_eps = p->q_norm_eps;
+  } else if (p->q_norm_weight || p->q_inv_rms) {
     // the raw q projection: normalised, then rotated, as it is loaded
     if (!p->q_norm_weight || !p->q_inv_rms || !p->rope_freqs) return SDV2_ERR_INVALID_ARG;
     if (!aligned16(p->q_norm_weight) || (reinterpret_cast<uintptr_t>(p->q_inv_rms) & 3)) return SDV2_ERR_INVALID_ARG;
@@ -1350,8 +1395,7 @@ int attn_fwd(const sdv2_attn_params* p, void* workspace, size_t workspace_bytes)
   // (A grid has fewer than 2^32 threads: up to eight times the workgroups must not carry an accepted call past that.)
   constexpr int64_t kMostWaveItems = 1 << 22;
   if (splits == 1 && work_items(kQBlock) <= kMostWaveItems &&
-      wave_kernel_us(p->rows, p->q_tokens, p->heads, p->max_seq_len) <
-          tile_kernels_us(p->rows, p->q_tokens, p->heads, p->max_seq_len, 1, 0)) {
+      waves_share_queries(p->rows, p->q_tokens, p->heads, p->max_seq_len)) {
     set_work_list(&a, kQBlock);
     return sdv2::attn::launch_wave(a, 8u * (((uint32_t)a.total_items + 7u) / 8u), stream);
   }
@@ -1362,7 +1406,6 @@ int attn_fwd(const sdv2_attn_params* p, void* workspace, size_t workspace_bytes)
   // one key range: 768 keys 30.5 against 30.7 us, 384 keys 22.1 against 21.3, 3072 keys 84.5 against 90.4).  With the
   // mask inside the chunk likewise (3807 queries x 12 heads in blocks of 1269 against 11421 keys, the layer call: 264
   // against 274 us).
-  constexpr int kTilesForM16 = 12;
   if ((p->max_seq_len + kKTile - 1) / kKTile >= kTilesForM16 * plan.base)
     return sdv2::attn::launch_m16(a, grid.x, stream);
   // The tile buffers (96 KB) or the epilogue staging (16 KB per wave) exceed the static limit:

@@ -414,6 +414,7 @@ def swa_attention(
     static_scratch: bool = False,
     rope: Optional[Tuple[torch.Tensor, Sequence[int], Sequence[int]]] = None,
     q_norm: Optional[Tuple[torch.Tensor, torch.Tensor]] = None,
+    q_row_squares: Optional[Tuple[torch.Tensor, torch.Tensor, float]] = None,
 ) -> torch.Tensor:
     """out[b] = softmax(q[b] k_cache[b,:seq_lens[b]]^T * scale) v_cache[b,:seq_lens[b]].
 
@@ -423,6 +424,9 @@ def swa_attention(
     caller-owned ``workspace`` must come from :func:`new_workspace` (zero-filled).
     With ``q_norm`` = (q norm weight, q_inv_rms from :func:`kv_append_rope`) as
     well, q is the raw q projection and is RMS-normalised before the rotation.
+    ``q_row_squares`` = (q norm weight, sums of squares of 32 columns each of q as
+    :func:`linear_or_none` stores them, eps): q is a raw projection, normalised and
+    not rotated, for shapes that ``sdv2_swa_attn_folds_norm`` names.
 
     ``static_scratch`` takes the library's allocation-free entry point
     (``sdv2_swa_attn_fwd_static``): partial results of a split call go to device
@@ -504,6 +508,14 @@ def swa_attention(
                 or inv_rms.device != dev:
             raise RuntimeError(f"q_inv_rms must be a contiguous float32 tensor of {rows} x {q_tokens} elements on {dev}")
         p.q_norm_weight, p.q_inv_rms = weight.data_ptr(), inv_rms.data_ptr()
+    if q_row_squares is not None:
+        weight, squares, eps = q_row_squares
+        if weight.dtype != q.dtype or weight.numel() != heads * HEAD_DIM or not weight.is_contiguous() or weight.device != dev:
+            raise RuntimeError(f"the q norm weight must be a contiguous {q.dtype} tensor of {heads * HEAD_DIM} elements on {dev}")
+        if squares.dtype != torch.float32 or squares.numel() != rows * q_tokens * heads * HEAD_DIM // 32 \
+                or not squares.is_contiguous() or squares.device != dev:
+            raise RuntimeError(f"q_row_squares must be a contiguous float32 tensor of {rows} x {q_tokens} x {heads * 4} elements on {dev}")
+        p.q_norm_weight, p.q_row_squares, p.q_norm_eps = weight.data_ptr(), squares.data_ptr(), eps
     with _on_device(dev):
         if static_scratch:
             _capi.check(lib.sdv2_swa_attn_fwd_static(C.byref(p)), "sdv2_swa_attn_fwd_static")
@@ -1063,10 +1075,13 @@ _PLAIN_TENSORS = (torch.Tensor, torch.nn.Parameter)
 _LINEAR_PREFERRED: dict = {}
 
 
-def linear_or_none(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor]) -> Optional[torch.Tensor]:
+def linear_or_none(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor],
+                   row_squares: bool = False):
     """``x weight^T + bias`` by the library's kernel where that is the faster one
     (``sdv2_linear_preferred``: bf16, a chunk's worth of rows), else None: the
-    caller's nn.Linear, for everything the kernel does not take too."""
+    caller's nn.Linear, for everything the kernel does not take too.  With
+    ``row_squares`` the result comes with the sums of squares of every 32 columns
+    of its rows, float32 [..., n / 32]."""
     bf16 = torch.bfloat16
     if not (x.is_cuda and x.dtype == bf16 and weight.dtype == bf16 and type(x) in _PLAIN_TENSORS
             and type(weight) in _PLAIN_TENSORS and weight.dim() == 2 and x.dim() >= 2 and x.numel() and _plain_call()):
@@ -1093,9 +1108,21 @@ def linear_or_none(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.T
     out = torch.empty((*x.shape[:-1], n), dtype=bf16, device=dev)
     p = _capi.LinearParams(x.data_ptr(), weight.data_ptr(), bias.data_ptr() if bias is not None else None, out.data_ptr(),
                            rows[1], k, n, m, n, k, _capi.DTYPE_BF16, _stream_ptr(dev))
+    squares = torch.empty((*x.shape[:-1], n // 32), dtype=torch.float32, device=dev) if row_squares else None
+    if row_squares:
+        p.row_squares = squares.data_ptr()
     with _on_device(dev):
         _capi.check(_capi.lib().sdv2_linear(C.byref(p)), "sdv2_linear")
-    return out
+    return (out, squares) if row_squares else out
+
+
+def folds_query_norm(q_shape, max_seq_len: int, weight: torch.Tensor, device) -> bool:
+    """Does the attention of a query [B, S, heads * 128] against max_seq_len keys take the raw projection and
+    normalise it itself (``swa_attention(q_row_squares=)``)?"""
+    rows, tokens, width = q_shape
+    return (width % HEAD_DIM == 0 and type(weight) in _PLAIN_TENSORS and weight.dtype == torch.bfloat16 and weight.is_contiguous()
+            and weight.device == device and weight.numel() == width and weight.data_ptr() % 16 == 0
+            and bool(_capi.lib().sdv2_swa_attn_folds_norm(rows, tokens, width // HEAD_DIM, max_seq_len)))
 
 
 def copy_bytes(dst: torch.Tensor, src: torch.Tensor) -> None:
