@@ -202,6 +202,9 @@ __device__ __forceinline__ void dma16(const char* uniform_base, uint32_t lane_of
 // barrier), and the last one reads only after it has drawn.  The 16-byte
 // accesses have no atomic spelling in the language, so they are asm (8-byte
 // atomics were measured 4 % of the whole kernel slower).
+// A store of 16 bytes reads its data up to two cycles after its issue, which the
+// compiler does not know of a store inside a statement: two wait states end it, or
+// the next instruction might write those registers.
 // ---------------------------------------------------------------------------
 __device__ __forceinline__ void store_coherent_x4(void* base, const u32x4& w0, const u32x4& w1, const u32x4& w2,
                                                   const u32x4& w3) {
@@ -209,7 +212,8 @@ __device__ __forceinline__ void store_coherent_x4(void* base, const u32x4& w0, c
       "global_store_dwordx4 %0, %1, off sc1\n\t"
       "global_store_dwordx4 %0, %2, off offset:1024 sc1\n\t"
       "global_store_dwordx4 %0, %3, off offset:2048 sc1\n\t"
-      "global_store_dwordx4 %0, %4, off offset:3072 sc1"
+      "global_store_dwordx4 %0, %4, off offset:3072 sc1\n\t"
+      "s_nop 1"
       :
       : "v"(base), "v"(w0), "v"(w1), "v"(w2), "v"(w3)
       : "memory");
@@ -248,7 +252,8 @@ __device__ __forceinline__ void load_coherent_4x4(const char* b0, const char* b1
 __device__ __forceinline__ void store_coherent_x2(void* base, const f32x4& w0, const f32x4& w1) {
   asm volatile(
       "global_store_dwordx4 %0, %1, off sc1\n\t"
-      "global_store_dwordx4 %0, %2, off offset:16 sc1"
+      "global_store_dwordx4 %0, %2, off offset:16 sc1\n\t"
+      "s_nop 1"
       :
       : "v"(base), "v"(w0), "v"(w1)
       : "memory");
