@@ -592,12 +592,14 @@ def module_path_section(args, w, headline_ms):
     out["cross_attention_forward"] = {
         "ms_per_layer_call": cross_per_layer, "ms_per_step": cross_per_layer * w.layers, "layers_timed": layers,
         "context_tokens": 512,
-        "what": "WanT2VCrossAttention.forward on the cached prompt: q projection (vendor GEMM), q RMSNorm (one launch "
-                "of the library), attention, o projection; scaled to the layer count"}
+        "what": "WanT2VCrossAttention.forward on the cached prompt: q projection (the library's product, or the vendor's "
+                "where that is faster), q RMSNorm (inside the attention, or one launch), attention, o projection; scaled "
+                "to the layer count"}
     out["module_forward"] = {"ms_per_layer_call": per_layer, "ms_per_step": per_layer * w.layers, "layers_timed": layers,
                              "ms_per_step_with_three_projection_launches": per_layer_apart * w.layers,
                              "what": "CausalWanSelfAttention.forward with its defaults: q / k / v as one vendor GEMM "
-                                     "on the packed weights, the path, the o projection; scaled to the layer count"}
+                                     "on the packed weights, the path, the o projection (the library's product, or "
+                                     "the vendor's where that is faster); scaled to the layer count"}
     return out
 
 
