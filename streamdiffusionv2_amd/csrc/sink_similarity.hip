@@ -43,7 +43,7 @@
 namespace {
 
 constexpr int kLanesPerRow = 16;            // 16 lanes x 8 elements = 128
-constexpr int kTokenLanes = 16;             // 256 threads
+constexpr int kTokenLanes = 32;             // 512 threads
 constexpr int kTokenSplits = 8;             // workgroups per (frame, head): token ranges summed apart
 constexpr int kMaxHeads = 64;
 constexpr int kThreads = kLanesPerRow * kTokenLanes;
@@ -210,7 +210,7 @@ __device__ __forceinline__ void decide(const SinkSimKernelArgs& a, int row) {
   auto live = [&](int i) { return raw_col(i) < width ? 1.f : 0.f; };
   // means of matrix m at this thread's columns: the token ranges in order and
   // the rounding of a stored mean, or the mean kept from an earlier call.  The
-  // token sums are fetched for eight columns at a time (64 loads in flight).
+  // token sums are fetched for four columns at a time.
   auto means = [&](int m, float (&out)[kCols]) {
     if (summed_now(a, row, m)) {
       const float* p = sums_of(a, row, m);
@@ -256,7 +256,7 @@ __device__ __forceinline__ void decide(const SinkSimKernelArgs& a, int row) {
   // ahead of the new chunk's sums: loads return in order, so nothing the dot
   // products need is still on its way when the sums have arrived.  (A batch that
   // reaches past the last frame repeats it; its results are dropped.)
-  constexpr int kBatch = kCols <= 8 ? 4 : (kCols <= 20 ? 2 : 1);
+  constexpr int kBatch = kCols <= 4 ? 4 : 2;
   float ks[kBatch][kCols], vs[kBatch][kCols];
   auto fetch_frames = [&](int j0) {
 #pragma unroll
@@ -268,29 +268,22 @@ __device__ __forceinline__ void decide(const SinkSimKernelArgs& a, int row) {
   };
   fetch_frames(0);
   float k_new[kCols], v_new[kCols];
-  if constexpr (kCols <= 8) {
-    // two column groups per thread: all the token sums of a new matrix come in one trip to memory
-    static_assert(kCols == 8, "two column groups per thread");
-    f32x4 part[2][2][kTokenSplits];          // matrix, column group, token range
+  // the token sums of both new matrices, a column group at a time, in one trip to memory
 #pragma unroll
-    for (int m = 0; m < 2; ++m) {
-      const float* p = sums_of(a, row, 2 * sink + m);
-      load_coherent_ranges2(ranges_of(p, 0), ranges_of(p, 4), part[m][0], part[m][1]);
-    }
+  for (int i0 = 0; i0 < kCols; i0 += 4) {
+    f32x4 part[2][kTokenSplits];             // matrix, token range
+    load_coherent_ranges2(ranges_of(sums_of(a, row, 2 * sink), i0), ranges_of(sums_of(a, row, 2 * sink + 1), i0), part[0], part[1]);
 #pragma unroll
-    for (int i = 0; i < kCols; ++i) {
+    for (int e = 0; e < 4; ++e) {
       float sum_k = 0.f, sum_v = 0.f;
 #pragma unroll
       for (int j = 0; j < kTokenSplits; ++j) {
-        sum_k += part[0][i >> 2][j][i & 3];
-        sum_v += part[1][i >> 2][j][i & 3];
+        sum_k += part[0][j][e];
+        sum_v += part[1][j][e];
       }
-      k_new[i] = round_to_storage<T>(sum_k * inv_tokens);
-      v_new[i] = round_to_storage<T>(sum_v * inv_tokens);
+      k_new[i0 + e] = round_to_storage<T>(sum_k * inv_tokens);
+      v_new[i0 + e] = round_to_storage<T>(sum_v * inv_tokens);
     }
-  } else {
-    means(2 * sink, k_new);
-    means(2 * sink + 1, v_new);
   }
   float n[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
@@ -364,17 +357,22 @@ __device__ __forceinline__ void decide(const SinkSimKernelArgs& a, int row) {
 }
 
 // grid (heads, matrices summed in this call, rows * kTokenSplits): one workgroup sums one head's
-// 128 columns of one frame over one eighth of its tokens.  (With every sink
-// frame's mean kept, the matrices are the new K and V alone: first_matrix.)  (One workgroup per
+// 128 columns of one frame over one eighth of its tokens, of the new K and V both.  (With every sink
+// frame's mean kept, those are all: first_matrix.)  (One workgroup per
 // frame and head would leave most of the chip idle: 96 workgroups for three
 // sink frames of twelve heads.)  Then it draws its row's ticket, after its
 // sums have been acknowledged by memory; the workgroup that draws the last one
 // finds every sum of the row in memory, decides, and leaves the ticket at zero
 // for the next call.
+//
+// What bounds it is the chain of trips to memory: tokens with their table entries, sums acknowledged, ticket, sums of
+// the row, results.  512 threads take a range of 195 tokens in one trip and the row's sums in another (256 threads took
+// two each): 2 x 1560 tokens x 12 heads, means kept, 25.2 -> 22 us, and with the new K and V in one workgroup 18.0
+// (one row 17.5 -> 17.2, four 34.2 -> 26.4; 1 x 1560 x 40 heads 39.5 -> 34.0, 4 x 3600 x 40 143 -> 108).
 template <typename T, int kCols>
 __global__ __launch_bounds__(kThreads)
 void sink_similarity_kernel(const SinkSimKernelArgs a) {
-  __shared__ float part[kTokenLanes][kLanesPerRow * 8];
+  __shared__ float part[2][kTokenLanes][kLanesPerRow * 8];    // of the matrix, of V beside the new K
   __shared__ int is_last;
   const int lane = threadIdx.x & (kLanesPerRow - 1);
   const int tl = threadIdx.x >> 4;
@@ -384,29 +382,29 @@ void sink_similarity_kernel(const SinkSimKernelArgs a) {
   const int split = blockIdx.z - row * kTokenSplits;
   const int sink = a.sink_frames;
 
-  const bool is_new = m >= 2 * sink;
-  const bool is_k = is_new ? (m == 2 * sink) : (m < sink);
+  const bool is_new = m == 2 * sink;         // the new K, and the new V with it
+  const bool is_k = is_new || m < sink;
   const int frame = is_new ? 0 : (m < sink ? m : m - sink);
   // a kept frame mean stands until the caller calls it stale
   if (!summed_now(a, row, m)) return;
-  const sdv2_stride3 st = is_new ? (is_k ? a.k_in_st : a.v_in_st) : (is_k ? a.k_st : a.v_st);
-  const T* base = static_cast<const T*>(is_new ? (is_k ? a.k_in : a.v_in) : (is_k ? a.k_cache : a.v_cache));
+  const sdv2_stride3 st = is_new ? a.k_in_st : (is_k ? a.k_st : a.v_st);
+  const T* base = static_cast<const T*>(is_new ? a.k_in : (is_k ? a.k_cache : a.v_cache));
   base += row * st.row + static_cast<int64_t>(frame) * a.tokens * st.token + head * st.head + lane * 8;
 
   const int per = (a.tokens + kTokenSplits - 1) / kTokenSplits;
   const int t_end = (split + 1) * per < a.tokens ? (split + 1) * per : a.tokens;
-  float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-  // A token lane walks every sixteenth token of the range.  The range is short
-  // (195 tokens of a 1560-token frame: 12 or 13 per lane) and every trip to
+  float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f}, acc_v[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+  // A token lane walks every 32nd token of the range.  The range is short (195
+  // tokens of a 1560-token frame: 6 or 7 per lane) and every trip to
   // memory costs the same few microseconds whatever it carries, so a lane asks
   // for up to kFlight of its tokens at once; past the end of the range it asks
   // for the last token again and leaves it out of the sum.  The order of the
   // adds is the token order.
-  constexpr int kFlight = 16;
-  if (is_new && is_k) {
-    // the new keys are rotated on the way in; their table entries (four per lane and token) are fetched for
-    // half a flight at a time, which is what the registers hold beside the tokens themselves
-    constexpr int kHalf = kFlight / 2;
+  constexpr int kFlight = sizeof(T) == 2 ? 8 : 4;        // (what the registers hold)
+  if (is_new) {
+    const T* base_v = static_cast<const T*>(a.v_in) + row * a.v_in_st.row + head * a.v_in_st.head + lane * 8;
+    // the new keys are rotated on the way in; their table entries (four per lane and token) ride along, and so do the
+    // new values: with a workgroup for each, two rows' 384 had one CU's registers each, 256 at a time
     auto rotation = [&](int t, double2 (&cs)[4]) {
       const int hi = t / a.grid_w;
       sdv2::load_rotation(a.freqs, a.pairs, a.split_t, a.split_h, lane, a.start_frame[row], hi, t - hi * a.grid_w, cs);
@@ -415,31 +413,28 @@ void sink_similarity_kernel(const SinkSimKernelArgs a) {
     sdv2::Vec8<T> weight;
     if (a.k_norm_w) weight = sdv2::Vec8<T>::load(static_cast<const T*>(a.k_norm_w) + head * 128 + lane * 8);
     for (int t0 = split * per + tl; t0 < t_end; t0 += kFlight * kTokenLanes) {
-      sdv2::Vec8<T> x[kFlight];
+      sdv2::Vec8<T> x[kFlight], xv[kFlight];
       float r[kFlight];
+      double2 cs[kFlight][4];
 #pragma unroll
       for (int u = 0; u < kFlight; ++u) {
+        if (t0 - tl + u * kTokenLanes >= t_end) break;       // (uniform: nobody's)
         const int t = t0 + u * kTokenLanes < t_end ? t0 + u * kTokenLanes : t_end - 1;
         x[u] = sdv2::Vec8<T>::load(base + t * st.token);
         r[u] = a.k_norm_w ? a.inv_rms[static_cast<int64_t>(row) * a.tokens + t] : 1.0f;
+        rotation(t, cs[u]);
+        xv[u] = sdv2::Vec8<T>::load(base_v + t * a.v_in_st.token);
       }
 #pragma unroll
-      for (int half = 0; half < 2; ++half) {
-        if (t0 + half * kHalf * kTokenLanes >= t_end) break;
-        double2 cs[kHalf][4];
+      for (int u = 0; u < kFlight; ++u) {
+        if (t0 + u * kTokenLanes < t_end) {
+          sdv2::Vec8<T> xx = x[u];
+          if (a.k_norm_w) xx = sdv2::normalise(xx, r[u], weight);
+          const sdv2::Vec8<T> y = sdv2::rotate(xx, cs[u]);
 #pragma unroll
-        for (int u = 0; u < kHalf; ++u) {
-          const int t = t0 + (half * kHalf + u) * kTokenLanes;
-          rotation(t < t_end ? t : t_end - 1, cs[u]);
-        }
-#pragma unroll
-        for (int u = 0; u < kHalf; ++u) {
-          if (t0 + (half * kHalf + u) * kTokenLanes < t_end) {
-            sdv2::Vec8<T> xx = x[half * kHalf + u];
-            if (a.k_norm_w) xx = sdv2::normalise(xx, r[half * kHalf + u], weight);
-            const sdv2::Vec8<T> y = sdv2::rotate(xx, cs[u]);
-#pragma unroll
-            for (int i = 0; i < 8; ++i) acc[i] += static_cast<float>(y.get(i));
+          for (int i = 0; i < 8; ++i) {
+            acc[i] += static_cast<float>(y.get(i));
+            acc_v[i] += static_cast<float>(xv[u].get(i));
           }
         }
       }
@@ -460,19 +455,23 @@ void sink_similarity_kernel(const SinkSimKernelArgs a) {
     }
   }
 #pragma unroll
-  for (int i = 0; i < 8; ++i) part[tl][lane * 8 + i] = acc[i];
+  for (int i = 0; i < 8; ++i) {
+    part[0][tl][lane * 8 + i] = acc[i];
+    if (is_new) part[1][tl][lane * 8 + i] = acc_v[i];
+  }
   __syncthreads();
-  if (threadIdx.x < kLanesPerRow * 8) {
+  const int of = threadIdx.x >> 7, column = threadIdx.x & 127;
+  if (of < (is_new ? 2 : 1)) {
     float sum = 0.f;
 #pragma unroll
-    for (int j = 0; j < kTokenLanes; ++j) sum += part[j][threadIdx.x];
-    store_coherent(sums_of(a, row, m) + (head * kTokenSplits + split) * 128 + threadIdx.x, sum);
+    for (int j = 0; j < kTokenLanes; ++j) sum += part[of][j][column];
+    store_coherent(sums_of(a, row, m + of) + (head * kTokenSplits + split) * 128 + column, sum);
   }
   __builtin_amdgcn_s_waitcnt(0x0F70);       // vmcnt(0): the stores have been acknowledged
   __syncthreads();
   if (threadIdx.x == 0) {
     // workgroups of this row that sum anything in this call
-    int matrices = 2;
+    int matrices = 1;                        // (the new K and V go together)
     for (int f = 0; f < sink; ++f) matrices += summed_now(a, row, f) ? 2 : 0;
     const int expected = matrices * a.heads * kTokenSplits;
     const int drawn = __hip_atomic_fetch_add(a.tickets + row, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -605,7 +604,7 @@ extern "C" int sdv2_sink_similarity(const sdv2_sink_sim_params* p) {
   bool any_stale = false;
   for (int i = 0; i < p->rows; ++i) any_stale |= (a.stale[i] & ((1u << p->sink_frames) - 1u)) != 0;
   a.first_matrix = any_stale ? 0 : 2 * p->sink_frames;
-  const dim3 grid(p->heads, 2 * p->sink_frames + 2 - a.first_matrix, p->rows * kTokenSplits);
+  const dim3 grid(p->heads, 2 * p->sink_frames + 1 - a.first_matrix, p->rows * kTokenSplits);
   if (p->k_norm_weight) {
     const dim3 grid_rms((p->tokens + 3) / 4, 1, p->rows);
     const int steps = (p->heads + 3) / 4;
@@ -618,7 +617,7 @@ extern "C" int sdv2_sink_similarity(const sdv2_sink_sim_params* p) {
     else if (steps <= 10) launch(std::integral_constant<int, 10>{});
     else launch(std::integral_constant<int, 16>{});
   }
-  // columns per thread of the deciding workgroup: 8 up to 16 heads, 20 up to 40, 32 up to 64
+  // columns per thread of the deciding workgroup: 4 up to 16 heads, 12 up to 48, 16 up to 64
   auto launch = [&](auto cols_c) {
     constexpr int kCols = decltype(cols_c)::value;
     if (p->dtype == SDV2_BF16)
@@ -627,8 +626,9 @@ extern "C" int sdv2_sink_similarity(const sdv2_sink_sim_params* p) {
       sdv2::launch_timed(SDV2_KERNEL_SINK, sink_similarity_kernel<float, kCols>, grid, block, 0, stream, a);
   };
   const int width = p->heads * SDV2_HEAD_DIM;
-  if (width <= 8 * kThreads) launch(std::integral_constant<int, 8>{});
-  else if (width <= 20 * kThreads) launch(std::integral_constant<int, 20>{});
-  else launch(std::integral_constant<int, 32>{});
+  if (width <= 4 * kThreads) launch(std::integral_constant<int, 4>{});
+  else if (width <= 12 * kThreads) launch(std::integral_constant<int, 12>{});
+  else launch(std::integral_constant<int, 16>{});
+  static_assert(16 * kThreads >= kMaxHeads * SDV2_HEAD_DIM, "columns of the deciding workgroup");
   return hipGetLastError() == hipSuccess ? SDV2_OK : SDV2_ERR_LAUNCH;
 }

@@ -144,9 +144,9 @@ def test_similarity_operator(gpu_device, dtype, tol, head_major):
 @pytest.mark.gpu
 @pytest.mark.parametrize("heads,sink", [(40, 3), (17, 16), (64, 2), (1, 1)])
 def test_similarity_operator_wide_and_deep(gpu_device, heads, sink):
-    """The kernel has builds for up to 16, 40 and 64 heads (8, 20 and 32 columns
-    per thread of the deciding workgroup, which takes the sink frames four,
-    two or one at a time) and room for 16 sink frames; the slot hand-over is
+    """The kernel has builds for up to 16, 48 and 64 heads (4, 12 and 16 columns
+    per thread of the deciding workgroup, which takes the sink frames four or
+    two at a time) and room for 16 sink frames; the slot hand-over is
     checked on the way (rows 0 and 2 flagged as evicting)."""
     from streamdiffusionv2_amd import ops, rope
 
