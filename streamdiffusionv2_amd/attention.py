@@ -584,6 +584,7 @@ class WanT2VCrossAttention(nn.Module):
         else:
             if context_lens is not None:
                 context_lens = context_lens.to(device=q.device, dtype=torch.int32).contiguous()
+            k, v = k.to(q.dtype), v.to(q.dtype)              # (as flash_attention does)
             out = ops.swa_attention(q, k, v, context_lens, q_row_squares=(self.norm_q.weight, raw[1], self.norm_q.eps))
         return _linear(self.o, out.flatten(2))
 
@@ -593,13 +594,7 @@ class WanT2VCrossAttention(nn.Module):
         if not (x.dim() == 3 and self.head_dim == ops.HEAD_DIM and _unwatched(self.q) and _unwatched(self.norm_q, WanRMSNorm)
                 and self.q.weight.shape[0] == self.dim):
             return None
-        keys = context
-        if crossattn_cache is not None and crossattn_cache["is_init"]:
-            keys = crossattn_cache["k"]
-            if keys.dtype != x.dtype or crossattn_cache["v"].dtype != x.dtype:
-                return None
-        elif keys.dtype != x.dtype or self.k.weight.dtype != x.dtype or self.v.weight.dtype != x.dtype:
-            return None
+        keys = crossattn_cache["k"] if crossattn_cache is not None and crossattn_cache["is_init"] else context
         if not ops.folds_query_norm((x.size(0), x.size(1), self.dim), keys.shape[1], self.norm_q.weight, x.device):
             return None
         return ops.linear_or_none(x, self.q.weight, self.q.bias, row_squares=True)

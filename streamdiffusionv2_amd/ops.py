@@ -1073,6 +1073,7 @@ def _plain_call() -> bool:
 
 _PLAIN_TENSORS = (torch.Tensor, torch.nn.Parameter)
 _LINEAR_PREFERRED: dict = {}
+_FOLDS_NORM: dict = {}
 
 
 def linear_or_none(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor],
@@ -1120,9 +1121,17 @@ def folds_query_norm(q_shape, max_seq_len: int, weight: torch.Tensor, device) ->
     """Does the attention of a query [B, S, heads * 128] against max_seq_len keys take the raw projection and
     normalise it itself (``swa_attention(q_row_squares=)``)?"""
     rows, tokens, width = q_shape
-    return (width % HEAD_DIM == 0 and type(weight) in _PLAIN_TENSORS and weight.dtype == torch.bfloat16 and weight.is_contiguous()
-            and weight.device == device and weight.numel() == width and weight.data_ptr() % 16 == 0
-            and bool(_capi.lib().sdv2_swa_attn_folds_norm(rows, tokens, width // HEAD_DIM, max_seq_len)))
+    if not (device.type == "cuda" and width % HEAD_DIM == 0 and type(weight) in _PLAIN_TENSORS and _plain_call()
+            and weight.dtype == torch.bfloat16 and weight.is_contiguous() and weight.device == device
+            and weight.numel() == width and weight.data_ptr() % 16 == 0):
+        return False
+    key = (rows, tokens, width, max_seq_len)
+    folds = _FOLDS_NORM.get(key)
+    if folds is None:
+        if len(_FOLDS_NORM) >= _MAX_ATTN_LAYOUTS:
+            _FOLDS_NORM.clear()
+        folds = _FOLDS_NORM[key] = bool(_capi.lib().sdv2_swa_attn_folds_norm(rows, tokens, width // HEAD_DIM, max_seq_len))
+    return folds
 
 
 def copy_bytes(dst: torch.Tensor, src: torch.Tensor) -> None:

@@ -113,5 +113,13 @@ def test_module_folds_only_what_nobody_watches(gpu_device, monkeypatch):
         assert (watched.float() - first.float()).abs().max() <= 2e-2 * max(1.0, first.float().abs().max().item())
         short = module(x[:1, :256], text[:1], None)            # another kernel: the norm's own launch
         assert (1, 256, 1536) in norms and torch.isfinite(short.float()).all()
+        # keys that are not bf16, from projections that have no weight of their own: cast, as without the fold
+        module.norm_k.float()
+        inner = module.v
+        module.v = torch.nn.Sequential(inner)
+        mixed = module(x, text, None)
+        module.norm_k.bfloat16()
+        module.v = inner
+        assert norms.count(query) == 1 and (mixed.float() - first.float()).abs().max() <= 2e-2 * max(1.0, first.float().abs().max().item())
     module(x, text, None).sum()                                # autograd: the module's own expression
     assert norms.count(query) == 1
