@@ -53,6 +53,7 @@ struct AttnKernelArgs {
   // (Uniform: group_pairs = rows * heads, more_pairs = 0.)
   int32_t num_splits, group_pairs, more_pairs;
   int32_t q_tiles, per_group, total_items;        // query tiles per (row, head); work items per group and in all
+  int32_t q_tile_rows;         // rows of a query tile
   FastDiv div_group, div_q_tiles, div_splits, div_splits_more, div_heads;
   float scale_log2;            // softmax_scale * log2(e)
   int32_t mask_block_tokens;   // 0 = no mask inside the chunk
@@ -392,6 +393,7 @@ struct WorkItem {
 };
 // host: everything decode() needs, for query tiles of q_tile_rows rows
 inline void set_work_list(AttnKernelArgs* a, int q_tile_rows) {
+  a->q_tile_rows = q_tile_rows;
   a->q_tiles = (a->q_tokens + q_tile_rows - 1) / q_tile_rows;
   a->per_group = a->q_tiles * ((a->group_pairs - a->more_pairs) * a->num_splits + a->more_pairs * (a->num_splits + 1));
   a->total_items = a->rows * a->heads / a->group_pairs * a->per_group;

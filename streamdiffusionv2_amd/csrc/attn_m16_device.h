@@ -1,5 +1,5 @@
 // The streaming loop of the bf16 attention on 16x16x32 matrix instructions (gfx950
-// only): 8 waves = 256 query rows of one (row, head) against a range of its keys, for
+// only): 8 waves = up to 256 query rows of one (row, head) against a range of its keys, for
 // the kernels that give a workgroup one such range (swa_attn_fwd_m16.hip) or a
 // share of several (swa_attn_fwd_even.hip).
 //
@@ -428,9 +428,8 @@ __device__ __forceinline__ void exact_pass(LaneConst& c, const bf16x8 (&qf)[2][4
 // are hidden from every query of the workgroup (from the last one, that is) are left out, and key ranges are cut from
 // what is left.
 template <bool kMask>
-__device__ __forceinline__ TileSpan tile_list(late_args<AttnKernelArgs>& a, int qtile, int chunk_start, int seq) {
-  const int q_last = qtile * kQTile + kQTile < a.q_tokens ? qtile * kQTile + kQTile - 1 : a.q_tokens - 1;
-  return visible_tiles(kKTile, seq, q_last, a.q_tokens, chunk_start, kMask ? a.mask_block_tokens : 0,
+__device__ __forceinline__ TileSpan tile_list(late_args<AttnKernelArgs>& a, int q_end, int chunk_start, int seq) {
+  return visible_tiles(kKTile, seq, q_end - 1, a.q_tokens, chunk_start, kMask ? a.mask_block_tokens : 0,
                        read_div(a.div_mask_block));
 }
 
@@ -440,9 +439,10 @@ __device__ __forceinline__ int row_keys(late_args<AttnKernelArgs>& a, int row) {
   return seq < 0 ? 0 : seq;
 }
 
-// no query row of this wave exists
-__device__ __forceinline__ bool block_idle(late_args<AttnKernelArgs>& a, int qtile, int wave) {
-  return __builtin_amdgcn_readfirstlane(qtile * kQTile + wave * kQBlock >= a.q_tokens);
+// The row behind the last one of query tile `qtile`, of tiles of `rows` rows
+__device__ __forceinline__ int tile_end_row(late_args<AttnKernelArgs>& a, int qtile, int rows) {
+  const int end = (qtile + 1) * rows;
+  return end < a.q_tokens ? end : a.q_tokens;
 }
 
 // A word of memory looked at by thread 0 before the range's last matrix instructions, for the time behind them.
@@ -462,12 +462,12 @@ struct NoPeek {
   __device__ __forceinline__ void end(int) const {}
 };
 
-// The workgroup's 256 query rows against entries [tile_begin, tile_end) of a tile list, the first
+// The workgroup's query rows, q_first .. q_end - 1, 32 a wave, against entries [tile_begin, tile_end) of a tile list, the first
 // key of entry t being key0_of(t): sums of the weighted values
 // (oacc), the queries' row sums (l_sum) and the exponent references both are relative to (c.neg_ref).  Behind it every
 // wave is done with the tile buffers.
 template <bool kMask, typename KeyOf, typename LookAt = NoPeek>
-__device__ __forceinline__ void stream_range(late_args<AttnKernelArgs>& a, lds_char* lds, int qtile, int head, int row, int seq,
+__device__ __forceinline__ void stream_range(late_args<AttnKernelArgs>& a, lds_char* lds, int q_first, int q_end, int head, int row, int seq,
                                              KeyOf key0_of, int tile_begin, int tile_end, LaneConst& c,
                                              f32x4 (&oacc)[8][2], float (&l_sum)[2], LookAt look = LookAt()) {
   lds_int* flags = reinterpret_cast<lds_int*>(lds + kLdsFlags);
@@ -503,7 +503,7 @@ __device__ __forceinline__ void stream_range(late_args<AttnKernelArgs>& a, lds_c
   // memory; one that is to be rotated here needs several trips for the rotation
   // table and is fetched behind the tiles the first two slots need, the rest of
   // the look-ahead after it.
-  const int q_row = qtile * kQTile + wave * kQBlock + n16;      // and q_row + 16
+  const int q_row = q_first + wave * kQBlock + n16;      // and q_row + 16
   bf16x8 qf[2][4];
   const uint16_t* q_ptr[2];
   int q_tok[2];
@@ -568,7 +568,7 @@ __device__ __forceinline__ void stream_range(late_args<AttnKernelArgs>& a, lds_c
   if constexpr (kMask) {
     c.m_block = a.mask_block_tokens;
     c.m_div = read_div(a.div_mask_block);
-    c.q_first = qtile * kQTile + wave_u * kQBlock;
+    c.q_first = q_first + wave_u * kQBlock;
     c.m_first = __builtin_amdgcn_readfirstlane(row_chunk_start(a, row));
     c.m_hi = c.m_first + a.q_tokens;
     c.m_lo = __builtin_amdgcn_readfirstlane(c.m_first + (c.m_div(c.q_first) + 1) * c.m_block);
@@ -640,7 +640,7 @@ __device__ __forceinline__ void stream_range(late_args<AttnKernelArgs>& a, lds_c
   using B2 = std::integral_constant<int, 2>;
   using B3 = std::integral_constant<int, 3>;
 
-  const bool idle = block_idle(a, qtile, wave);
+  const bool idle = __builtin_amdgcn_readfirstlane(q_first + wave * kQBlock >= q_end);       // no query row is this wave's
   int seen = 0;
   if (n > 0) {
     // K tiles 0 and 1 and V tile 0 have landed once at most the four tiles requested behind them are in flight
@@ -762,9 +762,8 @@ __device__ __forceinline__ void stage_out(lds_char* stage, int lane, int db, con
     *reinterpret_cast<__attribute__((address_space(3))) u32x2*>(stage + r * 256 + ((chunk ^ n16) << 4) + (g & 1) * 8) = x;
   }
 }
-__device__ __forceinline__ void write_block(late_args<AttnKernelArgs>& a, lds_char* stage, int qtile, int head, int row, int wave, int lane) {
+__device__ __forceinline__ void write_block(late_args<AttnKernelArgs>& a, lds_char* stage, int q0, int head, int row, int lane) {
   const int n16 = lane & 15, g = lane >> 4;
-  const int q0 = qtile * kQTile + wave * kQBlock;
   uint16_t* dst = a.out + row * a.o_st.row + head * a.o_st.head + (int64_t)q0 * a.o_st.token;
 #pragma unroll
   for (int it = 0; it < 8; ++it) {

@@ -161,7 +161,7 @@ void swa_attn_fwd_even_kernel(const EvenArgs args) {
 
       if (!is_block) {
         const int seq = row_keys(a.call, row);
-        const TileSpan list = tile_list<kMask>(a.call, item, kMask ? row_chunk_start(a.call, row) : 0, seq);
+        const TileSpan list = tile_list<kMask>(a.call, tile_end_row(a.call, item, kQTile), kMask ? row_chunk_start(a.call, row) : 0, seq);
         // (a row may hold fewer keys than the longest one)
         tile_begin = tile_begin < list.count ? tile_begin : list.count;
         tile_end = tile_end < list.count ? tile_end : list.count;
@@ -179,7 +179,7 @@ void swa_attn_fwd_even_kernel(const EvenArgs args) {
         float l_sum[2];
         // (a piece that ends the share finds the others of its item done, more often than not)
         const bool ends = !whole && next_off >= end && tile_end > tile_begin;
-        stream_range<kMask>(a.call, lds, item, head, row, seq, key0_of, tile_begin, tile_end, c, oacc, l_sum,
+        stream_range<kMask>(a.call, lds, item * kQTile, tile_end_row(a.call, item, kQTile), head, row, seq, key0_of, tile_begin, tile_end, c, oacc, l_sum,
                             Peek{ends ? ticket : nullptr, parts - 1, flags});
 
         late_args<EvenArgs>& b = read_late<EvenArgs>();
@@ -197,7 +197,7 @@ void swa_attn_fwd_even_kernel(const EvenArgs args) {
           if (!idle) {
 #pragma unroll
             for (int db = 0; db < 8; ++db) stage_out(stage, lane, db, oacc[db], inv);
-            write_block(b.call, stage, item, head, row, wave, lane);
+            write_block(b.call, stage, item * kQTile + wave * kQBlock, head, row, lane);
           }
         } else {
           float lse[2];
@@ -295,7 +295,7 @@ void swa_attn_fwd_even_kernel(const EvenArgs args) {
                   for (int db = 0; db < 4; ++db) stage_out(stage, lane, 4 * half + db, acc[db], inv);
                 }
               }
-              write_block(b.call, stage, item, head, row, wave, lane);
+              write_block(b.call, stage, item * kQTile + wave * kQBlock, head, row, lane);
             }
           }
         }

@@ -17,7 +17,7 @@
 // matrix pipe too (mfma_row_sum): v_dot2c_f32_bf16, which adds up two packed weights,
 // waits some 20 cycles for it to run empty, a fifth of the whole loop.
 //
-// Work decomposition: workgroup = 8 waves = 256 query rows of one (row, head),
+// Work decomposition: workgroup = 8 waves = up to 256 query rows of one (row, head),
 // one workgroup per CU, two waves per SIMD with 256 registers each; wave w owns
 // the 32-row block 32w..32w+31.  Keys stream through LDS in tiles of 64, four
 // buffers per matrix, filled three tiles ahead by global->LDS transfers that never
@@ -56,7 +56,8 @@ void swa_attn_fwd_m16_kernel(const AttnKernelArgs args) {
   const int qtile = w.qtile, head = w.head, row = w.row, split = w.split, nsplits = w.nsplits;
 
   const int seq = row_keys(a, row);
-  const TileSpan list = tile_list<kMask>(a, qtile, kMask ? row_chunk_start(a, row) : 0, seq);
+  const int q_first = qtile * a.q_tile_rows, q_end = tile_end_row(a, qtile, a.q_tile_rows);
+  const TileSpan list = tile_list<kMask>(a, q_end, kMask ? row_chunk_start(a, row) : 0, seq);
   const int per_split = (list.count + nsplits - 1) / nsplits;
   const int tile_begin = split * per_split;
   int tile_end = tile_begin + per_split;
@@ -66,13 +67,14 @@ void swa_attn_fwd_m16_kernel(const AttnKernelArgs args) {
   f32x4 oacc[8][2];
   float l_tot[2];
   auto key0_of = [=](int tile) { return (kMask && tile >= list.hole ? tile + list.skipped : tile) * kKTile; };
-  stream_range<kMask>(a, lds, qtile, head, row, seq, key0_of, tile_begin, tile_end, c, oacc, l_tot);
+  stream_range<kMask>(a, lds, q_first, q_end, head, row, seq, key0_of, tile_begin, tile_end, c, oacc, l_tot);
   late_args<AttnKernelArgs>& b = read_late<AttnKernelArgs>();
-  const bool idle = __builtin_amdgcn_readfirstlane(qtile * kQTile + wave * kQBlock >= b.q_tokens);
+  const int q0 = qtile * b.q_tile_rows + wave * kQBlock;           // of this wave
+  const bool idle = __builtin_amdgcn_readfirstlane(q0 >= tile_end_row(b, qtile, b.q_tile_rows));
 
   // ---- epilogue ---------------------------------------------------------------
   // (every wave is done with the K / V buffers: the barrier above, or the last one of the exact pass)
-  const int block = qtile * kWaves + wave;              // this wave's 32-row block within the (row, head)
+  const int block = q0 / kQBlock;                       // this wave's 32-row block within the (row, head)
   float inv[2];
 #pragma unroll
   for (int qt = 0; qt < 2; ++qt) {
@@ -212,7 +214,7 @@ void swa_attn_fwd_m16_kernel(const AttnKernelArgs args) {
     for (int db = 0; db < 8; ++db) stage_out(stage, lane, db, oacc[db], inv);
   }
 
-  write_block(b, stage, qtile, head, row, wave, lane);
+  write_block(b, stage, q0, head, row, lane);
 }
 
 }  // namespace

@@ -546,3 +546,35 @@ def test_masked_calls_with_host_starts_on_two_streams(gpu_device):
         torch.cuda.synchronize()
         assert torch.equal(out.view(torch.int16), want[64].view(torch.int16))
         assert torch.equal(eager.view(torch.int16), want[200].view(torch.int16))
+
+
+@pytest.mark.parametrize("rows,S,H,L,seq,block,splits", [
+    (1, 2688, 12, 200, None, 0, 1),             # four blocks of 32 rows a tile, 252 of them; 32x32x16
+    (1, 2689, 12, 833, None, 0, 1),             # five: one row past what four reach; 16x16x32
+    (1, 3361, 12, 130, [65], 0, 1),             # six
+    (2, 300, 12, 2400, [2400, 1], 0, 3),        # four, three key ranges, the last tile 44 rows; 16x16x32
+    (2, 513, 8, 700, [64, 700], 0, 2),          # four, one row in the last tile, a row whose second range is empty; 32x32x16
+    (3, 801, 7, 2500, None, 0, 2),              # five, two ranges
+    (1, 1560, 12, 2304, None, 0, 3),            # seven, as many tiles as of eight
+    (2, 900, 12, 1500, None, 300, 1),           # four, the chunk's blocks end inside a tile
+    (1, 1290, 12, 2600, None, 129, 2),          # four, a block is one row longer than a tile
+    (1, 2700, 12, 2700, None, 900, 1),          # five
+])
+def test_query_tiles_of_fewer_rows(gpu_device, rows, S, H, L, seq, block, splits):
+    from streamdiffusionv2_amd import ops
+
+    print(f"fewer rows a tile: {rows} x {S} x {H} against {L} ({seq}), block {block}, {splits} ranges", flush=True)
+    torch.manual_seed(21)
+    q, k, v = (torch.randn(rows, n, H, 128).bfloat16() for n in (S, L, L))
+    lens = seq or [L] * rows
+    mask, starts = {}, None
+    if block:
+        starts = [(L - S) // (r + 1) for r in range(rows)]
+        mask = dict(chunk_key_start=starts, mask_block_tokens=block)
+    want = oracle.attention_fp32_reference(q, k, v, lens, *((starts, block) if block else ()))
+    sl = torch.tensor(lens, dtype=torch.int32, device=gpu_device) if seq else None
+    args = [t.to(gpu_device) for t in (q, k, v)]
+    got = [ops.swa_attention(*args, sl, num_splits=splits, **mask) for _ in range(2)]
+    torch.cuda.synchronize()
+    assert torch.equal(*got)
+    _check(got[0].cpu(), want)
