@@ -41,8 +41,9 @@ extern "C" {
  * 17: sdv2_linear, sdv2_linear_preferred
  * 18: sdv2_linear_params.row_squares, sdv2_attn_params.q_row_squares and
  *     q_norm_eps, sdv2_swa_attn_folds_norm
- * 19: sdv2_swa_attn_plan_masked */
-#define SDV2KV_ABI_VERSION 19
+ * 19: sdv2_swa_attn_plan_masked
+ * 20: sdv2_append_params.k_inv_rms, sdv2_sink_sim_params.q_in and what follows it */
+#define SDV2KV_ABI_VERSION 20
 #define SDV2_HEAD_DIM 128      /* causal_stream_inference.py:99-100 fixes 128 */
 #define SDV2_MAX_ROWS 16       /* rows (B) per sdv2_kv_append_rope call       */
 #define SDV2_MAX_SINK_FRAMES 16 /* sink frames per sdv2_sink_similarity call  */
@@ -147,6 +148,11 @@ typedef struct sdv2_append_params {
    * no rotated query is written, and sdv2_swa_attn_fwd normalises and rotates
    * the raw q itself (its q_norm_weight / q_inv_rms), to the same bits.       */
   float* q_inv_rms;
+  /* Optional: device float [B * S], 1 / rms of every key token as
+   * sdv2_sink_similarity leaves them (its k_inv_rms).  k_in is then normalised
+   * with these and k_norm_weight, to the same bits; q_in and q_norm_weight are
+   * NULL (the query is rotated beside that decision too).                     */
+  const float* k_inv_rms;
 } sdv2_append_params;
 
 int sdv2_kv_append_rope(const sdv2_append_params* p);
@@ -371,6 +377,17 @@ typedef struct sdv2_sink_sim_params {
   float* frame_sums;
   const uint32_t* stale_frames;
   const int32_t* planned_frame;
+  /* Optional, SDV2_BF16: the chunk's query, rotated by workgroups that have
+   * nothing to do with the decision, as sdv2_kv_append_rope would (same bits),
+   * so that the append that follows moves K and V only.  q_norm_weight, together
+   * with k_norm_weight: q_in is the raw q projection.                          */
+  const void* q_in;            /* [B,S,H,128], or NULL together with q_out      */
+  void* q_out;
+  sdv2_stride3 q_in_stride, q_out_stride;
+  const void* q_norm_weight;
+  /* Optional, with k_norm_weight: device float [B * S] that receives 1 / rms of
+   * every new key token, for sdv2_append_params.k_inv_rms.                     */
+  float* k_inv_rms;
 } sdv2_sink_sim_params;
 
 size_t sdv2_sink_similarity_workspace_bytes(int32_t rows, int32_t tokens, int32_t heads, int32_t sink_frames);

@@ -12,7 +12,7 @@ from typing import Optional
 
 LIB_PATH = Path(__file__).resolve().parent / "_lib" / "libsdv2kv.so"
 
-ABI_VERSION = 19
+ABI_VERSION = 20
 HEAD_DIM = 128
 MAX_ROWS = 16
 
@@ -90,6 +90,7 @@ class AppendParams(C.Structure):
         ("norm_eps", C.c_float),
         ("dst_start_override", C.c_void_p),
         ("q_inv_rms", C.c_void_p),
+        ("k_inv_rms", C.c_void_p),
     ]
 
 
@@ -145,6 +146,10 @@ class SinkSimParams(C.Structure):
         ("frame_sums", C.c_void_p),
         ("stale_frames", C.POINTER(C.c_uint32)),
         ("planned_frame", C.POINTER(C.c_int32)),
+        ("q_in", C.c_void_p), ("q_out", C.c_void_p),
+        ("q_in_stride", Stride3), ("q_out_stride", Stride3),
+        ("q_norm_weight", C.c_void_p),
+        ("k_inv_rms", C.c_void_p),
     ]
 
 

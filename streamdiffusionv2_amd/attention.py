@@ -333,7 +333,7 @@ class RingKVPath:
         try:
             # planned as if no row refreshed; _settle() corrects the host state later where one did
             plan = ring.plan_append(kv_cache, self._evict_idx, starts, q.shape[1], frame_tokens, self.sink_size)
-            override = None
+            override = rotated = None
             if adaptive:
                 # adaptive sink refresh (causal_model.py:284-299): one fused
                 # reduction on the device, whose decision goes straight to the
@@ -349,6 +349,12 @@ class RingKVPath:
                     planned = [d // frame_tokens if d < self.sink_size * frame_tokens else -1 for d in plan.dst_start]
                     extra = dict(frame_sums=kept["sums"], stale_frames=list(kept["stale"]), planned_frames=planned)
                     kept["stale"] = [0] * rows        # summed now, and kept current by the decision kernel from here on
+                if q.dtype == torch.bfloat16 and rows <= ops._capi.MAX_ROWS:
+                    # the query rides along with the decision, and 1 / rms of the keys is handed on: the append
+                    # has K and V left to move (tensors of this call's own, as in LayerLauncher.patch)
+                    rotated = (torch.empty(q.shape, dtype=q.dtype, device=q.device),
+                               torch.empty((rows, q.shape[1]), dtype=torch.float32, device=q.device) if k_norm is not None else None)
+                    extra.update(query=(q, rotated[0], qk_norm[0] if qk_norm is not None else None), k_inv_rms=rotated[1])
                 ops.sink_similarity(
                     k, v, kv_cache["k"], kv_cache["v"], table, (h, w), [c // frame_tokens for c in starts],
                     self.sink_size, self.adapt_sink_thr, dst_start_override=override, override_rows=plan.evicting,
@@ -374,6 +380,7 @@ class RingKVPath:
                 # (cache, shape) and only patched per call
                 launcher = self._layer_launcher(q, k, v, kv_cache, table, (f, h, w), qk_norm)
                 start_frames = [c // frame_tokens for c in starts]
+                launcher.rotated = rotated
                 out = launcher.launch(q, k, v, start_frames, plan, seq, mask_tokens, override)
                 # (not held from call to call: the allocator hands the memory to the next layer)
                 roped_q, launcher.roped_q = launcher.roped_q, None

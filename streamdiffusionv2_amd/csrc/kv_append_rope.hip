@@ -43,6 +43,7 @@ struct AppendKernelArgs {
   int64_t* local_end;
   const int64_t* dst_override;              // device [rows] or null; a value >= 0 replaces dst_start[row]
   float* q_inv_rms;                         // device [rows][tokens] or null: 1 / rms of every q token (fused norm)
+  const float* k_inv_rms;                   // device [rows][tokens]: 1 / rms of every k token, taken by an earlier launch
   int64_t cache_tokens;
   int32_t tokens, heads, grid_w, frame_tokens;
   int32_t split_t, split_h;                 // pair index bounds: [0,split_t) temporal, [split_t,split_h) height
@@ -67,7 +68,10 @@ __device__ __forceinline__ int64_t row_dst_start(const AppendKernelArgs& a, int 
 
 // kWithKV = false: rotation of q alone (the stand-alone causal_rope_apply,
 // causal_model.py:94-108), no cache and no index is touched.
-template <typename T, bool kWithQ, bool kWithKV>
+// kNormK: k is the raw projection, normalised with the 1 / rms that the sink decision ahead of this launch took.  With
+// the query rotated there too, what is left is bound by the copy: 2 x 1560 tokens x 12 heads 8.4 us = 4.6 TB/s, where
+// the launch that does it all (kv_append_norm_rope_kernel) takes 16.3.
+template <typename T, bool kWithQ, bool kWithKV, bool kNormK = false>
 __global__ __launch_bounds__(kLanesPerRow * kTokensPerBlock)
 void kv_append_rope_kernel(const AppendKernelArgs a) {
   sdv2::fetch_arguments<AppendKernelArgs>();
@@ -100,11 +104,14 @@ void kv_append_rope_kernel(const AppendKernelArgs a) {
   T* kc = static_cast<T*>(a.k_cache) + row * a.k_st.row + dst_tok * a.k_st.token + e0;
   T* vc = static_cast<T*>(a.v_cache) + row * a.v_st.row + dst_tok * a.v_st.token + e0;
 
-  sdv2::Vec8<T> q[kHeadsPerThread], k[kHeadsPerThread], v[kHeadsPerThread];
+  sdv2::Vec8<T> q[kHeadsPerThread], k[kHeadsPerThread], v[kHeadsPerThread], wk[kHeadsPerThread];
+  float rk = 1.f;
+  if constexpr (kNormK) rk = a.k_inv_rms[static_cast<int64_t>(row) * a.tokens + tok];
 #pragma unroll
   for (int j = 0; j < kHeadsPerThread; ++j) {
     const int h = head0 + j;
     if (h < a.heads) {
+      if constexpr (kNormK) wk[j] = sdv2::Vec8<T>::load(static_cast<const T*>(a.k_norm_w) + h * 128 + e0);
       if (kWithKV) {
         k[j] = sdv2::Vec8<T>::load(ki + h * a.k_in_st.head);
         v[j] = sdv2::Vec8<T>::load(vi + h * a.v_in_st.head);
@@ -118,6 +125,7 @@ void kv_append_rope_kernel(const AppendKernelArgs a) {
     if (h < a.heads) {
       if (kWithKV) {
         v[j].store(vc + h * a.v_st.head);
+        if constexpr (kNormK) k[j] = sdv2::normalise(k[j], rk, wk[j]);
         sdv2::rotate(k[j], cs).store(kc + h * a.k_st.head);
       }
       if (kWithQ) sdv2::rotate(q[j], cs).store(qo + h * a.q_out_st.head);
@@ -300,7 +308,11 @@ extern "C" int sdv2_kv_append_rope(const sdv2_append_params* p) {
   if (p->grid_f <= 0 || p->grid_h <= 0 || p->grid_w <= 0) return SDV2_ERR_INVALID_ARG;
   if (static_cast<int64_t>(p->grid_f) * p->grid_h * p->grid_w != p->tokens) return SDV2_ERR_INVALID_ARG;
   if (!p->freqs) return SDV2_ERR_INVALID_ARG;
-  const bool with_norm = p->q_norm_weight != nullptr || p->k_norm_weight != nullptr;
+  // k normalised with 1 / rms values that are there already: the query is elsewhere
+  const bool norm_k = p->k_inv_rms != nullptr;
+  if (norm_k && (!p->k_in || !p->k_norm_weight || p->q_norm_weight || p->q_in)) return SDV2_ERR_INVALID_ARG;
+  if (norm_k && (!aligned16(p->k_norm_weight) || (reinterpret_cast<uintptr_t>(p->k_inv_rms) & 3))) return SDV2_ERR_INVALID_ARG;
+  const bool with_norm = !norm_k && (p->q_norm_weight != nullptr || p->k_norm_weight != nullptr);
   // q comes with the tensor its rotation goes to - or, with the norm folded in, with the place for its 1 / rms
   if (p->q_inv_rms && !with_norm) return SDV2_ERR_INVALID_ARG;
   if (p->q_in == nullptr ? (p->q_out != nullptr || p->q_inv_rms != nullptr) : (p->q_out == nullptr && p->q_inv_rms == nullptr))
@@ -355,6 +367,7 @@ extern "C" int sdv2_kv_append_rope(const sdv2_append_params* p) {
   a.local_end = p->local_end_index;
   a.dst_override = p->dst_start_override;
   a.q_inv_rms = p->q_inv_rms;
+  a.k_inv_rms = p->k_inv_rms;
   a.cache_tokens = p->cache_tokens;
   a.tokens = p->tokens; a.heads = p->heads; a.grid_w = p->grid_w;
   a.frame_tokens = p->grid_h * p->grid_w;
@@ -399,11 +412,13 @@ extern "C" int sdv2_kv_append_rope(const sdv2_append_params* p) {
     sdv2::launch_timed(SDV2_KERNEL_APPEND, kernel, grid, block, 0, stream, a);
   };
   if (p->dtype == SDV2_BF16) {
-    if (!with_kv) launch(kv_append_rope_kernel<uint16_t, true, false>);
+    if (norm_k) launch(kv_append_rope_kernel<uint16_t, false, true, true>);
+    else if (!with_kv) launch(kv_append_rope_kernel<uint16_t, true, false>);
     else if (with_q) launch(kv_append_rope_kernel<uint16_t, true, true>);
     else launch(kv_append_rope_kernel<uint16_t, false, true>);
   } else {
-    if (!with_kv) launch(kv_append_rope_kernel<float, true, false>);
+    if (norm_k) launch(kv_append_rope_kernel<float, false, true, true>);
+    else if (!with_kv) launch(kv_append_rope_kernel<float, true, false>);
     else if (with_q) launch(kv_append_rope_kernel<float, true, true>);
     else launch(kv_append_rope_kernel<float, false, true>);
   }

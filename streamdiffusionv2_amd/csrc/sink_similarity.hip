@@ -63,13 +63,19 @@ struct SinkSimKernelArgs {
   const void* k_norm_w;                     // RMSNorm weight of k over heads * 128, or null
   float* inv_rms;                           // [rows][tokens]: 1 / rms of every new key token (with k_norm_w)
   float norm_eps;
+  // the chunk's query, rotated (and normalised, with q_norm_w) beside the decision, or null
+  const uint16_t* q_in;
+  uint16_t* q_out;
+  sdv2_stride3 q_in_st, q_out_st;
+  const uint16_t* q_norm_w;                 // RMSNorm weight of q over heads * 128, or null
+  int32_t q_workgroups;
   uint32_t stale[SDV2_MAX_ROWS];            // bit j: sink frame j of the row is summed from the cache in this call
   int32_t planned_frame[SDV2_MAX_ROWS];     // sink frame the host's plan writes this call's chunk to, or -1
   float* similarity;                        // [rows][sink]
   int32_t* refresh;                         // [rows]
   int64_t* dst_override;                    // [rows] or null: slot start for the append that follows
   uint32_t override_rows;                   // bit i: row i is about to evict, so a refresh moves its write
-  int32_t tokens, heads, grid_w, sink_frames;
+  int32_t rows, tokens, heads, grid_w, sink_frames;
   int32_t first_matrix;                     // matrices below this one are not summed in this call: the grid leaves them out
   int32_t split_t, split_h, pairs;
   float threshold;
@@ -356,7 +362,78 @@ __device__ __forceinline__ void decide(const SinkSimKernelArgs& a, int row) {
   }
 }
 
-// grid (heads, matrices summed in this call, rows * kTokenSplits): one workgroup sums one head's
+// The query's part of a layer call, by the workgroups of the grid that sum nothing: a wave takes two tokens at a time (one of
+// more than sixteen heads), with the append's arithmetic (same order of additions, same roundings).  The decision is a chain of trips to memory
+// for which all but one workgroup per row have ended, so this work is next to free there: 2 x 1560 tokens x 12 heads
+// 20.7 -> 21.8 us, against 8 and more that it takes in the append that waits for the decision.
+constexpr int query_tokens(int steps) { return (steps <= 4 ? 2 : 1) * (kThreads / 64); }       // of a workgroup at a time
+constexpr int kMostQueryWorkgroups = 2048;
+
+template <int kSteps>
+__device__ __forceinline__ void rotate_queries(const SinkSimKernelArgs& a, int workgroup, float (&scratch)[2][64 * 8]) {
+#pragma clang fp contract(off)
+  using Vec = sdv2::Vec8<uint16_t>;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int sub = lane & (kLanesPerRow - 1), head0 = lane >> 4;
+  constexpr int kTokens = query_tokens(kSteps), kEach = kTokens / (kThreads / 64);
+  const int per_row = (a.tokens + kTokens - 1) / kTokens;
+  const bool norm = a.q_norm_w != nullptr;
+  for (int at = workgroup; at < per_row * a.rows; at += a.q_workgroups) {
+    const int row = at / per_row;
+    const int t0 = (at - row * per_row) * kTokens + kEach * wave;
+    if (t0 >= a.tokens) continue;            // (wave-uniform)
+    const int t1 = kEach > 1 && t0 + 1 < a.tokens ? t0 + 1 : t0;
+    Vec q[kEach][kSteps];
+    const uint16_t* qi = a.q_in + row * a.q_in_st.row + sub * 8;
+#pragma unroll
+    for (int j = 0; j < kSteps; ++j) {
+      const int h = 4 * j + head0, hh = h < a.heads ? h : a.heads - 1;
+      if (4 * j < a.heads) {                 // (uniform; lanes whose head does not exist ask for the last one's)
+        q[0][j] = Vec::load(qi + t0 * a.q_in_st.token + hh * a.q_in_st.head);
+        if constexpr (kEach > 1) q[1][j] = Vec::load(qi + t1 * a.q_in_st.token + hh * a.q_in_st.head);
+      } else {
+        q[0][j] = q[kEach - 1][j] = Vec::zero();
+      }
+    }
+    float r[2] = {1.f, 1.f};
+    if (norm) {
+      float ssq[2];
+      sdv2::wave_sum_squares<uint16_t, kSteps>(q[0], q[kEach - 1], a.heads, scratch, lane, ssq[0], ssq[1]);
+      const float width = static_cast<float>(a.heads * 128);
+#pragma unroll
+      for (int u = 0; u < 2; ++u) r[u] = 1.0f / sqrtf(ssq[u] / width + a.norm_eps);
+    }
+    // (what else they need, a second trip: it does not fit beside forty heads' slices)
+    __builtin_amdgcn_sched_barrier(0);
+    double2 cs[kEach][4];
+    Vec w[kSteps];
+#pragma unroll
+    for (int u = 0; u < kEach; ++u) {
+      const int t = u ? t1 : t0, hi = t / a.grid_w;
+      sdv2::load_rotation(a.freqs, a.pairs, a.split_t, a.split_h, sub, a.start_frame[row], hi, t - hi * a.grid_w, cs[u]);
+    }
+    if (norm)
+#pragma unroll
+      for (int j = 0; j < kSteps; ++j) {
+        const int h = 4 * j + head0;
+        if (4 * j < a.heads) w[j] = Vec::load(a.q_norm_w + (h < a.heads ? h : a.heads - 1) * 128 + sub * 8);
+      }
+#pragma unroll
+    for (int u = 0; u < kEach; ++u) {
+      if (u == 1 && t1 == t0) break;
+      uint16_t* qo = a.q_out + row * a.q_out_st.row + (u ? t1 : t0) * a.q_out_st.token + sub * 8;
+#pragma unroll
+      for (int j = 0; j < kSteps; ++j) {
+        const int h = 4 * j + head0;
+        if (4 * j >= a.heads) break;
+        const Vec y = sdv2::rotate(norm ? sdv2::normalise(q[u][j], r[u], w[j]) : q[u][j], cs[u]);
+        if (h < a.heads) y.store(qo + h * a.q_out_st.head);
+      }
+    }
+  }
+}
+
+// grid (heads, matrices summed in this call, rows * kTokenSplits, and behind those the query's workgroups): one workgroup sums one head's
 // 128 columns of one frame over one eighth of its tokens, of the new K and V both.  (With every sink
 // frame's mean kept, those are all: first_matrix.)  (One workgroup per
 // frame and head would leave most of the chip idle: 96 workgroups for three
@@ -379,6 +456,16 @@ void sink_similarity_kernel(const SinkSimKernelArgs a) {
   const int head = blockIdx.x;
   const int m = blockIdx.y + a.first_matrix;
   const int row = blockIdx.z / kTokenSplits;
+  if constexpr (std::is_same<T, uint16_t>::value) {
+    if (row >= a.rows) {
+      const int workgroup = (blockIdx.z - a.rows * kTokenSplits) * a.heads + head;
+      static_assert(sizeof(part) == kThreads / 64 * sizeof(float[2][64 * 8]), "the waves' scratch");
+      // (kCols columns a thread are 512 kCols columns, 4 kCols heads)
+      if (blockIdx.y == 0 && workgroup < a.q_workgroups)
+        rotate_queries<kCols>(a, workgroup, reinterpret_cast<float(*)[2][64 * 8]>(&part[0][0][0])[threadIdx.x >> 6]);
+      return;
+    }
+  }
   const int split = blockIdx.z - row * kTokenSplits;
   const int sink = a.sink_frames;
 
@@ -563,6 +650,14 @@ extern "C" int sdv2_sink_similarity(const sdv2_sink_sim_params* p) {
   if (!p->workspace || p->workspace_bytes < need || (reinterpret_cast<uintptr_t>(p->workspace) & 15))
     return SDV2_ERR_WORKSPACE;
   if (p->k_norm_weight && (!aligned16(p->k_norm_weight) || !(p->norm_eps >= 0.f))) return SDV2_ERR_INVALID_ARG;
+  if (p->k_inv_rms && (!p->k_norm_weight || (reinterpret_cast<uintptr_t>(p->k_inv_rms) & 3))) return SDV2_ERR_INVALID_ARG;
+  if ((p->q_in != nullptr) != (p->q_out != nullptr)) return SDV2_ERR_INVALID_ARG;
+  if (p->q_norm_weight && (!p->q_in || !p->k_norm_weight)) return SDV2_ERR_INVALID_ARG;
+  if (p->q_in) {
+    if (p->dtype != SDV2_BF16) return SDV2_ERR_UNSUPPORTED;
+    if (!aligned16(p->q_in) || !aligned16(p->q_out) || !aligned16(p->q_norm_weight)) return SDV2_ERR_INVALID_ARG;
+    if (!stride_ok(p->q_in_stride, vec) || !stride_ok(p->q_out_stride, vec)) return SDV2_ERR_INVALID_ARG;
+  }
   if (p->frame_sums) {
     if (reinterpret_cast<uintptr_t>(p->frame_sums) & 15) return SDV2_ERR_INVALID_ARG;
     if (!p->stale_frames || !p->planned_frame) return SDV2_ERR_INVALID_ARG;
@@ -578,6 +673,16 @@ extern "C" int sdv2_sink_similarity(const sdv2_sink_sim_params* p) {
   a.sums = reinterpret_cast<float*>(static_cast<char*>(p->workspace) + kTicketBytes);
   a.inv_rms = reinterpret_cast<float*>(static_cast<char*>(p->workspace) + kTicketBytes +
                                        sums_bytes(p->rows, p->heads, p->sink_frames));
+  if (p->k_inv_rms) a.inv_rms = p->k_inv_rms;
+  a.q_in = static_cast<const uint16_t*>(p->q_in);
+  a.q_out = static_cast<uint16_t*>(p->q_out);
+  a.q_in_st = p->q_in_stride; a.q_out_st = p->q_out_stride;
+  a.q_norm_w = static_cast<const uint16_t*>(p->q_norm_weight);
+  if (p->q_in) {
+    const int each = query_tokens(p->heads <= 16 ? 4 : 16);
+    const int64_t all = (int64_t)p->rows * ((p->tokens + each - 1) / each);
+    a.q_workgroups = all < kMostQueryWorkgroups ? (int32_t)all : kMostQueryWorkgroups;
+  }
   a.kept = p->frame_sums;
   a.k_norm_w = p->k_norm_weight;
   a.norm_eps = p->norm_eps;
@@ -585,7 +690,7 @@ extern "C" int sdv2_sink_similarity(const sdv2_sink_sim_params* p) {
   a.refresh = p->refresh;
   a.dst_override = p->dst_start_override;
   a.override_rows = p->override_rows;
-  a.tokens = p->tokens; a.heads = p->heads; a.grid_w = p->grid_w; a.sink_frames = p->sink_frames;
+  a.rows = p->rows; a.tokens = p->tokens; a.heads = p->heads; a.grid_w = p->grid_w; a.sink_frames = p->sink_frames;
   a.pairs = p->head_dim / 2;
   const int third = a.pairs / 3;
   a.split_t = a.pairs - 2 * third;
@@ -604,7 +709,7 @@ extern "C" int sdv2_sink_similarity(const sdv2_sink_sim_params* p) {
   bool any_stale = false;
   for (int i = 0; i < p->rows; ++i) any_stale |= (a.stale[i] & ((1u << p->sink_frames) - 1u)) != 0;
   a.first_matrix = any_stale ? 0 : 2 * p->sink_frames;
-  const dim3 grid(p->heads, 2 * p->sink_frames + 1 - a.first_matrix, p->rows * kTokenSplits);
+  const dim3 grid(p->heads, 2 * p->sink_frames + 1 - a.first_matrix, p->rows * kTokenSplits + (a.q_workgroups + p->heads - 1) / p->heads);
   if (p->k_norm_weight) {
     const dim3 grid_rms((p->tokens + 3) / 4, 1, p->rows);
     const int steps = (p->heads + 3) / 4;

@@ -546,6 +546,36 @@ def swa_attention(
 
 
 _SIM_WORKSPACES: dict = {}
+_SIM_LAYOUTS: dict = {}
+
+
+def _sim_layout(lib, k, v, k_cache, v_cache, freq_rows: int, grid_hw, sink_frames: int, q, q_out):
+    """What a sink decision of these shapes and strides passes down whatever the pointers: the descriptor with all
+    else filled in, and the bytes of its workspace and of the kept means.  (Filled anew it was 15 us of the call.)"""
+    if not (k.dtype == v.dtype == k_cache.dtype == v_cache.dtype):
+        raise RuntimeError("k, v and the caches must share one dtype")
+    rows, tokens, heads, _ = k.shape
+    if tuple(v.shape) != tuple(k.shape):
+        raise RuntimeError("k and v must have one shape")
+    if k_cache.shape[0] < rows or v_cache.shape != k_cache.shape or k_cache.shape[2] != heads:
+        raise RuntimeError(f"cache {tuple(k_cache.shape)} does not match the chunk {tuple(k.shape)}")
+    p = _capi.SinkSimParams()
+    p.k_in_stride, p.v_in_stride = _stride3(k, "k"), _stride3(v, "v")
+    p.k_cache_stride, p.v_cache_stride = _stride3(k_cache, "k_cache"), _stride3(v_cache, "v_cache")
+    p.freq_rows = freq_rows
+    if k.dtype not in _DTYPES:
+        raise RuntimeError(f"unsupported dtype {k.dtype}")
+    p.dtype = _DTYPES[k.dtype]
+    p.rows, p.tokens, p.heads, p.head_dim = rows, tokens, heads, HEAD_DIM
+    p.grid_h, p.grid_w = int(grid_hw[0]), int(grid_hw[1])
+    p.sink_frames = int(sink_frames)
+    p.cache_tokens = k_cache.shape[1]
+    if q is not None:
+        if q.shape != k.shape or q_out.shape != k.shape or not q.dtype == q_out.dtype == k.dtype:
+            raise RuntimeError("query and rotated query must have the key's shape and dtype")
+        p.q_in_stride, p.q_out_stride = _stride3(q, "q"), _stride3(q_out, "rotated q")
+    return p, lib.sdv2_sink_similarity_workspace_bytes(rows, tokens, heads, sink_frames), \
+        lib.sdv2_sink_frame_sums_bytes(rows, heads, sink_frames)
 
 
 def sink_similarity(
@@ -565,6 +595,8 @@ def sink_similarity(
     frame_sums: Optional[torch.Tensor] = None,
     stale_frames: Sequence[int] = (),
     planned_frames: Sequence[int] = (),
+    query: Optional[Tuple[torch.Tensor, torch.Tensor, Optional[torch.Tensor]]] = None,
+    k_inv_rms: Optional[torch.Tensor] = None,
 ):
     """Adaptive sink refresh decision (causal_model.py:284-299) for a
     one-frame chunk, before its append.
@@ -587,21 +619,30 @@ def sink_similarity(
     or never summed), ``planned_frames[i]`` the sink frame the append that
     follows writes to by the host's plan, or -1.
 
+    ``query`` = (q, rotated q, q norm weight or None), bf16: the chunk's query is
+    rotated (and normalised) in the same launch, by workgroups the decision has no
+    use for; with ``k_norm``, ``k_inv_rms`` (float32 [B, S]) receives 1 / rms of
+    every key token.  The append that follows then moves K and V only.
+
     k is the chunk's key BEFORE RoPE, v its value, both [B,S,H,128]; the caches
     are read as they are.  Returns (similarity float32 [B, sink_frames],
     refresh int32 [B]) on the device: refresh[i] is the sink frame of row i to
     overwrite next, or -1.
     """
     dev = _require_gpu(k, v, k_cache, v_cache, freqs_table)
-    if not (k.dtype == v.dtype == k_cache.dtype == v_cache.dtype):
-        raise RuntimeError("k, v and the caches must share one dtype")
-    rows, tokens, heads, _ = k.shape
-    if tuple(v.shape) != tuple(k.shape):
-        raise RuntimeError("k and v must have one shape")
-    if k_cache.shape[0] < rows or v_cache.shape != k_cache.shape or k_cache.shape[2] != heads:
-        raise RuntimeError(f"cache {tuple(k_cache.shape)} does not match the chunk {tuple(k.shape)}")
     lib = _capi.lib()
-    need = lib.sdv2_sink_similarity_workspace_bytes(rows, tokens, heads, sink_frames)
+    q, q_out, q_weight = query if query is not None else (None, None, None)
+    like = (k.shape, v.shape, k_cache.shape, v_cache.shape, k.stride(), v.stride(), k_cache.stride(), v_cache.stride(),
+            k.dtype, v.dtype, k_cache.dtype, v_cache.dtype, tuple(grid_hw), sink_frames, freqs_table.shape[0])
+    if query is not None:
+        like += (q.shape, q_out.shape, q.stride(), q_out.stride(), q.dtype, q_out.dtype)
+    layout = _SIM_LAYOUTS.get(like)
+    if layout is None:
+        if len(_SIM_LAYOUTS) >= _MAX_ATTN_LAYOUTS:
+            _SIM_LAYOUTS.clear()
+        layout = _SIM_LAYOUTS[like] = _sim_layout(lib, k, v, k_cache, v_cache, freqs_table.shape[0], grid_hw, sink_frames, q, q_out)
+    filled, need, kept_need = layout
+    rows, tokens, heads = filled.rows, filled.tokens, filled.heads
     ws = _workspace(dev, need, _SIM_WORKSPACES)      # (zero-filled: its ticket words start at zero)
     similarity = torch.empty((rows, sink_frames), dtype=torch.float32, device=dev)
     if refresh_out is None:
@@ -612,22 +653,11 @@ def sink_similarity(
         if refresh.dtype != torch.int32 or refresh.numel() < rows or not refresh.is_contiguous() or not on_device:
             raise RuntimeError(f"refresh_out must be a contiguous int32 tensor with one entry per row, on {dev} or pinned")
 
-    p = _capi.SinkSimParams()
-    p.k_in, p.k_in_stride = k.data_ptr(), _stride3(k, "k")
-    p.v_in, p.v_in_stride = v.data_ptr(), _stride3(v, "v")
-    p.k_cache, p.k_cache_stride = k_cache.data_ptr(), _stride3(k_cache, "k_cache")
-    p.v_cache, p.v_cache_stride = v_cache.data_ptr(), _stride3(v_cache, "v_cache")
-    p.freqs, p.freq_rows = freqs_table.data_ptr(), freqs_table.shape[0]
-    if k.dtype not in _DTYPES:
-        raise RuntimeError(f"unsupported dtype {k.dtype}")
-    p.dtype = _DTYPES[k.dtype]
-    p.rows, p.tokens, p.heads, p.head_dim = rows, tokens, heads, HEAD_DIM
-    p.grid_h, p.grid_w = int(grid_hw[0]), int(grid_hw[1])
-    p.sink_frames = int(sink_frames)
+    p = _capi.SinkSimParams.from_buffer_copy(filled)
+    p.k_in, p.v_in, p.k_cache, p.v_cache = k.data_ptr(), v.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr()
+    p.freqs = freqs_table.data_ptr()
     p.threshold = float(threshold)
-    p.cache_tokens = k_cache.shape[1]
-    starts = _i64_array(start_frames)
-    p.start_frame = C.cast(starts, C.POINTER(C.c_int64))
+    p.start_frame = _i64_array(start_frames)
     p.similarity, p.refresh = similarity.data_ptr(), refresh.data_ptr()
     p.workspace, p.workspace_bytes = ws.data_ptr(), ws.numel()
     p.stream = _stream_ptr(dev)
@@ -644,17 +674,28 @@ def sink_similarity(
             raise RuntimeError(f"the k norm weight must be a contiguous {k.dtype} tensor of {heads * HEAD_DIM} elements on {dev}")
         p.k_norm_weight, p.norm_eps = weight.data_ptr(), float(eps)
     if frame_sums is not None:
-        want = lib.sdv2_sink_frame_sums_bytes(rows, heads, sink_frames)
         if frame_sums.device != dev or not frame_sums.is_contiguous() \
-                or frame_sums.numel() * frame_sums.element_size() < want:
-            raise RuntimeError(f"frame_sums must be a contiguous buffer of at least {want} bytes on {dev}")
+                or frame_sums.numel() * frame_sums.element_size() < kept_need:
+            raise RuntimeError(f"frame_sums must be a contiguous buffer of at least {kept_need} bytes on {dev}")
         if len(stale_frames) != rows or len(planned_frames) != rows:
             raise RuntimeError("frame_sums needs stale_frames and planned_frames with one entry per row")
-        stale = (C.c_uint32 * rows)(*[int(x) & 0xffffffff for x in stale_frames])
-        planned = (C.c_int32 * rows)(*[int(x) for x in planned_frames])
         p.frame_sums = frame_sums.data_ptr()
-        p.stale_frames = C.cast(stale, C.POINTER(C.c_uint32))
-        p.planned_frame = C.cast(planned, C.POINTER(C.c_int32))
+        p.stale_frames = (C.c_uint32 * rows)(*[int(x) & 0xffffffff for x in stale_frames])
+        p.planned_frame = (C.c_int32 * rows)(*[int(x) for x in planned_frames])
+    if query is not None:
+        if q.device != dev or q_out.device != dev:
+            raise RuntimeError(f"query and rotated query must lie on {dev}")
+        if (q_weight is None) != (k_norm is None):
+            raise RuntimeError("the q and k norms are folded in together")
+        p.q_in, p.q_out = q.data_ptr(), q_out.data_ptr()
+        if q_weight is not None:
+            _check_norm((q_weight, *k_norm), q.dtype, heads, dev)
+            p.q_norm_weight = q_weight.data_ptr()
+    if k_inv_rms is not None:
+        if k_inv_rms.dtype != torch.float32 or k_inv_rms.numel() < rows * tokens or not k_inv_rms.is_contiguous() \
+                or k_inv_rms.device != dev:
+            raise RuntimeError(f"k_inv_rms must be a contiguous float32 tensor with one entry per token on {dev}")
+        p.k_inv_rms = k_inv_rms.data_ptr()
     with _on_device(dev):
         _capi.check(lib.sdv2_sink_similarity(C.byref(p)), "sdv2_sink_similarity")
     return similarity, refresh
@@ -749,6 +790,9 @@ class LayerLauncher:
         # may append on the same stream between this call's two launches, and a graph that captured
         # them keeps the memory in its pool.  (None when the attention rotates.)
         self.roped_q = None
+        # Set for the next call by one whose sink decision has made them: the rotated query, and 1 / rms of the key
+        # tokens with the norm folded in (which that caller holds).
+        self.rotated = None
         self.q_inv_rms = torch.empty((rows, tokens), dtype=torch.float32, device=dev) \
             if self.rope_in_attention and qk_norm is not None else None
         self.sf = (C.c_int64 * rows)()
@@ -844,10 +888,17 @@ class LayerLauncher:
             at.q = q.data_ptr()
             if self.q_inv_rms is not None:
                 ap.q_in = q.data_ptr()
+        elif self.rotated is not None:
+            (self.roped_q, inv_rms), self.rotated = self.rotated, None
+            at.q = self.roped_q.data_ptr()
+            ap.q_in = ap.q_out = ap.q_norm_weight = None
+            ap.k_inv_rms = inv_rms.data_ptr() if inv_rms is not None else None
         else:
             self.roped_q = torch.empty(self.in_shape, dtype=torch.bfloat16, device=self.dev)
             ap.q_in = q.data_ptr()
             ap.q_out = at.q = self.roped_q.data_ptr()
+            if self.norm_args is not None:
+                ap.q_norm_weight, ap.k_inv_rms = self.norm_args[0], None
         ap.stream = at.stream = stream
         span = plan.max_seq_len
         mask_plan = (mask_block_tokens, _starts_alike(plan.dst_start)) if mask_block_tokens else None

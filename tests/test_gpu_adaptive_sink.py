@@ -589,3 +589,62 @@ def test_module_with_fused_norm_and_adaptive_sink(gpu_device):
     ik1, ik0 = k1.cpu().view(torch.int16).int(), k0.cpu().view(torch.int16).int()
     assert (ik1 - ik0).abs().max().item() <= 1
     assert (y1.float() - y0.float()).abs().max().item() <= 3e-2
+
+
+@pytest.mark.parametrize("rows,grid,H,norm,strided", [
+    (1, (1, 1), 1, True, False),              # one token, one head: half of a wave's pair, three quarters of its lanes idle
+    (2, (3, 5), 12, True, True),              # an odd number of tokens: the last pair is one
+    (1, (16, 1), 16, True, False),            # a whole workgroup of pairs; the most heads of two tokens a wave
+    (3, (1, 17), 17, True, True),             # one token a wave; one head in the last step of four
+    (2, (9, 16), 40, True, False),
+    (1, (5, 7), 64, True, False),
+    (2, (3, 5), 12, False, True),             # no norm
+    (1, (30, 52), 40, False, False),
+    (16, (37, 61), 1, False, False),          # more groups of tokens than workgroups
+])
+def test_query_beside_the_decision(gpu_device, rows, grid, H, norm, strided):
+    """The query rotated by the decision's launch, and K, V appended with the 1 / rms values it leaves, have the bits of
+    the append that does it all; the decision is that of a call without them."""
+    from streamdiffusionv2_amd import ops, rope
+
+    S, sink = grid[0] * grid[1], 2
+    print(f"query beside the decision: {rows} x {S} x {H}, norm {norm}, strided {strided}", flush=True)
+    gen = torch.Generator(device=gpu_device).manual_seed(S + H)
+    wide = torch.randn(rows, S, 3 * H * 128, generator=gen, device=gpu_device).bfloat16()
+    parts = [wide[..., i * H * 128:(i + 1) * H * 128] for i in range(3)]
+    q, k, v = ((t if strided else t.contiguous()).view(rows, S, H, 128) for t in parts)
+    caches = [torch.randn(rows, 4 * S, H, 128, generator=gen, device=gpu_device).bfloat16() for _ in range(2)]
+    wq, wk = ((1 + 0.1 * torch.randn(H * 128, generator=gen, device=gpu_device)).bfloat16() for _ in range(2))
+    table = ops.device_freqs(rope.build_freqs(), gpu_device)
+    starts, dst = list(range(rows)), [S] * rows
+    args = (k, v, *caches, table, grid, starts, sink, 0.5)
+    k_norm = (wk, 1e-6) if norm else None
+    want_sim, want_refresh = ops.sink_similarity(*args, k_norm=k_norm)
+    roped = torch.full((rows, S, H, 128), 7.0, device=gpu_device).bfloat16()
+    inv = torch.empty(rows, S, device=gpu_device) if norm else None
+    sim, refresh = ops.sink_similarity(*args, k_norm=k_norm, query=(q, roped, wq if norm else None), k_inv_rms=inv)
+    assert torch.equal(sim, want_sim) and torch.equal(refresh, want_refresh)
+
+    want = [c.clone() for c in caches]
+    want_q = ops.kv_append_rope(q, k, v, *want, table, (1, *grid), starts, dst, qk_norm=(wq, wk, 1e-6) if norm else None)
+    assert torch.equal(roped.view(torch.int16), want_q.view(torch.int16))
+
+    import ctypes as C
+    from streamdiffusionv2_amd import _capi
+
+    p = _capi.AppendParams()
+    p.k_in, p.k_in_stride, p.v_in, p.v_in_stride = k.data_ptr(), ops._stride3(k, "k"), v.data_ptr(), ops._stride3(v, "v")
+    p.k_cache, p.k_cache_stride = caches[0].data_ptr(), ops._stride3(caches[0], "k")
+    p.v_cache, p.v_cache_stride = caches[1].data_ptr(), ops._stride3(caches[1], "v")
+    p.freqs, p.freq_rows, p.dtype = table.data_ptr(), table.shape[0], _capi.DTYPE_BF16
+    p.rows, p.tokens, p.heads, p.head_dim = rows, S, H, 128
+    p.grid_f, p.grid_h, p.grid_w, p.cache_tokens = 1, *grid, 4 * S
+    host = [(C.c_int64 * rows)(*x) for x in (starts, dst)]
+    p.start_frame, p.dst_start = (C.cast(x, C.POINTER(C.c_int64)) for x in host)
+    p.stream = torch.cuda.current_stream().cuda_stream
+    if norm:
+        p.k_norm_weight, p.norm_eps, p.k_inv_rms = wk.data_ptr(), 1e-6, inv.data_ptr()
+    _capi.check(_capi.lib().sdv2_kv_append_rope(C.byref(p)), "sdv2_kv_append_rope")
+    torch.cuda.synchronize()
+    for got, expected in zip(caches, want):
+        assert torch.equal(got.view(torch.int16), expected.view(torch.int16))
