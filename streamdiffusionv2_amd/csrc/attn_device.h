@@ -36,6 +36,12 @@ constexpr int kKTile = 64;                  // keys per tile
 constexpr int kTileBytes = kKTile * kD * 2; // 16 KB per matrix
 constexpr int kIssuers = 4;                 // waves that issue the global->LDS transfers
 constexpr int kPieces = 16 / kIssuers;      // global->LDS instructions per issuing wave and matrix tile
+// The first of them, of eight waves.  Where a query tile has rows for four only, the other four move the tiles, so that
+// nothing holds up a wave that has its SIMD to itself: 1 x 2560 x 12 heads against 9360 keys 144.2 -> 131.2 us, 1 x 1560 x
+// 12 against themselves 30.4 -> 27.6, 1 x 640 x 40 against 512 15.0 -> 14.4.  (With rows for five to seven it is the other
+// way round, 64.2 -> 67.8 us for 3120 x 12 against themselves, 83.0 -> 84.9 for 3840 x 12, and two of the spare waves for
+// all transfers, 65.8 and 82.9, no better: waves that share a SIMD and do not run in step share it better.)
+__host__ __device__ constexpr int first_issuer(int q_tile_rows) { return q_tile_rows <= kIssuers * kQBlock ? kIssuers : 0; }
 constexpr int kStageBytes = 16384;          // epilogue staging per wave
 constexpr int kMaxDevices = 64;
 constexpr int kPartBlockHalves = kQBlock * kD;   // one block's partial output: 32 x 128 fp16 = 8 KB

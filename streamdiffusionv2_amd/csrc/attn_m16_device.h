@@ -112,7 +112,7 @@ struct LaneFetch {
 };
 __device__ __forceinline__ void issue_tile(const char* base, uint32_t tok_bytes, uint32_t chunk, uint32_t row_off, int key0,
                                            int seq, uint32_t lds_dst, int wave_u, int lane) {
-  if (wave_u >= kIssuers) return;
+  if ((unsigned)wave_u >= kIssuers) return;
   const char* tile = base + (int64_t)key0 * tok_bytes;      // wave-uniform
   if (key0 + kKTile <= seq) {
 #pragma unroll
@@ -469,13 +469,14 @@ struct NoPeek {
 template <bool kMask, typename KeyOf, typename LookAt = NoPeek>
 __device__ __forceinline__ void stream_range(late_args<AttnKernelArgs>& a, lds_char* lds, int q_first, int q_end, int head, int row, int seq,
                                              KeyOf key0_of, int tile_begin, int tile_end, LaneConst& c,
-                                             f32x4 (&oacc)[8][2], float (&l_sum)[2], LookAt look = LookAt()) {
+                                             f32x4 (&oacc)[8][2], float (&l_sum)[2], int first_of_issuers = 0, LookAt look = LookAt()) {
   lds_int* flags = reinterpret_cast<lds_int*>(lds + kLdsFlags);
   int tid = threadIdx.x;
   asm volatile("" : "+v"(tid));      // (what is derived from it is worked out per range, not held across them)
   const int lane = tid & 63;
   const int wave = tid >> 6;
   const int wave_u = __builtin_amdgcn_readfirstlane(wave);
+  const int issuer = wave_u - first_of_issuers;
   const int n16 = lane & 15, g = lane >> 4;
   const int n = tile_end - tile_begin;       // tiles this workgroup streams
 
@@ -491,10 +492,10 @@ __device__ __forceinline__ void stream_range(late_args<AttnKernelArgs>& a, lds_c
   f.v_row = g * v_tok_bytes;
   // T is the tile index inside this workgroup's range
   auto issue_k = [&](int T, int buf) {
-    issue_tile(kbase, k_tok_bytes, f.chunk, f.k_row, key0_of(tile_begin + T), seq, lds_addr0 + kLdsBuf(buf), wave_u, lane);
+    issue_tile(kbase, k_tok_bytes, f.chunk, f.k_row, key0_of(tile_begin + T), seq, lds_addr0 + kLdsBuf(buf), issuer, lane);
   };
   auto issue_v = [&](int T, int buf) {
-    issue_tile(vbase, v_tok_bytes, f.chunk, f.v_row, key0_of(tile_begin + T), seq, lds_addr0 + kLdsVBase + kLdsBuf(buf), wave_u, lane);
+    issue_tile(vbase, v_tok_bytes, f.chunk, f.v_row, key0_of(tile_begin + T), seq, lds_addr0 + kLdsVBase + kLdsBuf(buf), issuer, lane);
   };
 
   // ---- this lane's two query rows, and the first tiles ------------------------
@@ -644,7 +645,7 @@ __device__ __forceinline__ void stream_range(late_args<AttnKernelArgs>& a, lds_c
   int seen = 0;
   if (n > 0) {
     // K tiles 0 and 1 and V tile 0 have landed once at most the four tiles requested behind them are in flight
-    if (wave_u < kIssuers) {
+    if ((unsigned)issuer < kIssuers) {
       __builtin_amdgcn_s_waitcnt(0x4070);   // vmcnt(16) = 4 * kPieces, and lgkmcnt(0) for the LDS clear
       static_assert(4 * kPieces == 16, "the wait above");
     } else {

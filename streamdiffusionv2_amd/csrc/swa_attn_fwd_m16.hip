@@ -67,7 +67,8 @@ void swa_attn_fwd_m16_kernel(const AttnKernelArgs args) {
   f32x4 oacc[8][2];
   float l_tot[2];
   auto key0_of = [=](int tile) { return (kMask && tile >= list.hole ? tile + list.skipped : tile) * kKTile; };
-  stream_range<kMask>(a, lds, q_first, q_end, head, row, seq, key0_of, tile_begin, tile_end, c, oacc, l_tot);
+  stream_range<kMask>(a, lds, q_first, q_end, head, row, seq, key0_of, tile_begin, tile_end, c, oacc, l_tot,
+                      first_issuer(a.q_tile_rows));
   late_args<AttnKernelArgs>& b = read_late<AttnKernelArgs>();
   const int q0 = qtile * b.q_tile_rows + wave * kQBlock;           // of this wave
   const bool idle = __builtin_amdgcn_readfirstlane(q0 >= tile_end_row(b, qtile, b.q_tile_rows));

@@ -548,6 +548,19 @@ def test_masked_calls_with_host_starts_on_two_streams(gpu_device):
         assert torch.equal(eager.view(torch.int16), want[200].view(torch.int16))
 
 
+@pytest.mark.parametrize("S,L", [(2600, 900), (2600, 300), (3120, 900)])       # four blocks, 16x16x32 and 32x32x16; five
+def test_rows_redone_in_query_tiles_of_fewer_rows(gpu_device, S, L):
+    """A later key far above the exponent reference: the tiles are streamed a second time, by the waves that always do."""
+    from streamdiffusionv2_amd import ops
+
+    print(f"redone rows of fewer a tile: {S} x 12 against {L}", flush=True)
+    torch.manual_seed(22)
+    q, k, v = (torch.randn(1, n, 12, 128).bfloat16() for n in (S, L, L))
+    k[:, L - 100:L - 98] *= 100
+    got = ops.swa_attention(*(t.to(gpu_device) for t in (q, k, v)), None, num_splits=1)
+    _check(got.cpu(), oracle.attention_fp32_reference(q, k, v, [L]))
+
+
 @pytest.mark.parametrize("rows,S,H,L,seq,block,splits", [
     (1, 2688, 12, 200, None, 0, 1),             # four blocks of 32 rows a tile, 252 of them; 32x32x16
     (1, 2689, 12, 833, None, 0, 1),             # five: one row past what four reach; 16x16x32
