@@ -240,3 +240,13 @@ def test_equal_shares_in_a_graph(gpu_device):
         torch.cuda.synchronize()
         assert torch.equal(out, ops.swa_attention(q, k, v, num_splits=EVEN))
         assert torch.equal(other, ops.swa_attention(q2, k2, v2, num_splits=EVEN))
+
+
+def test_calls_left_whole():
+    """Two ranges become one where tiles of four blocks make one round; what is not cut in two stays as it is."""
+    lib = _capi.lib()
+    for shape, plan in (((2, 1083, 12, 2166), 1), ((1, 672, 40, 2016), 1), ((3, 754, 12, 2262), 1), ((1, 1024, 24, 2048), 2),
+                        ((1, 1560, 12, 9360), 3), ((1, 756, 12, 4536), 4), ((1, 1560, 40, 9360), EVEN), ((1, 256, 12, 1536), 1)):
+        assert lib.sdv2_swa_attn_plan(*shape) == plan, (shape, lib.sdv2_swa_attn_plan(*shape))
+        if plan == 1:
+            assert lib.sdv2_swa_attn_default_splits(*shape) == 1 and lib.sdv2_swa_attn_workspace_bytes(*shape, 0) == 0
