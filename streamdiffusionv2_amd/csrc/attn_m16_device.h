@@ -743,7 +743,7 @@ __device__ __forceinline__ void stream_range(late_args<AttnKernelArgs>& a, lds_c
     const int redo = flags[0];
     if (redo)
       exact_pass<kMask>(c, qf, oacc, l_sum, unsafe, kbase, vbase, k_tok_bytes, v_tok_bytes, f, tile_begin, n,
-                 seq, key0_of, lds_addr0, wave_u, lane);
+                 seq, key0_of, lds_addr0, issuer, lane);
   }
 }
 
