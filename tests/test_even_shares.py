@@ -246,6 +246,8 @@ def test_calls_left_whole():
     """Two ranges become one where tiles of four blocks make one round; what is not cut in two stays as it is."""
     lib = _capi.lib()
     for shape, plan in (((2, 1083, 12, 2166), 1), ((1, 672, 40, 2016), 1), ((3, 754, 12, 2262), 1), ((1, 1024, 24, 2048), 2),
+                        # (plans of two counts: three ranges, or two, and one more for some pairs)
+                        ((4, 567, 12, 10958), 3 | 3 << 8), ((2, 565, 24, 7152), 3 | 3 << 8), ((3, 343, 24, 3632), 2 | 4 << 8),
                         ((1, 1560, 12, 9360), 3), ((1, 756, 12, 4536), 4), ((1, 1560, 40, 9360), EVEN), ((1, 256, 12, 1536), 1)):
         assert lib.sdv2_swa_attn_plan(*shape) == plan, (shape, lib.sdv2_swa_attn_plan(*shape))
         if plan == 1:
