@@ -591,6 +591,7 @@ def test_module_with_fused_norm_and_adaptive_sink(gpu_device):
     assert (y1.float() - y0.float()).abs().max().item() <= 3e-2
 
 
+@pytest.mark.gpu
 @pytest.mark.parametrize("rows,grid,H,norm,strided", [
     (1, (1, 1), 1, True, False),              # one token, one head: half of a wave's pair, three quarters of its lanes idle
     (2, (3, 5), 12, True, True),              # an odd number of tokens: the last pair is one
