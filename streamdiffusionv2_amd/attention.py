@@ -349,7 +349,8 @@ class RingKVPath:
                     planned = [d // frame_tokens if d < self.sink_size * frame_tokens else -1 for d in plan.dst_start]
                     extra = dict(frame_sums=kept["sums"], stale_frames=list(kept["stale"]), planned_frames=planned)
                     kept["stale"] = [0] * rows        # summed now, and kept current by the decision kernel from here on
-                if q.dtype == torch.bfloat16 and rows <= ops._capi.MAX_ROWS:
+                if q.dtype == torch.bfloat16 and rows <= ops._capi.MAX_ROWS \
+                        and ops.query_beside_decision(rows, q.shape[1], q.shape[2], k_norm is not None):
                     # the query rides along with the decision, and 1 / rms of the keys is handed on: the append
                     # has K and V left to move (tensors of this call's own, as in LayerLauncher.patch)
                     rotated = (torch.empty(q.shape, dtype=q.dtype, device=q.device),

@@ -545,6 +545,17 @@ def swa_attention(
     return out
 
 
+def query_beside_decision(rows: int, tokens: int, heads: int, norm: bool) -> bool:
+    """Should the query be rotated by the sink decision's launch (``sink_similarity(query=...)``) and the append behind it
+    move K and V only?  The workgroups that rotate are next to free while the decision waits on its trips to memory; where
+    its sums fill the chip's bandwidth they hold those up, the more with the norm of more than sixteen heads, whose waves
+    take one token at a time.  Both launches together, beside / in the append, 41 shapes each way: up to 160 000
+    (token, head) pairs 0.83 to 0.97 (2 x 1560 x 12 with the norm 29.7 / 35.8 us, 1 x 3600 x 40 94.9 / 101.7); above,
+    norm of more than 16 heads 0.97 to 1.14 (4 x 1560 x 40 171 / 164, 4 x 3600 x 40 320 / 291); the others 0.87 to 0.99
+    up to 240 000 (4 x 3600 x 12 with the norm 96 / 110) and 0.94 to 1.05 above (8 x 1560 x 20 without 152 / 147)."""
+    return rows * tokens * heads <= (160_000 if norm and heads > 16 else 240_000)
+
+
 _SIM_WORKSPACES: dict = {}
 _SIM_LAYOUTS: dict = {}
 

@@ -591,6 +591,44 @@ def test_module_with_fused_norm_and_adaptive_sink(gpu_device):
     assert (y1.float() - y0.float()).abs().max().item() <= 3e-2
 
 
+def test_which_calls_rotate_the_query_beside_the_decision():
+    """Where the sums of the decision fill the chip's bandwidth the query held them up by 4 to 14 %."""
+    from streamdiffusionv2_amd import ops
+
+    for shape in ((4, 3600, 40, True), (2, 3600, 40, True), (4, 1560, 40, True), (3, 1560, 40, True), (3, 1560, 64, True),
+                  (8, 1560, 20, True), (8, 3600, 16, True), (8, 1560, 20, False), (16, 1560, 12, False)):
+        assert not ops.query_beside_decision(*shape), shape
+    for shape in ((1, 256, 12, True), (2, 1560, 12, True), (4, 3600, 12, True), (2, 1560, 40, True), (1, 3600, 40, True),
+                  (3, 1560, 40, False), (1, 3600, 64, False)):
+        assert ops.query_beside_decision(*shape), shape
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("H,norm", [(12, True), (17, True), (12, False)])
+def test_both_routes_of_the_query_give_the_same_bits(gpu_device, monkeypatch, H, norm):
+    """attend() with the query rotated by the decision's launch and by the append: cache, output, rotated query, decisions."""
+    from streamdiffusionv2_amd import ops, ring, rope
+    from streamdiffusionv2_amd.attention import RingKVPath
+
+    print(f"both routes of the query: {H} heads, norm {norm}", flush=True)
+    grid, S, rows = (5, 7), 35, 2
+    seen = []
+    for beside in (True, False):
+        monkeypatch.setattr(ops, "query_beside_decision", lambda *a: beside)
+        gen = torch.Generator(device=gpu_device).manual_seed(H)
+        w = [(1 + 0.1 * torch.randn(H * 128, generator=gen, device=gpu_device)).bfloat16() for _ in range(2)]
+        cache = ring.new_kv_cache(1, 1, 4 * S, H, total_steps=1, dtype=torch.bfloat16, device=gpu_device)
+        ring.replicate_for_stream_batch(cache, rows)
+        path, got = RingKVPath(sink_size=2, adapt_sink_thr=0.2), []
+        for i in range(7):
+            q, k, v = ((torch.randn(rows, S, H, 128, generator=gen, device=gpu_device) + (1 if i < 5 else -1)).bfloat16() for _ in range(3))
+            got += path.attend(q, k, v, torch.tensor([[1, *grid]] * rows), rope.build_freqs(), cache[0], [min(i, 3) * S] * rows,
+                               return_roped_query=True, qk_norm=(*w, 1e-6) if norm else None)
+            got += [cache[0][n].clone() for n in ("k", "v", "global_end_index", "local_end_index")]
+        seen.append(got)
+    assert all(torch.equal(a, b) for a, b in zip(*seen))
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("rows,grid,H,norm,strided", [
     (1, (1, 1), 1, True, False),              # one token, one head: half of a wave's pair, three quarters of its lanes idle
