@@ -15,6 +15,7 @@ LIB_PATH = Path(__file__).resolve().parent / "_lib" / "libsdv2kv.so"
 ABI_VERSION = 20
 HEAD_DIM = 128
 MAX_ROWS = 16
+SPLITS_EVEN = 1 << 20
 
 SDV2_OK = 0
 SDV2_ERR_INVALID_ARG = -1

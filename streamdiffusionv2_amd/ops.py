@@ -370,11 +370,10 @@ _MAX_ATTN_LAYOUTS = 256
 def _library_plan(lib, rows: int, q_tokens: int, heads: int, max_seq_len: int, even: bool, mask_block_tokens: int,
                   starts_alike: bool) -> int:
     """num_splits as the library picks it; ``even``: equal shares of the key tiles are among what it may pick."""
-    if not even:
+    plan = lib.sdv2_swa_attn_plan_masked(rows, q_tokens, heads, max_seq_len, mask_block_tokens, starts_alike)
+    if plan == _capi.SPLITS_EVEN and not even:
         return lib.sdv2_swa_attn_default_splits(rows, q_tokens, heads, max_seq_len)
-    if not mask_block_tokens:
-        return lib.sdv2_swa_attn_plan(rows, q_tokens, heads, max_seq_len)
-    return lib.sdv2_swa_attn_plan_masked(rows, q_tokens, heads, max_seq_len, mask_block_tokens, starts_alike)
+    return plan
 
 
 def _starts_alike(starts) -> bool:

@@ -252,3 +252,48 @@ def test_calls_left_whole():
         assert lib.sdv2_swa_attn_plan(*shape) == plan, (shape, lib.sdv2_swa_attn_plan(*shape))
         if plan == 1:
             assert lib.sdv2_swa_attn_default_splits(*shape) == 1 and lib.sdv2_swa_attn_workspace_bytes(*shape, 0) == 0
+
+
+def test_masked_calls_left_whole():
+    """With the mask two ranges lose less to one, whichever entry asks: of shapes that stay whole without it, some do not."""
+    lib = _capi.lib()
+    for shape, block, ranges in (((1, 687, 40, 1374), 343, 1), ((4, 447, 12, 1341), 149, 1), ((2, 1278, 12, 2556), 426, 2),
+                                 ((1, 2055, 12, 2950), 1027, 2)):
+        assert lib.sdv2_swa_attn_default_splits(*shape) == 1
+        for alike in (0, 1):
+            assert lib.sdv2_swa_attn_plan_masked(*shape, block, alike) == ranges, shape
+            for even in (False, True):
+                assert ops._library_plan(lib, *shape, even, block, bool(alike)) == ranges, shape
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows,S,H,L,block", [(2, 1278, 12, 2556, 426), (1, 687, 40, 1374, 343)])
+def test_a_masked_shape_has_one_plan(gpu_device, rows, S, H, L, block):
+    """The same ranges, and so the same bits, from every entry that chooses them."""
+    import ctypes as C
+
+    print(f"masked, one plan: {rows} x {S} x {H} against {L}, block {block}", flush=True)
+    torch.manual_seed(31)
+    q, k, v = (torch.randn(rows, n, H, 128).bfloat16().to(gpu_device) for n in (S, L, L))
+    starts, lib = [L - S] * rows, _capi.lib()
+    mask = dict(chunk_key_start=starts, mask_block_tokens=block)
+    ranges = lib.sdv2_swa_attn_plan_masked(rows, S, H, L, block, 1)
+    want = ops.swa_attention(q, k, v, num_splits=ranges, **mask)
+    assert torch.equal(ops.swa_attention(q, k, v, **mask), want)
+    assert torch.equal(ops.swa_attention(q, k, v, static_scratch=True, **mask), want)
+    # the library's own choice behind the C entries, with a workspace and with none
+    p = _capi.AttnParams.from_buffer_copy(ops._attn_layout(q, k, v, None, ranges, False, False, block, True)[0])
+    whole = ops.swa_attention(q, k, v, num_splits=1, **mask)
+    host = (C.c_int64 * rows)(*starts)
+    ws = ops.new_workspace(gpu_device, max(1, lib.sdv2_swa_attn_workspace_bytes(rows, S, H, L, 2)))
+    p.num_splits, p.mask_block_tokens, p.chunk_key_start_host = 0, block, C.cast(host, C.POINTER(C.c_int64))
+    p.q, p.k_cache, p.v_cache = q.data_ptr(), k.data_ptr(), v.data_ptr()
+    p.stream = torch.cuda.current_stream().cuda_stream
+    for entry, workspace, expected in ((lib.sdv2_swa_attn_fwd_static, None, want), (lib.sdv2_swa_attn_fwd, ws, want),
+                                       (lib.sdv2_swa_attn_fwd, None, whole)):
+        out = torch.empty_like(q)
+        p.out, p.workspace, p.workspace_bytes = out.data_ptr(), None if workspace is None else workspace.data_ptr(), \
+            0 if workspace is None else workspace.numel()
+        _capi.check(entry(C.byref(p)), "masked, one plan")
+        torch.cuda.synchronize()
+        assert torch.equal(out, expected)
