@@ -420,8 +420,9 @@ struct EvenArgs {
 constexpr int kEvenPartFloats = 256 * kD;
 constexpr int kEvenPartRows = 256;
 
-// the kernel on 16x16x32 matrix instructions (swa_attn_fwd_m16.hip)
+// the kernel on 16x16x32 matrix instructions (swa_attn_fwd_m16.hip), and for query tiles of at most four blocks
 int launch_m16(const AttnKernelArgs& a, uint32_t workgroups, hipStream_t stream);
+int launch_m16_few(const AttnKernelArgs& a, uint32_t workgroups, hipStream_t stream);
 // the kernel whose waves share the keys of one query block (swa_attn_fwd_wave.hip)
 int launch_wave(const AttnKernelArgs& a, uint32_t workgroups, hipStream_t stream);
 

@@ -111,21 +111,21 @@ struct LaneFetch {
   uint32_t k_row, v_row;  // bytes from the wave's first row to this lane's of a piece: (l / 16) * token stride
 };
 __device__ __forceinline__ void issue_tile(const char* base, uint32_t tok_bytes, uint32_t chunk, uint32_t row_off, int key0,
-                                           int seq, uint32_t lds_dst, int wave_u, int lane) {
-  if ((unsigned)wave_u >= kIssuers) return;
+                                           int seq, uint32_t lds_dst, int issuer, int lane) {
+  if ((unsigned)issuer >= kIssuers) return;
   const char* tile = base + (int64_t)key0 * tok_bytes;      // wave-uniform
   if (key0 + kKTile <= seq) {
 #pragma unroll
     for (int j = 0; j < kPieces; ++j)
-      dma16(tile + (uint64_t)((wave_u * kPieces + j) * 4) * tok_bytes, (chunk ^ (uint32_t)(piece_swizzle(j) << 4)) + row_off,
-            lds_dst + (wave_u * kPieces + j) * 1024);
+      dma16(tile + (uint64_t)((issuer * kPieces + j) * 4) * tok_bytes, (chunk ^ (uint32_t)(piece_swizzle(j) << 4)) + row_off,
+            lds_dst + (issuer * kPieces + j) * 1024);
   } else {
     const int last_rel = seq - 1 - key0;
 #pragma unroll
     for (int j = 0; j < kPieces; ++j) {
-      const int r = 4 * (wave_u * kPieces + j) + (lane >> 4);
+      const int r = 4 * (issuer * kPieces + j) + (lane >> 4);
       const int rr = r < last_rel ? r : last_rel;
-      dma16(tile, (uint32_t)rr * tok_bytes + (chunk ^ (uint32_t)(piece_swizzle(j) << 4)), lds_dst + (wave_u * kPieces + j) * 1024);
+      dma16(tile, (uint32_t)rr * tok_bytes + (chunk ^ (uint32_t)(piece_swizzle(j) << 4)), lds_dst + (issuer * kPieces + j) * 1024);
     }
   }
 }
@@ -337,7 +337,7 @@ __device__ __forceinline__ void exact_pass(LaneConst& c, const bf16x8 (&qf)[2][4
                                            bool compute, const char* kbase, const char* vbase,
                                            uint32_t k_tok_bytes, uint32_t v_tok_bytes, const LaneFetch& f, int tile_begin,
                                            int n, int seq,
-                                           KeyOf key0_of, uint32_t lds_addr0, int wave_u, int lane) {
+                                           KeyOf key0_of, uint32_t lds_addr0, int issuer, int lane) {
   float m_run[2] = {-INFINITY, -INFINITY}, l_run[2] = {0.f, 0.f};
   if (compute) {
 #pragma unroll
@@ -348,8 +348,8 @@ __device__ __forceinline__ void exact_pass(LaneConst& c, const bf16x8 (&qf)[2][4
   }
   auto issue = [&](int T) {
     const int key0 = key0_of(tile_begin + T);
-    issue_tile(kbase, k_tok_bytes, f.chunk, f.k_row, key0, seq, lds_addr0 + kLdsBuf(T & 1), wave_u, lane);
-    issue_tile(vbase, v_tok_bytes, f.chunk, f.v_row, key0, seq, lds_addr0 + kLdsVBase + kLdsBuf(T & 1), wave_u, lane);
+    issue_tile(kbase, k_tok_bytes, f.chunk, f.k_row, key0, seq, lds_addr0 + kLdsBuf(T & 1), issuer, lane);
+    issue_tile(vbase, v_tok_bytes, f.chunk, f.v_row, key0, seq, lds_addr0 + kLdsVBase + kLdsBuf(T & 1), issuer, lane);
   };
   __syncthreads();       // everyone is done with the buffers of the fast pass
   issue(0);
@@ -466,17 +466,17 @@ struct NoPeek {
 // key of entry t being key0_of(t): sums of the weighted values
 // (oacc), the queries' row sums (l_sum) and the exponent references both are relative to (c.neg_ref).  Behind it every
 // wave is done with the tile buffers.
-template <bool kMask, typename KeyOf, typename LookAt = NoPeek>
+template <bool kMask, int kFirstIssuer = 0, typename KeyOf, typename LookAt = NoPeek>
 __device__ __forceinline__ void stream_range(late_args<AttnKernelArgs>& a, lds_char* lds, int q_first, int q_end, int head, int row, int seq,
                                              KeyOf key0_of, int tile_begin, int tile_end, LaneConst& c,
-                                             f32x4 (&oacc)[8][2], float (&l_sum)[2], int first_of_issuers = 0, LookAt look = LookAt()) {
+                                             f32x4 (&oacc)[8][2], float (&l_sum)[2], LookAt look = LookAt()) {
   lds_int* flags = reinterpret_cast<lds_int*>(lds + kLdsFlags);
   int tid = threadIdx.x;
   asm volatile("" : "+v"(tid));      // (what is derived from it is worked out per range, not held across them)
   const int lane = tid & 63;
   const int wave = tid >> 6;
   const int wave_u = __builtin_amdgcn_readfirstlane(wave);
-  const int issuer = wave_u - first_of_issuers;
+  const int issuer = wave_u - kFirstIssuer;
   const int n16 = lane & 15, g = lane >> 4;
   const int n = tile_end - tile_begin;       // tiles this workgroup streams
 

@@ -180,7 +180,7 @@ void swa_attn_fwd_even_kernel(const EvenArgs args) {
         // (a piece that ends the share finds the others of its item done, more often than not)
         const bool ends = !whole && next_off >= end && tile_end > tile_begin;
         stream_range<kMask>(a.call, lds, item * kQTile, tile_end_row(a.call, item, kQTile), head, row, seq, key0_of, tile_begin, tile_end, c, oacc, l_sum,
-                            0, Peek{ends ? ticket : nullptr, parts - 1, flags});
+                            Peek{ends ? ticket : nullptr, parts - 1, flags});
 
         late_args<EvenArgs>& b = read_late<EvenArgs>();
         int tid = threadIdx.x;
