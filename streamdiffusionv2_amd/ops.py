@@ -577,8 +577,8 @@ def _sim_layout(lib, k, v, k_cache, v_cache, freq_rows: int, grid_hw, sink_frame
         raise RuntimeError(f"unsupported dtype {k.dtype}")
     p.dtype = _DTYPES[k.dtype]
     p.rows, p.tokens, p.heads, p.head_dim = rows, tokens, heads, HEAD_DIM
-    p.grid_h, p.grid_w = int(grid_hw[0]), int(grid_hw[1])
-    p.sink_frames = int(sink_frames)
+    p.grid_h, p.grid_w = grid_hw
+    p.sink_frames = sink_frames
     p.cache_tokens = k_cache.shape[1]
     if q is not None:
         if q.shape != k.shape or q_out.shape != k.shape or not q.dtype == q_out.dtype == k.dtype:
@@ -642,8 +642,9 @@ def sink_similarity(
     dev = _require_gpu(k, v, k_cache, v_cache, freqs_table)
     lib = _capi.lib()
     q, q_out, q_weight = query if query is not None else (None, None, None)
+    grid_hw, sink_frames = (int(grid_hw[0]), int(grid_hw[1])), int(sink_frames)      # (a key of values, whatever they came in)
     like = (k.shape, v.shape, k_cache.shape, v_cache.shape, k.stride(), v.stride(), k_cache.stride(), v_cache.stride(),
-            k.dtype, v.dtype, k_cache.dtype, v_cache.dtype, tuple(grid_hw), sink_frames, freqs_table.shape[0])
+            k.dtype, v.dtype, k_cache.dtype, v_cache.dtype, grid_hw, sink_frames, freqs_table.shape[0])
     if query is not None:
         like += (q.shape, q_out.shape, q.stride(), q_out.stride(), q.dtype, q_out.dtype)
     layout = _SIM_LAYOUTS.get(like)

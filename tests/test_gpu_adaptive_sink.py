@@ -591,6 +591,30 @@ def test_module_with_fused_norm_and_adaptive_sink(gpu_device):
     assert (y1.float() - y0.float()).abs().max().item() <= 3e-2
 
 
+@pytest.mark.gpu
+def test_the_kept_descriptor_goes_by_the_grids_values(gpu_device):
+    """A grid of tensors that the caller writes to between calls, or of 0-d arrays, is read at every call."""
+    import numpy as np
+    from streamdiffusionv2_amd import ops, rope
+
+    gen = torch.Generator(device=gpu_device).manual_seed(3)
+    k, v = (torch.randn(1, 15, 2, 128, generator=gen, device=gpu_device).bfloat16() for _ in range(2))
+    caches = [torch.randn(1, 30, 2, 128, generator=gen, device=gpu_device).bfloat16() for _ in range(2)]
+    table = ops.device_freqs(rope.build_freqs(), gpu_device)
+
+    def similarity(grid):
+        return ops.sink_similarity(k, v, *caches, table, grid, [0], 1, 0.5)[0].item()
+
+    wide, tall = similarity((3, 5)), similarity((5, 3))
+    assert wide != tall
+    grid = (torch.tensor(3), torch.tensor(5))
+    assert similarity(grid) == wide
+    grid[0].fill_(5)
+    grid[1].fill_(3)
+    assert similarity(grid) == tall
+    assert similarity((np.array(3), np.array(5))) == wide
+
+
 def test_which_calls_rotate_the_query_beside_the_decision():
     """Where the sums of the decision fill the chip's bandwidth the query held them up by 4 to 14 %."""
     from streamdiffusionv2_amd import ops
