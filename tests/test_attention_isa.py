@@ -141,6 +141,22 @@ def test_register_budget(assembly):
     assert len(counts) == 2 and max(counts) <= 256, counts
 
 
+def test_the_first_tiles_are_asked_for_without_a_detour(assembly):
+    """Up to the first barrier no register goes to scratch memory, and behind the last tiles' transfers only the kernel's own
+    waits stand: one that the compiler puts there, for a register some path reloads, waits for the transfers too (loads
+    return in order)."""
+    for name, body in kernel_bodies(assembly).items():
+        ins = instructions(body)
+        first = next(i for i, (mn, _) in enumerate(ins) if mn == "s_barrier")
+        assert not [i for i, (mn, _) in enumerate(ins[:first]) if mn.startswith("scratch_")], name
+        transfers = [i for i, (mn, _) in enumerate(ins[:first]) if mn.startswith("global_load_lds")]
+        assert len(transfers) == 40                  # five tiles, whole or ragged, of four transfers
+        if "ILb0" not in name:
+            continue                                 # (with the mask the chunk's start may come from memory here)
+        waits = [ins[i][1][0] for i in range(transfers[24], first) if ins[i][0] == "s_waitcnt" and "vmcnt" in ins[i][1][0]]
+        assert sorted(waits) == ["vmcnt(0) lgkmcnt(0)", "vmcnt(8) lgkmcnt(0)"], (name, waits)      # no transfers of its own; eight
+
+
 @pytest.fixture(scope="module")
 def assembly_m16():
     out = os.path.join(ROOT, "build", "isa_check")
