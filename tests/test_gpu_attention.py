@@ -550,7 +550,8 @@ def test_masked_calls_with_host_starts_on_two_streams(gpu_device):
 
 @pytest.mark.parametrize("S,L", [(2600, 900), (2600, 300), (3120, 900)])       # four blocks, 16x16x32 and 32x32x16; five
 def test_rows_redone_in_query_tiles_of_fewer_rows(gpu_device, S, L):
-    """A later key far above the exponent reference: the tiles are streamed a second time, by the waves that always do."""
+    """A later key far above the exponent reference: the tiles are streamed a second time (by the waves that moved them the
+    first time with 16x16x32, by waves 0 to 3 with 32x32x16)."""
     from streamdiffusionv2_amd import ops
 
     print(f"redone rows of fewer a tile: {S} x 12 against {L}", flush=True)
@@ -561,21 +562,29 @@ def test_rows_redone_in_query_tiles_of_fewer_rows(gpu_device, S, L):
     _check(got.cpu(), oracle.attention_fp32_reference(q, k, v, [L]))
 
 
-@pytest.mark.parametrize("rows,S,H,L,seq,block,splits", [
-    (1, 2688, 12, 200, None, 0, 1),             # four blocks of 32 rows a tile, 252 of them; 32x32x16
-    (1, 2689, 12, 833, None, 0, 1),             # five: one row past what four reach; 16x16x32
-    (1, 3361, 12, 130, [65], 0, 1),             # six
-    (2, 300, 12, 2400, [2400, 1], 0, 3),        # four, three key ranges, the last tile 44 rows; 16x16x32
-    (2, 513, 8, 700, [64, 700], 0, 2),          # four, one row in the last tile, a row whose second range is empty; 32x32x16
-    (3, 801, 7, 2500, None, 0, 2),              # five, two ranges
-    (1, 1560, 12, 2304, None, 0, 3),            # seven, as many tiles as of eight
-    (2, 900, 12, 1500, None, 300, 1),           # four, the chunk's blocks end inside a tile
-    (1, 1290, 12, 2600, None, 129, 2),          # four, a block is one row longer than a tile
-    (1, 2700, 12, 2700, None, 900, 1),          # five
+@pytest.mark.parametrize("rows,S,H,L,seq,block,splits,blocks", [
+    (1, 2688, 12, 200, None, 0, 1, 4),          # blocks of 32 rows a tile, 252 tiles; 32x32x16
+    (1, 2689, 12, 833, None, 0, 1, 5),          # one row past what four reach; 16x16x32
+    (1, 3361, 12, 130, [65], 0, 1, 6),
+    (2, 300, 12, 2400, [2400, 1], 0, 3, 4),     # three key ranges, the last tile 44 rows; 16x16x32
+    (2, 513, 8, 700, [64, 700], 0, 2, 4),       # one row in the last tile, a row whose second range is empty; 32x32x16
+    (3, 801, 7, 2500, None, 0, 2, 5),           # two ranges
+    (1, 1560, 12, 2304, None, 0, 3, 7),         # as many tiles as of eight
+    (2, 900, 12, 1500, None, 300, 1, 4),        # the chunk's blocks end inside a tile
+    (1, 1290, 12, 2600, None, 129, 2, 5),
+    (1, 1270, 12, 2600, None, 129, 2, 4),       # two ranges, a block one row longer than a tile
+    (1, 700, 40, 700, None, 100, 1, 4),         # 11 key tiles: 32x32x16
+    (1, 500, 30, 1400, None, 129, 2, 4),        # 11 of each range
+    (1, 2700, 12, 2700, None, 900, 1, 5),
 ])
-def test_query_tiles_of_fewer_rows(gpu_device, rows, S, H, L, seq, block, splits):
+def test_query_tiles_of_fewer_rows(gpu_device, rows, S, H, L, seq, block, splits, blocks):
     from streamdiffusionv2_amd import ops
 
+    def one_round(n):
+        return rows * H * -(-S // (32 * n)) * splits <= 256
+
+    assert one_round(blocks) and not any(one_round(n) for n in range(4, blocks))       # the fewest from four on ...
+    assert blocks < 7 or -(-S // 224) == -(-S // 256)
     print(f"fewer rows a tile: {rows} x {S} x {H} against {L} ({seq}), block {block}, {splits} ranges", flush=True)
     torch.manual_seed(21)
     q, k, v = (torch.randn(rows, n, H, 128).bfloat16() for n in (S, L, L))
