@@ -711,3 +711,40 @@ def test_query_beside_the_decision(gpu_device, rows, grid, H, norm, strided):
     torch.cuda.synchronize()
     for got, expected in zip(caches, want):
         assert torch.equal(got.view(torch.int16), expected.view(torch.int16))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows,grid,H", [(2, (3, 5), 12), (1, (1, 17), 17), (1, (16, 1), 40), (1, (1, 1), 1)])
+def test_keys_appended_with_the_decisions_inverse_rms_in_fp32(gpu_device, rows, grid, H):
+    """The fp32 append that normalises with 1 / rms values of the decision has the bits of the one that takes them itself."""
+    import ctypes as C
+    from streamdiffusionv2_amd import _capi, ops, rope
+
+    S = grid[0] * grid[1]
+    print(f"fp32 append behind the decision: {rows} x {S} x {H}", flush=True)
+    gen = torch.Generator(device=gpu_device).manual_seed(S + H)
+    q, k, v = (torch.randn(rows, S, H, 128, generator=gen, device=gpu_device) for _ in range(3))
+    caches = [torch.randn(rows, 3 * S, H, 128, generator=gen, device=gpu_device) for _ in range(2)]
+    wq, wk = (1 + 0.1 * torch.randn(H * 128, generator=gen, device=gpu_device) for _ in range(2))
+    table = ops.device_freqs(rope.build_freqs(), gpu_device)
+    starts, dst = list(range(rows)), [2 * S] * rows
+    inv = torch.empty(rows, S, device=gpu_device)
+    ops.sink_similarity(k, v, *caches, table, grid, starts, 1, 0.5, k_norm=(wk, 1e-6), k_inv_rms=inv)
+    want = [c.clone() for c in caches]
+    ops.kv_append_rope(q, k, v, *want, table, (1, *grid), starts, dst, qk_norm=(wq, wk, 1e-6))
+
+    p = _capi.AppendParams()
+    p.k_in, p.k_in_stride, p.v_in, p.v_in_stride = k.data_ptr(), ops._stride3(k, "k"), v.data_ptr(), ops._stride3(v, "v")
+    p.k_cache, p.k_cache_stride = caches[0].data_ptr(), ops._stride3(caches[0], "k")
+    p.v_cache, p.v_cache_stride = caches[1].data_ptr(), ops._stride3(caches[1], "v")
+    p.freqs, p.freq_rows, p.dtype = table.data_ptr(), table.shape[0], _capi.DTYPE_F32
+    p.rows, p.tokens, p.heads, p.head_dim = rows, S, H, 128
+    p.grid_f, p.grid_h, p.grid_w, p.cache_tokens = 1, *grid, 3 * S
+    host = [(C.c_int64 * rows)(*x) for x in (starts, dst)]
+    p.start_frame, p.dst_start = (C.cast(x, C.POINTER(C.c_int64)) for x in host)
+    p.k_norm_weight, p.norm_eps, p.k_inv_rms = wk.data_ptr(), 1e-6, inv.data_ptr()
+    p.stream = torch.cuda.current_stream().cuda_stream
+    _capi.check(_capi.lib().sdv2_kv_append_rope(C.byref(p)), "sdv2_kv_append_rope")
+    torch.cuda.synchronize()
+    for got, expected in zip(caches, want):
+        assert torch.equal(got.view(torch.int32), expected.view(torch.int32))
