@@ -379,7 +379,9 @@ typedef struct sdv2_sink_sim_params {
   const int32_t* planned_frame;
   /* Optional, SDV2_BF16: the chunk's query, rotated by workgroups that have
    * nothing to do with the decision, as sdv2_kv_append_rope would (same bits),
-   * so that the append that follows moves K and V only.  q_norm_weight, together
+   * so that the append that follows moves K and V only: faster where the decision
+   * is bound by its trips to memory, not where its sums fill the bandwidth (some
+   * 160 000 tokens x heads and more).  q_norm_weight, together
    * with k_norm_weight: q_in is the raw q projection.                          */
   const void* q_in;            /* [B,S,H,128], or NULL together with q_out      */
   void* q_out;

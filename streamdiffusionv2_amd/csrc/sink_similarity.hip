@@ -365,7 +365,8 @@ __device__ __forceinline__ void decide(const SinkSimKernelArgs& a, int row) {
 // The query's part of a layer call, by the workgroups of the grid that sum nothing: a wave takes two tokens at a time (one of
 // more than sixteen heads), with the append's arithmetic (same order of additions, same roundings).  The decision is a chain of trips to memory
 // for which all but one workgroup per row have ended, so this work is next to free there: 2 x 1560 tokens x 12 heads
-// 20.7 -> 21.8 us, against 8 and more that it takes in the append that waits for the decision.
+// 20.7 -> 21.8 us, against 8 and more that it takes in the append that waits for the decision.  (Where the sums are bound by
+// bandwidth it holds them up: the caller chooses, ops.query_beside_decision.)
 constexpr int query_tokens(int steps) { return (steps <= 4 ? 2 : 1) * (kThreads / 64); }       // of a workgroup at a time
 constexpr int kMostQueryWorkgroups = 2048;
 
@@ -440,7 +441,8 @@ __device__ __forceinline__ void rotate_queries(const SinkSimKernelArgs& a, int w
 // sink frames of twelve heads.)  Then it draws its row's ticket, after its
 // sums have been acknowledged by memory; the workgroup that draws the last one
 // finds every sum of the row in memory, decides, and leaves the ticket at zero
-// for the next call.
+// for the next call.  (With a frame to be summed from the cache there are the query's workgroups once per matrix, all but
+// the first ending at once: that costs nothing one can measure.)
 //
 // What bounds it is the chain of trips to memory: tokens with their table entries, sums acknowledged, ticket, sums of
 // the row, results.  512 threads take a range of 195 tokens in one trip and the row's sums in another (256 threads took
