@@ -195,8 +195,11 @@ typedef struct sdv2_attn_params {
   int32_t rows, q_tokens, heads, head_dim;        /* B, S, H, 128              */
   int32_t max_seq_len;                            /* L = k_cache.shape[1]      */
   int32_t num_splits;          /* key ranges per (row, head); 0 = choose from the
-                                * shape and whether mask_block_tokens hides anything.  Bits 0-7: the count s (<= 64).  Bits 8-15
-                                * (optional, needs rows * heads divisible by 8): of
+                                * shape and whether mask_block_tokens hides anything
+                                * (where only the mask asks for more than one range and
+                                * the workspace does not hold them: one).
+                                * Bits 0-7: the count s (<= 64).  Bits 8-15 (optional,
+                                * needs rows * heads divisible by 8): of
                                 * every eighth of the (row, head) list - one XCD's
                                 * share - that many pairs take s + 1 ranges instead,
                                 * which fills the last round of workgroups better.
