@@ -30,6 +30,7 @@ void swa_attn_fwd_m16_kernel(const AttnKernelArgs args) {
   const int wave = tid >> 6;
   const int n16 = lane & 15, g = lane >> 4;
 
+  sdv2::fetch_arguments<AttnKernelArgs>();
   WorkItem w;
   if (!w.decode(args, blockIdx.x)) return;
   late_args<AttnKernelArgs>& a = read_late<AttnKernelArgs>();

@@ -102,6 +102,7 @@ void swa_attn_fwd_even_kernel(const EvenArgs args) {
 
   // Workgroups are dealt to the XCDs round robin by id; each XCD takes runs of neighbouring items and shares.
   const int per_xcd = gridDim.x >> 3, xcd = blockIdx.x & 7, in_xcd = blockIdx.x >> 3;
+  sdv2::fetch_arguments<EvenArgs>();
   int round = 0;
   int begin = 0, end = 0, off = 0, pair = 0, item = 0;
   for (bool again = false;; again = true) {
