@@ -38,8 +38,8 @@ constexpr int kIssuers = 4;                 // waves that issue the global->LDS 
 constexpr int kPieces = 16 / kIssuers;      // global->LDS instructions per issuing wave and matrix tile
 // The first of them, of eight waves.  Where a query tile has rows for four only, the other four move the tiles, so that
 // nothing holds up a wave that has its SIMD to itself: 1 x 2560 x 12 heads against 9360 keys 144.2 -> 131.2 us, 1 x 1560 x
-// 12 against themselves 30.4 -> 27.6, 1 x 640 x 40 against 512 15.0 -> 14.4.  (With rows for five to seven it is the other
-// way round, 64.2 -> 67.8 us for 3120 x 12 against themselves, 83.0 -> 84.9 for 3840 x 12, and two of the spare waves for
+// 12 against themselves 30.4 -> 27.6, 1 x 640 x 40 against 512 15.0 -> 14.4.  (With a wave each for five to seven it is the
+// other way round, 64.2 -> 67.8 us for 3120 x 12 against themselves, 83.0 -> 84.9 for 3840 x 12, and two of the spare waves for
 // all transfers, 65.8 and 82.9, no better: waves that share a SIMD and do not run in step share it better.)
 __host__ __device__ constexpr int first_issuer(int q_tile_rows) { return q_tile_rows <= kIssuers * kQBlock ? kIssuers : 0; }
 constexpr int kStageBytes = 16384;          // epilogue staging per wave
@@ -423,6 +423,8 @@ constexpr int kEvenPartRows = 256;
 // the kernel on 16x16x32 matrix instructions (swa_attn_fwd_m16.hip), and for query tiles of at most four blocks
 int launch_m16(const AttnKernelArgs& a, uint32_t workgroups, hipStream_t stream);
 int launch_m16_few(const AttnKernelArgs& a, uint32_t workgroups, hipStream_t stream);
+// ... of five or six blocks, the last ones shared by several waves (no mask)
+int launch_m16_shared(const AttnKernelArgs& a, uint32_t workgroups, hipStream_t stream);
 // the kernel whose waves share the keys of one query block (swa_attn_fwd_wave.hip)
 int launch_wave(const AttnKernelArgs& a, uint32_t workgroups, hipStream_t stream);
 

@@ -1,5 +1,6 @@
-// The kernel of swa_attn_fwd_m16.hip (which see), for the two sources that compile it: kFirstIssuer is the first of the
-// waves that move the tiles, 0, or 4 in query tiles with rows for four waves (first_issuer).
+// The kernel of swa_attn_fwd_m16.hip (which see), for the sources that compile it: kFirstIssuer is the first of the
+// waves that move the tiles, 0, or 4 in query tiles with rows for four waves (first_issuer) and in those whose waves 4 to 7
+// share a block (kShare: SharedBlock).
 #ifndef SDV2KV_ATTN_M16_KERNEL_H
 #define SDV2KV_ATTN_M16_KERNEL_H
 
@@ -18,7 +19,7 @@ namespace {
 using namespace sdv2::attn;
 using namespace sdv2::attn::m16;
 
-template <bool kMask, int kFirstIssuer>
+template <bool kMask, int kFirstIssuer, int kShare>
 __global__ __launch_bounds__(kThreads, 1)
 void swa_attn_fwd_m16_kernel(const AttnKernelArgs args) {
   extern __shared__ __attribute__((aligned(1024))) char smem[];
@@ -48,10 +49,10 @@ void swa_attn_fwd_m16_kernel(const AttnKernelArgs args) {
   f32x4 oacc[8][2];
   float l_tot[2];
   auto key0_of = [=](int tile) { return (kMask && tile >= list.hole ? tile + list.skipped : tile) * kKTile; };
-  stream_range<kMask, kFirstIssuer>(a, lds, q_first, q_end, head, row, seq, key0_of, tile_begin, tile_end, c, oacc, l_tot);
+  stream_range<kMask, kFirstIssuer, kShare>(a, lds, q_first, q_end, head, row, seq, key0_of, tile_begin, tile_end, c, oacc, l_tot);
   late_args<AttnKernelArgs>& b = read_late<AttnKernelArgs>();
-  const int q0 = qtile * b.q_tile_rows + wave * kQBlock;           // of this wave
-  const bool idle = __builtin_amdgcn_readfirstlane(q0 >= tile_end_row(b, qtile, b.q_tile_rows));
+  const int q0 = qtile * b.q_tile_rows + wave_block<kShare>(wave) * kQBlock;           // of this wave
+  const bool idle = __builtin_amdgcn_readfirstlane(q0 >= tile_end_row(b, qtile, b.q_tile_rows) || share_part<kShare>(wave) > 0);
 
   // ---- epilogue ---------------------------------------------------------------
   // (every wave is done with the K / V buffers: the barrier above, or the last one of the exact pass)
@@ -198,22 +199,26 @@ void swa_attn_fwd_m16_kernel(const AttnKernelArgs args) {
   write_block(b, stage, q0, head, row, lane);
 }
 
-template <int kFirstIssuer>
-int launch(const AttnKernelArgs& a, uint32_t workgroups, hipStream_t stream) {
-  // the tile buffers exceed the static limit: ask for the dynamic size once per device
+// the tile buffers exceed the static limit: ask for the dynamic size once per device
+template <bool kMask, int kFirstIssuer, int kShare>
+int launch_one(const AttnKernelArgs& a, uint32_t workgroups, hipStream_t stream) {
+  constexpr int kLds = kShare > 0 ? kLdsSharedBytes : kLdsBytes;
+  auto kernel = swa_attn_fwd_m16_kernel<kMask, kFirstIssuer, kShare>;
   static std::atomic<bool> lds_ready[kMaxDevices];
   int device = 0;
   if (hipGetDevice(&device) != hipSuccess || device < 0 || device >= kMaxDevices) return SDV2_ERR_LAUNCH;
   if (!lds_ready[device].load(std::memory_order_acquire)) {
-    for (const void* kernel : {reinterpret_cast<const void*>(swa_attn_fwd_m16_kernel<false, kFirstIssuer>),
-                               reinterpret_cast<const void*>(swa_attn_fwd_m16_kernel<true, kFirstIssuer>)})
-      if (hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, kLdsBytes) != hipSuccess) return SDV2_ERR_LAUNCH;
+    if (hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, kLds) != hipSuccess)
+      return SDV2_ERR_LAUNCH;
     lds_ready[device].store(true, std::memory_order_release);
   }
-  auto go = [&](auto kernel) { sdv2::launch_timed(SDV2_KERNEL_ATTENTION, kernel, dim3(workgroups), dim3(kThreads), kLdsBytes, stream, a); };
-  if (a.mask_block_tokens > 0) go(swa_attn_fwd_m16_kernel<true, kFirstIssuer>);
-  else go(swa_attn_fwd_m16_kernel<false, kFirstIssuer>);
+  sdv2::launch_timed(SDV2_KERNEL_ATTENTION, kernel, dim3(workgroups), dim3(kThreads), kLds, stream, a);
   return hipGetLastError() == hipSuccess ? SDV2_OK : SDV2_ERR_LAUNCH;
+}
+template <int kFirstIssuer>
+int launch(const AttnKernelArgs& a, uint32_t workgroups, hipStream_t stream) {
+  return a.mask_block_tokens > 0 ? launch_one<true, kFirstIssuer, 0>(a, workgroups, stream)
+                                 : launch_one<false, kFirstIssuer, 0>(a, workgroups, stream);
 }
 
 }  // namespace

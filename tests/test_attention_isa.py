@@ -185,13 +185,14 @@ def test_the_same_promises_for_the_16x16_kernel(assembly_m16):
     assert len(counts) == 2 and max(counts) <= 256, counts
 
 
-def test_the_same_promises_in_query_tiles_of_few_rows():
-    """(the same kernel, the tiles moved by the waves that have no rows: compiled apart)"""
+@pytest.mark.parametrize("name", ["swa_attn_fwd_m16_few", "swa_attn_fwd_m16_shared"])
+def test_the_same_promises_in_query_tiles_of_few_rows(name):
+    """(the same kernel, the tiles moved by the waves that have no rows, or the last blocks shared: compiled apart)"""
     out = os.path.join(ROOT, "build", "isa_check")
     os.makedirs(out, exist_ok=True)
-    path = os.path.join(out, "swa_attn_fwd_m16_few.s")
+    path = os.path.join(out, name + ".s")
     cmd = [build_ext.hipcc_path(), *build_ext.HIPCC_FLAGS, f"-I{os.path.join(ROOT, 'include')}", f"-I{build_ext.CSRC}",
-           "-S", "--cuda-device-only", str(build_ext.CSRC / "swa_attn_fwd_m16_few.hip"), "-o", path]
+           "-S", "--cuda-device-only", str(build_ext.CSRC / (name + ".hip")), "-o", path]
     res = subprocess.run(cmd, capture_output=True, text=True)
     assert res.returncode == 0, res.stderr[-2000:]
     test_the_same_promises_for_the_16x16_kernel(open(path).read().split("\n"))

@@ -600,3 +600,35 @@ def test_query_tiles_of_fewer_rows(gpu_device, rows, S, H, L, seq, block, splits
     torch.cuda.synchronize()
     assert torch.equal(*got)
     _check(got[0].cpu(), want)
+
+
+@pytest.mark.parametrize("rows,S,H,L,seq,splits,blocks,redo", [
+    (1, 3041, 12, 512, None, 1, 5, False),          # the fewest key tiles; one row in the last query tile, no fifth block in it
+    (1, 3120, 12, 530, None, 1, 5, False),          # an odd number of tiles, the last one of 18 keys
+    (1, 3200, 12, 577, [1], 1, 5, False),           # one key, in a tile that has no second one
+    (2, 1500, 12, 900, [900, 65], 1, 5, True),      # a key far above the reference, in the fourth wave's part of a tile
+    (3, 801, 7, 2500, [2500, 1664, 100], 2, 5, False),      # two ranges: one with 26 tiles, one empty
+    (1, 3777, 12, 520, None, 1, 6, False),          # five blocks in the last query tile
+    (1, 3649, 12, 577, [33], 1, 6, False),          # one row in it
+    (4, 900, 12, 1100, [1100, 1, 64, 1057], 1, 6, True),
+    (2, 900, 12, 1600, None, 2, 6, False),
+])
+def test_query_tiles_whose_last_blocks_are_shared(gpu_device, rows, S, H, L, seq, splits, blocks, redo):
+    """Waves 4 to 7 take the fifth block, or the fifth and sixth, by key, 16 or 32 keys of every tile each."""
+    from streamdiffusionv2_amd import ops
+
+    tiles = [rows * H * -(-S // (32 * n)) * splits for n in (blocks - 1, blocks)]
+    assert tiles[1] <= 256 < tiles[0] and L >= (512 if splits == 1 else 768 * splits)
+    print(f"shared blocks: {rows} x {S} x {H} against {L} ({seq}), {splits} ranges", flush=True)
+    torch.manual_seed(23)
+    q, k, v = (torch.randn(rows, n, H, 128).bfloat16() for n in (S, L, L))
+    lens = seq or [L] * rows
+    if redo:
+        k[:, 64 * 9 + 60:64 * 9 + 62] *= 100
+    want = oracle.attention_fp32_reference(q, k, v, lens)
+    sl = torch.tensor(lens, dtype=torch.int32, device=gpu_device) if seq else None
+    args = [t.to(gpu_device) for t in (q, k, v)]
+    got = [ops.swa_attention(*args, sl, num_splits=splits) for _ in range(2)]
+    torch.cuda.synchronize()
+    assert torch.equal(*got)
+    _check(got[0].cpu(), want)
