@@ -42,8 +42,9 @@ extern "C" {
  * 18: sdv2_linear_params.row_squares, sdv2_attn_params.q_row_squares and
  *     q_norm_eps, sdv2_swa_attn_folds_norm
  * 19: sdv2_swa_attn_plan_masked
- * 20: sdv2_append_params.k_inv_rms, sdv2_sink_sim_params.q_in and what follows it */
-#define SDV2KV_ABI_VERSION 20
+ * 20: sdv2_append_params.k_inv_rms, sdv2_sink_sim_params.q_in and what follows it
+ * 21: sdv2_linear_one_round */
+#define SDV2KV_ABI_VERSION 21
 #define SDV2_HEAD_DIM 128      /* causal_stream_inference.py:99-100 fixes 128 */
 #define SDV2_MAX_ROWS 16       /* rows (B) per sdv2_kv_append_rope call       */
 #define SDV2_MAX_SINK_FRAMES 16 /* sink frames per sdv2_sink_similarity call  */
@@ -497,7 +498,9 @@ typedef struct sdv2_linear_params {
 } sdv2_linear_params;
 
 int sdv2_linear(const sdv2_linear_params* p);
-/* 1 where the call is one round of the chip and faster than a general library's */
+/* 1 where the call (with row_squares or without) is one round of the chip, and by that faster than a general library's */
+int sdv2_linear_one_round(int64_t m, int32_t n, int32_t k, int32_t row_squares);
+/* the same of k up to 2048 and tiles of up to 160 rows, as versions 17 to 20 answered */
 int sdv2_linear_preferred(int64_t m, int32_t n, int32_t k);
 
 #ifdef __cplusplus

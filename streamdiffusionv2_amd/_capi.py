@@ -12,7 +12,7 @@ from typing import Optional
 
 LIB_PATH = Path(__file__).resolve().parent / "_lib" / "libsdv2kv.so"
 
-ABI_VERSION = 20
+ABI_VERSION = 21
 HEAD_DIM = 128
 MAX_ROWS = 16
 SPLITS_EVEN = 1 << 20
@@ -51,6 +51,7 @@ EXPORTED_SYMBOLS = (
     "sdv2_cache_relayout",
     "sdv2_cache_relayout_pair",
     "sdv2_linear",
+    "sdv2_linear_one_round",
     "sdv2_linear_preferred",
     "sdv2_rms_norm",
     "sdv2_event_create",
@@ -252,6 +253,8 @@ def lib() -> C.CDLL:
     handle.sdv2_cache_relayout_pair.argtypes = [C.POINTER(RelayoutParams)] * 2
     handle.sdv2_linear.restype = C.c_int
     handle.sdv2_linear.argtypes = [C.POINTER(LinearParams)]
+    handle.sdv2_linear_one_round.restype = C.c_int
+    handle.sdv2_linear_one_round.argtypes = [C.c_int64, C.c_int32, C.c_int32, C.c_int32]
     handle.sdv2_linear_preferred.restype = C.c_int
     handle.sdv2_linear_preferred.argtypes = [C.c_int64, C.c_int32, C.c_int32]
     handle.sdv2_rms_norm.restype = C.c_int

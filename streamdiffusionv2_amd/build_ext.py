@@ -19,7 +19,7 @@ LIB_PATH = LIB_DIR / "libsdv2kv.so"
 SOURCES = ["sdv2kv_api.hip", "kv_append_rope.hip", "swa_attn_fwd.hip", "swa_attn_fwd_m16.hip", "swa_attn_fwd_m16_few.hip",
            "swa_attn_fwd_m16_shared.hip", "swa_attn_fwd_even.hip", "swa_attn_fwd_wave.hip",
            "swa_attn_fwd_f32.hip", "sink_similarity.hip",
-           "cache_relayout.hip", "rms_norm.hip", "linear.hip", "mfma_ceiling.hip"]
+           "cache_relayout.hip", "rms_norm.hip", "linear.hip", "linear_wide.hip", "mfma_ceiling.hip"]
 
 # -packed-fp32-ops is switched off: the compiler would otherwise form
 # v_pk_*_f32 from ordinary float code.

@@ -1163,7 +1163,7 @@ _FOLDS_NORM: dict = {}
 def linear_or_none(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor],
                    row_squares: bool = False):
     """``x weight^T + bias`` by the library's kernel where that is the faster one
-    (``sdv2_linear_preferred``: bf16, a chunk's worth of rows), else None: the
+    (``sdv2_linear_one_round``: bf16, a chunk's worth of rows), else None: the
     caller's nn.Linear, for everything the kernel does not take too.  With
     ``row_squares`` the result comes with the sums of squares of every 32 columns
     of its rows, float32 [..., n / 32]."""
@@ -1175,12 +1175,12 @@ def linear_or_none(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.T
     if x.shape[-1] != k:
         return None
     m = x.numel() // k
-    key = (m, n, k)
+    key = (m, n, k, row_squares)
     preferred = _LINEAR_PREFERRED.get(key)
     if preferred is None:
         if len(_LINEAR_PREFERRED) >= _MAX_ATTN_LAYOUTS:
             _LINEAR_PREFERRED.clear()
-        preferred = _LINEAR_PREFERRED[key] = bool(_capi.lib().sdv2_linear_preferred(m, n, k))
+        preferred = _LINEAR_PREFERRED[key] = bool(_capi.lib().sdv2_linear_one_round(m, n, k, row_squares))
     if not preferred:
         return None
     dev = x.device
