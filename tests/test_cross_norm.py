@@ -123,3 +123,12 @@ def test_module_folds_only_what_nobody_watches(gpu_device, monkeypatch):
         assert norms.count(query) == 1 and (mixed.float() - first.float()).abs().max() <= 2e-2 * max(1.0, first.float().abs().max().item())
     module(x, text, None).sum()                                # autograd: the module's own expression
     assert norms.count(query) == 1
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows,S,heads,L,lens", [(1, 200, 40, 100, None), (2, 97, 63, 65, [65, 3]), (1, 161, 64, 77, None),
+                                                 (1, 129, 67, 64, None)])
+def test_folded_norm_of_many_heads(gpu_device, rows, S, heads, L, lens):
+    """Sums of more heads than one trip brings (40), of as many as a wave's part of LDS holds (64), and of more; few rows, so
+    that the last block of a query tile is short."""
+    test_folded_norm_matches_the_oracle(gpu_device, rows, S, heads, L, lens)
