@@ -197,17 +197,6 @@ __device__ __forceinline__ void dma16(const char* uniform_base, uint32_t lane_of
       : "memory");
 }
 
-// the same from an address of each lane's own
-__device__ __forceinline__ void dma16_from(const void* lane_address, uint32_t lds_dst) {
-  asm volatile(
-      "s_mov_b32 m0, %1\n\t"
-      "s_nop 0\n\t"
-      "global_load_lds_dwordx4 %0, off"
-      :
-      : "v"(lane_address), "s"(lds_dst)
-      : "memory");
-}
-
 // ---------------------------------------------------------------------------
 // Partial results travel between workgroups that may sit on different XCDs,
 // each behind its own L2.  Fences would make that safe by writing back and
