@@ -36,7 +36,7 @@ PEAK_HBM_GBS = 8000.0       # MI355X HBM3E
 # kernel sources (hash below); otherwise `traffic` is null and stderr says why.
 TRAFFIC_JSON = os.path.join(ROOT, "profiles", "hbm_traffic.json")
 KERNEL_SOURCES = ("swa_attn_fwd.hip", "swa_attn_fwd_m16.hip", "swa_attn_fwd_m16_few.hip", "swa_attn_fwd_m16_shared.hip",
-                  "swa_attn_fwd_even.hip", "swa_attn_fwd_wave.hip", "attn_device.h", "attn_m16_device.h", "attn_m16_kernel.h", "attn_wave_device.h", "attn_tiles.h", "attn_even_plan.h", "kv_append_rope.hip",
+                  "swa_attn_fwd_even.hip", "swa_attn_fwd_wave.hip", "swa_attn_fwd_wave_half.hip", "attn_device.h", "attn_m16_device.h", "attn_m16_kernel.h", "attn_wave_device.h", "attn_tiles.h", "attn_even_plan.h", "kv_append_rope.hip",
                   "rope_device.h", "sdv2kv_internal.h")
 
 

@@ -17,7 +17,7 @@ CSRC = PKG_DIR / "csrc"
 LIB_DIR = PKG_DIR / "_lib"
 LIB_PATH = LIB_DIR / "libsdv2kv.so"
 SOURCES = ["sdv2kv_api.hip", "kv_append_rope.hip", "swa_attn_fwd.hip", "swa_attn_fwd_m16.hip", "swa_attn_fwd_m16_few.hip",
-           "swa_attn_fwd_m16_shared.hip", "swa_attn_fwd_even.hip", "swa_attn_fwd_wave.hip",
+           "swa_attn_fwd_m16_shared.hip", "swa_attn_fwd_even.hip", "swa_attn_fwd_wave.hip", "swa_attn_fwd_wave_half.hip",
            "swa_attn_fwd_f32.hip", "sink_similarity.hip",
            "cache_relayout.hip", "rms_norm.hip", "linear.hip", "linear_wide.hip", "mfma_ceiling.hip"]
 

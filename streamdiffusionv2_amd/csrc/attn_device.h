@@ -398,9 +398,9 @@ struct WorkItem {
   }
 };
 // host: everything decode() needs, for query tiles of q_tile_rows rows
-inline void set_work_list(AttnKernelArgs* a, int q_tile_rows) {
+inline void set_work_list(AttnKernelArgs* a, int q_tile_rows, int parts = 1) {
   a->q_tile_rows = q_tile_rows;
-  a->q_tiles = (a->q_tokens + q_tile_rows - 1) / q_tile_rows;
+  a->q_tiles = (a->q_tokens + q_tile_rows - 1) / q_tile_rows * parts;       // (every tile as often as it has parts)
   a->per_group = a->q_tiles * ((a->group_pairs - a->more_pairs) * a->num_splits + a->more_pairs * (a->num_splits + 1));
   a->total_items = a->rows * a->heads / a->group_pairs * a->per_group;
   a->div_group = FastDiv::by((uint32_t)a->per_group);
@@ -427,6 +427,8 @@ int launch_m16_few(const AttnKernelArgs& a, uint32_t workgroups, hipStream_t str
 int launch_m16_shared(const AttnKernelArgs& a, uint32_t workgroups, hipStream_t stream);
 // the kernel whose waves share the keys of one query block (swa_attn_fwd_wave.hip)
 int launch_wave(const AttnKernelArgs& a, uint32_t workgroups, hipStream_t stream);
+// ... and two workgroups a block, each with half of V's columns: query tile 2 i + part of the work list (no rotation)
+int launch_wave_half(const AttnKernelArgs& a, uint32_t workgroups, hipStream_t stream);
 
 // the same with equal shares of the key tiles for all workgroups (swa_attn_fwd_even.hip)
 int launch_even(const EvenArgs& a, hipStream_t stream);

@@ -8,6 +8,9 @@
 // (K fragments straight from memory into registers, which would leave room for a block
 // more in flight, are 64-byte pieces of 16 rows: 2.2 us per 256 keys and workgroup.)
 //
+// Or two workgroups share a query block, each with half of V's columns (kParts = 2): both take all of K, nothing has to meet
+// between them, and each brings three quarters of the bytes; every number is the one a workgroup by itself comes to.
+//
 // Matrix layout (v_mfma_f32_16x16x32_bf16) and V^T fragments as in swa_attn_fwd_m16.hip.
 // Softmax: exp2 of the scaled scores against a running maximum per query and wave.
 #ifndef SDV2KV_ATTN_WAVE_DEVICE_H
@@ -57,7 +60,8 @@ __device__ __forceinline__ void read_k_now(uint32_t at, u32x4 (&k)[2][4]) {
       : "v"(at), "v"(at ^ 64u), "v"(at ^ 128u), "v"(at ^ 192u), "n"(kSub)
       : "memory");
 }
-// Four V^T fragments: dimension blocks db .. db + 3, address `at ^ (db << 5)`
+// Four V^T fragments: dimension blocks db .. db + 3, address `at ^ (db << 5)`, second 16 keys as far on as 16 rows take
+template <int kParts>
 __device__ __forceinline__ void read_v_now(uint32_t at, bf16x8 (&f)[4]) {
   u32x2 lo[4], hi[4];
   asm volatile(
@@ -71,17 +75,21 @@ __device__ __forceinline__ void read_v_now(uint32_t at, bf16x8 (&f)[4]) {
       "ds_read_b64_tr_b16 %7, %11 offset:%12\n\t"
       "s_waitcnt lgkmcnt(0)"
       : "=&v"(lo[0]), "=&v"(hi[0]), "=&v"(lo[1]), "=&v"(hi[1]), "=&v"(lo[2]), "=&v"(hi[2]), "=&v"(lo[3]), "=&v"(hi[3])
-      : "v"(at), "v"(at ^ 32u), "v"(at ^ 64u), "v"(at ^ 96u), "n"(kSub)
+      : "v"(at), "v"(at ^ 32u), "v"(at ^ 64u), "v"(at ^ 96u), "n"(kSub / kParts)
       : "memory");
 #pragma unroll
   for (int i = 0; i < 4; ++i) f[i] = __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo[i], hi[i], 0, 1, 2, 3));
 }
 
-// All but the newest block (eight transfers, if there is one) have landed
+// All but the newest block (kTransfers, if there is one) have landed
+template <int kTransfers>
 __device__ __forceinline__ void land(bool newer) {
-  if (newer) asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
+  if (newer) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kTransfers) : "memory");
   else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 }
+// Where 16-byte chunk c of row r of half of V is stored: position c ^ swz_half(r).  Two rows lie side by side in the banks, and
+// the four of a parity among eight consecutive rows, two chunks of each read together, must not meet.
+__device__ __forceinline__ int swz_half(int r) { return (r >> 1 & 3) << 1; }
 // A query that arrives rotated, ahead of everything else: it has landed with the first block
 __device__ __forceinline__ void load_rotated(bf16x8 (&qf)[2][4], const uint16_t* p0, const uint16_t* p1) {
   asm volatile(
@@ -100,12 +108,15 @@ __device__ __forceinline__ void load_rotated(bf16x8 (&qf)[2][4], const uint16_t*
 }
 
 // Queries q0 .. q0 + 31 of (row, head) against 32-key blocks [first_block, end_block) of those they see.  Every thread
-// gets eight columns, 8 (tid % 16) and on, of row tid / 16 of the normalised result.  kEarly: a query that arrives
+// gets eight columns, 8 (tid % 16) and on, of row tid / 16 of the normalised result; of two parts four, 64 part + 4 (tid %
+// 16) and on.  kEarly: a query that arrives
 // rotated is requested ahead of the first keys and waited for with them, which rests on the compiler leaving its
 // registers alone until then (checked on the assembly of the kernel that uses it).
-template <bool kMask, bool kRope, bool kEarly, typename Args>
+template <bool kMask, bool kRope, bool kEarly, int kParts = 1, typename Args>
 __device__ __forceinline__ void stream_block(Args& a, lds_char* lds, int head, int row, int q0, int first_block, int end_block,
-                                             f32x4 (&sum)[2]) {
+                                             f32x4 (&sum)[2 / kParts], int part = 0) {
+  static_assert(kParts == 1 || kParts == 2, "columns of V");
+  constexpr int kDb = 8 / kParts, kVTransfers = 8 / kParts, kVRow = 256 / kParts;       // dimension blocks, transfers and bytes of a row of V
   int tid = threadIdx.x;
   asm volatile("" : "+v"(tid));
   const int lane = tid & 63;
@@ -180,19 +191,26 @@ __device__ __forceinline__ void stream_block(Args& a, lds_char* lds, int head, i
   const int last_key0 = seq > kKeys ? seq - kKeys : 0;
   auto loaded_from = [&](int key0) { return key0 < last_key0 ? key0 : last_key0; };
   const int second = seq >= kKeys ? 16 : seq > 16 ? seq - 16 : 0;         // where the second 16 keys start
-  uint32_t k_off[4], v_off[4];
+  uint32_t k_off[4], v_off[kVTransfers / 2];
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
     const int r = 4 * j + g;
     const uint32_t rr = r < seq ? r : seq - 1, chunk = (uint32_t)((n16 ^ swz16(r)) << 4);
     k_off[j] = rr * k_tok_bytes + chunk;
-    v_off[j] = rr * v_tok_bytes + chunk;
+    if constexpr (kParts == 1) v_off[j] = rr * v_tok_bytes + chunk;
   }
-  auto fetch = [&](const char* base, uint32_t tok_bytes, const uint32_t (&off)[4], int b, uint32_t dst) {
+  if constexpr (kParts == 2)
+#pragma unroll
+    for (int j = 0; j < kVTransfers / 2; ++j) {
+      const int r = 8 * j + (lane >> 3);
+      v_off[j] = (uint32_t)(r < seq ? r : seq - 1) * v_tok_bytes + (uint32_t)(((lane & 7) ^ swz_half(r)) << 4) + part * kVRow;
+    }
+  auto fetch = [&](const char* base, uint32_t tok_bytes, const auto& off, int b, uint32_t dst) {
+    constexpr int kEach = sizeof(off) / sizeof(uint32_t);        // transfers of 16 keys
     const char* first = base + (int64_t)loaded_from(key0_of(b)) * tok_bytes;
     const char* half = first + (int64_t)second * tok_bytes;
 #pragma unroll
-    for (int j = 0; j < 8; ++j) dma16(j < 4 ? first : half, off[j & 3], dst + j * 1024);
+    for (int j = 0; j < 2 * kEach; ++j) dma16(j < kEach ? first : half, off[j % kEach], dst + j * 1024);
   };
   auto fetch_k = [&](int b) { fetch(kbase, k_tok_bytes, k_off, b, mine); };
   auto fetch_v = [&](int b) { fetch(vbase, v_tok_bytes, v_off, b, mine + kBlockBytes); };
@@ -205,14 +223,14 @@ __device__ __forceinline__ void stream_block(Args& a, lds_char* lds, int head, i
   // this lane's fragment addresses, for d-step / d block 0 (see swa_attn_fwd_m16.hip)
   const uint32_t k_at = mine + n16 * 256 + ((g ^ swz16(n16)) << 4);
   const int v_row = 4 * g + (n16 >> 2);
-  const uint32_t v_at = mine + kBlockBytes + v_row * 256 + ((((n16 & 3) >> 1) ^ swz16(v_row)) << 4) + (n16 & 1) * 8;
+  const uint32_t v_at = mine + kBlockBytes + v_row * kVRow + ((((n16 & 3) >> 1) ^ (kParts == 1 ? swz16(v_row) : swz_half(v_row))) << 4) + (n16 & 1) * 8;
   const bf16x8 ones = __builtin_bit_cast(bf16x8, u32x4{0x3f803f80u, 0x3f803f80u, 0x3f803f80u, 0x3f803f80u});
 
-  f32x4 oacc[8][2], lacc[2];
+  f32x4 oacc[kDb][2], lacc[2];
 #pragma unroll
   for (int qt = 0; qt < 2; ++qt) {
 #pragma unroll
-    for (int db = 0; db < 8; ++db) oacc[db][qt] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int db = 0; db < kDb; ++db) oacc[db][qt] = f32x4{0.f, 0.f, 0.f, 0.f};
     lacc[qt] = f32x4{0.f, 0.f, 0.f, 0.f};
   }
   float m_run[2] = {-INFINITY, -INFINITY}, neg_ref[2] = {0.f, 0.f};
@@ -220,7 +238,7 @@ __device__ __forceinline__ void stream_block(Args& a, lds_char* lds, int head, i
   for (int b = block0; b < nblocks; b += kWaves) {
     const bool more = b + kWaves < nblocks;
     u32x4 k[2][4];
-    land(true);                                // (V of this block is the newest)
+    land<kVTransfers>(true);                   // (V of this block is the newest)
     read_k_now(k_at, k);
     if (more) fetch_k(b + kWaves);
 #pragma unroll
@@ -272,7 +290,7 @@ __device__ __forceinline__ void stream_block(Args& a, lds_char* lds, int head, i
         for (int i = 0; i < 4; ++i) {
           lacc[qt][i] *= alpha;
 #pragma unroll
-          for (int db = 0; db < 8; ++db) oacc[db][qt][i] *= alpha;
+          for (int db = 0; db < kDb; ++db) oacc[db][qt][i] *= alpha;
         }
       }
     }
@@ -288,13 +306,13 @@ __device__ __forceinline__ void stream_block(Args& a, lds_char* lds, int head, i
 #pragma unroll
     for (int qt = 0; qt < 2; ++qt)
       lacc[qt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones, __builtin_bit_cast(bf16x8, p[qt]), lacc[qt], 0, 0, 0);
-    land(more);
-    bf16x8 v[2][4];
-    read_v_now(v_at, v[0]);
-    read_v_now(v_at ^ 128u, v[1]);
+    land<8>(more);
+    bf16x8 v[kDb / 4][4];
+    read_v_now<kParts>(v_at, v[0]);
+    if constexpr (kParts == 1) read_v_now<kParts>(v_at ^ 128u, v[1]);
     if (more) fetch_v(b + kWaves);
 #pragma unroll
-    for (int db = 0; db < 8; ++db)
+    for (int db = 0; db < kDb; ++db)
 #pragma unroll
       for (int qt = 0; qt < 2; ++qt)
         oacc[db][qt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(v[db >> 2][db & 3], __builtin_bit_cast(bf16x8, p[qt]), oacc[db][qt], 0, 0, 0);
@@ -329,22 +347,24 @@ __device__ __forceinline__ void stream_block(Args& a, lds_char* lds, int head, i
     const float f = to_top(m_run[qt]) * (total > 0.f ? 1.0f / total : 0.f);
     const int r = 16 * qt + n16;
 #pragma unroll
-    for (int db = 0; db < 8; ++db) {
+    for (int db = 0; db < kDb; ++db) {
       f32x4 o = oacc[db][qt];
 #pragma unroll
       for (int i = 0; i < 4; ++i) o[i] *= f;
-      *reinterpret_cast<lds_f32x4*>(lds + wave * kWaveLds + r * 512 + (((4 * db + g) ^ n16) << 4)) = o;
+      *reinterpret_cast<lds_f32x4*>(lds + wave * kWaveLds + r * (512 / kParts) + (((4 * db + g) ^ n16) << 4)) = o;
     }
   }
   __syncthreads();
   {
-    const int r = tid >> 4, c = 2 * (tid & 15);          // row, first of two 16-byte pieces of it
-    sum[0] = sum[1] = f32x4{0.f, 0.f, 0.f, 0.f};
+    constexpr int kPieces = 2 / kParts;
+    const int r = tid >> 4, c = kPieces * (tid & 15);    // row, first of its 16-byte pieces
+#pragma unroll
+    for (int e = 0; e < kPieces; ++e) sum[e] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int u = 0; u < kWaves; ++u)
 #pragma unroll
-      for (int e = 0; e < 2; ++e) {
-        const f32x4 x = *reinterpret_cast<lds_f32x4*>(lds + u * kWaveLds + r * 512 + (((c + e) ^ (r & 15)) << 4));
+      for (int e = 0; e < kPieces; ++e) {
+        const f32x4 x = *reinterpret_cast<lds_f32x4*>(lds + u * kWaveLds + r * (512 / kParts) + (((c + e) ^ (r & 15)) << 4));
 #pragma unroll
         for (int i = 0; i < 4; ++i) sum[e][i] += x[i];
       }
@@ -376,6 +396,14 @@ __device__ __forceinline__ void write_row(Args& a, int head, int row, int q0, co
     x[2 * e + 1] = pack_bf16x2(sum[e][2], sum[e][3]);
   }
   *reinterpret_cast<u32x4*>(a.out + row * a.o_st.row + head * a.o_st.head + (int64_t)token * a.o_st.token + 8 * (threadIdx.x & 15)) = x;
+}
+
+template <typename Args>
+__device__ __forceinline__ void write_half_row(Args& a, int head, int row, int q0, int part, const f32x4& sum) {
+  const int token = q0 + (threadIdx.x >> 4);
+  if (token >= a.q_tokens) return;
+  const u32x2 x = {pack_bf16x2(sum[0], sum[1]), pack_bf16x2(sum[2], sum[3])};
+  *reinterpret_cast<u32x2*>(a.out + row * a.o_st.row + head * a.o_st.head + (int64_t)token * a.o_st.token + part * (kD / 2) + 4 * (threadIdx.x & 15)) = x;
 }
 
 }  // namespace wave

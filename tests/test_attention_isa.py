@@ -237,3 +237,26 @@ def test_nothing_touches_a_query_on_its_way(assembly_wave):
     counts = [int(x) for x in re.findall(r"\.vgpr_count:\s+(\d+)", "\n".join(assembly_wave))]
     assert len(counts) == 4 and max(counts) <= 256, counts
     assert not any(re.search(r"\bscratch_(load|store)", l) for l in assembly_wave)
+
+
+def test_nothing_touches_a_query_on_its_way_to_half_of_the_values():
+    """The same of two workgroups to a block, where four transfers of V are the newest at the first wait."""
+    out = os.path.join(ROOT, "build", "isa_check")
+    os.makedirs(out, exist_ok=True)
+    path = os.path.join(out, "swa_attn_fwd_wave_half.s")
+    cmd = [build_ext.hipcc_path(), *build_ext.HIPCC_FLAGS, f"-I{os.path.join(ROOT, 'include')}", f"-I{build_ext.CSRC}",
+           "-S", "--cuda-device-only", str(build_ext.CSRC / "swa_attn_fwd_wave_half.hip"), "-o", path]
+    res = subprocess.run(cmd, capture_output=True, text=True)
+    assert res.returncode == 0, res.stderr[-2000:]
+    text = open(path).read()
+    asked = [m.start() for m in re.finditer("Q requested", text)]
+    assert len(asked) == 2
+    for at in asked:
+        lines = text[:at].rsplit("\n", 8)[-8:] + [""]
+        query = set().union(*(registers(ops[0]) for mn, ops in instructions(lines) if mn == "global_load_dwordx4"))
+        assert len(query) == 32
+        for mn, ops in instructions(text[at:].split("\n")[1:]):
+            if mn == "s_waitcnt" and ops[0].startswith("vmcnt(4)"):
+                break
+            assert not any(registers(o) & query for o in ops), (mn, ops)
+    assert max(int(x) for x in re.findall(r"\.vgpr_count:\s+(\d+)", text)) <= 256 and not re.search(r"\bscratch_(load|store)", text)

@@ -632,3 +632,12 @@ def test_query_tiles_whose_last_blocks_are_shared(gpu_device, rows, S, H, L, seq
     torch.cuda.synchronize()
     assert torch.equal(*got)
     _check(got[0].cpu(), want)
+
+
+@pytest.mark.parametrize("rows,S,H,L,seq,block", [
+    (2, 31, 65, 16, [15, 16], 0), (2, 33, 40, 40, [17, 31], 0), (3, 32, 43, 64, [32, 33, 0], 0), (1, 64, 65, 255, None, 0),
+    (1, 90, 45, 333, None, 30), (1, 120, 33, 120, None, 10),
+])
+def test_attention_of_small_calls_with_a_workgroup_a_block(gpu_device, rows, S, H, L, seq, block):
+    """(up to 128 query blocks, as most of the above are, have two workgroups each)"""
+    test_attention_of_small_calls(gpu_device, rows, S, H, L, seq, block, True)
