@@ -303,7 +303,8 @@ class RingKVPath:
             self._evict_idx = [list(self._evict_idx[0]) for _ in range(cache_rows)]
 
         table = ops.device_freqs(freqs, q.device)
-        self._last_refresh = None
+        own = self.__dict__               # (plain attributes: a module's own way of setting one takes three microseconds)
+        own["_last_refresh"] = None
         adaptive = self.sink_size * frame_tokens > 0 and self.adapt_sink_thr > -1 and q.shape[1] <= frame_tokens
         k_norm = (qk_norm[1], qk_norm[2]) if qk_norm is not None else None
         if adaptive:
@@ -371,7 +372,7 @@ class RingKVPath:
                 # rows differ only while the stream batch is still filling; the
                 # lengths are a handful of host ints, shipped asynchronously
                 seq = torch.tensor(plan.new_local_end, dtype=torch.int32).to(q.device, non_blocking=True)
-            self._last_plan = plan
+            own["_last_plan"] = plan
             mask_tokens = 0
             if self.block_frames is not None and self.block_frames * frame_tokens < q.shape[1]:
                 mask_tokens = self.block_frames * frame_tokens
@@ -470,21 +471,23 @@ class CausalWanSelfAttention(nn.Module, RingKVPath):
         """(weight [3 * dim, dim], bias [3 * dim] or None) of the q, k and v
         Linears laid end to end, rebuilt when any of the six tensors has been
         replaced (another tensor, dtype or device) or written in place."""
-        layers = (self.q, self.k, self.v)
+        modules = self._modules
+        layers = (modules["q"], modules["k"], modules["v"])
+        key = []
         for layer in layers:
             # only plain Linears that nobody watches: a wrapped or replaced layer (an adapter, a quantised
             # Linear) computes something else than x W^T + b, and a hook expects its layer to be called
             if type(layer) is not nn.Linear or layer._forward_hooks or layer._forward_pre_hooks:
                 return None
-        tensors = [t for layer in layers for t in (layer.weight, layer.bias)]
-
-        def edits(t):
-            try:
-                return t._version
-            except RuntimeError:                   # a tensor made under inference_mode() counts no edits:
-                return -1                          # after writing such a weight in place, set _packed = None
-
-        key = tuple((t.data_ptr(), edits(t), t.dtype, t.device) if t is not None else None for t in tensors)
+            for t in (layer.weight, layer.bias):
+                if t is None:
+                    key.append(None)
+                    continue
+                try:
+                    edits = t._version
+                except RuntimeError:               # a tensor made under inference_mode() counts no edits:
+                    edits = -1                     # after writing such a weight in place, set _packed = None
+                key.append((t.data_ptr(), edits, t.dtype, t.device))
         packed = self._packed
         if packed is None or packed[0] != key:
             with torch.no_grad():

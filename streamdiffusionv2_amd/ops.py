@@ -47,6 +47,13 @@ def _stream_ptr(dev: torch.device) -> int:
     return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if index is None else index)
 
 
+def _empty_as(t: torch.Tensor) -> torch.Tensor:
+    """A contiguous plain tensor of t's shape, dtype and device."""
+    if type(t) is torch.Tensor and t.is_contiguous():
+        return torch.empty_like(t)                # (a third of the time it takes to spell them out)
+    return torch.empty(t.shape, dtype=t.dtype, device=t.device)
+
+
 class _NoSwitch:
     def __enter__(self):
         return self
@@ -479,7 +486,7 @@ def swa_attention(
     if seq_lens is not None and (seq_lens.dtype != torch.int32 or seq_lens.numel() != rows or not seq_lens.is_contiguous()):
         raise RuntimeError("seq_lens must be a contiguous int32 tensor with one entry per row")
     if out is None:
-        out = torch.empty(q.shape, dtype=q.dtype, device=dev)
+        out = _empty_as(q)
 
     lib = _capi.lib()
     stream = _stream_ptr(dev)
@@ -905,7 +912,7 @@ class LayerLauncher:
             ap.q_in = ap.q_out = ap.q_norm_weight = None
             ap.k_inv_rms = inv_rms.data_ptr() if inv_rms is not None else None
         else:
-            self.roped_q = torch.empty(self.in_shape, dtype=torch.bfloat16, device=self.dev)
+            self.roped_q = _empty_as(q) if q.device == self.dev else torch.empty(self.in_shape, dtype=torch.bfloat16, device=self.dev)
             ap.q_in = q.data_ptr()
             ap.q_out = at.q = self.roped_q.data_ptr()
             if self.norm_args is not None:
@@ -925,7 +932,7 @@ class LayerLauncher:
             # and the launch: the one this call carries is held)
             self.workspace = ws = _workspace(self.dev, self.workspace_need, stream=stream)
             at.workspace, at.workspace_bytes = ws.data_ptr(), ws.numel()
-        out = torch.empty(self.in_shape, dtype=torch.bfloat16, device=self.dev)
+        out = torch.empty(self.in_shape, dtype=torch.bfloat16, device=self.dev) if self.rope_in_attention else _empty_as(self.roped_q)
         at.out = out.data_ptr()
         at.seq_lens = seq_lens.data_ptr() if seq_lens is not None else None
         return out
@@ -1002,27 +1009,43 @@ def flash_attention(q, k, v, q_lens=None, k_lens=None, dropout_p=0.0, softmax_sc
     return out if out_dtype == torch.bfloat16 else out.to(out_dtype)
 
 
-def _relayout_params(dst, src, dst_indices, src_indices, global_end_shift):
-    flat = [dst, src] + list(dst_indices or ()) + list(src_indices or ())
-    dev = _require_gpu(*flat)
+_RELAYOUT_LAYOUTS: dict = {}
+
+
+def _relayout_layout(dst, src) -> bytes:
+    """The descriptor of such a pair of tensors, but for what changes from call to call."""
     if src.dtype not in _DTYPES or dst.dtype != src.dtype:
         raise RuntimeError(f"unsupported dtype pair {dst.dtype} / {src.dtype}")
     if tuple(dst.shape) != tuple(src.shape):
         raise RuntimeError(f"shape mismatch: {tuple(dst.shape)} vs {tuple(src.shape)}")
-    if (dst_indices is None) != (src_indices is None):
-        raise RuntimeError("index tensors are handed over as two pairs or not at all")
     rows, tokens, heads, _ = src.shape
     p = _capi.RelayoutParams()
-    p.src, p.src_stride = src.data_ptr(), _stride3(src, "src")
-    p.dst, p.dst_stride = dst.data_ptr(), _stride3(dst, "dst")
+    p.src_stride, p.dst_stride = _stride3(src, "src"), _stride3(dst, "dst")
     p.dtype = _DTYPES[src.dtype]
     p.rows, p.heads, p.head_dim, p.tokens = rows, heads, HEAD_DIM, tokens
+    return bytes(p)
+
+
+def _relayout_params(dst, src, dst_indices, src_indices, global_end_shift):
+    dev = _require_gpu(dst, src, *(dst_indices or ()), *(src_indices or ()))
+    key = (src.shape, dst.shape, src.stride(), dst.stride(), src.dtype, dst.dtype)
+    layout = _RELAYOUT_LAYOUTS.get(key)
+    if layout is None:
+        layout = _relayout_layout(dst, src)
+        if len(_RELAYOUT_LAYOUTS) >= _MAX_ATTN_LAYOUTS:
+            _RELAYOUT_LAYOUTS.clear()
+        _RELAYOUT_LAYOUTS[key] = layout
+    if (dst_indices is None) != (src_indices is None):
+        raise RuntimeError("index tensors are handed over as two pairs or not at all")
+    p = _capi.RelayoutParams.from_buffer_copy(layout)
+    p.src, p.dst = src.data_ptr(), dst.data_ptr()
     if dst_indices is not None:
+        rows = src.shape[0]
         for idx in (*dst_indices, *src_indices):
             if idx.dtype != torch.int64 or idx.numel() < rows or not idx.is_contiguous():
                 raise RuntimeError("end-index tensors must be contiguous int64 with one entry per row")
-        p.dst_global_end_index, p.dst_local_end_index = (t.data_ptr() for t in dst_indices)
-        p.src_global_end_index, p.src_local_end_index = (t.data_ptr() for t in src_indices)
+        p.dst_global_end_index, p.dst_local_end_index = dst_indices[0].data_ptr(), dst_indices[1].data_ptr()
+        p.src_global_end_index, p.src_local_end_index = src_indices[0].data_ptr(), src_indices[1].data_ptr()
         p.global_end_shift = int(global_end_shift)
     p.stream = _stream_ptr(dev)
     return p, dev
@@ -1156,8 +1179,24 @@ def _plain_call() -> bool:
 
 
 _PLAIN_TENSORS = (torch.Tensor, torch.nn.Parameter)
-_LINEAR_PREFERRED: dict = {}
+_LINEAR_LAYOUTS: dict = {}
 _FOLDS_NORM: dict = {}
+
+
+def _linear_layout(x: torch.Tensor, weight: torch.Tensor, row_squares: bool):
+    """(descriptor as bytes, but for what changes from call to call, shape of the result, shape of the sums) of a product
+    of such tensors, or None where it is not the library's."""
+    if weight.dim() != 2 or x.dim() < 2 or x.numel() == 0:
+        return None
+    n, k = weight.shape
+    if x.shape[-1] != k:
+        return None
+    m = x.numel() // k
+    rows = _norm_rows(x)
+    if rows is None or not _capi.lib().sdv2_linear_one_round(m, n, k, row_squares):
+        return None
+    lead = tuple(x.shape[:-1])
+    return bytes(_capi.LinearParams(None, None, None, None, rows[1], k, n, m, n, k, _capi.DTYPE_BF16)), (*lead, n), (*lead, n // 32)
 
 
 def linear_or_none(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor],
@@ -1169,32 +1208,32 @@ def linear_or_none(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.T
     of its rows, float32 [..., n / 32]."""
     bf16 = torch.bfloat16
     if not (x.is_cuda and x.dtype == bf16 and weight.dtype == bf16 and type(x) in _PLAIN_TENSORS
-            and type(weight) in _PLAIN_TENSORS and weight.dim() == 2 and x.dim() >= 2 and x.numel() and _plain_call()):
+            and type(weight) in _PLAIN_TENSORS and _plain_call()):
         return None
-    n, k = weight.shape
-    if x.shape[-1] != k:
+    key = (x.shape, x.stride(), weight.shape, row_squares)
+    layout = _LINEAR_LAYOUTS.get(key, _LINEAR_LAYOUTS)
+    if layout is _LINEAR_LAYOUTS:                   # (not seen yet)
+        if len(_LINEAR_LAYOUTS) >= _MAX_ATTN_LAYOUTS:
+            _LINEAR_LAYOUTS.clear()
+        layout = _LINEAR_LAYOUTS[key] = _linear_layout(x, weight, row_squares)
+    if layout is None:
         return None
-    m = x.numel() // k
-    key = (m, n, k, row_squares)
-    preferred = _LINEAR_PREFERRED.get(key)
-    if preferred is None:
-        if len(_LINEAR_PREFERRED) >= _MAX_ATTN_LAYOUTS:
-            _LINEAR_PREFERRED.clear()
-        preferred = _LINEAR_PREFERRED[key] = bool(_capi.lib().sdv2_linear_one_round(m, n, k, row_squares))
-    if not preferred:
-        return None
+    template, out_shape, squares_shape = layout
     dev = x.device
-    rows = _norm_rows(x)
-    if rows is None or weight.device != dev or not weight.is_contiguous() or x.data_ptr() % 16 or weight.data_ptr() % 16:
+    x_ptr, weight_ptr = x.data_ptr(), weight.data_ptr()
+    if weight.device != dev or not weight.is_contiguous() or x_ptr % 16 or weight_ptr % 16:
         return None
-    if bias is not None and not (type(bias) in _PLAIN_TENSORS and bias.dtype == bf16 and bias.device == dev
-                                 and bias.dim() == 1 and bias.is_contiguous() and bias.data_ptr() % 8 == 0):
-        return None
-    out = torch.empty((*x.shape[:-1], n), dtype=bf16, device=dev)
-    p = _capi.LinearParams(x.data_ptr(), weight.data_ptr(), bias.data_ptr() if bias is not None else None, out.data_ptr(),
-                           rows[1], k, n, m, n, k, _capi.DTYPE_BF16, _stream_ptr(dev))
-    squares = torch.empty((*x.shape[:-1], n // 32), dtype=torch.float32, device=dev) if row_squares else None
+    p = _capi.LinearParams.from_buffer_copy(template)
+    if bias is not None:
+        if not (type(bias) in _PLAIN_TENSORS and bias.dtype == bf16 and bias.device == dev and bias.dim() == 1 and bias.is_contiguous()):
+            return None
+        p.bias = bias_ptr = bias.data_ptr()
+        if bias_ptr % 8:
+            return None
+    out = _empty_as(x) if x.shape == out_shape else torch.empty(out_shape, dtype=bf16, device=dev)
+    p.x, p.weight, p.out, p.stream = x_ptr, weight_ptr, out.data_ptr(), _stream_ptr(dev)
     if row_squares:
+        squares = torch.empty(squares_shape, dtype=torch.float32, device=dev)
         p.row_squares = squares.data_ptr()
     with _on_device(dev):
         _capi.check(_capi.lib().sdv2_linear(C.byref(p)), "sdv2_linear")
