@@ -41,7 +41,8 @@ inline void launch_timed(int which, Kernel kernel, dim3 grid, dim3 block, uint32
 // memory, and the compiler loads them where they are used: four or five trips one after another at the start of
 // every workgroup.  Behind this the rest come from the scalar cache.  Eight layers of 256
 // tokens x 12 heads against 1536 keys 178 -> 167 us; in the 16x16x32 attention 0.7 to 1 us of a launch (2560 x 12 heads
-// against 1024 keys 22.3 -> 21.7, 1560 x 12 in three ranges of 9360 84.8 -> 83.8, in equal shares 97.6 -> 96.9).  (In the
+// against 1024 keys 22.3 -> 21.7, 1560 x 12 in three ranges of 9360 84.8 -> 83.8, in equal shares 97.6 -> 96.9), 0.4 to 1 in the sink decision.  (In
+// sdv2_linear it makes no difference; in the
 // 32x32x16 kernel it costs 0.5 to 1 %: that one is short of scalar registers at its start.)
 template <typename Args>
 __device__ __forceinline__ void fetch_arguments() {

@@ -214,6 +214,10 @@ __device__ __forceinline__ void decide(const SinkSimKernelArgs& a, int row) {
   // where the eight ranges' sums of the column group that starts at column i of this thread begin
   auto ranges_of = [&](const float* p, int i) { return p + (col(i) >> 7) * (kTokenSplits * 128) + (col(i) & 127); };
   auto live = [&](int i) { return raw_col(i) < width ? 1.f : 0.f; };
+  auto store_kept = [&](float* keep, const float (&x)[kCols]) {
+#pragma unroll
+    for (int i0 = 0; i0 < kCols; i0 += 4) *reinterpret_cast<f32x4*>(keep + col(i0)) = f32x4{x[i0], x[i0 + 1], x[i0 + 2], x[i0 + 3]};
+  };
   // means of matrix m at this thread's columns: the token ranges in order and
   // the rounding of a stored mean, or the mean kept from an earlier call.  The
   // token sums are fetched for four columns at a time.
@@ -232,15 +236,15 @@ __device__ __forceinline__ void decide(const SinkSimKernelArgs& a, int row) {
           out[i0 + e] = round_to_storage<T>(sum * inv_tokens);
         }
       }
-      if (a.kept && m < 2 * sink) {
-        float* keep = kept_of(a, row, m);
-#pragma unroll
-        for (int i = 0; i < kCols; ++i) keep[col(i)] = out[i];      // (clamped columns repeat the last one's value)
-      }
+      if (a.kept && m < 2 * sink) store_kept(kept_of(a, row, m), out);      // (clamped columns repeat the last group's values)
     } else {
       const float* keep = kept_of(a, row, m);
 #pragma unroll
-      for (int i = 0; i < kCols; ++i) out[i] = keep[col(i)];
+      for (int i0 = 0; i0 < kCols; i0 += 4) {
+        const f32x4 x = *reinterpret_cast<const f32x4*>(keep + col(i0));
+#pragma unroll
+        for (int e = 0; e < 4; ++e) out[i0 + e] = x[e];
+      }
     }
   };
   // this wave's share of four sums, in a fixed order, parked in LDS
@@ -351,13 +355,8 @@ __device__ __forceinline__ void decide(const SinkSimKernelArgs& a, int row) {
     const bool evicting = (a.override_rows >> row) & 1u;
     const int target = evicting && a.dst_override && chosen >= 0 ? chosen : a.planned_frame[row];
     if (target >= 0 && target < sink) {
-      float* keep_k = kept_of(a, row, target);
-      float* keep_v = kept_of(a, row, sink + target);
-#pragma unroll
-      for (int i = 0; i < kCols; ++i) {
-        keep_k[col(i)] = k_new[i];
-        keep_v[col(i)] = v_new[i];
-      }
+      store_kept(kept_of(a, row, target), k_new);
+      store_kept(kept_of(a, row, sink + target), v_new);
     }
   }
 }
@@ -447,12 +446,17 @@ __device__ __forceinline__ void rotate_queries(const SinkSimKernelArgs& a, int w
 // What bounds it is the chain of trips to memory: tokens with their table entries, sums acknowledged, ticket, sums of
 // the row, results.  512 threads take a range of 195 tokens in one trip and the row's sums in another (256 threads took
 // two each): 2 x 1560 tokens x 12 heads, means kept, 25.2 -> 22 us, and with the new K and V in one workgroup 18.0
-// (one row 17.5 -> 17.2, four 34.2 -> 26.4; 1 x 1560 x 40 heads 39.5 -> 34.0, 4 x 3600 x 40 143 -> 108).
+// (one row 17.5 -> 17.2, four 34.2 -> 26.4; 1 x 1560 x 40 heads 39.5 -> 34.0, 4 x 3600 x 40 143 -> 108).  Of what was left,
+// with the query beside it, 6.5 us were the tokens, 1.9 the meeting of the token lanes, 1.5 acknowledgement and ticket, 6.9 the
+// decision (11 with forty heads, whose kept means came four bytes at a time); arguments asked for together, lanes that meet in
+// registers and kept means in 16-byte accesses: 21.5 -> 20.0, 1 x 399 x 40 24.8 -> 20.5.
 template <typename T, int kCols>
 __global__ __launch_bounds__(kThreads)
 void sink_similarity_kernel(const SinkSimKernelArgs a) {
-  __shared__ float part[2][kTokenLanes][kLanesPerRow * 8];    // of the matrix, of V beside the new K
+  // sums of the waves, of the matrix and of V beside the new K; the query's workgroups have their scratch in it
+  __shared__ __attribute__((aligned(16))) float part[kThreads / 64][2][64 * 8];
   __shared__ int is_last;
+  sdv2::fetch_arguments<SinkSimKernelArgs>();
   const int lane = threadIdx.x & (kLanesPerRow - 1);
   const int tl = threadIdx.x >> 4;
   const int head = blockIdx.x;
@@ -461,10 +465,9 @@ void sink_similarity_kernel(const SinkSimKernelArgs a) {
   if constexpr (std::is_same<T, uint16_t>::value) {
     if (row >= a.rows) {
       const int workgroup = (blockIdx.z - a.rows * kTokenSplits) * a.heads + head;
-      static_assert(sizeof(part) == kThreads / 64 * sizeof(float[2][64 * 8]), "the waves' scratch");
       // (kCols columns a thread are 512 kCols columns, 4 kCols heads)
       if (blockIdx.y == 0 && workgroup < a.q_workgroups)
-        rotate_queries<kCols>(a, workgroup, reinterpret_cast<float(*)[2][64 * 8]>(&part[0][0][0])[threadIdx.x >> 6]);
+        rotate_queries<kCols>(a, workgroup, part[threadIdx.x >> 6]);
       return;
     }
   }
@@ -543,17 +546,35 @@ void sink_similarity_kernel(const SinkSimKernelArgs a) {
           for (int i = 0; i < 8; ++i) acc[i] += static_cast<float>(x[u].get(i));
     }
   }
+  // The four token lanes of a wave meet in registers, the waves in LDS.  (All 32 token lanes through LDS, a number at a time
+  // and eight ways into a bank, took 1.9 us of the launch's 18.)
+  auto over_token_lanes = [](float x) {
+    auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+    x = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+    r = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+    return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+  };
 #pragma unroll
   for (int i = 0; i < 8; ++i) {
-    part[0][tl][lane * 8 + i] = acc[i];
-    if (is_new) part[1][tl][lane * 8 + i] = acc_v[i];
+    acc[i] = over_token_lanes(acc[i]);
+    if (is_new) acc_v[i] = over_token_lanes(acc_v[i]);
+  }
+  const int wave = threadIdx.x >> 6;
+  if ((threadIdx.x & 63) < kLanesPerRow) {
+#pragma unroll
+    for (int half = 0; half < 2; ++half) {
+      *reinterpret_cast<f32x4*>(&part[wave][0][lane * 8 + 4 * half]) = f32x4{acc[4 * half], acc[4 * half + 1], acc[4 * half + 2], acc[4 * half + 3]};
+      if (is_new)
+        *reinterpret_cast<f32x4*>(&part[wave][1][lane * 8 + 4 * half]) =
+            f32x4{acc_v[4 * half], acc_v[4 * half + 1], acc_v[4 * half + 2], acc_v[4 * half + 3]};
+    }
   }
   __syncthreads();
   const int of = threadIdx.x >> 7, column = threadIdx.x & 127;
   if (of < (is_new ? 2 : 1)) {
     float sum = 0.f;
 #pragma unroll
-    for (int j = 0; j < kTokenLanes; ++j) sum += part[of][j][column];
+    for (int j = 0; j < kThreads / 64; ++j) sum += part[j][of][column];
     store_coherent(sums_of(a, row, m + of) + (head * kTokenSplits + split) * 128 + column, sum);
   }
   __builtin_amdgcn_s_waitcnt(0x0F70);       // vmcnt(0): the stores have been acknowledged
@@ -579,6 +600,7 @@ void sink_similarity_kernel(const SinkSimKernelArgs a) {
 template <typename T, int kSteps>
 __global__ __launch_bounds__(256)
 void key_inv_rms_kernel(const SinkSimKernelArgs a) {
+  sdv2::fetch_arguments<SinkSimKernelArgs>();
   const int lane = threadIdx.x & 63;
   const int tok = blockIdx.x * 4 + (threadIdx.x >> 6);
   const int row = blockIdx.z;
