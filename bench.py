@@ -84,7 +84,7 @@ def record_traffic(args, w):
         total, count = collections.defaultdict(float), collections.Counter()
         for row in csv.DictReader(open(files[0])):
             for short, names in (("swa_attn_fwd_kernel", ("swa_attn_fwd_kernel", "swa_attn_fwd_m16_kernel", "swa_attn_fwd_even_kernel",
-                                                          "swa_attn_fwd_wave_kernel")),
+                                                          "swa_attn_fwd_wave_kernel", "swa_attn_fwd_wave_half_kernel")),
                                  ("kv_append_rope_kernel", ("kv_append_rope_kernel",)), ("copy16_kernel", ("copy16_kernel",))):
                 if any(n in row["Kernel_Name"] for n in names):
                     total[short] += float(row["Counter_Value"])
