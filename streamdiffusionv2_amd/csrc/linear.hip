@@ -84,6 +84,9 @@ extern "C" int sdv2_linear_one_round(int64_t m, int32_t n, int32_t k, int32_t ro
   // time on the geometric mean (1560 x 4608 x 1536 24.3 against 28.3 us, 528 x 3712 x 3712 23.6 and 32.6, 1560 x 5120 x
   // 5120 73.4 and 88); 528 to 640 rows of 5120 x 5120 lose up to 7 %, 352 rows 17.  A second round costs a launch's
   // start and end again and leaves CUs idle: 480 tiles 1.1 to 1.23 of the vendor's time.
+  // Of few rows and a long contraction the vendor's cuts the contraction (16 x 5120 x 5120 14.9 against 22.1 us, 64 x 5120 x
+  // 5120 21.3 and 29.6, 64 x 7680 x 2560 15.6 and 17.6; 100 x 5120 x 5120 27.5 and 25.7, 100 x 3712 x 3712 18.8 and 17.4).
+  if (m <= 96 && k > 2048) return 0;
   const int i = best_tile(m, n, k, row_squares != 0);
   return i >= 0 && tiles_of(kTiles[i], m, n) <= kCus;
 }

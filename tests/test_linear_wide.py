@@ -17,7 +17,7 @@ def test_which_products_are_one_round():
     lib = _capi.lib()
     for m, n, k, squares, want in ((1560, 4608, 1536, 0, 1), (1560, 5120, 5120, 0, 1), (1792, 5120, 64, 0, 1), (1793, 5120, 64, 0, 0),
                                    (1560, 5120, 5120, 1, 0), (1536, 5120, 64, 1, 1), (1280, 5120, 5120, 1, 1),
-                                   (9360, 1536, 1536, 0, 0), (1560, 15360, 5120, 0, 0), (0, 64, 64, 0, 0), (16, 96, 64, 0, 0), (16, 64, 96, 0, 0)):
+                                   (96, 5120, 5120, 0, 0), (97, 5120, 5120, 0, 1), (1, 5120, 2048, 0, 1), (9360, 1536, 1536, 0, 0), (1560, 15360, 5120, 0, 0), (0, 64, 64, 0, 0), (16, 96, 64, 0, 0), (16, 64, 96, 0, 0)):
         assert lib.sdv2_linear_one_round(m, n, k, squares) == want, (m, n, k, squares)
 
 
