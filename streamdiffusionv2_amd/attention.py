@@ -472,7 +472,7 @@ class CausalWanSelfAttention(nn.Module, RingKVPath):
         Linears laid end to end, rebuilt when any of the six tensors has been
         replaced (another tensor, dtype or device) or written in place."""
         modules = self._modules
-        layers = (modules["q"], modules["k"], modules["v"])
+        layers = (modules.get("q"), modules.get("k"), modules.get("v"))
         key = []
         for layer in layers:
             # only plain Linears that nobody watches: a wrapped or replaced layer (an adapter, a quantised

@@ -55,6 +55,18 @@ def test_the_packed_copy_follows_the_weights():
     assert _close(mod, x.double()) and mod._packed[1].dtype == torch.float64
 
 
+def test_a_layer_that_is_no_registered_module_is_called():
+    torch.manual_seed(3)
+    mod = CausalWanSelfAttention(256, 2)
+    x = torch.randn(1, 5, 256)
+    q, want = mod.q, mod.q(x) * 2
+    del mod.q
+    object.__setattr__(mod, "q", lambda t: q(t) * 2)
+    with torch.no_grad():
+        assert mod._packed_qkv() is None
+        assert torch.equal(mod.project_qkv(x)[0], want)
+
+
 def test_three_launches_when_asked_or_when_training():
     torch.manual_seed(2)
     mod = CausalWanSelfAttention(256, 2)
