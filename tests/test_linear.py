@@ -180,6 +180,12 @@ def test_infinities_and_nans_stay_in_their_row(gpu_device):
     _check(got[ok], x[ok], w, None)
 
 
+def test_results_are_contiguous_whatever_the_strides_of_ones():
+    t = torch.empty(4096).as_strided((1, 4, 2, 128), (3, 256, 128, 1))
+    assert t.is_contiguous() and ops._empty_as(t).stride() == (1024, 256, 128, 1)
+    assert ops._empty_as(t.transpose(1, 2)).stride() == (1024, 512, 128, 1)
+
+
 @pytest.mark.gpu
 def test_the_modules_take_it(gpu_device):
     """A chunk's q, k, v and o, of a strided input too; one product for q, k and v gives the bits of three (every element
