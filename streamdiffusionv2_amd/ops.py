@@ -1181,6 +1181,7 @@ def _plain_call() -> bool:
 
 _PLAIN_TENSORS = (torch.Tensor, torch.nn.Parameter)
 _LINEAR_LAYOUTS: dict = {}
+_MAX_LINEAR_STRIDE = 1 << 22           # elements between x's rows, as sdv2_linear takes them
 _FOLDS_NORM: dict = {}
 
 
@@ -1194,7 +1195,7 @@ def _linear_layout(x: torch.Tensor, weight: torch.Tensor, row_squares: bool):
         return None
     m = x.numel() // k
     rows = _norm_rows(x)
-    if rows is None or not _capi.lib().sdv2_linear_one_round(m, n, k, row_squares):
+    if rows is None or rows[1] > _MAX_LINEAR_STRIDE or not _capi.lib().sdv2_linear_one_round(m, n, k, row_squares):
         return None
     lead = tuple(x.shape[:-1])
     return bytes(_capi.LinearParams(None, None, None, None, rows[1], k, n, m, n, k, _capi.DTYPE_BF16)), (*lead, n), (*lead, n // 32)

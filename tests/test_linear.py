@@ -180,6 +180,16 @@ def test_infinities_and_nans_stay_in_their_row(gpu_device):
     _check(got[ok], x[ok], w, None)
 
 
+def test_layouts_that_stay_with_the_caller():
+    """Rows further apart than the kernel's offsets reach (sdv2_linear refuses them), and what is no product."""
+    w = torch.empty(64, 64, dtype=torch.bfloat16)
+    flat = torch.empty((1 << 22) + 72, dtype=torch.bfloat16)
+    for step, want in ((1 << 22, True), ((1 << 22) + 8, False), (68, False), (0, False)):
+        assert (ops._linear_layout(flat.as_strided((2, 64), (step, 1)), w, False) is not None) == want, step
+    assert ops._linear_layout(flat[:64], w, False) is None and ops._linear_layout(flat[:32].view(1, 32), w, False) is None
+    assert ops._linear_layout(flat[:0].view(0, 64), w, False) is None
+
+
 def test_results_are_contiguous_whatever_the_strides_of_ones():
     t = torch.empty(4096).as_strided((1, 4, 2, 128), (3, 256, 128, 1))
     assert t.is_contiguous() and ops._empty_as(t).stride() == (1024, 256, 128, 1)
