@@ -809,7 +809,8 @@ __device__ __forceinline__ void stream_range(late_args<AttnKernelArgs>& a, lds_c
             end_tile(T);
           }
         } else {
-          // 16 keys of two tiles make one product; a last tile without a second one meets its values again, with weights of zero
+          // 16 keys of two tiles make one product; a last tile without a second one has zeros there, weights and values (its own
+          // values again could hold an infinity, and that times zero is no number)
           for (int T = 0; T < n; T += 2) {
             const uint32_t off = offset(T);
             uint32_t off2 = off;
@@ -826,6 +827,8 @@ __device__ __forceinline__ void stream_range(late_args<AttnKernelArgs>& a, lds_c
             } else {
               b.p[0][2] = b.p[0][3] = b.p[1][2] = b.p[1][3] = 0u;
               b.fetch_v(off, off2, vf);
+#pragma unroll
+              for (int db = 0; db < 8; ++db) vf[db] = __builtin_shufflevector(vf[db], bf16x8{}, 0, 1, 2, 3, 8, 9, 10, 11);
             }
             b.values(vf);
             end_tile(T + 1 < n ? T + 1 : T);

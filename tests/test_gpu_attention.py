@@ -641,3 +641,20 @@ def test_query_tiles_whose_last_blocks_are_shared(gpu_device, rows, S, H, L, seq
 def test_attention_of_small_calls_with_a_workgroup_a_block(gpu_device, rows, S, H, L, seq, block):
     """(up to 128 query blocks, as most of the above are, have two workgroups each)"""
     test_attention_of_small_calls(gpu_device, rows, S, H, L, seq, block, True)
+
+
+@pytest.mark.parametrize("S,L", [(3120, 530), (3041, 640), (3777, 530)])
+def test_an_infinite_value_stays_one_where_blocks_are_shared(gpu_device, S, L):
+    """A value of infinity in the last tile, which has no second one where their number is odd: its column of every query is
+    infinite, and nothing else is touched."""
+    from streamdiffusionv2_amd import ops
+
+    print(f"an infinite value: {S} x 12 against {L}", flush=True)
+    torch.manual_seed(24)
+    q, k, v = (torch.randn(1, n, 12, 128, device=gpu_device).bfloat16() for n in (S, L, L))
+    clean = ops.swa_attention(q, k, v, num_splits=1)
+    v[0, (L - 1) // 64 * 64 + 8, :, 77] = float("inf")
+    got = ops.swa_attention(q, k, v, num_splits=1)
+    assert (got[..., 77] == float("inf")).all()
+    others = [d for d in range(128) if d != 77]
+    assert torch.equal(got[..., others], clean[..., others])
