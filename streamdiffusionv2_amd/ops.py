@@ -1045,8 +1045,8 @@ def _relayout_params(dst, src, dst_indices, src_indices, global_end_shift):
         for idx in (*dst_indices, *src_indices):
             if idx.dtype != torch.int64 or idx.numel() < rows or not idx.is_contiguous():
                 raise RuntimeError("end-index tensors must be contiguous int64 with one entry per row")
-        p.dst_global_end_index, p.dst_local_end_index = dst_indices[0].data_ptr(), dst_indices[1].data_ptr()
-        p.src_global_end_index, p.src_local_end_index = src_indices[0].data_ptr(), src_indices[1].data_ptr()
+        p.dst_global_end_index, p.dst_local_end_index = (t.data_ptr() for t in dst_indices)
+        p.src_global_end_index, p.src_local_end_index = (t.data_ptr() for t in src_indices)
         p.global_end_shift = int(global_end_shift)
     p.stream = _stream_ptr(dev)
     return p, dev

@@ -240,6 +240,8 @@ def test_relayout_indices_and_errors(gpu_device):
         ops.cache_relayout(dst.float(), src)
     with pytest.raises(RuntimeError):            # one index pair only
         ops.cache_relayout(dst, src, (dg, dl), None)
+    with pytest.raises(ValueError):              # more than a pair
+        ops.cache_relayout(dst, src, (dg, dl, dl), (sg, sl, sl))
     with pytest.raises(RuntimeError):            # destination rows alias each other
         ops.cache_relayout(dst[:1].expand(2, -1, -1, -1), src)
     with pytest.raises(RuntimeError):            # no CPU path
