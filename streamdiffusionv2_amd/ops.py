@@ -1227,7 +1227,8 @@ def linear_or_none(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.T
         return None
     p = _capi.LinearParams.from_buffer_copy(template)
     if bias is not None:
-        if not (type(bias) in _PLAIN_TENSORS and bias.dtype == bf16 and bias.device == dev and bias.dim() == 1 and bias.is_contiguous()):
+        if not (type(bias) in _PLAIN_TENSORS and bias.dtype == bf16 and bias.device == dev and bias.shape == weight.shape[:1]
+                and bias.is_contiguous()):
             return None
         p.bias = bias_ptr = bias.data_ptr()
         if bias_ptr % 8:

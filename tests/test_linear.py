@@ -197,6 +197,15 @@ def test_results_are_contiguous_whatever_the_strides_of_ones():
 
 
 @pytest.mark.gpu
+def test_a_bias_of_another_length_stays_with_the_caller(gpu_device):
+    x, w = torch.randn(32, 64, device=gpu_device).bfloat16(), torch.randn(128, 64, device=gpu_device).bfloat16()
+    bias = torch.randn(128, device=gpu_device).bfloat16()
+    with torch.no_grad():
+        _check(ops.linear_or_none(x, w, bias), x, w, bias)
+        assert ops.linear_or_none(x, w, bias[:1]) is None and ops.linear_or_none(x, w, bias[:64]) is None
+
+
+@pytest.mark.gpu
 def test_the_modules_take_it(gpu_device):
     """A chunk's q, k, v and o, of a strided input too; one product for q, k and v gives the bits of three (every element
     is the same sum in the same order, whatever the tile)."""
