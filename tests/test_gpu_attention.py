@@ -658,3 +658,27 @@ def test_an_infinite_value_stays_one_where_blocks_are_shared(gpu_device, S, L):
     assert (got[..., 77] == float("inf")).all()
     others = [d for d in range(128) if d != 77]
     assert torch.equal(got[..., others], clean[..., others])
+
+
+@pytest.mark.parametrize("S,H,blocks", [(1026, 40, 8), (1560, 12, 7)])
+@pytest.mark.parametrize("normed", [False, True])
+def test_a_row_without_keys_in_tiles_of_seven_and_eight_blocks(gpu_device, S, H, blocks, normed):
+    """Seven and eight blocks of 32 queries: the part of LDS that one wave turns its result in is where other waves' queries
+    lay, and without keys there is no streaming between the two.  The other rows are what they are by themselves."""
+    from streamdiffusionv2_amd import ops
+
+    lens, L = [122, 0, 5], 122
+    tiles = -(-S // (32 * blocks))
+    assert (3 * H * tiles <= 256 < 3 * H * -(-S // (32 * (blocks - 1)))) if blocks < 8 else 3 * H * -(-S // 224) > 256
+    print(f"a row without keys: 3 x {S} x {H} against {lens}, norm {normed}", flush=True)
+    torch.manual_seed(25)
+    q, k, v = (torch.randn(3, n, H, 128, device=gpu_device).bfloat16() for n in (S, L, L))
+    kw = {}
+    if normed:
+        weight = torch.rand(H * 128, device=gpu_device).add(0.5).bfloat16()
+        kw["q_row_squares"] = (weight, q.float().pow(2).view(3, S, 4 * H, 32).sum(-1), 1e-6)
+    sl = torch.tensor(lens, dtype=torch.int32, device=gpu_device)
+    got = [ops.swa_attention(q, k, v, sl, num_splits=1, **kw) for _ in range(3)]
+    assert all((g[1] == 0).all() for g in got) and torch.equal(got[0], got[1]) and torch.equal(got[0], got[2])
+    full = ops.swa_attention(q, k, v, torch.tensor([122, 122, 5], dtype=torch.int32, device=gpu_device), num_splits=1, **kw)
+    assert torch.equal(got[0][0], full[0]) and torch.equal(got[0][2], full[2])
