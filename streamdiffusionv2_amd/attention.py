@@ -471,8 +471,7 @@ class CausalWanSelfAttention(nn.Module, RingKVPath):
         """(weight [3 * dim, dim], bias [3 * dim] or None) of the q, k and v
         Linears laid end to end, rebuilt when any of the six tensors has been
         replaced (another tensor, dtype or device) or written in place."""
-        modules = self._modules
-        layers = (modules.get("q"), modules.get("k"), modules.get("v"))
+        layers = (self.q, self.k, self.v)          # (by name, not from _modules: an attribute may hide the registered layer)
         key = []
         for layer in layers:
             # only plain Linears that nobody watches: a wrapped or replaced layer (an adapter, a quantised

@@ -67,6 +67,32 @@ def test_a_layer_that_is_no_registered_module_is_called():
         assert torch.equal(mod.project_qkv(x)[0], want)
 
 
+@pytest.mark.parametrize("name", ["q", "k", "v"])
+def test_what_hides_a_registered_layer_is_called(name):
+    """An instance attribute over the registered Linear, and a property of a subclass: the mode without gradients calls what
+    the one with gradients does."""
+    torch.manual_seed(4)
+    x = torch.randn(1, 5, 256)
+    at = "qkv".index(name)
+
+    mod = CausalWanSelfAttention(256, 2)
+    layer = getattr(mod, name)
+    assert mod._packed_qkv() is not None
+    object.__setattr__(mod, name, lambda t: layer(t) * 2)
+    with torch.no_grad():
+        assert torch.equal(mod.project_qkv(x)[at], layer(x) * 2) and mod._packed_qkv() is None
+    assert torch.equal(mod.project_qkv(x)[at], layer(x) * 2)
+
+    class Doubled(CausalWanSelfAttention):
+        pass
+
+    setattr(Doubled, name, property(lambda self: lambda t: self._modules[name](t) * 2))
+    mod = Doubled(256, 2)
+    with torch.no_grad():
+        assert torch.equal(mod.project_qkv(x)[at], mod._modules[name](x) * 2)
+    assert torch.equal(mod.project_qkv(x)[at], mod._modules[name](x) * 2)
+
+
 def test_three_launches_when_asked_or_when_training():
     torch.manual_seed(2)
     mod = CausalWanSelfAttention(256, 2)
