@@ -476,7 +476,7 @@ class CausalWanSelfAttention(nn.Module, RingKVPath):
         for layer in layers:
             # only plain Linears that nobody watches: a wrapped or replaced layer (an adapter, a quantised
             # Linear) computes something else than x W^T + b, and a hook expects its layer to be called
-            if type(layer) is not nn.Linear or layer._forward_hooks or layer._forward_pre_hooks:
+            if type(layer) is not nn.Linear or "forward" in layer.__dict__ or layer._forward_hooks or layer._forward_pre_hooks:
                 return None
             for t in (layer.weight, layer.bias):
                 if t is None:

@@ -93,6 +93,16 @@ def test_what_hides_a_registered_layer_is_called(name):
     assert torch.equal(mod.project_qkv(x)[at], mod._modules[name](x) * 2)
 
 
+def test_a_layer_whose_own_forward_was_replaced_is_called():
+    torch.manual_seed(5)
+    mod = CausalWanSelfAttention(256, 2)
+    x = torch.randn(1, 5, 256)
+    plain = mod.k.forward
+    mod.k.forward = lambda t: plain(t) * 2           # as a wrapper does that keeps the module's type
+    with torch.no_grad():
+        assert torch.equal(mod.project_qkv(x)[1], plain(x) * 2)
+
+
 def test_three_launches_when_asked_or_when_training():
     torch.manual_seed(2)
     mod = CausalWanSelfAttention(256, 2)
