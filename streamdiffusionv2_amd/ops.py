@@ -49,7 +49,7 @@ def _stream_ptr(dev: torch.device) -> int:
 
 def _empty_as(t: torch.Tensor) -> torch.Tensor:
     """A contiguous plain tensor of t's shape, dtype and device."""
-    if type(t) is torch.Tensor and t.is_contiguous():
+    if type(t) is torch.Tensor and t.is_contiguous() and not t.has_names():
         # (a third of the time it takes to spell them out; by itself it would take over odd strides of dimensions of one)
         return torch.empty_like(t, memory_format=torch.contiguous_format)
     return torch.empty(t.shape, dtype=t.dtype, device=t.device)

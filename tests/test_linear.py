@@ -196,6 +196,11 @@ def test_results_are_contiguous_whatever_the_strides_of_ones():
     assert ops._empty_as(t.transpose(1, 2)).stride() == (1024, 512, 128, 1)
 
 
+@pytest.mark.filterwarnings("ignore:Named tensors")
+def test_results_have_no_names():
+    assert ops._empty_as(torch.zeros(2, 3, names=("a", "b"))).names == (None, None)
+
+
 @pytest.mark.gpu
 def test_a_bias_of_another_length_stays_with_the_caller(gpu_device):
     x, w = torch.randn(32, 64, device=gpu_device).bfloat16(), torch.randn(128, 64, device=gpu_device).bfloat16()
