@@ -1210,7 +1210,7 @@ def linear_or_none(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.T
     of its rows, float32 [..., n / 32]."""
     bf16 = torch.bfloat16
     if not (x.is_cuda and x.dtype == bf16 and weight.dtype == bf16 and type(x) in _PLAIN_TENSORS
-            and type(weight) in _PLAIN_TENSORS and _plain_call()):
+            and type(weight) in _PLAIN_TENSORS and x.layout is weight.layout is torch.strided and _plain_call()):
         return None
     key = (x.shape, x.stride(), weight.shape, row_squares)
     layout = _LINEAR_LAYOUTS.get(key, _LINEAR_LAYOUTS)

@@ -202,6 +202,17 @@ def test_results_have_no_names():
 
 
 @pytest.mark.gpu
+@pytest.mark.filterwarnings("ignore:Sparse CSR")
+def test_sparse_operands_stay_with_the_caller(gpu_device):
+    """(they have no strides to look at)"""
+    x, w = torch.randn(256, 128, device=gpu_device).bfloat16(), torch.eye(128, device=gpu_device).bfloat16()
+    with torch.no_grad():
+        assert ops.linear_or_none(x, w, None) is not None
+        for sparse in (w.to_sparse_csr(), w.to_sparse()):
+            assert ops.linear_or_none(x, sparse, None) is None and ops.linear_or_none(sparse, w, None) is None
+
+
+@pytest.mark.gpu
 def test_a_bias_of_another_length_stays_with_the_caller(gpu_device):
     x, w = torch.randn(32, 64, device=gpu_device).bfloat16(), torch.randn(128, 64, device=gpu_device).bfloat16()
     bias = torch.randn(128, device=gpu_device).bfloat16()
