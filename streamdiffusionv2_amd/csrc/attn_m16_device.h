@@ -414,6 +414,16 @@ struct SharedBlock {
       vf[db] = __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3));
     }
   }
+  // Behind the next barrier transfers fill the buffers that this tile's K and V were read from.  The compiler knows nothing of
+  // that, and what takes the fragments up touches no memory: it could wait for them, and use them, behind the barrier.
+  // So what K was read for is in registers ahead of it, and so are V's fragments.  (Text for the check of the assembly.)
+  __device__ __forceinline__ void k_has_been_read() const {
+    asm volatile("; shared block: K has been read" ::"v"(p[0]), "v"(p[1]));
+  }
+  __device__ __forceinline__ void v_has_been_read(const bf16x8 (&vf)[8]) const {
+    asm volatile("; shared block: V has been read" ::"v"(vf[0]), "v"(vf[1]), "v"(vf[2]), "v"(vf[3]), "v"(vf[4]), "v"(vf[5]), "v"(vf[6]),
+                 "v"(vf[7]));
+  }
   __device__ __forceinline__ void values(const bf16x8 (&vf)[8]) {
     const bf16x8 pf[2] = {__builtin_bit_cast(bf16x8, p[0]), __builtin_bit_cast(bf16x8, p[1])};
 #pragma unroll
@@ -806,6 +816,8 @@ __device__ __forceinline__ void stream_range(late_args<AttnKernelArgs>& a, lds_c
             b.template weights<0>(s[0], first_key(T), seq);
             b.template weights<1>(s[1], first_key(T) + 16, seq);
             b.values(vf);
+            b.k_has_been_read();
+            b.v_has_been_read(vf);
             end_tile(T);
           }
         } else {
@@ -817,6 +829,7 @@ __device__ __forceinline__ void stream_range(late_args<AttnKernelArgs>& a, lds_c
             b.template scores<kSubs>(kf, s);
             b.template fetch_k<kSubs>(offset(T + 1), kf);
             b.template weights<0>(s[0], first_key(T), seq);
+            b.k_has_been_read();
             if (T + 1 < n) {
               end_tile(T);
               off2 = offset(T + 1);
@@ -831,6 +844,8 @@ __device__ __forceinline__ void stream_range(late_args<AttnKernelArgs>& a, lds_c
               for (int db = 0; db < 8; ++db) vf[db] = __builtin_shufflevector(vf[db], bf16x8{}, 0, 1, 2, 3, 8, 9, 10, 11);
             }
             b.values(vf);
+            b.k_has_been_read();
+            b.v_has_been_read(vf);
             end_tile(T + 1 < n ? T + 1 : T);
           }
         }

@@ -198,6 +198,85 @@ def test_the_same_promises_in_query_tiles_of_few_rows(name):
     test_the_same_promises_for_the_16x16_kernel(open(path).read().split("\n"))
 
 
+def reads_at_barriers(body):
+    """Every way through a kernel: what a wave has asked LDS for ("k" rows, "v" transposed) and not waited for at each barrier
+    that a text "shared block: ..." stands ahead of, as (texts since the barrier before, reads)."""
+    blocks, names = [], {}
+    for line in body:
+        label = re.match(r"^(\.LBB\w+):", line)
+        if label or not blocks:
+            blocks.append([])
+            if label:
+                names[label.group(1)] = len(blocks) - 1
+        blocks[-1].append(line)
+    found, seen, todo = set(), set(), [(0, (), frozenset())]
+    while todo:
+        at, flying, texts = todo.pop()
+        if at >= len(blocks) or (at, flying, texts) in seen:
+            continue
+        seen.add((at, flying, texts))
+        ended = False
+        for line in blocks[at]:
+            text = re.search(r"shared block: (\w)", line)
+            if text:
+                texts |= {text.group(1)}
+                continue
+            ins = list(instructions([line]))
+            if not ins:
+                continue
+            mn, ops = ins[0]
+            if mn.startswith("ds_read_b128"):
+                flying += ("k",)
+            elif mn.startswith("ds_read_b64_tr"):
+                flying += ("v",)
+            elif mn.startswith("ds_"):
+                flying += ("other",)
+            elif mn == "s_waitcnt" and "lgkmcnt" in line:
+                left = int(re.search(r"lgkmcnt\((\d+)\)", line).group(1))
+                flying = flying[len(flying) - left:] if left else ()          # (in order; what else counts can only make it fewer)
+            elif mn == "s_barrier":
+                if texts:
+                    found.add((texts, flying))
+                texts = frozenset()
+            elif mn in ("s_branch", "s_endpgm") or mn.startswith("s_cbranch"):
+                if mn != "s_endpgm":
+                    todo.append((names[ops[0]], flying, texts))
+                if not mn.startswith("s_cbranch"):
+                    ended = True
+                    break
+        if not ended:
+            todo.append((at + 1, flying, texts))
+    return found
+
+
+def test_shared_blocks_have_read_a_tile_before_its_buffers_are_filled_again():
+    """Of waves that share a query block, at the barrier that ends a tile: V's fragments have all arrived, and no more of K is
+    on its way than was asked for last, the next tile's."""
+    toy = ["\tds_read_b64_tr_b16 v[2:3], v1", "\tds_read_b128 v[4:7], v1", "\ts_waitcnt lgkmcnt(1)", "\t; shared block: V has been read",
+           "\ts_cbranch_scc0 .LBB0_1", "\tds_read_b64_tr_b16 v[2:3], v1", ".LBB0_1:", "\ts_barrier", "\ts_endpgm"]
+    assert reads_at_barriers(toy) == {(frozenset("V"), ("k",)), (frozenset("V"), ("k", "v"))}
+    out = os.path.join(ROOT, "build", "isa_check")
+    os.makedirs(out, exist_ok=True)
+    path = os.path.join(out, "swa_attn_fwd_m16_shared.s")
+    cmd = [build_ext.hipcc_path(), *build_ext.HIPCC_FLAGS, f"-I{os.path.join(ROOT, 'include')}", f"-I{build_ext.CSRC}",
+           "-S", "--cuda-device-only", str(build_ext.CSRC / "swa_attn_fwd_m16_shared.hip"), "-o", path]
+    res = subprocess.run(cmd, capture_output=True, text=True)
+    assert res.returncode == 0, res.stderr[-2000:]
+    lines = open(path).read().split("\n")
+    shares = []
+    for start in (i for i, l in enumerate(lines) if re.match(r"^_Z\S*swa_attn_fwd_m16_kernel\S*:", l)):
+        body = lines[start:next(i for i in range(start, len(lines)) if lines[i].strip().startswith(".Lfunc_end"))]
+        share = int(re.search(r"Li(\d)EEEv", body[0]).group(1))
+        shares.append(share)
+        found = reads_at_barriers(body)
+        # two blocks of sixteen keys: a tile at a time; four: two, and V with the second
+        assert {t for t, _ in found} == ({frozenset("KV")} if share == 2 else {frozenset("K"), frozenset("KV")}), found
+        for texts, reads in found:
+            # (behind the first barrier of two tiles only K's buffer is filled)
+            assert ("V" not in texts or "v" not in reads) and "other" not in reads and reads.count("k") <= 16 // share, (share, texts, reads)
+    assert sorted(shares) == [2, 4]
+
+
 @pytest.fixture(scope="module")
 def assembly_wave():
     out = os.path.join(ROOT, "build", "isa_check")
