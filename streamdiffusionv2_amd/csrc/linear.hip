@@ -19,9 +19,10 @@
 // 13.1 us).  Bringing lines to L2 ahead of that, by the waves that multiply, costs
 // more than it gives: 64 rows are 64 lines to ask for (736 x 5120 x 5120 51 -> 65 us).
 //
-// A workgroup alone runs its matrix pipe 76 to 87 % full (a stage of 128 x 128 0.28 us, of
-// 224 x 128 0.43); on all CUs the same stages take 0.4 and 0.65, 1.2 and 1.4 PFLOP/s, what a
-// large product reaches on the board's power.  So what counts is one round of workgroups,
+// With x and the weights in L2 a workgroup alone runs its matrix pipe 76 to 87 % full (a stage of 128 x 128
+// 0.28 us, of 224 x 128 0.43); on all CUs the same stages take 0.4 and 0.65, 1.2 and 1.4 PFLOP/s, what a
+// large product reaches on the board's power.  (What a stage takes with weights that come from memory:
+// linear_tiles.h.)  So what counts is one round of workgroups,
 // whatever the tile that takes, and the larger the tile the less energy: 224 x 128 and
 // 224 x 160 where 160 x 128 would be two rounds (linear_wide.hip), 1560 x 4608 x 1536 31.6
 // -> 24.3 us, 3648 x 1536 x 1536 25.6 -> 20.8, 1560 x 5120 x 5120 117 -> 73.
@@ -36,56 +37,21 @@
 // lane ends up with four neighbouring columns of a row; each wave turns its part
 // through LDS and writes whole lines.
 #include "linear_kernel.h"
-
-namespace {
-
-// The tiles there are.  us: what a stage of 64 takes a workgroup that has the chip to itself.
-struct Tile {
-  int m, n;
-  float us;
-};
-constexpr Tile kTiles[] = {{64, 64, 0.115f},  {96, 64, 0.148f},  {160, 64, 0.229f},  {96, 128, 0.262f},  {128, 128, 0.322f},
-                           {160, 128, 0.377f}, {192, 128, 0.435f}, {224, 128, 0.501f}, {256, 128, 0.554f}, {224, 160, 0.591f}};
-constexpr int kTileCount = sizeof(kTiles) / sizeof(kTiles[0]);
-constexpr int kCus = 256;
-
-int64_t tiles_of(const Tile& t, int64_t m, int64_t n) { return (m + t.m - 1) / t.m * (n / t.n); }
-
-// A stage takes 1.5 times as long where every CU has a tile (the board's power, and what L2 brings), and up to 0.1 us more
-// where a long contraction's weights come from memory.  159 products that fit one round, 144 to 7020 rows of 4 to 40
-// heads, weights cold: the tile this picks takes 1.01 of the best one's time (1.35 at worst, 352 x 5120 x 5120).
-double tile_us(const Tile& t, int64_t m, int64_t n, int64_t k) {
-  const int64_t tiles = tiles_of(t, m, n), rounds = (tiles + kCus - 1) / kCus;
-  const double load = tiles < kCus ? (double)tiles / kCus : 1.0, stages = (double)k / kDepth;
-  const double longer = stages < 24 ? 0 : stages < 80 ? stages - 24 : 56;
-  return (double)rounds * (3.4 + stages * (t.us * (1 + 0.53 * load) + longer / 56 * 0.097 * load));
-}
-
-// The tile that takes least, or -1 where none divides n.
-int best_tile(int64_t m, int64_t n, int64_t k, bool squares) {
-  int best = -1;
-  double best_us = 0;
-  for (int i = 0; i < kTileCount; ++i) {
-    if (n % kTiles[i].n != 0 || (squares && kTiles[i].n == 160)) continue;        // (80 columns of a wave are no groups of 32)
-    const double us = tile_us(kTiles[i], m, n, k);
-    if (best < 0 || us < best_us) {
-      best = i;
-      best_us = us;
-    }
-  }
-  return best;
-}
-
-}  // namespace
+#include "linear_tiles.h"
 
 extern "C" int sdv2_linear_one_round(int64_t m, int32_t n, int32_t k, int32_t row_squares) {
   if (m <= 0 || n <= 0 || k <= 0 || n % 64 != 0 || k % kDepth != 0) return 0;
-  // One round of tiles, of which each CU has one.  Of the 159 products above 155 are faster than the vendor's, 0.79 of its
-  // time on the geometric mean (1560 x 4608 x 1536 24.3 against 28.3 us, 528 x 3712 x 3712 23.6 and 32.6, 1560 x 5120 x
-  // 5120 73.4 and 88); 528 to 640 rows of 5120 x 5120 lose up to 7 %, 352 rows 17.  A second round costs a launch's
+  // One round of tiles, of which each CU has one.  1441 such products of 97 to 7020 rows, 4 to 64 heads (q, k and v in one among
+  // them), weights cold, in graphs: contractions of up to 2048 take 0.77 of the vendor's time on the geometric mean, 2 of 549
+  // are slower by more than 2 %; longer ones 0.88 (1560 x 5120 x 5120 72.8 and 88.7 us, 352 x 4352 x 4352 27.3 and 34.1), 58 of
+  // 892 are slower by more than 2 %, 6 of those by more than 10.  These lie at 97 to 960 rows in 64-column or 96-row tiles whose
+  // row tiles are full, so that none goes ahead (464 x 3840 x 3840 34.6 and 29.2 us, 496 rows 26.1 and 30.9): with whatever
+  // tile is best 37 would stay, and a line that leaves them out loses as much on their neighbours (of contractions past 3000 in
+  // tiles of 160 x 64 and 96 x 128, 96 % full, 14 of 28 are the slower ones, 1.016 together).  A second round costs a launch's
   // start and end again and leaves CUs idle: 480 tiles 1.1 to 1.23 of the vendor's time.
   // Of few rows and a long contraction the vendor's cuts the contraction (16 x 5120 x 5120 14.9 against 22.1 us, 64 x 5120 x
-  // 5120 21.3 and 29.6, 64 x 7680 x 2560 15.6 and 17.6; 100 x 5120 x 5120 27.5 and 25.7, 100 x 3712 x 3712 18.8 and 17.4).
+  // 5120 21.3 and 29.6, 64 x 7680 x 2560 15.6 and 17.6; the other way round 100 x 5120 x 5120, 27.5 and 25.7, and 100 x 3712 x
+  // 3712, 18.8 and 17.4).
   if (m <= 96 && k > 2048) return 0;
   const int i = best_tile(m, n, k, row_squares != 0);
   return i >= 0 && tiles_of(kTiles[i], m, n) <= kCus;

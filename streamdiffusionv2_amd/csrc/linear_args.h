@@ -5,10 +5,10 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "linear_tiles.h"
+
 namespace sdv2 {
 namespace linear {
-
-constexpr int kDepth = 64;                   // of a stage, along the contraction
 
 struct LinearArgs {
   const uint16_t* x;

@@ -3,6 +3,7 @@ and their results at the edges of the tiles."""
 import ctypes as C
 import os
 import re
+import shutil
 import subprocess
 
 import pytest
@@ -19,6 +20,30 @@ def test_which_products_are_one_round():
                                    (1560, 5120, 5120, 1, 0), (1536, 5120, 64, 1, 1), (1280, 5120, 5120, 1, 1),
                                    (96, 5120, 5120, 0, 0), (97, 5120, 5120, 0, 1), (1, 5120, 2048, 0, 1), (9360, 1536, 1536, 0, 0), (1560, 15360, 5120, 0, 0), (0, 64, 64, 0, 0), (16, 96, 64, 0, 0), (16, 64, 96, 0, 0)):
         assert lib.sdv2_linear_one_round(m, n, k, squares) == want, (m, n, k, squares)
+
+
+@pytest.mark.skipif(shutil.which("g++") is None, reason="no g++")
+def test_the_tile_a_product_takes(tmp_path):
+    """Measured (us, weights cold): within 5 % of the fastest tile, among them products whose row tiles differ in how full they
+    are.  With sums of squares never the tile of 160 columns."""
+    measured = [
+        ((352, 4352, 4352), {(160, 64): 27.28, (96, 128): 37.27, (160, 128): 37.42}),
+        ((359, 5120, 5120), {(160, 64): 32.98, (96, 128): 46.67, (160, 128): 45.28}),
+        ((320, 6144, 6144), {(160, 64): 49.95, (96, 128): 43.41}),
+        ((508, 6144, 6144), {(128, 128): 62.45, (160, 128): 53.06}),
+        ((1561, 3712, 3712), {(224, 128): 48.21, (256, 128): 43.44}),
+        ((1567, 5120, 5120), {(224, 160): 72.81}),
+        ((256, 1536, 1536), {(64, 64): 7.76}),
+    ]
+    exe = str(tmp_path / "linear_tile_check")
+    subprocess.run(["g++", "-std=c++17", "-O2", "-Wall", "-Werror", f"-I{build_ext.CSRC}",
+                    os.path.join(ROOT, "tests", "c_abi", "linear_tile_check.cpp"), "-o", exe], check=True)
+    asked = [*(size + (0,) for size, _ in measured), (1567, 5120, 5120, 1), (64, 96, 64, 0)]
+    run = subprocess.run([exe, *(str(x) for a in asked for x in a)], capture_output=True, text=True, timeout=60)
+    got = [tuple(int(x) for x in line.split()) for line in run.stdout.splitlines()]
+    for (size, times), tile in zip(measured, got):
+        assert times[tile] <= 1.05 * min(times.values()), (size, tile)
+    assert got[-2][1] != 160 and got[-1] == (0, 0)
 
 
 def test_nothing_touches_a_fragment_on_its_way():
