@@ -682,3 +682,44 @@ def test_a_row_without_keys_in_tiles_of_seven_and_eight_blocks(gpu_device, S, H,
     assert all((g[1] == 0).all() for g in got) and torch.equal(got[0], got[1]) and torch.equal(got[0], got[2])
     full = ops.swa_attention(q, k, v, torch.tensor([122, 122, 5], dtype=torch.int32, device=gpu_device), num_splits=1, **kw)
     assert torch.equal(got[0][0], full[0]) and torch.equal(got[0][2], full[2])
+
+
+@pytest.mark.parametrize("grid,blocks", [((2, 30, 52), 5), ((3, 27, 47), 6)])
+@pytest.mark.parametrize("normed", [False, True])
+def test_shared_blocks_rotate_their_query(gpu_device, grid, blocks, normed):
+    """The query as it was before its rotation (or norm and rotation): every wave that shares a block loads that block's rows,
+    and the bits are those of the query that the append wrote."""
+    from streamdiffusionv2_amd import ops, rope
+
+    H, S, L = 12, grid[0] * grid[1] * grid[2], 4100
+    assert H * -(-S // (32 * blocks)) <= 256 < H * -(-S // (32 * (blocks - 1)))
+    print(f"shared blocks, rotating: {S} x {H} against {L}, norm {normed}", flush=True)
+    torch.manual_seed(26)
+    q, k, v = (torch.randn(1, S, H, 128, device=gpu_device).bfloat16() for _ in range(3))
+    caches = [torch.randn(1, L, H, 128, device=gpu_device).bfloat16() for _ in range(2)]
+    table = ops.device_freqs(rope.build_freqs(), gpu_device)
+    weights = [torch.rand(H * 128, device=gpu_device).add(0.5).bfloat16() for _ in range(2)]
+    norm = dict(qk_norm=(*weights, 1e-6)) if normed else {}
+    inv = torch.empty(1, S, device=gpu_device)
+    rotated = ops.kv_append_rope(q, k, v, *caches, table, grid, [4], [100], **norm)
+    want = ops.swa_attention(rotated, *caches, None, num_splits=1)
+    if normed:
+        assert ops.kv_append_rope(q, k, v, *caches, table, grid, [4], [100], q_inv_rms=inv, **norm) is None
+    got = ops.swa_attention(q, *caches, None, num_splits=1, rope=(table, grid[1:], [4]), **(dict(q_norm=(weights[0], inv)) if normed else {}))
+    assert torch.equal(got.view(torch.int16), want.view(torch.int16))
+    _check(got.cpu(), oracle.attention_fp32_reference(rotated.cpu(), *(c.cpu() for c in caches), [L]))
+
+
+@pytest.mark.parametrize("S,L,lens,blocks", [(1000, 900, [900, 0, 65], 5), (1269, 700, [0, 700, 1], 6)])
+def test_a_row_without_keys_where_blocks_are_shared(gpu_device, S, L, lens, blocks):
+    from streamdiffusionv2_amd import ops
+
+    H, rows = 12, 3
+    assert rows * H * -(-S // (32 * blocks)) <= 256 < rows * H * -(-S // (32 * (blocks - 1)))
+    print(f"a row without keys, shared blocks: {rows} x {S} x {H} against {lens}", flush=True)
+    torch.manual_seed(27)
+    q, k, v = (torch.randn(rows, n, H, 128).bfloat16() for n in (S, L, L))
+    got = ops.swa_attention(*(t.to(gpu_device) for t in (q, k, v)), torch.tensor(lens, dtype=torch.int32, device=gpu_device), num_splits=1).cpu()
+    live = [r for r in range(rows) if lens[r]]
+    assert not got[lens.index(0)].any()
+    _check(got[live], oracle.attention_fp32_reference(q[live], k[live], v[live], [lens[r] for r in live]))

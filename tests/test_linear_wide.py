@@ -9,7 +9,7 @@ import subprocess
 import pytest
 import torch
 
-from streamdiffusionv2_amd import _capi, build_ext
+from streamdiffusionv2_amd import _capi, build_ext, ops
 from test_attention_isa import instructions, registers
 from test_linear import ROOT, _check
 
@@ -111,3 +111,25 @@ def test_wide_products(gpu_device, m, n, k, tile):
         if squared:                                        # 32 terms in fp32, 2^-24 each
             want = out[:m, :n].double().pow(2).view(m, n // 32, 32).sum(-1)
             assert ((squares[:m].double() - want).abs() <= 32 * 2.0 ** -24 * want).all() and (squares[m:] == -1).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("m,n,k,squared", [
+    (97, 2176, 2176, True), (300, 2176, 2176, False), (352, 3712, 3712, True), (464, 3712, 3712, True), (820, 3712, 3712, False),
+    (352, 5120, 5120, True), (640, 5120, 5120, True), (1080, 5120, 5120, True), (1560, 5120, 5120, False), (130, 15360, 5120, False),
+])
+def test_long_contractions(gpu_device, m, n, k, squared):
+    """Past 2048: all of the width of a model of 17, 29 and 40 heads, against 64 bits, with sums of squares or without."""
+    print(f"linear {m} x {n} x {k}", flush=True)
+    assert _capi.lib().sdv2_linear_one_round(m, n, k, squared)
+    gen = torch.Generator(device=gpu_device).manual_seed(m + n + k)
+    x, w, b = (torch.randn(*s, generator=gen, device=gpu_device).bfloat16() for s in ((m, k), (n, k), (n,)))
+    with torch.no_grad():
+        out = ops.linear_or_none(x, w, b, row_squares=squared)
+        again = ops.linear_or_none(x, w, b)
+    if squared:                                            # 32 terms in fp32, 2^-24 each
+        out, squares = out
+        want = out.double().pow(2).view(m, n // 32, 32).sum(-1)
+        assert ((squares.double() - want).abs() <= 32 * 2.0 ** -24 * want).all()
+    assert torch.equal(out, again)
+    _check(out, x, w, b)
