@@ -443,7 +443,7 @@ class CausalWanSelfAttention(nn.Module, RingKVPath):
         # The q, k and v projections (causal_model.py:212-218 calls the three
         # Linears one after the other) run as ONE product on the three
         # weights laid end to end: at 1560 tokens x 1536 three launches of the vendor's take
-        # 60 us and one 26 us (the library's own loses to it where the weights come from memory),
+        # 60 us, one 30 us and the library's own 26 us (weights from memory),
         # with the same bits out (every output element is the same dot product over `dim`).  q, k and v are then strided views
         # of one [B, S, 3 * dim] tensor, which the kernels of the path read as
         # they are.  The packed copy of the weights (3 * dim * dim elements per
