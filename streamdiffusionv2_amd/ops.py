@@ -913,7 +913,9 @@ class LayerLauncher:
             ap.q_in = ap.q_out = ap.q_norm_weight = None
             ap.k_inv_rms = inv_rms.data_ptr() if inv_rms is not None else None
         else:
-            self.roped_q = _empty_as(q) if q.device == self.dev else torch.empty(self.in_shape, dtype=torch.bfloat16, device=self.dev)
+            # (a caller that fills in its own calls may bring the same memory in another form)
+            alike = q.shape == self.in_shape and q.dtype == torch.bfloat16 and q.device == self.dev
+            self.roped_q = _empty_as(q) if alike else torch.empty(self.in_shape, dtype=torch.bfloat16, device=self.dev)
             ap.q_in = q.data_ptr()
             ap.q_out = at.q = self.roped_q.data_ptr()
             if self.norm_args is not None:

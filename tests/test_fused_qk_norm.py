@@ -308,6 +308,26 @@ def test_a_patched_call_keeps_its_workspace_until_it_is_launched(monkeypatch):
     assert carried() is not None and carried() is not ops._WORKSPACES[(launcher.dev, 0)]
 
 
+def test_a_patched_call_has_the_launchers_shape(monkeypatch):
+    """... whatever form its query's memory comes in."""
+    import types
+
+    from streamdiffusionv2_amd import ops
+
+    monkeypatch.setattr(ops, "_require_gpu", lambda *t: t[0].device)          # (nothing is launched)
+    monkeypatch.setattr(ops, "_stream_ptr", lambda dev: 0)
+    heads, tokens, cap = 2, 6, 12
+    cache = [torch.zeros(1, cap, heads, 128, dtype=torch.bfloat16) for _ in range(2)]
+    index = [torch.zeros(1, dtype=torch.long) for _ in range(2)]
+    q = torch.zeros(1, tokens, heads, 128, dtype=torch.bfloat16)
+    launcher = ops.LayerLauncher(*cache, *index, torch.zeros(16, 64, 2, dtype=torch.float64), (1, 2, 3), q,
+                                 rope_in_attention=False)
+    plan = types.SimpleNamespace(dst_start=[0], new_global_end=[6], new_local_end=[6], max_seq_len=cap)
+    for form in (q, q.flatten(2), q.view(torch.int16)):
+        out = launcher.patch(form, q, q, [0], plan)
+        assert out.shape == launcher.roped_q.shape == q.shape and out.dtype == launcher.roped_q.dtype == torch.bfloat16
+
+
 def test_workspaces_under_capture(monkeypatch):
     """(on the host, nothing is launched) A workspace that a capture has taken outlives the pool's growth; one made inside
     a capture is not handed to later eager calls."""
